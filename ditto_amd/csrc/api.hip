@@ -270,16 +270,25 @@ int plan_bmm(const ditto_bmm_chain_desc* d, BmmPlan* plan, bool need_device) {
         d->f_row_stride > 0x7fffffff)
       return fail(DITTO_EINVAL, "row stride too large");
     plan->family = 1;
+    const bool f64 = in == DITTO_F64;
+    // fp32 workgroups of 16 or of 32 rows: a 32-row one does twice the work in 0.9 of the time two 16-row ones take
+    // (every B and C fragment fetched from L2 feeds two row tiles), and the fewer rounds over the compute units win.
+    // Measured, us per launch, 16 / 32 rows: 12 x 512 x 512 x 64 16.0 / 14.4, 1 x 512 x 512 x 64 8.8 / 13.9,
+    // 16 x 700 x 700 x 64 28.2 / 33.4, 64 x 512 x 512 x 64 51.6 / 52.7 (B [K][L]: 62.6 / 57.1).  Beyond 80 columns two row
+    // tiles do not fit the registers.
+    const int cus = need_device ? device_cus() : 256;
+    auto rounds = [&](int rows) { return (((d->M + rows - 1) / rows) * d->batch + cus - 1) / cus; };
+    plan->qt = !f64 && (d->K > 80 || d->N > 80 || (double)rounds(16) < 1.8 * (double)rounds(32)) ? 1 : 2;
     ditto_tile_param& t = plan->tile;
-    t.block_threads = 256;
-    t.block_m = 32;
+    t.block_threads = f64 ? 256 : 512;
+    t.block_m = 16 * plan->qt;
     t.block_n = (int)d->N;
     t.head_pad = 0;
-    t.block_l = in == DITTO_F64 ? 32 : 64;
-    t.lds_bytes = ditto::f32_chain_lds_bytes_host((int)d->K, (int)d->N, in == DITTO_F64);
-    t.grid_x = (int)(((d->M + 31) / 32) * d->batch);
+    t.block_l = f64 ? 32 : 128;
+    t.lds_bytes = ditto::f32_chain_lds_bytes_host((int)d->K, (int)d->N, f64, plan->qt);
+    t.grid_x = (int)(((d->M + t.block_m - 1) / t.block_m) * d->batch);
     t.grid_y = t.grid_z = 1;
-    t.variant = in == DITTO_F64 ? 1001 : 1000;  // fp32 / fp64 FMA chain
+    t.variant = f64 ? 1001 : 1000;  // fp32 (MFMA) / fp64 (FMA) chain
     return DITTO_OK;
   }
   if (in == DITTO_I8) {
@@ -1076,7 +1085,8 @@ int ditto_bmm_chain_run(const ditto_bmm_chain_desc* d, const void* a, const void
     args.K = (int)d->K;
     args.L = (int)d->L;
     args.batch = (int)d->batch;
-    args.mblocks = (int)((d->M + 31) / 32);
+    args.mblocks = (int)((d->M + plan.tile.block_m - 1) / plan.tile.block_m);
+    args.row_tiles = plan.qt;
     args.b_lk = d->b_layout == DITTO_B_LK;
     args.relu = d->inter_op == DITTO_INTER_RELU;
     args.relu_out = d->relu_out;

@@ -1,4 +1,4 @@
-// Arguments and launcher of the fp32 / fp64 GEMM chain kernel (gemm_chain_f32.hip).
+// Arguments and launcher of the fp32 / fp64 GEMM chain kernels (gemm_chain_f32.hip).
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -12,7 +12,8 @@ struct F32ChainArgs {
   long long a_bs, b_bs, c_bs, f_bs;  // batch strides, elements
   int a_rs, b_rs, c_rs, f_rs;        // row strides, elements
   int M, N, K, L, batch;
-  int mblocks;  // workgroups (32 rows each) per batch entry
+  int mblocks;    // workgroups per batch entry
+  int row_tiles;  // fp32: rows of a workgroup / 16 (1 or 2); fp64: workgroups own 32 rows
   int b_lk;     // B stored [L][K]
   int relu;
   int relu_out;  // ReLU on the output
@@ -21,8 +22,8 @@ struct F32ChainArgs {
   int f64;       // elements are doubles
 };
 
-int f32_chain_lds_bytes_host(int K, int N, int f64);
-int f32_chain_max_dim();  // largest K and N the kernel takes
+int f32_chain_lds_bytes_host(int K, int N, int f64, int row_tiles);
+int f32_chain_max_dim();  // largest K and N the kernels take
 hipError_t launch_gemm_chain_f32(const F32ChainArgs& args, hipStream_t stream);
 
 }  // namespace ditto

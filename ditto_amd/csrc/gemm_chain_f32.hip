@@ -1,111 +1,324 @@
-// fp32 / fp64 GEMM -> cast|relu|softmax -> GEMM chain  F = inter(A.B).C  for the reference's fp32, CPU-sized
-// configurations (python_test/auto_tensorize/test_hyper_fusion.py:16-21: 512x64 . 64x64 . 64x64; the fp32
-// BMM -> softmax -> BMM of benchmark/chimera/cpu/bmm_softmax_bmm.py:64-170).
+// fp32 / fp64 GEMM -> cast|relu|softmax -> GEMM chain  F = inter(A.B).C  for the reference's fp32 configurations
+// (python_test/auto_tensorize/test_hyper_fusion.py:16-21: 512x64 . 64x64 . 64x64; the fp32 BMM -> softmax -> BMM of
+// benchmark/chimera/cpu/bmm_softmax_bmm.py:64-170) and its ("80", "float64", "float64") row
+// (benchmark/chimera/cuda/bmm_bmm_cuda.py:273-288).
 //
-// That configuration is plumbing, not a hot path (0.5 MFLOP per row block), so this kernel is
-// plain fp32 FMAs over LDS tiles: a workgroup owns 32 rows of A for one batch entry, walks L in
-// tiles of 64, keeps the 32x64 intermediate tile in LDS and its 32xN slice of F in registers.
-// (fp64, the reference's ("80", "float64", "float64") row of benchmark/chimera/cuda/bmm_bmm_cuda.py:273-288: the
-// same kernel on doubles with tiles of 32 along L, so that K, N up to 128 still fit LDS.)
-// Sums run over k, then l, in ascending order in the element type.  Softmax is the online form over the tiles of L: the eight
-// threads of a row share its running maximum (exchanged by lane shuffles), each keeps the sum of its own
-// probabilities, and the row's slice of F is rescaled when the maximum rises.
+// fp32: gemm_chain_f32_kernel below, on v_mfma_f32_16x16x4_f32.  fp64: plain FMAs over LDS tiles
+// (gemm_chain_f64_kernel), the arithmetic type the matrix cores' fp32 path does not cover.
+#include "common.h"
 #include "gemm_chain_f32.h"
 
 namespace ditto {
 
 namespace {
-constexpr int kBM = 32, kMaxD = 128;
-template <typename F>
-constexpr int tile_l() { return sizeof(F) == 8 ? 32 : 64; }  // intermediate columns per step
-
-__device__ inline float fp_exp2(float x) { return exp2f(x); }
-__device__ inline double fp_exp2(double x) { return exp2(x); }
-__device__ inline float fp_max(float a, float b) { return fmaxf(a, b); }
-__device__ inline double fp_max(double a, double b) { return fmax(a, b); }
-__device__ inline float fp_fma(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
-__device__ inline double fp_fma(double a, double b, double c) { return __builtin_fma(a, b, c); }
+constexpr int kMaxD = 128;
+constexpr int kWaves = 8;  // waves of an fp32 workgroup: they split the keys
 }
 
-template <typename F>
-__host__ __device__ inline int fp_chain_lds_bytes(int K, int N) {
-  constexpr int kBL = tile_l<F>();
-  return (kBM * (K + 1) + K * (kBL + 1) + kBL * (N + 1) + kBM * (kBL + 1)) * (int)sizeof(F);
-}
-
-template <typename F>
-__global__ __launch_bounds__(256) void gemm_chain_fp_kernel(F32ChainArgs p) {
-  constexpr int kBL = tile_l<F>();
-  extern __shared__ __attribute__((aligned(16))) char smem_fp[];
+// ---- fp32 ------------------------------------------------------------------------------------
+// A workgroup owns 16 * RT rows of A; its eight waves split L: wave w takes the steps w, w + 8, ... of 16 keys, and the
+// eight partial results of a row meet once, in LDS, at the end (with the softmax: each wave has its own reference
+// exponent and sum).  Sixteen rows of one head are too little work for eight waves any other way, and at the sizes
+// this type is used at (6144 rows in all on 256 compute units) splitting the rows alone leaves most SIMDs idle.
+//
+// Nothing but that merge goes through LDS.  With S^T = B^T.A^T on the 16x16x4 MFMA a lane (c = lane % 16, q = lane / 16)
+// ends with keys 4q + r, r = 0..3, of row c, which is operand r of a second contraction over the four keys
+// {4q + r : q}: F^T = C^T.P^T takes the probabilities where they are.  The contraction index of either product may run
+// in any order both operands agree on, so every operand is loaded as 16-byte pieces of its own rows straight from
+// memory: k = 16 s + 4 q + t is k step (s, t) of the first product, and column n = 64 g + 4 c + t is output tile (g, t) of
+// the second.  K fragments are fetched during the second product of the step before, V fragments during the first.
+//
+// Bound: the fp32 matrix pipe (256 flop per cycle and compute unit) from a few rounds of workgroups on, the chain of
+// first loads, steps and merge below that.  12 x 512 x 512 x 64 (BERT-base, batch 1), softmax: 14.4 us per launch,
+// 56 TFLOP/s, where the plain fp32 FMAs over LDS tiles that this kernel replaced took 143 us (one row per eight threads,
+// an LDS read per operand of every FMA); 64 x 512 x 512 x 64: 52.7 us, 82 TFLOP/s; 4 x 1024 x 1024 x 128: 28.9 us, 74 TFLOP/s.
+//
+// DT: column tiles of 16 that K and N are padded to.  EXACT: K = N = 16 DT and every row starts on a 16-byte boundary;
+// otherwise elements are loaded one by one and columns past K or N are zeros.
+template <int DT, int RT, bool EXACT, bool KL, bool SM>
+__global__ __launch_bounds__(64 * kWaves) void gemm_chain_f32_kernel(F32ChainArgs p) {
+  constexpr int G = DT / 4, REM = DT % 4;  // column groups of 64 (16-byte pieces), column tiles beyond them
+  constexpr int ORS = 16 * DT + 4;         // row stride of a parked partial result, floats
+  static_assert(REM <= 1, "columns beyond the groups of 64: at most one tile of 16");
+  extern __shared__ __attribute__((aligned(16))) float smem_f32[];
+  float* const Om = smem_f32;                              // [wave][16 RT][ORS]
+  float* const Ml = smem_f32 + kWaves * 16 * RT * ORS;     // [wave][16 RT][reference exponent, sum]
   const int K = p.K, N = p.N, L = p.L, M = p.M;
-  F* As = reinterpret_cast<F*>(smem_fp);  // [32][K+1]
-  F* Bs = As + kBM * (K + 1);             // [K][kBL+1]
-  F* Cs = Bs + K * (kBL + 1);             // [kBL][N+1]
-  F* Ms = Cs + kBL * (N + 1);             // [32][kBL+1]
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, c = lane & 15, q = lane >> 4;
+  const unsigned bid = xcd_remap(blockIdx.x, gridDim.x);  // the row blocks of a batch entry read the same B and C
+  const int bz = bid / (unsigned)p.mblocks, m0 = (bid - bz * (unsigned)p.mblocks) * 16 * RT;
+  const float* const Ag = static_cast<const float*>(p.a) + (long long)bz * p.a_bs;
+  const float* const Bg = static_cast<const float*>(p.b) + (long long)bz * p.b_bs;
+  const float* const Cg = static_cast<const float*>(p.c) + (long long)bz * p.c_bs;
+  float* const Fg = static_cast<float*>(p.f) + (long long)bz * p.f_bs;
+
+  // columns k0 .. k0 + 3 of a row, zeros from `n` on
+  auto load4 = [](const float* row, int k0, int n) -> f32x4 {
+    if constexpr (EXACT) return *reinterpret_cast<const f32x4*>(row + k0);
+    f32x4 v;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) v[t] = k0 + t < n ? row[k0 + t] : 0.f;
+    return v;
+  };
+
+  const int nsteps = (L + 15) / 16;
+  f32x4 kf[DT], qf[RT][DT], vf[4][G + REM], o[RT][DT];
+  auto load_k = [&](int step) __attribute__((always_inline)) {
+    const int key = min(16 * step + c, L - 1);  // keys past the last are masked below
+#pragma unroll
+    for (int s = 0; s < DT; ++s) {
+      if constexpr (KL) {
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          const int k = 16 * s + 4 * q + t;
+          kf[s][t] = EXACT || k < K ? Bg[(long long)k * p.b_rs + key] : 0.f;
+        }
+      } else {
+        kf[s] = load4(Bg + (long long)key * p.b_rs, 16 * s + 4 * q, K);
+      }
+    }
+  };
+  if (w < nsteps) load_k(w);
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt) {
+    const float* const row = Ag + (long long)min(m0 + 16 * rt + c, M - 1) * p.a_rs;
+#pragma unroll
+    for (int s = 0; s < DT; ++s) qf[rt][s] = load4(row, 16 * s + 4 * q, K);
+#pragma unroll
+    for (int j = 0; j < DT; ++j) o[rt][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  }
+  // softmax in the exp2 domain: a row's reference exponent is its maximum over the wave's first keys, raised only when a
+  // later score exceeds it by 2^kSlack (a row sum stays below L 2^kSlack, far inside the fp32 range)
+  constexpr float kSlack = 20.f;
+  const float c2 = p.softmax_scale * 1.4426950408889634f;
+  float ref[RT], lsum[RT];
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt) ref[rt] = -INFINITY, lsum[rt] = 0.f;
+
+  for (int step = w; step < nsteps; step += kWaves) {
+    const int key0 = 16 * step;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const float* const row = Cg + (long long)min(key0 + 4 * q + r, L - 1) * p.c_rs;
+#pragma unroll
+      for (int g = 0; g < G; ++g) vf[r][g] = load4(row, 64 * g + 4 * c, N);
+      if constexpr (REM > 0) vf[r][G][0] = EXACT || 64 * G + c < N ? row[64 * G + c] : 0.f;
+    }
+    f32x4 st[RT];
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) st[rt] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < DT; ++s)
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt)
+          st[rt] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[s][t], qf[rt][s][t], st[rt], 0, 0, 0);
+    if (step + kWaves < nsteps) load_k(step + kWaves);
+    const bool tail = key0 + 16 > L;
+    if constexpr (SM) {
+      bool raise = false;
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          st[rt][r] *= c2;
+          if (tail && key0 + 4 * q + r >= L) st[rt][r] = -INFINITY;
+          raise |= st[rt][r] > ref[rt] + kSlack;
+        }
+      }
+      if (__any(raise)) {
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) {
+          float mx = fmaxf(fmaxf(st[rt][0], st[rt][1]), fmaxf(st[rt][2], st[rt][3]));
+          mx = fmaxf(mx, __shfl_xor(mx, 16));
+          mx = fmaxf(mx, __shfl_xor(mx, 32));
+          const float up = fmaxf(ref[rt], mx), alpha = exp2f(ref[rt] - up);
+          ref[rt] = up;
+          lsum[rt] *= alpha;
+#pragma unroll
+          for (int j = 0; j < DT; ++j) o[rt][j] *= alpha;
+        }
+      }
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          st[rt][r] = __builtin_amdgcn_exp2f(st[rt][r] - ref[rt]);
+          lsum[rt] += st[rt][r];
+        }
+    } else {
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          if (p.relu) st[rt][r] = fmaxf(st[rt][r], 0.f);
+          if (tail && key0 + 4 * q + r >= L) st[rt][r] = 0.f;
+        }
+    }
+    if (tail) {  // the clamped rows stand for nothing, whatever the last row holds
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int g = 0; g < G + REM; ++g)
+          if (key0 + 4 * q + r >= L) vf[r][g] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int j = 0; j < DT; ++j)
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt)
+          o[rt][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[r][j / 4][j % 4], st[rt][r], o[rt][j], 0, 0, 0);
+  }
+
+  // lane (c, q) holds of row c: columns 64 g + 16 q + 4 r + t in register r of tile 4 g + t, and 64 G + 4 q + r in the last
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt) {
+    float* const row = Om + (w * 16 * RT + 16 * rt + c) * ORS;
+#pragma unroll
+    for (int g = 0; g < G; ++g)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        *reinterpret_cast<f32x4*>(row + 64 * g + 16 * q + 4 * r) =
+            (f32x4){o[rt][4 * g][r], o[rt][4 * g + 1][r], o[rt][4 * g + 2][r], o[rt][4 * g + 3][r]};
+    if constexpr (REM > 0) *reinterpret_cast<f32x4*>(row + 64 * G + 4 * q) = o[rt][4 * G];
+    if constexpr (SM) {
+      float s = lsum[rt];
+      s += __shfl_xor(s, 16);
+      s += __shfl_xor(s, 32);
+      if (q == 0) {
+        Ml[2 * (w * 16 * RT + 16 * rt + c)] = ref[rt];
+        Ml[2 * (w * 16 * RT + 16 * rt + c) + 1] = s;
+      }
+    }
+  }
+  wg_sync();
+  for (int e = tid; e < 16 * RT * 4 * DT; e += 64 * kWaves) {
+    const int row = e / (4 * DT), n0 = 4 * (e - row * 4 * DT);
+    float wt[kWaves];
+    if constexpr (SM) {
+      float mx = -INFINITY, s = 0.f;
+#pragma unroll
+      for (int i = 0; i < kWaves; ++i) mx = fmaxf(mx, Ml[2 * (i * 16 * RT + row)]);
+#pragma unroll
+      for (int i = 0; i < kWaves; ++i) {
+        wt[i] = exp2f(Ml[2 * (i * 16 * RT + row)] - mx);
+        s += wt[i] * Ml[2 * (i * 16 * RT + row) + 1];
+      }
+      const float inv = 1.f / s;
+#pragma unroll
+      for (int i = 0; i < kWaves; ++i) wt[i] *= inv;
+    } else {
+#pragma unroll
+      for (int i = 0; i < kWaves; ++i) wt[i] = 1.f;
+    }
+    f32x4 x = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < kWaves; ++i) {
+      const f32x4 part = *reinterpret_cast<const f32x4*>(Om + (i * 16 * RT + row) * ORS + n0);
+#pragma unroll
+      for (int t = 0; t < 4; ++t) x[t] = __builtin_fmaf(wt[i], part[t], x[t]);
+    }
+    if (p.relu_out)
+#pragma unroll
+      for (int t = 0; t < 4; ++t) x[t] = fmaxf(x[t], 0.f);
+    if (m0 + row < M) {
+      float* const dst = Fg + (long long)(m0 + row) * p.f_rs + n0;
+      if constexpr (EXACT) {
+        *reinterpret_cast<f32x4*>(dst) = x;
+      } else {
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+          if (n0 + t < N) dst[t] = x[t];
+      }
+    }
+  }
+}
+
+// ---- fp64 ------------------------------------------------------------------------------------
+// A workgroup owns 32 rows of A for one batch entry, walks L in tiles of 32, keeps the 32x32 intermediate tile in LDS and
+// its 32xN slice of F in registers.  Sums run over k, then l, in ascending order.  Softmax is the online form over the tiles
+// of L: the eight threads of a row share its running maximum (exchanged by lane shuffles), each keeps the sum of its own
+// probabilities, and the row's slice of F is rescaled when the maximum rises.
+namespace {
+constexpr int kBM = 32, kBL = 32;
+}
+
+static int f64_chain_lds_bytes(int K, int N) {
+  return (kBM * (K + 1) + K * (kBL + 1) + kBL * (N + 1) + kBM * (kBL + 1)) * (int)sizeof(double);
+}
+
+__global__ __launch_bounds__(256) void gemm_chain_f64_kernel(F32ChainArgs p) {
+  extern __shared__ __attribute__((aligned(16))) double smem_f64[];
+  const int K = p.K, N = p.N, L = p.L, M = p.M;
+  double* As = smem_f64;             // [32][K+1]
+  double* Bs = As + kBM * (K + 1);   // [K][kBL+1]
+  double* Cs = Bs + K * (kBL + 1);   // [kBL][N+1]
+  double* Ms = Cs + kBL * (N + 1);   // [32][kBL+1]
   const int tid = threadIdx.x;
   const int mb = blockIdx.x % p.mblocks, bz = blockIdx.x / p.mblocks;
   const int m0 = mb * kBM;
-  const F* Ag = static_cast<const F*>(p.a) + (long long)bz * p.a_bs;
-  const F* Bg = static_cast<const F*>(p.b) + (long long)bz * p.b_bs;
-  const F* Cg = static_cast<const F*>(p.c) + (long long)bz * p.c_bs;
-  F* Fg = static_cast<F*>(p.f) + (long long)bz * p.f_bs;
-  const F zero = 0;
+  const double* Ag = static_cast<const double*>(p.a) + (long long)bz * p.a_bs;
+  const double* Bg = static_cast<const double*>(p.b) + (long long)bz * p.b_bs;
+  const double* Cg = static_cast<const double*>(p.c) + (long long)bz * p.c_bs;
+  double* Fg = static_cast<double*>(p.f) + (long long)bz * p.f_bs;
 
   for (int e = tid; e < kBM * K; e += 256) {
     const int r = e / K, k = e % K;
-    As[r * (K + 1) + k] = m0 + r < M ? Ag[(long long)(m0 + r) * p.a_rs + k] : zero;
+    As[r * (K + 1) + k] = m0 + r < M ? Ag[(long long)(m0 + r) * p.a_rs + k] : 0.0;
   }
   const int r = tid >> 3, c8 = tid & 7;  // this thread's row and its column phase
-  F acc[kMaxD / 8];
+  double acc[kMaxD / 8];
 #pragma unroll
-  for (int i = 0; i < kMaxD / 8; ++i) acc[i] = zero;
+  for (int i = 0; i < kMaxD / 8; ++i) acc[i] = 0.0;
 
-  F mrow = -INFINITY, lsum = zero;  // softmax: running maximum (exp2 domain), this thread's share of the row sum
-  const F c2 = (F)p.softmax_scale * (F)1.4426950408889634;
+  double mrow = -INFINITY, lsum = 0.0;  // softmax: running maximum (exp2 domain), this thread's share of the row sum
+  const double c2 = (double)p.softmax_scale * 1.4426950408889634;
 
   for (int l0 = 0; l0 < L; l0 += kBL) {
     __syncthreads();
     for (int e = tid; e < K * kBL; e += 256) {
       // consecutive threads read along the contiguous axis of B
       const int k = p.b_lk ? e % K : e / kBL, l = p.b_lk ? e / K : e % kBL;
-      F v = zero;
+      double v = 0.0;
       if (l0 + l < L) v = p.b_lk ? Bg[(long long)(l0 + l) * p.b_rs + k] : Bg[(long long)k * p.b_rs + l0 + l];
       Bs[k * (kBL + 1) + l] = v;
     }
     for (int e = tid; e < kBL * N; e += 256) {
       const int l = e / N, n = e % N;
-      Cs[l * (N + 1) + n] = l0 + l < L ? Cg[(long long)(l0 + l) * p.c_rs + n] : zero;
+      Cs[l * (N + 1) + n] = l0 + l < L ? Cg[(long long)(l0 + l) * p.c_rs + n] : 0.0;
     }
     __syncthreads();
-    F sv[kBL / 8];
+    double sv[kBL / 8];
 #pragma unroll
     for (int j = 0; j < kBL / 8; ++j) {
       const int l = c8 + 8 * j;
-      F s = zero;
-      for (int k = 0; k < K; ++k) s = fp_fma(As[r * (K + 1) + k], Bs[k * (kBL + 1) + l], s);
-      if (p.relu) s = fp_max(s, zero);
+      double s = 0.0;
+      for (int k = 0; k < K; ++k) s = __builtin_fma(As[r * (K + 1) + k], Bs[k * (kBL + 1) + l], s);
+      if (p.relu) s = fmax(s, 0.0);
       sv[j] = s;
     }
     if (p.softmax) {
-      F mx = -INFINITY;
+      double mx = -INFINITY;
 #pragma unroll
       for (int j = 0; j < kBL / 8; ++j) {
-        sv[j] = l0 + c8 + 8 * j < L ? sv[j] * c2 : (F)-INFINITY;  // keys past L take no part
-        mx = fp_max(mx, sv[j]);
+        sv[j] = l0 + c8 + 8 * j < L ? sv[j] * c2 : (double)-INFINITY;  // keys past L take no part
+        mx = fmax(mx, sv[j]);
       }
       // the row's eight threads are eight consecutive lanes
-      mx = fp_max(mx, __shfl_xor(mx, 1));
-      mx = fp_max(mx, __shfl_xor(mx, 2));
-      mx = fp_max(mx, __shfl_xor(mx, 4));
-      const F mnew = fp_max(mrow, mx);  // finite: every tile holds at least one key
-      const F alpha = fp_exp2(mrow - mnew);
+      mx = fmax(mx, __shfl_xor(mx, 1));
+      mx = fmax(mx, __shfl_xor(mx, 2));
+      mx = fmax(mx, __shfl_xor(mx, 4));
+      const double mnew = fmax(mrow, mx);  // finite: every tile holds at least one key
+      const double alpha = exp2(mrow - mnew);
       mrow = mnew;
       lsum *= alpha;
 #pragma unroll
       for (int i = 0; i < kMaxD / 8; ++i) acc[i] *= alpha;
 #pragma unroll
       for (int j = 0; j < kBL / 8; ++j) {
-        sv[j] = fp_exp2(sv[j] - mnew);
+        sv[j] = exp2(sv[j] - mnew);
         lsum += sv[j];
       }
     }
@@ -116,51 +329,86 @@ __global__ __launch_bounds__(256) void gemm_chain_fp_kernel(F32ChainArgs p) {
     for (int i = 0; i < kMaxD / 8; ++i) {
       const int n = c8 + 8 * i;
       if (n < N) {
-        F s = acc[i];
-        for (int l = 0; l < kBL; ++l) s = fp_fma(Ms[r * (kBL + 1) + l], Cs[l * (N + 1) + n], s);
+        double s = acc[i];
+        for (int l = 0; l < kBL; ++l) s = __builtin_fma(Ms[r * (kBL + 1) + l], Cs[l * (N + 1) + n], s);
         acc[i] = s;
       }
     }
   }
-  F inv = 1;
+  double inv = 1.0;
   if (p.softmax) {
     lsum += __shfl_xor(lsum, 1);
     lsum += __shfl_xor(lsum, 2);
     lsum += __shfl_xor(lsum, 4);
-    inv = (F)1 / lsum;
+    inv = 1.0 / lsum;
   }
   if (m0 + r < M) {
 #pragma unroll
     for (int i = 0; i < kMaxD / 8; ++i) {
       const int n = c8 + 8 * i;
-      if (n < N) Fg[(long long)(m0 + r) * p.f_rs + n] = p.relu_out ? fp_max(acc[i] * inv, zero) : acc[i] * inv;
+      if (n < N) Fg[(long long)(m0 + r) * p.f_rs + n] = p.relu_out ? fmax(acc[i] * inv, 0.0) : acc[i] * inv;
     }
   }
 }
 
-int f32_chain_lds_bytes_host(int K, int N, int f64) { return f64 ? fp_chain_lds_bytes<double>(K, N) : fp_chain_lds_bytes<float>(K, N); }
+// ---- launch ----------------------------------------------------------------------------------
 int f32_chain_max_dim() { return kMaxD; }
 
-template <typename F>
-static hipError_t launch_fp(const F32ChainArgs& args, hipStream_t stream) {
-  const int lds = fp_chain_lds_bytes<F>(args.K, args.N);
-  static thread_local int configured_dev = -1;
+static int f32_tiles(int K, int N) {  // column tiles of 16 the fp32 kernel is built for
+  const int d = K > N ? K : N;
+  return d <= 64 ? 4 : d <= 80 ? 5 : 8;
+}
+int f32_chain_lds_bytes_host(int K, int N, int f64, int rt) {
+  if (f64) return f64_chain_lds_bytes(K, N);
+  return kWaves * 16 * rt * (16 * f32_tiles(K, N) + 4 + 2) * (int)sizeof(float);
+}
+
+template <typename Tag, typename Kernel>
+static hipError_t launch_with_lds(Kernel kernel, unsigned threads, int lds, const F32ChainArgs& args, hipStream_t stream) {
+  static thread_local int configured_dev = -1;  // one per kernel (Tag names it), device and thread
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
   if (e != hipSuccess) return e;
   if (configured_dev != dev) {
-    e = hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_chain_fp_kernel<F>),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
     if (e != hipSuccess) return e;
     configured_dev = dev;
   }
-  const unsigned grid = (unsigned)args.mblocks * (unsigned)args.batch;
-  hipLaunchKernelGGL(gemm_chain_fp_kernel<F>, dim3(grid), dim3(256), lds, stream, args);
+  hipLaunchKernelGGL(kernel, dim3((unsigned)args.mblocks * (unsigned)args.batch), dim3(threads), lds, stream, args);
   return hipGetLastError();
 }
 
-hipError_t launch_gemm_chain_f32(const F32ChainArgs& args, hipStream_t stream) {
-  return args.f64 ? launch_fp<double>(args, stream) : launch_fp<float>(args, stream);
+template <int DT, int RT, bool EXACT, bool KL, bool SM>
+struct F32Tag {};
+
+template <int DT, int RT, bool EXACT>
+static hipError_t launch_f32(const F32ChainArgs& a, hipStream_t stream) {
+  const int lds = f32_chain_lds_bytes_host(a.K, a.N, 0, RT), threads = 64 * kWaves;
+  if (a.softmax)
+    return a.b_lk ? launch_with_lds<F32Tag<DT, RT, EXACT, false, true>>(gemm_chain_f32_kernel<DT, RT, EXACT, false, true>, threads, lds, a, stream)
+                  : launch_with_lds<F32Tag<DT, RT, EXACT, true, true>>(gemm_chain_f32_kernel<DT, RT, EXACT, true, true>, threads, lds, a, stream);
+  return a.b_lk ? launch_with_lds<F32Tag<DT, RT, EXACT, false, false>>(gemm_chain_f32_kernel<DT, RT, EXACT, false, false>, threads, lds, a, stream)
+                : launch_with_lds<F32Tag<DT, RT, EXACT, true, false>>(gemm_chain_f32_kernel<DT, RT, EXACT, true, false>, threads, lds, a, stream);
+}
+
+template <int DT>
+static hipError_t launch_f32_rows(const F32ChainArgs& a, bool exact, hipStream_t stream) {
+  if constexpr (DT <= 5)
+    if (a.row_tiles == 2) return exact ? launch_f32<DT, 2, true>(a, stream) : launch_f32<DT, 2, false>(a, stream);
+  if (a.row_tiles != 1) return hipErrorInvalidValue;
+  return exact ? launch_f32<DT, 1, true>(a, stream) : launch_f32<DT, 1, false>(a, stream);
+}
+
+hipError_t launch_gemm_chain_f32(const F32ChainArgs& a, hipStream_t stream) {
+  if (a.f64) return launch_with_lds<double>(gemm_chain_f64_kernel, 256, f64_chain_lds_bytes(a.K, a.N), a, stream);
+  const int dt = f32_tiles(a.K, a.N);
+  // 16-byte pieces of the rows of A, B (stored [L][K]), C and F; a [K][L] B is read one element per lane either way
+  long long strides = a.a_bs | a.c_bs | a.f_bs | a.a_rs | a.c_rs | a.f_rs;
+  if (a.b_lk) strides |= a.b_bs | a.b_rs;
+  const bool exact = a.K == 16 * dt && a.N == 16 * dt && strides % 4 == 0;
+  return dt == 4 ? launch_f32_rows<4>(a, exact, stream)
+         : dt == 5 ? launch_f32_rows<5>(a, exact, stream)
+                   : launch_f32_rows<8>(a, exact, stream);
 }
 
 }  // namespace ditto

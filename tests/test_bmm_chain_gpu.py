@@ -141,6 +141,25 @@ def test_fp32_chain_vs_oracle(oracle, shape, inter):
         assert mx <= 1e-4 and rel <= 1e-5, (b_layout, mx, rel)  # fp32 sums of <= 200 terms
 
 
+@pytest.mark.parametrize("shape", [
+    # (batch, M, N, K, L): one key, steps of 16 keys that do not fill a round of eight waves, ragged ends of both
+    (1, 1, 64, 64, 1), (2, 17, 64, 64, 16), (1, 33, 64, 64, 129), (3, 50, 80, 80, 77), (1, 40, 128, 128, 300),
+    (1, 20, 4, 6, 33), (2, 20, 70, 66, 50),   # columns loaded one by one
+    (9, 512, 64, 64, 140), (9, 500, 80, 80, 40),  # 32-row workgroups
+])
+@pytest.mark.parametrize("inter", ["relu", "softmax"])
+def test_fp32_chain_at_the_edges_of_its_tiles(oracle, shape, inter):
+    batch, M, N, K, L = shape
+    A, B, C = oracle.make_gemm_chain_inputs(batch, M, N, K, L, "float32", seed=M + L, std=1.0 if inter == "softmax" else 0.25)
+    # scores that climb by far more than the slack of the running reference as the keys go on
+    B = B * np.linspace(0.1, 8.0, L, dtype=np.float32)[None, None, :]
+    want = oracle.bmm_chain_f64(A, B, C, inter=inter, scale=0.5 if inter == "softmax" else 1.0)
+    for b_layout in ("KL", "LK"):
+        got = run_chain(A, B, C, "float32", inter, 0.5 if inter == "softmax" else 1.0, b_layout)
+        mx, rel = errors(got, want)
+        assert np.isfinite(got).all() and rel <= 1e-5, (b_layout, mx, rel)
+
+
 @pytest.mark.parametrize("shape", [(1, 512, 64, 64, 64), (3, 100, 24, 40, 72), (2, 64, 128, 128, 200)])
 @pytest.mark.parametrize("inter", ["cast", "relu", "softmax"])
 def test_fp64_chain_vs_oracle(oracle, shape, inter):
