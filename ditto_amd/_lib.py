@@ -159,6 +159,23 @@ def load():
     return _lib
 
 
+_host = None
+
+
+def host():
+    """The native call path over the library (``ditto_amd/_host.so``, ``csrc/host/host_call.cpp``), loaded once."""
+    global _host
+    if _host is None:
+        load()
+        try:
+            from . import _host as module
+        except ImportError as error:
+            raise ChainLibraryError("ditto_amd/_host.so cannot be loaded (%s): build it with `python -m ditto_amd.build_ext`"
+                                    % error)
+        _host = module
+    return _host
+
+
 def last_error():
     return load().ditto_last_error().decode("utf-8", "replace")
 

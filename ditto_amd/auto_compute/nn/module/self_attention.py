@@ -10,7 +10,7 @@ every head straight into its columns of the ``[batch, M, hidden]`` output.
 """
 import torch
 
-from .... import chain, te
+from .... import _lib, chain, te
 from ...graph import Layer
 
 MUTI_HEAD_ATTENTION_LAYER = "multi_head_attention_mma_layer"  # the reference's dispatch key (:7)
@@ -70,6 +70,13 @@ class MultiHeadAttentionMMA:
     def forward(self, query_key_value, out=None, tile_variant=0):
         """query_key_value: [batch, M, 3 * hidden] (query | key | value along the last axis).
         Returns [batch, M, hidden]; ``out`` may be given (destination passing)."""
+        done = _lib.host().run_attention(query_key_value, out, self.num_heads, self.hidden_size, self.scale, tile_variant)
+        if done is not None:
+            rc, out = done
+            if rc:
+                _lib.check(rc)
+            return out
+        # tensors the native call leaves to the general path (and to its errors): strided or misshapen ones
         q, k, v = self.head_views(query_key_value)
         batch, M = query_key_value.shape[0], query_key_value.shape[1]
         if out is None:

@@ -18,6 +18,10 @@ CPU_LIB = os.path.join(CSRC, "libditto_chain_cpu.so")
 CPU_SRC = os.path.join(CSRC, "cpu", "chain_cpu.cpp")
 CPU_FLAGS = ["-O3", "-std=c++17", "-mavx2", "-mfma", "-fopenmp", "-fPIC", "-fvisibility=hidden", "-shared"]
 
+# the native call path from torch tensors to the chain library: a Python extension module, built with g++ (host code only)
+HOST_MODULE = os.path.join(os.path.dirname(os.path.abspath(__file__)), "_host.so")
+HOST_SRC = os.path.join(CSRC, "host", "host_call.cpp")
+
 # -packed-fp32-ops is switched off: packed fp32 VALU forms are not wanted in these kernels.
 HIPCC_FLAGS = [
     "--offload-arch=gfx950",
@@ -95,8 +99,35 @@ def build_cpu(verbose=True):
     return CPU_LIB
 
 
+def build_host(verbose=True):
+    """The native call path; links against the chain library, which has to be built."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+
+    cxx = shutil.which("g++") or shutil.which("c++")
+    if not cxx:
+        raise RuntimeError("g++ not found; the native call path needs a host C++ compiler")
+    lib_dir = os.path.join(os.path.dirname(torch.__file__), "lib")
+    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    cmd = [cxx, "-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-shared",
+           # torch's HIP headers are read as HIP's own headers ask for it
+           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch._C._GLIBCXX_USE_CXX11_ABI,
+           *("-I" + p for p in [*cpp_extension.include_paths(), os.path.join(rocm, "include"), sysconfig.get_paths()["include"]]),
+           HOST_SRC, "-o", HOST_MODULE,
+           "-L" + lib_dir, "-ltorch_python", "-ltorch_cpu", "-ltorch", "-lc10_hip", "-lc10",
+           "-L" + CSRC, "-l:" + os.path.basename(LIB), "-Wl,-rpath,$ORIGIN/csrc"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError("building %s failed:\n%s" % (HOST_SRC, r.stderr))
+    if verbose:
+        print("built", HOST_MODULE)
+    return HOST_MODULE
+
+
 def build(verbose=True, jobs=None):
-    """Compile every translation unit and link the shared library.  Always rebuilds."""
+    """Compile every translation unit, link the shared library and build the call path over it.  Always rebuilds."""
     os.makedirs(OBJ_DIR, exist_ok=True)
     build_cpu(verbose)
     jobs = jobs or min(8, os.cpu_count() or 1)
@@ -108,6 +139,7 @@ def build(verbose=True, jobs=None):
         raise RuntimeError("link failed:\n%s" % r.stderr)
     if verbose:
         print("built", LIB)
+    build_host(verbose)
     return LIB
 
 

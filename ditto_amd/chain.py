@@ -49,22 +49,6 @@ def _check_device(*tensors):
     return dev
 
 
-def _as3d(t, name):
-    if t.dim() == 2:
-        t = t.unsqueeze(0)
-    if t.dim() != 3:
-        raise ValueError("%s must be [batch, rows, cols] or [rows, cols]" % name)
-    return t
-
-
-def _split_levels(t, name):
-    """[outer, inner, rows, cols] (any strides) -> (3-D view of the first outer entry with the inner
-    level as its batch, outer extent, outer stride); 2-D / 3-D tensors have a single level."""
-    if t.dim() == 4:
-        return t[0], t.shape[0], t.stride(0)
-    return _as3d(t, name), 1, 0
-
-
 def bmm_chain_desc(A, B, C, F, inter_op="cast", softmax_scale=1.0, requant_scale=1.0, tile_variant=0,
                    relu_out=False):
     """Fill a ``ditto_bmm_chain_desc`` from tensors A[b,M,K], B[b,K,L], C[b,L,N], F[b,M,N].
@@ -76,50 +60,8 @@ def bmm_chain_desc(A, B, C, F, inter_op="cast", softmax_scale=1.0, requant_scale
     is copied.  ``tile_variant`` forces a kernel variant (an id that
     ``select_tile`` reports); 0 leaves the choice to the library's per-shape table.
     """
-    (A, ao, a_so), (B, bo, b_so), (C, co, c_so), (F, fo, f_so) = (
-        _split_levels(A, "A"), _split_levels(B, "B"), _split_levels(C, "C"), _split_levels(F, "F"))
-    if not (ao == bo == co == fo):
-        raise ValueError("A, B, C, F must agree in their outer batch extent")
-    batch, M, K = A.shape
-    if B.shape[0] != batch or B.shape[1] != K:
-        raise ValueError("B must be [batch, K, L] = [%d, %d, L], got %s" % (batch, K, tuple(B.shape)))
-    L = B.shape[2]
-    if C.shape[0] != batch or C.shape[1] != L:
-        raise ValueError("C must be [batch, L, N] = [%d, %d, N], got %s" % (batch, L, tuple(C.shape)))
-    N = C.shape[2]
-    if tuple(F.shape) != (batch, M, N):
-        raise ValueError("F must be [%d, %d, %d], got %s" % (batch, M, N, tuple(F.shape)))
-    if not (A.dtype == B.dtype == C.dtype):
-        raise ValueError("A, B, C must share one dtype")
-    for t, name in ((A, "A"), (C, "C"), (F, "F")):
-        if t.shape[2] > 1 and t.stride(2) != 1:
-            raise ValueError("%s rows must be contiguous" % name)
     d = _lib.BmmChainDesc()
-    d.abi_version = _lib.ABI_VERSION
-    d.in_dtype = _code(A)
-    d.acc_dtype = _lib.I32 if A.dtype == torch.int8 else _lib.F64 if A.dtype == torch.float64 else _lib.F32
-    d.out_dtype = _code(F)
-    d.inter_op = INTER_OPS[inter_op] if isinstance(inter_op, str) else int(inter_op)
-    if B.stride(2) == 1 or L == 1:
-        d.b_layout = _lib.B_KL
-        d.b_row_stride = B.stride(1)
-    elif B.stride(1) == 1:
-        d.b_layout = _lib.B_LK
-        d.b_row_stride = B.stride(2)
-    else:
-        raise ValueError("B must be contiguous along L or along K")
-    d.batch, d.M, d.N, d.K, d.L = batch * ao, M, N, K, L
-    d.batch_inner = batch if ao > 1 else 0
-    d.a_batch_stride_outer, d.b_batch_stride_outer = a_so, b_so
-    d.c_batch_stride_outer, d.f_batch_stride_outer = c_so, f_so
-    d.a_batch_stride, d.a_row_stride = A.stride(0), A.stride(1)
-    d.b_batch_stride = B.stride(0)
-    d.c_batch_stride, d.c_row_stride = C.stride(0), C.stride(1)
-    d.f_batch_stride, d.f_row_stride = F.stride(0), F.stride(1)
-    d.softmax_scale = float(softmax_scale)
-    d.requant_scale = float(requant_scale)
-    d.tile_variant = int(tile_variant)
-    d.relu_out = int(bool(relu_out))
+    _lib.host().fill_bmm_desc(ctypes.addressof(d), A, B, C, F, inter_op, softmax_scale, requant_scale, tile_variant, relu_out)
     return d
 
 
@@ -140,24 +82,11 @@ def run_bmm_chain(A, B, C, F, inter_op="cast", softmax_scale=1.0, requant_scale=
 
     ``aux``: for ``inter_op="requant"`` an fp32 tensor of L per-column scales (``None``: use
     ``requant_scale`` for every column)."""
-    lib = _lib.load()
-    dev = _check_device(A, B, C, F)
+    host = _lib.host()
     if desc is None:
-        desc = bmm_chain_desc(A, B, C, F, inter_op, softmax_scale, requant_scale, tile_variant, relu_out)
-    aux_ptr = None
-    if aux is not None:
-        _check_device(A, aux)
-        if aux.dtype != torch.float32 or not aux.is_contiguous() or aux.numel() != desc.L:
-            raise ValueError("aux must be a contiguous fp32 tensor of L = %d scales" % desc.L)
-        aux_ptr = aux.data_ptr()
-    if torch.cuda.current_device() == dev.index:
-        # (the common case, kept short: for the smallest chains the host's call path is longer than the kernel)
-        rc = lib.ditto_bmm_chain_run(ctypes.byref(desc), A.data_ptr(), B.data_ptr(), C.data_ptr(), aux_ptr,
-                                     F.data_ptr(), None, 0, _raw_stream(dev.index))
+        rc = host.run_bmm(A, B, C, F, inter_op, softmax_scale, requant_scale, aux, tile_variant, relu_out)
     else:
-        with torch.cuda.device(dev):
-            rc = lib.ditto_bmm_chain_run(ctypes.byref(desc), A.data_ptr(), B.data_ptr(), C.data_ptr(), aux_ptr,
-                                         F.data_ptr(), None, 0, _raw_stream(dev.index))
+        rc = host.run_bmm_desc(ctypes.addressof(desc), A, B, C, F, aux)
     if rc:
         _lib.check(rc)
     return F

@@ -4,9 +4,11 @@ Replaces ``func = tvm.build(sch, layer.schedule_tensors, "cuda")`` followed by
 ``func(*inputs, *outputs)`` and ``func.time_evaluator(func.entry_name, ctx, min_repeat_ms=600)``
 (benchmark/chimera/cuda/bmm_softmax_bmm_cuda.py:23-42, 239, 256).
 """
+import ctypes
+
 import torch
 
-from . import chain
+from . import _lib, chain, te
 from .auto_tensorize.hyper_fusion import ChainSchedule
 
 _TORCH = {"float16": torch.float16, "bfloat16": torch.bfloat16, "float32": torch.float32, "float64": torch.float64,
@@ -28,8 +30,8 @@ class ChainFunction:
     in ``layer.schedule_tensors`` order; the output is written in place (destination passing)
     and the call returns without synchronising.
 
-    The C-ABI descriptor is filled once per distinct argument layout (shapes, strides, dtypes)
-    and reused.  A conv chain that takes a workspace owns one per device, sized by
+    A call goes through native code (``csrc/host/host_call.cpp``) that checks the arguments, fills the C-ABI
+    descriptor and launches.  A conv chain that takes a workspace owns one per device, sized by
     ``ditto_conv_chain_workspace_bytes`` at its first call and never replaced, so a HIP graph that
     captured a call keeps a valid pointer; calls of ONE function object on two streams still race
     on it (use ``specialize`` for a second object).  ``specialize(W1, W2)`` returns a function bound
@@ -54,14 +56,27 @@ class ChainFunction:
         self.tensors = list(tensors) if tensors is not None else sch.layer.schedule_tensors
         self.target = "hip"
         self.tile_variant = int(sch.tile_variant if tile_variant is None else tile_variant)
-        self._descs = {}        # argument layout -> filled descriptor
+        self._native = None     # the native call, made at the first one
+        self._descs = {}        # dtypes -> descriptor as filled for them first: what ran, for a caller that logs it
         self._workspaces = {}   # device -> uint8 tensor (conv chains)
         self._prepared = None   # (W1, W2, W1._version, W2._version): what the workspace holds the repacked form of
+
+    def _make_native(self):
+        host, s = _lib.host(), self.sch
+        shapes = [(t.name, tuple(t.shape)) for t in self.tensors]
+        if s.kind == "bmm_chain":
+            self._native = host.BmmCall(shapes, s.inter_op, s.softmax_scale, s.requant_scale, self.tile_variant, s.relu_out,
+                                        s.scale_tensor)
+        elif s.kind == "conv_chain":
+            self._native = host.ConvCall(shapes)
+        else:
+            raise NotImplementedError("no kernel family for chain kind %r" % s.kind)
+        return self._native
 
     def _check_args(self, args):
         if len(args) != len(self.tensors):
             raise ValueError("expected %d tensors (inputs then outputs), got %d" % (len(self.tensors), len(args)))
-        if self.sch.kind == "conv_chain" and args[0].dim() == 5:
+        if args[0].dim() == 5:
             return  # the reference's packed placeholders: checked in _call_packed
         for a, t in zip(args, self.tensors):
             if tuple(a.shape) != tuple(t.shape):
@@ -100,22 +115,12 @@ class ChainFunction:
 
             sch = copy.copy(self.sch)
             sch.dims = dict(d, H=H + 2 * pad1, W=W + 2 * pad1, pad1=0)
-            f = self._packed_fn = ChainFunction(sch, [None] * 4, self.target, self.tile_variant)
-            f._check_args = lambda args: None
+            shapes = ((N, C0, H + 2 * pad1, W + 2 * pad1), want1, (d["C2"], d["C1"], d["R2"], d["S2"]), (N, d["C2"], P, Q))
+            tensors = [te.placeholder(list(s), name=t.name, dtype=t.dtype) for s, t in zip(shapes, self.tensors)]
+            f = self._packed_fn = ChainFunction(sch, tensors, self.target, self.tile_variant)
         y = torch.empty((N, d["C2"], P, Q), device=x.device, dtype=out_p.dtype)
         f(x, w1, w2, y)
         layout.pack_output_into(y, out_p)
-
-    @staticmethod
-    def _layout(args):
-        return tuple((tuple(a.shape), tuple(a.stride()), a.dtype) for a in args)
-
-    def _desc(self, args, make):
-        key = self._layout(args)
-        d = self._descs.get(key)
-        if d is None:
-            d = self._descs[key] = make()
-        return d
 
     def _workspace(self, desc, dev):
         ws = self._workspaces.get(dev)
@@ -126,9 +131,16 @@ class ChainFunction:
 
     def _conv_desc(self, X, W1, W2, Y):
         s, d = self.sch, self.sch.dims
-        return self._desc((X, W1, W2, Y), lambda: chain.conv_chain_desc(
-            X, W1, W2, Y, d["pad1"], d["stride1"], d["pad2"], d["stride2"], s.inter_op, s.relu_out,
-            d.get("groups1", 1)))
+        return chain.conv_chain_desc(X, W1, W2, Y, d["pad1"], d["stride1"], d["pad2"], d["stride2"], s.inter_op, s.relu_out,
+                                     d.get("groups1", 1))
+
+    def _remember(self, desc, X, W1, W2, Y, ws, prepared):
+        """Leave the next call with tensors like these (and, for bound weights, with those weights unchanged) to native
+        code."""
+        native = self._native or self._make_native()
+        self._descs[X.dtype, Y.dtype] = desc
+        native.remember(ctypes.addressof(desc), X, Y, ws if ws is not False else None, W1 if prepared else None,
+                        W2 if prepared else None)
 
     def specialize(self, W1, W2):
         """A copy of this conv chain function bound to the weight tensors ``W1``, ``W2``: they are
@@ -141,13 +153,12 @@ class ChainFunction:
         # the descriptor depends on shapes and dtypes only (all four tensors are contiguous)
         X = torch.empty(tuple(xt.shape), device="meta", dtype=dt)
         Y = torch.empty(tuple(yt.shape), device="meta", dtype=_TORCH[yt.dtype])
-        d = self.sch.dims
-        desc = chain.conv_chain_desc(X, W1, W2, Y, d["pad1"], d["stride1"], d["pad2"], d["stride2"],
-                                     self.sch.inter_op, self.sch.relu_out, d.get("groups1", 1))
+        desc = self._conv_desc(X, W1, W2, Y)
         ws = f._workspace(desc, W1.device)
         if ws is not False:
             chain.prepare_conv_chain(desc, W1, W2, ws)
             f._prepared = (W1, W2, W1._version, W2._version)
+            f._remember(desc, W1, W1, W2, Y, ws, True)
         return f
 
     def _is_prepared(self, W1, W2):
@@ -162,37 +173,47 @@ class ChainFunction:
         return same(p[0], W1) and same(p[1], W2) and p[2] == W1._version and p[3] == W2._version
 
     def __call__(self, *args):
-        self._check_args(args)
+        native = self._native
+        if native is None:
+            return self._first_call(*args)
+        rc = native(*args)
+        if rc is None:
+            return self._call_conv(*args)
+        if rc:
+            _lib.check(rc)
+
+    def _first_call(self, *args):
+        self._make_native()
+        self(*args)
         s = self.sch
         if s.kind == "bmm_chain":
-            aux = None
-            if s.scale_tensor:
-                A, B, C, aux, F = args
-            else:
-                A, B, C, F = args
-            desc = self._desc((A, B, C, F), lambda: chain.bmm_chain_desc(
-                A, B, C, F, s.inter_op, s.softmax_scale, s.requant_scale, self.tile_variant, s.relu_out))
-            chain.run_bmm_chain(A, B, C, F, aux=aux, desc=desc)
-        elif s.kind == "conv_chain":
-            X, W1, W2, Y = args
-            if X.dim() == 5:
-                return self._call_packed(X, W1, W2, Y)
-            desc = self._conv_desc(X, W1, W2, Y)
-            ws = self._workspace(desc, X.device)
-            prepared = ws is not False and self._is_prepared(W1, W2)
-            if ws is not False and self._prepared is not None and not prepared:
-                # a specialised function handed other weights (or the bound ones after an in-place update):
-                # repack them now; they are the bound weights from here on
-                self._prepared = None
-                try:
-                    chain.prepare_conv_chain(desc, W1, W2, ws)
-                    self._prepared = (W1, W2, W1._version, W2._version)
-                    prepared = True
-                except ValueError:
-                    pass  # pointers the prepared form cannot take: the one-call form below decides
-            chain.run_conv_chain(X, W1, W2, Y, desc=desc, workspace=ws, prepared=prepared)
-        else:
-            raise NotImplementedError("no kernel family for chain kind %r" % s.kind)
+            A, B, C, F = args[0], args[1], args[2], args[-1]
+            self._descs[A.dtype, F.dtype] = chain.bmm_chain_desc(A, B, C, F, s.inter_op, s.softmax_scale, s.requant_scale,
+                                                                 self.tile_variant, s.relu_out)
+
+    def _call_conv(self, *args):
+        """A conv chain call that the native one has not seen the like of: the first, or with other weights than the bound
+        ones, or packed."""
+        self._check_args(args)
+        X, W1, W2, Y = args
+        if X.dim() == 5:
+            return self._call_packed(X, W1, W2, Y)
+        desc = self._conv_desc(X, W1, W2, Y)
+        ws = self._workspace(desc, X.device)
+        prepared = ws is not False and self._is_prepared(W1, W2)
+        if ws is not False and self._prepared is not None and not prepared:
+            # a specialised function handed other weights (or the bound ones after an in-place update):
+            # repack them now; they are the bound weights from here on
+            self._prepared = None
+            self._native.forget()
+            try:
+                chain.prepare_conv_chain(desc, W1, W2, ws)
+                self._prepared = (W1, W2, W1._version, W2._version)
+                prepared = True
+            except ValueError:
+                pass  # pointers the prepared form cannot take: the one-call form below decides
+        chain.run_conv_chain(X, W1, W2, Y, desc=desc, workspace=ws, prepared=prepared)
+        self._remember(desc, X, W1, W2, Y, ws, prepared)
 
     def time_evaluator(self, func_name=None, ctx=None, number=1, repeat=1, min_repeat_ms=0):
         """Mean seconds per call measured with HIP events on the current stream: ``repeat``
