@@ -374,6 +374,8 @@ struct ConvPlan {
   bool rows31;         // 3x3 -> 1x1 with at most 64 -> 64 -> 256 channels: the row pipeline (cvargs), W1 fragments
                        // in the workspace
   ditto::ConvRowsArgs cvargs;
+  bool tiles;          // dense -> 1x1 on tiles of whole output rows (targs), both weights as fragments in the workspace
+  ditto::ConvTilesArgs targs;
   ditto_tile_param tile;
 };
 
@@ -395,6 +397,7 @@ struct ConvSteer {
   bool resident = true;  // 3600: the persistent kernel with W2 resident in LDS
   bool dw_rows = true;   // 4024
   bool dw16_rows = true; // 4025
+  bool tiles = true;     // 3200: tiles of whole output rows
   bool persist = false;  // 3900: the persistent 3x3 -> 1x1 kernel (switched off)
 };
 int conv_steer(int tv, ConvSteer* st) {
@@ -405,10 +408,11 @@ int conv_steer(int tv, ConvSteer* st) {
   const int fam = tv / 100 * 100;
   st->rows = fam == 3700 || fam == 3800;
   st->resident = fam == 3600;
+  st->tiles = fam == 3200;
   st->dw_rows = tv == 4024;
   st->dw16_rows = tv == 4025;
   st->persist = fam == 3900;
-  if (!(fam == 3000 || fam == 3100 || fam == 3500 || fam == 3600 || fam == 3700 || fam == 3800 || fam == 3900 || fam == 4000))
+  if (!(fam == 3000 || fam == 3100 || fam == 3200 || fam == 3500 || fam == 3600 || fam == 3700 || fam == 3800 || fam == 3900 || fam == 4000))
     return fail(DITTO_EINVAL, "tile_variant %d names no conv chain kernel family", tv);
   return DITTO_OK;
 }
@@ -666,6 +670,75 @@ int plan_dw_conv(const ditto_conv_chain_desc* d, const ConvSteer& steer, long lo
 
 int plan_conv_steered(const ditto_conv_chain_desc* d, const ConvSteer& steer, ConvPlan* plan, bool need_device,
                       int dw_vec_cap, bool allow_resident, bool allow_dw_rows);
+
+// Dense -> 1x1 on tiles of whole output rows (conv_tiles.h), where that is the kernel for the shape (`forced`: where it can
+// run it at all).
+bool plan_conv_tiles(const ditto_conv_chain_desc* d, long long P, long long Q, bool forced, ConvPlan* plan, int cus) {
+  const int slots = 16 * ditto::kCtMaxTiles;
+  if (d->W < 8 || Q > slots) return false;
+  const int c0p = (int)((d->C0 + 31) / 32 * 32), c1p = ditto::conv_tiles_c1p((int)d->C1);
+  const int cols_in = (int)((Q - 1) * d->stride1 + d->S1);
+  auto rows_in = [&](int th) { return (int)((th - 1) * d->stride1 + d->R1); };
+  auto lds_of = [&](int th) { return ditto::conv_tiles_lds_bytes(rows_in(th), cols_in, c0p, c1p, slots); };
+  if (lds_of(1) > 160 * 1024) return false;
+  // The general kernel stays ahead on stride-1 filters over few channels whose image rows are whole 16-byte vectors, with a
+  // tile of four rows and more for every compute unit (32 x 64 x 56 x 56 3x3 -> 64 -> 64 15.2 against 15.7 us, 32 x 32 x 56 x 56
+  // -> 32 -> 128 11.2 / 15.4, 10 x 64 x 72 x 72 -> 64 -> 256 16.4 / 18.2); with two rows per tile it is behind (8 x 64 x 104 x 104
+  // 39.3 / 26.2), and so it is everywhere else: 8 x 32 x 147 x 147 stride 2 -> 64 -> 80 21.5 / 13.3, one image of 128 x 28 x 28 ->
+  // 256 -> 128 45.6 / 9.2, 21 x 64 x 106 x 106 stride 2 -> 192 -> 128 109 / 31, 32 x 256 x 56 x 56 1x1 -> 256 -> 64 83 / 31.
+  const long long old_rows = d->W > 0 ? 256 / d->W : 0;
+  if (!forced && d->W % 8 == 0 && d->stride1 == 1 && d->R1 * d->S1 > 1 && d->C1 <= 64 && old_rows >= 3 &&
+      d->N * ((P + old_rows - 1) / old_rows) >= cus)
+    return false;
+  // Rows per workgroup.  A workgroup streams all of W1 whatever its rows, at 64 bytes per clock - as long as the MFMAs of
+  // four pixel tiles take - and fetches its halo rows; the fewest clocks over the rounds of workgroups win, a third more
+  // where only one workgroup fits a compute unit (its phases then overlap with nobody's).  Strided filters take few halo
+  // rows in common with their neighbours, so their workgroups stay at one output row as soon as that fills three pixel
+  // tiles or the grid is small (8 x 16 x 227 x 227 stride 4: one row 7.5 us, two 9.8; 32 x 32 x 112 x 112 stride 2 15.9 / 19.1).
+  const long long k_w1 = d->R1 * d->S1 * (c0p / 32) * (c1p / 16);
+  int th = 1;
+  double best = 0;
+  for (int t = 1; t <= P && t * Q <= slots && lds_of(t) <= 160 * 1024; ++t) {
+    const long long wgs = d->N * ((P + t - 1) / t), rounds = (wgs + cus - 1) / cus;
+    const double work = (double)k_w1 * std::max(16LL, 4 * ((t * Q + 15) / 16)) + rows_in(t) * (double)(d->W * c0p) / 12 + 300;
+    const double cost = rounds * work * (rounds > 1 && 2 * lds_of(t) > 160 * 1024 ? 1.35 : 1.0);
+    if (t == 1 || cost < best) best = cost, th = t;
+    if (d->stride1 > 1 && (t * Q > 32 || wgs <= 2 * cus)) {
+      th = t;
+      break;
+    }
+  }
+  ditto::ConvTilesArgs& a = plan->targs;
+  a.N = (int)d->N; a.C0 = (int)d->C0; a.H = (int)d->H; a.W = (int)d->W; a.C1 = (int)d->C1; a.C2 = (int)d->C2;
+  a.R = (int)d->R1; a.S = (int)d->S1; a.pad = (int)d->pad1; a.stride = (int)d->stride1;
+  a.P = (int)P; a.Q = (int)Q;
+  a.TH = th;
+  a.tiles_h = (int)((P + th - 1) / th);
+  a.rows_in = rows_in(th);
+  a.cols_in = cols_in;
+  a.c0p = c0p;
+  a.relu_mid = d->inter_op == DITTO_INTER_RELU;
+  a.relu_out = d->relu_out != 0;
+  a.out_f32 = d->out_dtype == DITTO_F32;
+  a.inv_cg = 1.f / (float)(c0p / 8), a.inv_ng = 1.f / (float)((d->W + 7) / 8);
+  a.inv_q = 1.f / (float)Q;
+  plan->tiles = true;
+  plan->w1p_bytes = ditto::conv_tiles_w1_bytes((int)d->C1, c0p, (int)(d->R1 * d->S1));
+  plan->w2p_bytes = ditto::conv_tiles_w2_bytes((int)d->C2, c1p);
+  ditto_tile_param& t = plan->tile;
+  const ditto::ConvTilesSplit w = ditto::conv_tiles_split((int)d->C1, (int)(d->R1 * d->S1) * c0p / 32);
+  t.block_threads = 64 * w.wc * w.wp;
+  t.block_m = th * (int)Q;
+  t.block_l = c1p;
+  t.block_n = (int)d->C2;
+  t.head_pad = c0p;
+  t.lds_bytes = lds_of(th);
+  t.grid_x = a.N * a.tiles_h;
+  t.grid_y = th;
+  t.grid_z = (int)Q;
+  t.variant = 3200 + th;  // tiles of whole output rows; rows per workgroup
+  return true;
+}
 
 // allow_resident = false: the general kernels only (pointers the specialised ones cannot take);
 // allow_dw_rows: y takes 16-byte stores
@@ -926,6 +999,8 @@ int plan_conv_steered(const ditto_conv_chain_desc* d, const ConvSteer& steer, Co
       return DITTO_OK;
     }
   }
+  if (allow_resident && steer.tiles && plan_conv_tiles(d, P, Q, steer.tv / 100 == 32, plan, need_device ? device_cus() : 256))
+    return DITTO_OK;
   // The persistent variant (conv_chain_persist.h: W1 resident in LDS, W2 in registers, one workgroup per
   // CU walking over the tiles) is switched off: it waits for its prefetched halo tile with a hand-counted
   // `s_waitcnt vmcnt` over loads the compiler does not track, and it is slower than the kernel below
@@ -1143,7 +1218,7 @@ size_t ditto_conv_chain_workspace_bytes(const ditto_conv_chain_desc* desc) {
   ConvPlan plan;
   if (plan_conv(desc, &plan, true) != DITTO_OK) return 0;
   size_t need = plan.w1p_bytes + plan.w2p_bytes;
-  if (plan.resident || plan.rows31 || plan.rows13) {
+  if (plan.resident || plan.rows31 || plan.rows13 || plan.tiles) {
     // a call with pointers these kernels cannot take falls back to the general one (tile_variant 0 only): the
     // larger of the two figures, whatever the device's compute-unit count makes of the choice
     ConvPlan general;
@@ -1239,6 +1314,38 @@ int conv_chain_call(int phase, const ditto_conv_chain_desc* d, const void* x, co
               : ditto::pack_conv_w2_resident_bf16(w1, workspace, r.C0, r.C1, st);
     if (e == hipSuccess && (phase & kConvCompute))
       e = f16 ? ditto::launch_conv_rows_f16(r, st) : ditto::launch_conv_rows_bf16(r, st);
+    if (e != hipSuccess) return fail(DITTO_EHIP, "kernel launch failed: %s", hipGetErrorString(e));
+    return DITTO_OK;
+  }
+  if (plan.tiles) {
+    // both weights as MFMA fragments in the workspace; x and y at any element
+    const size_t need = plan.w1p_bytes + plan.w2p_bytes;
+    const bool ok = workspace && workspace_bytes >= need && aligned(workspace, 16);
+    if (!ok && phase == kConvBoth && d->tile_variant == 0) {
+      rc = plan_conv(d, &plan, true, 4, false);  // the general kernel: workspace optional
+      if (rc != DITTO_OK) return rc;
+    } else if (!workspace || workspace_bytes < need) {
+      return fail(DITTO_EWORKSPACE, "prepared weights live in the workspace: need %zu bytes", need);
+    } else if (!ok) {
+      return fail(DITTO_EINVAL, "workspace must be 16-byte aligned");
+    }
+  }
+  if (plan.tiles) {
+    ditto::ConvTilesArgs r = plan.targs;
+    if (!aligned(x, 2) || !aligned(y, r.out_f32 ? 4 : 2) || !aligned(w1, 2) || !aligned(w2, 2))
+      return fail(DITTO_EINVAL, "misaligned data pointer");
+    r.x = x;
+    r.w1f = workspace;
+    r.w2f = static_cast<char*>(workspace) + plan.w1p_bytes;
+    r.y = y;
+    hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+    const bool f16 = d->in_dtype == DITTO_F16;
+    hipError_t e = hipSuccess;
+    if (phase & kConvPrepare)
+      e = f16 ? ditto::pack_conv_tiles_f16(r, w1, w2, const_cast<void*>(r.w1f), const_cast<void*>(r.w2f), st)
+              : ditto::pack_conv_tiles_bf16(r, w1, w2, const_cast<void*>(r.w1f), const_cast<void*>(r.w2f), st);
+    if (e == hipSuccess && (phase & kConvCompute))
+      e = f16 ? ditto::launch_conv_tiles_f16(r, st) : ditto::launch_conv_tiles_bf16(r, st);
     if (e != hipSuccess) return fail(DITTO_EHIP, "kernel launch failed: %s", hipGetErrorString(e));
     return DITTO_OK;
   }

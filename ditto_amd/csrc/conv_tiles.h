@@ -1,0 +1,369 @@
+// conv(RxS, any stride) -> cast|relu -> conv(1x1) on NCHW tensors, fp16 / bf16: tiles of whole output rows, any image
+// width from 8 pixels on, weights as MFMA fragments straight from L2.
+//
+// For the shapes the general kernel (conv_chain.h) is bad at: it stages halo tile and weights through LDS in chunks of 32
+// channels, four barriers and two exposed memory latencies each, computes 256 pixel slots whatever the tile holds, reads
+// image rows that are not whole 16-byte vectors two bytes at a time, and stores two bytes at a time where a tile is not a
+// run of such rows.  A workgroup here
+//   - owns TH whole output rows (at most 128 pixels) of one image and all channels: one contiguous run of every channel plane;
+//   - stages the halo rows of ALL input channels once, with 16-byte loads at element alignment (the hardware takes them at
+//     any address) and an 8x8 transposition in registers;
+//   - runs the first convolution without a barrier: W1 comes as ready fragments, 1 KB per wave and instruction, each by the
+//     one wave (or two, see conv_tiles_split) that owns those channels, four k steps ahead;
+//   - puts the cast result into LDS once and takes the second convolution's pixels in the order PO j + t (column j of tile t),
+//     which leaves a lane with 8 consecutive pixels of 4 channels: 16-byte stores, 256 contiguous bytes per 16 lanes.
+// Three barriers in all; several workgroups share a compute unit and cover one another's loads.
+//
+// Bound: for few pixels the stream of W1 through one compute unit (64 bytes per clock), otherwise load, compute and
+// store phases one after the other, which only other workgroups on the compute unit overlap.  Measured, us per launch with
+// prepared weights, general kernel -> this one: 8 x 32 x 147 x 147 stride 2 -> 64 -> 80 21.5 -> 13.3 (4 of them the loads, 2.4
+// the launch); one image 128 x 28 x 28 -> 256 -> 128 45.6 -> 9.2 (28 compute units, each streaming 590 KB of W1);
+// 21 x 64 x 106 x 106 stride 2 -> 192 -> 128 109 -> 31 (520 TFLOP/s); 32 x 128 x 28 x 28 -> 256 -> 128 46 -> 20.5 (800 TFLOP/s);
+// 32 x 256 x 56 x 56 1x1 -> 256 -> 64 83 -> 31.  Tried and left out: columns kept by remainder modulo the stride, so that a
+// strided tap reads neighbouring pixels without bank conflicts (level at 147 x 147, 0.3 us slower on small images: the
+// index arithmetic); W2 fragments fetched ahead of the first convolution (level).
+#pragma once
+#include "common.h"
+
+namespace ditto {
+
+struct ConvTilesArgs {
+  const void* x;
+  const void* w1f;  // W1 as fragments (pack_conv_fragments): [wave][k step][tile of the wave][64 lanes][8]
+  const void* w2f;  // W2 as fragments: [output tile][k step][64 lanes][8]
+  void* y;
+  int N, C0, H, W, C1, C2;
+  int R, S, pad, stride;
+  int P, Q;           // output extent
+  int TH, tiles_h;    // output rows per workgroup, workgroups per image
+  int rows_in, cols_in;  // halo rows and columns of a full tile
+  int c0p;               // input channels padded to 32
+  int relu_mid, relu_out, out_f32;
+  float inv_cg, inv_ng, inv_q;  // 1 / (c0p / 8), 1 / ceil(W / 8), 1 / Q
+};
+
+// n / d for 0 <= n < 2^21 and inv = 1 / d: the half keeps the product inside the quotient's interval whatever its
+// rounding.  (An integer division by a run-time value is some thirty instructions, and a workgroup's start is a chain of
+// them.)
+__device__ __forceinline__ int div_by(int n, float inv) { return (int)(((float)n + 0.5f) * inv); }
+
+template <int V>
+struct CtInt {
+  static constexpr int value = V;
+};
+
+constexpr int kCtMaxTiles = 8;  // tiles of 16 output pixels per workgroup
+
+// element stride of a pixel's channel vector in LDS: the 8 elements beyond the channels spread consecutive pixels over
+// the banks
+__host__ __device__ constexpr int conv_tiles_stride(int channels) { return channels + 8; }
+__host__ __device__ inline int conv_tiles_lds_bytes(int rows_in, int cols_in, int c0p, int c1p, int slots) {
+  const int x = rows_in * cols_in * conv_tiles_stride(c0p) * 2, mid = slots * conv_tiles_stride(c1p) * 2;
+  return x > mid ? x : mid;
+}
+
+// W[rows][cols][taps] -> [group of `per` row tiles][k step][tile][lane][8], zero padded: element e of lane l of tile t
+// is row 16 t + l % 16, column 32 (step % (colsp / 32)) + 8 (l / 16) + e, tap step / (colsp / 32)
+template <typename T>
+__global__ void pack_conv_fragments_kernel(const T* __restrict__ w, T* __restrict__ out, int rows, int cols, int colsp, int taps,
+                                           int per, unsigned total) {
+  const unsigned i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= total) return;
+  const int e = i & 7, l = (i >> 3) & 63;
+  const unsigned f = i >> 9;
+  const int cb = colsp / 32, steps = taps * cb;
+  const int m = f % (unsigned)per, step = f / (unsigned)per % (unsigned)steps, grp = f / (unsigned)per / (unsigned)steps;
+  const int row = 16 * (grp * per + m) + (l & 15), col = 32 * (step % cb) + 8 * (l >> 4) + e, tap = step / cb;
+  out[i] = row < rows && col < cols ? w[((long long)row * cols + col) * taps + tap] : (T)0.f;
+}
+
+// WC x WP waves: WC of them split the intermediate channels (MC tiles of 16 each), WP the pixels (PT tiles of 16 each).
+template <typename T, int WC, int WP, int MC, int PT>
+__global__ __launch_bounds__(64 * WC * WP) void conv_tiles_kernel(ConvTilesArgs p) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  typedef typename Elem<T>::v8 V8;
+  typedef typename Elem<T>::v4 V4;
+  typedef __attribute__((ext_vector_type(8), aligned(2))) T V8u;  // 16 bytes at any element's address
+  constexpr int NW = WC * WP, NT = 64 * NW, C1P = 16 * WC * MC, MS = conv_tiles_stride(C1P);
+  constexpr int PO = WP * PT <= 2 ? 2 : WP * PT <= 4 ? 4 : 8;  // consecutive output pixels of a lane
+  constexpr int D = NW == 8 ? 2 : 4;                 // W1 fragments in flight per tile
+  extern __shared__ __attribute__((aligned(16))) char smem_ct[];
+  T* const Xs = reinterpret_cast<T*>(smem_ct);  // [rows_in][cols_in][CHS]
+  T* const Ms = Xs;                             // [slot][MS], once everyone is done with Xs
+  const int tid = threadIdx.x, lane = tid & 63, c = lane & 15, q = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wc = wave % WC, wp = wave / WC;
+  const unsigned lid = xcd_remap(blockIdx.x, gridDim.x);
+  const int n = lid / (unsigned)p.tiles_h, p0 = (lid - n * (unsigned)p.tiles_h) * p.TH;
+  const int npx = min(p.TH, p.P - p0) * p.Q;
+  const int h0 = p0 * p.stride - p.pad;
+  const int CHS = conv_tiles_stride(p.c0p), cg = p.c0p / 8;
+  const long long hw = (long long)p.H * p.W;
+
+  const int cb = p.c0p / 32, KS = p.R * p.S * cb;
+  const T* const w1 = reinterpret_cast<const T*>(p.w1f) + (size_t)wc * KS * MC * 512;
+  V8 wf[D][MC];
+  auto load_w = [&](int d, int ks) __attribute__((always_inline)) {
+    const T* const src = w1 + (size_t)min(ks, KS - 1) * MC * 512;
+#pragma unroll
+    for (int m = 0; m < MC; ++m) wf[d][m] = *reinterpret_cast<const V8*>(src + m * 512 + lane * 8);
+  };
+#pragma unroll
+  for (int d = 0; d < D; ++d) load_w(d, d);
+
+  // ---- halo rows into LDS, channel fastest.  A task is 8 pixels x 8 channels of one image row: eight 16-byte loads (at
+  // element alignment: rows of any length), an 8x8 transposition in registers, eight 16-byte writes.  The last group of a
+  // row starts at W - 8 and repeats pixels of the one before it.  Two tasks of a thread are in flight together.
+  const int row_step = p.cols_in * CHS;
+  {
+    const T* const Xg = reinterpret_cast<const T*>(p.x) + (long long)n * p.C0 * hw;
+    const int ng = (p.W + 7) / 8, tasks = p.rows_in * ng * cg;
+    auto stage = [&](auto both, int t0) __attribute__((always_inline)) {
+      constexpr int U = decltype(both)::value;
+      i32x4 xr[U][8];
+      int col[U];
+      T* dst[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int t = t0 + u * NT, rest = div_by(t, p.inv_cg), ri = div_by(rest, p.inv_ng), chg = t - rest * cg;
+        const int w = min(8 * (rest - ri * ng), p.W - 8), h = h0 + ri;
+        col[u] = w + p.pad;
+        dst[u] = Xs + ri * row_step + (w + p.pad) * CHS + 8 * chg;
+        const bool live = t < tasks && h >= 0 && h < p.H;
+        const T* const src = Xg + (long long)(8 * chg) * hw + (long long)h * p.W + w;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+          i32x4 v = {0, 0, 0, 0};
+          if (live && 8 * chg + k < p.C0) v = __builtin_bit_cast(i32x4, (V8)*reinterpret_cast<const V8u*>(src + k * hw));
+          xr[u][k] = v;
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        if (t0 + u * NT >= tasks) break;
+#pragma unroll
+        for (int px = 0; px < 8; ++px) {
+          i32x4 o;
+#pragma unroll
+          for (int k = 0; k < 4; ++k)
+            o[k] = __builtin_amdgcn_perm(xr[u][2 * k + 1][px >> 1], xr[u][2 * k][px >> 1], (px & 1) ? 0x07060302 : 0x05040100);
+          if (col[u] + px < p.cols_in) *reinterpret_cast<i32x4*>(dst[u] + px * CHS) = o;
+        }
+      }
+    };
+    int t0 = tid;
+    for (; t0 - tid + NT < tasks; t0 += 2 * NT) stage(CtInt<2>(), t0);
+    if (t0 - tid < tasks) stage(CtInt<1>(), t0);
+    // the columns left and right of the image
+    const int right = max(0, p.cols_in - p.W - p.pad), nz = p.pad + right;
+    if (nz > 0) {
+      const float inv_nz = 1.f / (float)nz;
+      for (int t = tid; t < p.rows_in * nz * cg; t += NT) {
+        const int rest = div_by(t, p.inv_cg), chg = t - rest * cg, ri = div_by(rest, inv_nz), z = rest - ri * nz;
+        *reinterpret_cast<i32x4*>(Xs + ri * row_step + (z < p.pad ? z : p.W + z) * CHS + 8 * chg) = i32x4{0, 0, 0, 0};
+      }
+    }
+  }
+
+  int xb[PT];  // element offset of this lane's pixel of tile t at tap (0, 0)
+#pragma unroll
+  for (int t = 0; t < PT; ++t) {
+    int slot = 16 * (wp * PT + t) + c;
+    slot = slot < npx ? slot : 0;
+    const int ph = div_by(slot, p.inv_q), pw = slot - ph * p.Q;
+    xb[t] = (ph * p.cols_in + pw) * p.stride * CHS + 8 * q;
+  }
+  f32x4 acc[MC][PT];
+#pragma unroll
+  for (int m = 0; m < MC; ++m)
+#pragma unroll
+    for (int t = 0; t < PT; ++t) acc[m][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  wg_sync();
+
+  // ---- first convolution: k step = 32 channels of one tap
+  {
+    int kb = 0, ts = 0, off = 0;  // of the next pixel fragments to fetch: channel block, tap column, element offset
+    constexpr int XB = NW == 8 ? 1 : 2;  // (eight waves: four per SIMD hide the LDS latency, and registers are what they lack)
+    V8 xf[XB][PT];
+    auto load_x = [&](int d) __attribute__((always_inline)) {
+#pragma unroll
+      for (int t = 0; t < PT; ++t) xf[d][t] = *reinterpret_cast<const V8*>(Xs + xb[t] + off);
+      off += 32;
+      if (++kb == cb) {
+        kb = 0, off += CHS - p.c0p;
+        if (++ts == p.S) ts = 0, off += row_step - p.S * CHS;
+      }
+    };
+    if (XB == 2) load_x(0);
+    for (int ks = 0; ks < KS; ks += D) {
+#pragma unroll
+      for (int d = 0; d < D; ++d) {
+        if (ks + d >= KS) break;
+        if (XB == 1) load_x(0);
+        else if (ks + d + 1 < KS) load_x((d + 1) & 1);
+#pragma unroll
+        for (int m = 0; m < MC; ++m)
+#pragma unroll
+          for (int t = 0; t < PT; ++t) acc[m][t] = Elem<T>::mfma16(wf[d][m], xf[d & (XB - 1)][t], acc[m][t]);
+        load_w(d, ks + d + D);
+      }
+    }
+  }
+
+  // ---- second convolution (1x1): column j of output tile t is pixel PO j + t, so a lane ends with PO consecutive pixels
+  // of four channels
+  constexpr int KS2 = C1P / 32;
+  const int tiles2 = (p.C2 + 15) / 16;
+  V8 vf[KS2];
+  auto load_w2 = [&](int ct) __attribute__((always_inline)) {
+    const T* const src = reinterpret_cast<const T*>(p.w2f) + (size_t)min(ct, tiles2 - 1) * KS2 * 512;
+#pragma unroll
+    for (int k = 0; k < KS2; ++k) vf[k] = *reinterpret_cast<const V8*>(src + k * 512 + lane * 8);
+  };
+  load_w2(wave);
+  wg_sync();  // the halo rows are no longer read
+#pragma unroll
+  for (int m = 0; m < MC; ++m)
+#pragma unroll
+    for (int t = 0; t < PT; ++t) {
+      f32x4 v = acc[m][t];
+      if (p.relu_mid)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[r] = fmaxf(v[r], 0.f);
+      const typename Elem<T>::v2 lo = cvt2<T>(v[0], v[1]), hi = cvt2<T>(v[2], v[3]);
+      *reinterpret_cast<V4*>(Ms + (16 * (wp * PT + t) + c) * MS + 16 * (wc * MC + m) + 4 * q) = V4{lo[0], lo[1], hi[0], hi[1]};
+    }
+  wg_sync();
+  const T* const mb = Ms + PO * c * MS + 8 * q;
+  const long long plane = (long long)p.P * p.Q;
+  const int valid = npx - PO * c;  // of this lane's pixels
+  for (int ct = wave; ct < tiles2; ct += NW) {
+    f32x4 o[PO];
+#pragma unroll
+    for (int t = 0; t < PO; ++t) o[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    V8 mf[2][PO];
+#pragma unroll
+    for (int t = 0; t < PO; ++t) mf[0][t] = *reinterpret_cast<const V8*>(mb + t * MS);
+#pragma unroll
+    for (int k = 0; k < KS2; ++k) {
+      if (k + 1 < KS2)
+#pragma unroll
+        for (int t = 0; t < PO; ++t) mf[(k + 1) & 1][t] = *reinterpret_cast<const V8*>(mb + t * MS + 32 * (k + 1));
+#pragma unroll
+      for (int t = 0; t < PO; ++t) o[t] = Elem<T>::mfma16(vf[k], mf[k & 1][t], o[t]);
+      __builtin_amdgcn_sched_barrier(0);  // one step of reads ahead, not all of them (registers)
+    }
+    load_w2(ct + NW);
+    if (p.relu_out)
+#pragma unroll
+      for (int t = 0; t < PO; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) o[t][r] = fmaxf(o[t][r], 0.f);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int c2 = 16 * ct + 4 * q + r;
+      if (c2 >= p.C2) continue;
+      const long long at = ((long long)n * p.C2 + c2) * plane + (long long)p0 * p.Q + PO * c;
+      if (p.out_f32) {
+        float* const dst = reinterpret_cast<float*>(p.y) + at;
+#pragma unroll
+        for (int t = 0; t < PO; ++t)
+          if (t < valid) dst[t] = o[t][r];
+        continue;
+      }
+      typedef __attribute__((ext_vector_type(PO))) T VP;
+      typedef __attribute__((ext_vector_type(PO), aligned(2))) T VPu;
+      VP v;
+#pragma unroll
+      for (int t = 0; t < PO; t += 2) {
+        const typename Elem<T>::v2 two = cvt2<T>(o[t][r], o[t + 1][r]);
+        v[t] = two[0], v[t + 1] = two[1];
+      }
+      T* const dst = reinterpret_cast<T*>(p.y) + at;
+      if (valid >= PO) {
+        *reinterpret_cast<VPu*>(dst) = v;
+      } else {
+#pragma unroll
+        for (int t = 0; t < PO; ++t)
+          if (t < valid) dst[t] = v[t];
+      }
+    }
+  }
+#else
+  (void)p;
+#endif
+}
+
+template <typename T, int WC, int WP, int MC, int PT>
+hipError_t launch_conv_tiles_as(const ConvTilesArgs& a, hipStream_t stream) {
+  auto kern = conv_tiles_kernel<T, WC, WP, MC, PT>;
+  static thread_local int configured_dev = -1;
+  int dev = 0;
+  hipError_t e = hipGetDevice(&dev);
+  if (e != hipSuccess) return e;
+  if (configured_dev != dev) {
+    e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    if (e != hipSuccess) return e;
+    configured_dev = dev;
+  }
+  constexpr int slots = WP * PT <= 2 ? 32 : WP * PT <= 4 ? 64 : 128;
+  const int lds = conv_tiles_lds_bytes(a.rows_in, a.cols_in, a.c0p, 16 * WC * MC, slots);
+  hipLaunchKernelGGL(kern, dim3((unsigned)a.N * (unsigned)a.tiles_h), dim3(64 * WC * WP), lds, stream, a);
+  return hipGetLastError();
+}
+
+template <typename T, int WC, int WP, int MC>
+hipError_t launch_conv_tiles_rows(const ConvTilesArgs& a, hipStream_t stream) {
+  const int tiles = (a.TH * a.Q + 15) / 16, pt = (tiles + WP - 1) / WP;
+  if (tiles > kCtMaxTiles) return hipErrorInvalidValue;
+  if (pt == 1) return launch_conv_tiles_as<T, WC, WP, MC, WP == 1 ? 2 : 1>(a, stream);
+  if (pt == 2) return launch_conv_tiles_as<T, WC, WP, MC, 2>(a, stream);
+  if (pt == 3) return launch_conv_tiles_as<T, WC, WP, MC, 3>(a, stream);
+  if (pt == 4) return launch_conv_tiles_as<T, WC, WP, MC, 4>(a, stream);
+  if constexpr (WP == 1) {
+    if (pt == 5) return launch_conv_tiles_as<T, WC, WP, MC, 5>(a, stream);
+    if (pt == 6) return launch_conv_tiles_as<T, WC, WP, MC, 6>(a, stream);
+    if (pt == 7) return launch_conv_tiles_as<T, WC, WP, MC, 7>(a, stream);
+    if (pt == 8) return launch_conv_tiles_as<T, WC, WP, MC, 8>(a, stream);
+  }
+  return hipErrorInvalidValue;
+}
+
+// How the waves of a workgroup split the C1 x pixels product of the first convolution: wc of them the channels (mc tiles
+// of 16 each), wp the pixels.  Splitting channels alone reads every weight fragment once per workgroup and every pixel
+// fragment wc times out of LDS; at 64 channels that makes LDS the bound of a long contraction, and two waves by two halve
+// its reads for twice the weight fetches: 32 x 64 x 56 x 56 3x3 -> 64 -> 64 17.4 -> 15.7 us, -> 256 24.5 -> 22.7; with 9 k steps
+// (32 input channels) the weights are what counts: 32 x 32 x 147 x 147 stride 2 31.4 against 32.7 us.
+struct ConvTilesSplit {
+  int wc, wp, mc;
+};
+inline ConvTilesSplit conv_tiles_split(int C1, int k_steps) {
+  if (C1 <= 64) return k_steps >= 12 ? ConvTilesSplit{2, 2, 2} : ConvTilesSplit{4, 1, 1};
+  return C1 <= 128 ? ConvTilesSplit{4, 1, 2} : C1 <= 192 ? ConvTilesSplit{4, 1, 3} : ConvTilesSplit{8, 1, 2};
+}
+inline int conv_tiles_c1p(int C1) { return (C1 + 63) / 64 * 64; }
+inline size_t conv_tiles_w1_bytes(int C1, int c0p, int taps) { return (size_t)conv_tiles_c1p(C1) / 16 * taps * (c0p / 32) * 1024; }
+inline size_t conv_tiles_w2_bytes(int C2, int c1p) { return (size_t)((C2 + 15) / 16) * (c1p / 32) * 1024; }
+
+template <typename T>
+hipError_t launch_conv_tiles(const ConvTilesArgs& a, hipStream_t stream) {
+  const ConvTilesSplit w = conv_tiles_split(a.C1, a.R * a.S * a.c0p / 32);
+  if (w.wp == 2) return launch_conv_tiles_rows<T, 2, 2, 2>(a, stream);
+  if (w.wc == 8) return launch_conv_tiles_rows<T, 8, 1, 2>(a, stream);
+  if (w.mc == 1) return launch_conv_tiles_rows<T, 4, 1, 1>(a, stream);
+  if (w.mc == 2) return launch_conv_tiles_rows<T, 4, 1, 2>(a, stream);
+  return launch_conv_tiles_rows<T, 4, 1, 3>(a, stream);
+}
+
+template <typename T>
+hipError_t launch_pack_conv_tiles(const ConvTilesArgs& a, const void* w1, const void* w2, void* w1f, void* w2f, hipStream_t stream) {
+  const int c1p = conv_tiles_c1p(a.C1), taps = a.R * a.S;
+  const unsigned n1 = (unsigned)(conv_tiles_w1_bytes(a.C1, a.c0p, taps) / 2), n2 = (unsigned)(conv_tiles_w2_bytes(a.C2, c1p) / 2);
+  hipLaunchKernelGGL(pack_conv_fragments_kernel<T>, dim3((n1 + 255) / 256), dim3(256), 0, stream, static_cast<const T*>(w1),
+                     static_cast<T*>(w1f), a.C1, a.C0, a.c0p, taps, conv_tiles_split(a.C1, taps * a.c0p / 32).mc, n1);
+  hipLaunchKernelGGL(pack_conv_fragments_kernel<T>, dim3((n2 + 255) / 256), dim3(256), 0, stream, static_cast<const T*>(w2),
+                     static_cast<T*>(w2f), a.C2, a.C1, c1p, 1, 1, n2);
+  return hipGetLastError();
+}
+
+}  // namespace ditto

@@ -923,3 +923,42 @@ def test_packed_placeholders_of_the_reference(oracle, first):
     got2 = out_p.float().cpu().numpy().transpose(0, 1, 4, 2, 3).reshape(N, C2, H, W)
     want2 = oracle.conv_chain_f32(Xp, W1 * 0.5, W2, 0, 1, pad2, 1, round_mid="float16")
     assert errors(got2, oracle.np_round_to(want2, "float16"))[1] <= REL_L2
+
+
+CASES_TILES = [
+    # N, C0, H, W, C1, R, pad, stride, C2: tiles of whole output rows
+    (1, 16, 9, 8, 8, 3, 1, 1, 8),        # the narrowest image, one 16-pixel tile, channels that fill no tile
+    (2, 24, 7, 9, 72, 3, 1, 1, 40),      # a row's last 8-pixel group starts at W - 8; two row tiles per wave
+    (3, 40, 17, 23, 136, 3, 1, 2, 24),   # stride 2, three tiles per wave, a ragged last tile of rows
+    (1, 32, 6, 128, 200, 1, 0, 1, 16),   # the widest output row (8 pixel tiles), eight waves
+    (2, 64, 11, 29, 64, 3, 1, 1, 272),   # two waves by two; five rows per tile, more output tiles than waves
+    (1, 16, 21, 227, 64, 3, 1, 4, 16),   # stride 4
+    (2, 8, 30, 30, 24, 5, 2, 1, 33),     # 5x5, an odd number of output channels
+    (1, 64, 12, 57, 64, 3, 0, 1, 64),    # no padding
+]
+
+
+@pytest.mark.parametrize("case", CASES_TILES)
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+def test_conv_chain_on_row_tiles(oracle, case, dtype):
+    N, C0, H, W, C1, R, pad, stride, C2 = case
+    X, W1, W2 = oracle.make_conv_chain_inputs(N, C0, H, W, C1, C2, R, 1, dtype, seed=C0 + C2 + W, w_std=0.05)
+    for relu in (False, True):
+        inter = "relu" if relu else "cast"
+        want = oracle.conv_chain_f32(X, W1, W2, pad, stride, 0, 1, relu_mid=relu, relu_out=relu, round_mid=dtype)
+        got32 = run_conv(X, W1, W2, dtype, pad, stride, inter, relu, out_dtype="float32", tile_variant=3200)
+        got = run_conv(X, W1, W2, dtype, pad, stride, inter, relu, tile_variant=3200)
+        assert np.isfinite(got).all()
+        mx, rel = errors(got32, want)
+        assert mx <= MAX_ABS and rel <= REL_L2, (relu, mx, rel)
+        assert np.array_equal(got, oracle.np_round_to(got32, dtype)), relu
+    # tensors at any element's address, prepared weights
+    flat = to_dev(np.concatenate([np.zeros(1, np.float32), X.ravel()]), dtype)
+    x, w1, w2 = flat[1:].view(N, C0, H, W), to_dev(W1, dtype), to_dev(W2, dtype)
+    out = torch.full((got.size + 1,), float("nan"), device=x.device, dtype=x.dtype)
+    y = out[1:].view(got.shape)
+    desc = chain.conv_chain_desc(x, w1, w2, y, pad, stride, 0, 1, "relu", True, tile_variant=3200)
+    ws = chain.prepare_conv_chain(desc, w1, w2)
+    chain.run_conv_chain(x, w1, w2, y, desc=desc, workspace=ws, prepared=True)
+    torch.cuda.synchronize()
+    assert np.array_equal(y.float().cpu().numpy(), got) and bool(torch.isnan(out[0]))
