@@ -67,6 +67,8 @@ UNITS = [
      ["-DDITTO_INST_T=bf16", "-DDITTO_INST_INTER=0", "-DDITTO_INST_NAME=launch_bf16_cast", *FP_CHAIN_FLAGS]),
     ("fp_bf16_softmax", "bmm_chain_fp_inst.hip",
      ["-DDITTO_INST_T=bf16", "-DDITTO_INST_INTER=2", "-DDITTO_INST_NAME=launch_bf16_softmax", *FP_CHAIN_FLAGS]),
+    ("fp_split_f16", "bmm_chain_split_inst.hip", ["-DDITTO_INST_T=f16", "-DDITTO_SPLIT_NAME=launch_split_f16", *FP_CHAIN_FLAGS]),
+    ("fp_split_bf16", "bmm_chain_split_inst.hip", ["-DDITTO_INST_T=bf16", "-DDITTO_SPLIT_NAME=launch_split_bf16", *FP_CHAIN_FLAGS]),
 ]
 
 

@@ -15,6 +15,7 @@
 #include "bmm_chain_fp8.h"
 #include "bmm_chain_fp8m16.h"
 #include "bmm_chain_fp4m16.h"
+#include "bmm_chain_split.h"
 #include "chain_kernels.h"
 
 namespace {
@@ -47,6 +48,7 @@ int device_cus() {
 struct BmmPlan {
   int family;  // 0: fp16/bf16 register-resident chain, 1: fp32 chain, 2: int8 requant chain
   int d_pad, qt;  // fp chains: head pad and rows-per-wave code; int8 chain: row tiles and ring depth
+  int split_dt = 0, split_rt = 0;  // fp chains on few rows: column tiles and row tiles of the key-splitting kernel (0: none)
   int nb3 = 0, nb = 0;  // 16x16x32-MFMA kernel: row blocks of 384 rows / row blocks in all, per batch entry
   ditto_tile_param tile;
 };
@@ -206,6 +208,47 @@ int plan_bmm(const ditto_bmm_chain_desc* d, BmmPlan* plan, bool need_device) {
         rows64 = n64 <= cus;
       if (rows64) plan->qt = d->L >= 1024 ? 5 : 4;
       else if (sm && lk && n8 >= 2LL * cus) plan->qt = 6;
+    }
+    {
+      // Few rows: the kernel whose eight waves split the keys (bmm_chain_split.h), in workgroups of 16 or 32 rows.  Its cost
+      // beyond the launch is a start and a merge plus a share of the keys, `a + b L` us, for every round of workgroups over
+      // the compute units; the kernels above walk all keys in one go and their 64 or 128 rows per workgroup need fewer
+      // rounds.  Fitted to measurements at head sizes 64, 80 and 128 (us per launch, other kernel -> this one, LK):
+      // 16 x 176 x 176 x 80 8.4 -> 4.9, 8 x 461 x 461 x 80 12.7 -> 5.9, 16 x 512 x 512 x 80 12.4 -> 7.3 (32 rows),
+      // 2 x 2392 x 2392 x 80 38.5 -> 13.1, 2 x 4096 x 4096 x 128 60.9 -> 28.4, 8 x 512 x 2048 x 64 17.5 -> 8.8; but
+      // 40 x 300 x 300 x 80 10.1 against 11.2 and 60 x 58 x 58 x 64 3.7 against 4.1, which stay.
+      const int dt = dmax <= 64 ? 4 : dmax <= 80 ? 5 : 8;
+      const bool kl_b = d->b_layout == DITTO_B_KL;
+      int rt = 0;
+      if (d->tile_variant == 0 && (plan->qt == 1 || plan->qt == 4 || plan->qt == 5)) {
+        const double start[2] = {dt == 4 ? 1.2 : dt == 5 ? 2.0 : 3.0, dt == 4 ? 2.7 : dt == 5 ? 2.9 : 4.5};
+        const double per_key[2] = {dt == 4 ? 0.0022 : dt == 5 ? 0.0028 : 0.0044, dt == 4 ? 0.0029 : dt == 5 ? 0.0033 : 0.0053};
+        const long long n64 = ((d->M + 63) / 64) * d->batch, n128 = ((d->M + 127) / 128) * d->batch;
+        double best = dt == 4 ? (0.55 + 0.0065 * d->L) * (n64 <= cus ? 1.0 : 0.8 * ((n64 + cus - 1) / cus))
+                              : (sm ? 3.6 + 0.0134 * d->L : 3.2 + 0.0099 * d->L) * ((n128 + cus - 1) / cus);
+        best *= 0.95;
+        for (int r = 1; r <= 2; ++r) {
+          const long long rounds = (((d->M + 16 * r - 1) / (16 * r)) * d->batch + cus - 1) / cus;
+          const double cost = rounds * (start[r - 1] + per_key[r - 1] * d->L) * (!kl_b ? 1.0 : dt == 8 ? 1.3 : 1.15);
+          if (cost < best) best = cost, rt = r;
+        }
+      }
+      if (d->tile_variant == 2001 + 10 * dt || d->tile_variant == 2002 + 10 * dt) rt = d->tile_variant % 10;
+      if (rt > 0) {
+        plan->split_dt = dt, plan->split_rt = rt;
+        plan->nb = (int)((d->M + 16 * rt - 1) / (16 * rt));
+        ditto_tile_param& t = plan->tile;
+        t.block_threads = 64 * ditto::kSplitWaves;
+        t.block_m = 16 * rt;
+        t.block_l = 32 * ditto::kSplitWaves;
+        t.block_n = (int)d->N;
+        t.head_pad = 16 * dt;
+        t.lds_bytes = ditto::bmm_chain_split_lds(dt, rt, kl_b);
+        t.grid_x = (int)(plan->nb * d->batch);
+        t.grid_y = t.grid_z = 1;
+        t.variant = 2000 + 10 * dt + rt;
+        return DITTO_OK;
+      }
     }
     if (d->tile_variant != 0) {
       const int q = d->tile_variant % 10;
@@ -1131,7 +1174,10 @@ int ditto_bmm_chain_run(const ditto_bmm_chain_desc* d, const void* a, const void
     const bool kl = d->b_layout == DITTO_B_KL;
     const bool sm = d->inter_op == DITTO_INTER_SOFTMAX;
     hipError_t e;
-    if (d->in_dtype == DITTO_F16)
+    if (plan.split_rt > 0)
+      e = d->in_dtype == DITTO_F16 ? ditto::launch_split_f16(plan.split_dt, plan.split_rt, sm, kl, args, st)
+                                   : ditto::launch_split_bf16(plan.split_dt, plan.split_rt, sm, kl, args, st);
+    else if (d->in_dtype == DITTO_F16)
       e = sm ? ditto::launch_f16_softmax(plan.d_pad, plan.qt, kl, args, st)
              : ditto::launch_f16_cast(plan.d_pad, plan.qt, kl, args, st);
     else

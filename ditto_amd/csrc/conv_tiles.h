@@ -62,19 +62,27 @@ __host__ __device__ inline int conv_tiles_lds_bytes(int rows_in, int cols_in, in
   return x > mid ? x : mid;
 }
 
-// W[rows][cols][taps] -> [group of `per` row tiles][k step][tile][lane][8], zero padded: element e of lane l of tile t
+// Both weight tensors in one launch, each W[rows][cols][taps] -> [group of `per` row tiles][k step][tile][lane][8], zero padded: element e of lane l of tile t
 // is row 16 t + l % 16, column 32 (step % (colsp / 32)) + 8 (l / 16) + e, tap step / (colsp / 32)
+struct ConvFragments {
+  const void* w;
+  void* out;
+  int rows, cols, colsp, taps, per;
+  unsigned total;  // elements of `out`
+};
 template <typename T>
-__global__ void pack_conv_fragments_kernel(const T* __restrict__ w, T* __restrict__ out, int rows, int cols, int colsp, int taps,
-                                           int per, unsigned total) {
-  const unsigned i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= total) return;
+__global__ void pack_conv_fragments_kernel(ConvFragments w1, ConvFragments w2, unsigned blocks1) {
+  const bool first = blockIdx.x < blocks1;
+  const ConvFragments& a = first ? w1 : w2;
+  const unsigned i = (blockIdx.x - (first ? 0 : blocks1)) * blockDim.x + threadIdx.x;
+  if (i >= a.total) return;
   const int e = i & 7, l = (i >> 3) & 63;
   const unsigned f = i >> 9;
-  const int cb = colsp / 32, steps = taps * cb;
-  const int m = f % (unsigned)per, step = f / (unsigned)per % (unsigned)steps, grp = f / (unsigned)per / (unsigned)steps;
-  const int row = 16 * (grp * per + m) + (l & 15), col = 32 * (step % cb) + 8 * (l >> 4) + e, tap = step / cb;
-  out[i] = row < rows && col < cols ? w[((long long)row * cols + col) * taps + tap] : (T)0.f;
+  const int cb = a.colsp / 32, steps = a.taps * cb;
+  const int m = f % (unsigned)a.per, step = f / (unsigned)a.per % (unsigned)steps, grp = f / (unsigned)a.per / (unsigned)steps;
+  const int row = 16 * (grp * a.per + m) + (l & 15), col = 32 * (step % cb) + 8 * (l >> 4) + e, tap = step / cb;
+  static_cast<T*>(a.out)[i] =
+      row < a.rows && col < a.cols ? static_cast<const T*>(a.w)[((long long)row * a.cols + col) * a.taps + tap] : (T)0.f;
 }
 
 // WC x WP waves: WC of them split the intermediate channels (MC tiles of 16 each), WP the pixels (PT tiles of 16 each).
@@ -358,11 +366,11 @@ hipError_t launch_conv_tiles(const ConvTilesArgs& a, hipStream_t stream) {
 template <typename T>
 hipError_t launch_pack_conv_tiles(const ConvTilesArgs& a, const void* w1, const void* w2, void* w1f, void* w2f, hipStream_t stream) {
   const int c1p = conv_tiles_c1p(a.C1), taps = a.R * a.S;
-  const unsigned n1 = (unsigned)(conv_tiles_w1_bytes(a.C1, a.c0p, taps) / 2), n2 = (unsigned)(conv_tiles_w2_bytes(a.C2, c1p) / 2);
-  hipLaunchKernelGGL(pack_conv_fragments_kernel<T>, dim3((n1 + 255) / 256), dim3(256), 0, stream, static_cast<const T*>(w1),
-                     static_cast<T*>(w1f), a.C1, a.C0, a.c0p, taps, conv_tiles_split(a.C1, taps * a.c0p / 32).mc, n1);
-  hipLaunchKernelGGL(pack_conv_fragments_kernel<T>, dim3((n2 + 255) / 256), dim3(256), 0, stream, static_cast<const T*>(w2),
-                     static_cast<T*>(w2f), a.C2, a.C1, c1p, 1, 1, n2);
+  const ConvFragments f1 = {w1, w1f, a.C1, a.C0, a.c0p, taps, conv_tiles_split(a.C1, taps * a.c0p / 32).mc,
+                            (unsigned)(conv_tiles_w1_bytes(a.C1, a.c0p, taps) / 2)};
+  const ConvFragments f2 = {w2, w2f, a.C2, a.C1, c1p, 1, 1, (unsigned)(conv_tiles_w2_bytes(a.C2, c1p) / 2)};
+  const unsigned blocks1 = (f1.total + 255) / 256, blocks2 = (f2.total + 255) / 256;
+  hipLaunchKernelGGL(pack_conv_fragments_kernel<T>, dim3(blocks1 + blocks2), dim3(256), 0, stream, f1, f2, blocks1);
   return hipGetLastError();
 }
 

@@ -125,6 +125,35 @@ def test_cast_chain_vs_oracle(oracle, shape, dtype, inter):
             assert np.array_equal(got, oracle.np_round_to(got32, dtype)), (variant, b_layout)
 
 
+@pytest.mark.parametrize("shape", [
+    # (batch, M, N, K, L) for the kernel whose waves split the keys: one step of keys and one more key than eight waves take in
+    # one, single rows, head sizes at and between its three widths
+    (1, 1, 64, 64, 8), (2, 17, 64, 64, 264), (3, 33, 80, 80, 520), (2, 40, 72, 80, 96), (1, 50, 128, 128, 1000),
+    (2, 31, 96, 88, 256), (1, 16, 8, 8, 32), (1, 90, 24, 64, 40),
+])
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+@pytest.mark.parametrize("inter", ["relu", "softmax"])
+def test_key_splitting_kernel(oracle, shape, dtype, inter):
+    batch, M, N, K, L = shape
+    std = 1.0 if inter == "softmax" else 0.25
+    A, B, C = oracle.make_gemm_chain_inputs(batch, M, N, K, L, dtype, seed=700 + M + L, std=std)
+    # scores that climb past the slack of the running reference within a wave's keys
+    B = oracle.np_round_to(B * np.linspace(0.1, 4.0 if inter == "softmax" else 1.0, L, dtype=np.float32)[None, None, :], dtype)
+    scale = 0.5 if inter == "softmax" else 1.0
+    want = oracle.bmm_chain_f64(A, B, C, inter=inter, scale=scale, round_mid=None if inter == "softmax" else dtype)
+    width = 4 if max(K, N) <= 64 else 5 if max(K, N) <= 80 else 8
+    for rows in (1, 2):
+        variant = 2000 + 10 * width + rows
+        for b_layout in ("KL", "LK"):
+            got = run_chain(A, B, C, dtype, inter, scale, b_layout, "float32", variant)
+            assert np.isfinite(got).all()
+            mx, rel = errors(got, want)
+            bound = REL_L2 if inter != "softmax" or dtype == "float16" else 2.0e-3  # bf16: the probabilities' own rounding
+            assert rel <= bound and mx <= 4e-2, (variant, b_layout, mx, rel)
+            narrow = run_chain(A, B, C, dtype, inter, scale, b_layout, dtype, variant)
+            assert np.array_equal(narrow, oracle.np_round_to(got, dtype)), (variant, b_layout)
+
+
 @pytest.mark.parametrize("shape", [(1, 512, 64, 64, 64), (3, 100, 24, 40, 72), (2, 64, 128, 128, 200)])
 @pytest.mark.parametrize("inter", ["cast", "relu", "softmax"])
 def test_fp32_chain_vs_oracle(oracle, shape, inter):
