@@ -419,6 +419,7 @@ struct ConvPlan {
   ditto::ConvRowsArgs cvargs;
   bool tiles;          // dense -> 1x1 on tiles of whole output rows (targs), both weights as fragments in the workspace
   ditto::ConvTilesArgs targs;
+  ditto::DwTilesArgs dwtargs;
   ditto_tile_param tile;
 };
 
@@ -433,6 +434,7 @@ struct ConvPlan {
 // dw_mode 5: the row-streaming kernel for multiplier 16 (dw16_rows.h): 3x3, pad 1, stride 1, an even number of at
 // most 32 input channels, at most 64 output channels, image rows of whole 16-byte vectors whose ring of row slots
 // fits beside the filters in LDS, 16-bit output.  DITTO_DW16_ROWS=0 keeps such shapes on the persistent kernel.
+// dw_mode 6: tiles of whole output rows (dwtargs).
 // What a forced tile_variant allows (0: everything; see ditto_conv_chain_desc.tile_variant).
 struct ConvSteer {
   int tv = 0;
@@ -441,6 +443,7 @@ struct ConvSteer {
   bool dw_rows = true;   // 4024
   bool dw16_rows = true; // 4025
   bool tiles = true;     // 3200: tiles of whole output rows
+  bool dw_tiles = true;  // 4100: depthwise, tiles of whole output rows
   bool persist = false;  // 3900: the persistent 3x3 -> 1x1 kernel (switched off)
 };
 int conv_steer(int tv, ConvSteer* st) {
@@ -454,8 +457,10 @@ int conv_steer(int tv, ConvSteer* st) {
   st->tiles = fam == 3200;
   st->dw_rows = tv == 4024;
   st->dw16_rows = tv == 4025;
+  st->dw_tiles = fam == 4100;
   st->persist = fam == 3900;
-  if (!(fam == 3000 || fam == 3100 || fam == 3200 || fam == 3500 || fam == 3600 || fam == 3700 || fam == 3800 || fam == 3900 || fam == 4000))
+  if (!(fam == 3000 || fam == 3100 || fam == 3200 || fam == 3500 || fam == 3600 || fam == 3700 || fam == 3800 || fam == 3900 || fam == 4000 ||
+        fam == 4100))
     return fail(DITTO_EINVAL, "tile_variant %d names no conv chain kernel family", tv);
   return DITTO_OK;
 }
@@ -471,6 +476,57 @@ int conv_steer_check(const ConvSteer& st, int got) {
   }
   return fail(DITTO_EINVAL, "tile_variant %d cannot run this chain (the kernel that fits it under that constraint is %d)",
               st.tv, got);
+}
+
+// Depthwise 3x3 on tiles of whole output rows (dw_tiles.h), where it can run the shape at all.
+bool plan_dw_tiles(const ditto_conv_chain_desc* d, long long P, long long Q, ConvPlan* plan, int cus) {
+  const int mult = (int)(d->C1 / d->C0), slots = 16 * ditto::kDtMaxTiles;
+  if (!(mult == 16 || mult == 1) || d->R1 != 3 || d->S1 != 3 || d->pad1 != 1 || d->C2 > 64 || d->W < 8 || Q > slots ||
+      (mult == 1 && d->C0 % 8) || d->C0 * d->H * d->W > 0x3fffffff)
+    return false;
+  auto rows_in = [&](int th) { return (int)((th - 1) * d->stride1 + 3); };
+  auto lds_of = [&](int th) { return ditto::dw_tiles_lds_bytes(mult, rows_in(th), (int)d->W, d->C2 <= 32 ? 2 : 4); };
+  if (lds_of(1) > 160 * 1024) return false;
+  // Rows per workgroup.  A workgroup of one pixel tile per wave takes two units alone on a compute unit and three (multiplier
+  // 1: 2.6) beside another, one of two tiles 3 and 4.6 (5.2); a compute unit holds two.  The height with the fewest units on
+  // the busiest compute unit wins, the smaller one on ties (32 x 64 x 56 x 56 times 16: one row 63 us, two 38, four 29.5;
+  // times 1: 22, 16.2, 18.3).
+  int th = 1;
+  double best = 0;
+  for (int t = 1; t <= P && t * Q <= slots && lds_of(t) <= 160 * 1024; ++t) {
+    const bool two = t * Q > 16 * ditto::kDtWaves;
+    const double alone = two ? 3 : 2, pair = mult == 16 ? (two ? 4.6 : 3) : (two ? 5.2 : 2.6);
+    const long long wgs = d->N * ((P + t - 1) / t), per_round = 2LL * lds_of(t) <= 160 * 1024 ? 2 * cus : cus;
+    const long long full = wgs / per_round, rest = wgs % per_round;
+    const double cost = full * (per_round > cus ? pair : alone) + (rest > cus ? pair : rest > 0 ? alone : 0);
+    if (t == 1 || cost < best) best = cost, th = t;
+  }
+  ditto::DwTilesArgs& a = plan->dwtargs;
+  a.N = (int)d->N; a.C0 = (int)d->C0; a.H = (int)d->H; a.W = (int)d->W; a.C2 = (int)d->C2;
+  a.P = (int)P; a.Q = (int)Q; a.stride = (int)d->stride1;
+  a.TH = th;
+  a.tiles_h = (int)((P + th - 1) / th);
+  a.rows_in = rows_in(th);
+  a.relu_mid = d->inter_op == DITTO_INTER_RELU;
+  a.relu_out = d->relu_out != 0;
+  a.out_f32 = d->out_dtype == DITTO_F32;
+  a.inv_blocks = 1.f / (float)ditto::dw_tiles_row_blocks((int)d->W);
+  a.inv_rows = 1.f / (float)a.rows_in;
+  a.inv_group = 1.f / (float)ditto::dw_tiles_group_blocks(a.rows_in, (int)d->W);
+  a.inv_q = 1.f / (float)Q;
+  plan->dw_mode = 6;
+  ditto_tile_param& t = plan->tile;
+  t.block_threads = 64 * ditto::kDtWaves;
+  t.block_m = th * (int)Q;
+  t.block_l = ditto::dw_tiles_chunk(mult) * mult;
+  t.block_n = d->C2 <= 32 ? 32 : 64;
+  t.head_pad = 0;
+  t.lds_bytes = lds_of(th);
+  t.grid_x = a.N * a.tiles_h;
+  t.grid_y = th;
+  t.grid_z = (int)Q;
+  t.variant = 4100 + th;
+  return true;
 }
 
 int plan_dw_conv(const ditto_conv_chain_desc* d, const ConvSteer& steer, long long P, long long Q, ConvPlan* plan,
@@ -536,11 +592,11 @@ int plan_dw_conv(const ditto_conv_chain_desc* d, const ConvSteer& steer, long lo
       return DITTO_OK;
     }
   }
-  if (allow_rows && vec_cap >= 8 && steer.dw16_rows && mult == 16 && d->R1 == 3 && d->S1 == 3 && d->pad1 == 1 &&
-      d->stride1 == 1 && d->C0 <= 32 && d->C0 % 2 == 0 && d->C2 <= 64 && d->W % 8 == 0 && d->W >= 8 &&
-      ditto::dw16_rows_ni((int)d->C0, (int)d->W) <= 8 &&
-      ditto::dw16_rows_lds_bytes((int)d->C0, (int)d->W) <= 160 * 1024 && d->out_dtype != DITTO_F32 &&
-      d->H * d->W < (1 << 20)) {
+  const bool rows16 = mult == 16 && d->R1 == 3 && d->S1 == 3 && d->pad1 == 1 && d->stride1 == 1 && d->C0 <= 32 &&
+                      d->C0 % 2 == 0 && d->C2 <= 64 && d->W % 8 == 0 && d->W >= 8 &&
+                      ditto::dw16_rows_ni((int)d->C0, (int)d->W) <= 8 &&
+                      ditto::dw16_rows_lds_bytes((int)d->C0, (int)d->W) <= 160 * 1024 && d->H * d->W < (1 << 20);
+  if (allow_rows && vec_cap >= 8 && steer.dw16_rows && rows16 && d->out_dtype != DITTO_F32) {
     // Bands of whole output rows, one workgroup each, whose pixels eight waves take as one stream of 32-pixel
     // tiles: the band height with the fewest tiles on the busiest SIMD (waves w and w + 4 share one) over
     // the rounds of workgroups, a workgroup's start-up counted as three tiles.
@@ -579,6 +635,12 @@ int plan_dw_conv(const ditto_conv_chain_desc* d, const ConvSteer& steer, long lo
     t.variant = 4000 + 20 + 5;
     return DITTO_OK;
   }
+  // Tiles of whole output rows: what the two row-streaming kernels do not take (they keep all weights in LDS: 8 x 32 x 56 x
+  // 56 times 16 7.6 us against 8.9, 32 x 32 x 56 x 56 times 1 7.8 / 12.5), 1.3 to 7 times the kernels below: 32 x 64 x 56 x 56
+  // times 16 -> 64 52.5 / 29.5 us, 8 x 32 x 37 x 37 times 16 25.6 / 9.1, 32 x 16 x 147 x 147 times 16 stride 2 127 / 19, 32 x
+  // 64 x 112 x 112 times 1 73 / 48.  (The fp32 output of a shape the second one takes stays below, whose order of
+  // accumulation is that kernel's.)
+  if (steer.dw_tiles && (!rows16 || steer.tv > 0) && plan_dw_tiles(d, P, Q, plan, need_device ? device_cus() : 256)) return DITTO_OK;
   plan->dw_mode = dwv ? 3 : mfma ? 2 : mult % 8 == 0 ? 1 : 0;
   const int c2t = d->C2 <= 32 ? 1 : d->C2 <= 64 ? 2 : d->C2 <= 128 ? 4 : 8;
   const int pxw = mfma ? ditto::dw_mfma_pxw(c2t) : c2t == 8 ? 1 : 2;
@@ -1413,6 +1475,21 @@ int conv_chain_call(int phase, const ditto_conv_chain_desc* d, const void* x, co
               : ditto::pack_conv_w2_resident_bf16(w2, workspace, r.C1, r.C2, st);
     if (e == hipSuccess && (phase & kConvCompute))
       e = f16 ? ditto::launch_conv_resident_f16(r, plan.res_grid, st) : ditto::launch_conv_resident_bf16(r, plan.res_grid, st);
+    if (e != hipSuccess) return fail(DITTO_EHIP, "kernel launch failed: %s", hipGetErrorString(e));
+    return DITTO_OK;
+  }
+  if (plan.dw && plan.dw_mode == 6) {  // x, weights and y at any element
+    if (!(phase & kConvCompute)) return DITTO_OK;
+    ditto::DwTilesArgs r = plan.dwtargs;
+    if (!aligned(x, 2) || !aligned(w1, 2) || !aligned(w2, 2) || !aligned(y, r.out_f32 ? 4 : 2))
+      return fail(DITTO_EINVAL, "misaligned data pointer");
+    r.x = x;
+    r.w1 = w1;
+    r.w2 = w2;
+    r.y = y;
+    hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+    const int mult = (int)(d->C1 / d->C0);
+    hipError_t e = d->in_dtype == DITTO_F16 ? ditto::launch_dw_tiles_f16(mult, r, st) : ditto::launch_dw_tiles_bf16(mult, r, st);
     if (e != hipSuccess) return fail(DITTO_EHIP, "kernel launch failed: %s", hipGetErrorString(e));
     return DITTO_OK;
   }

@@ -10,6 +10,7 @@
 #include "dw_conv_chain.h"
 #include "dw_rows.h"
 #include "dw16_rows.h"
+#include "dw_tiles.h"
 #include "gemm_chain_f32.h"
 #include "gemm_chain_i8.h"
 
@@ -50,6 +51,9 @@ hipError_t launch_conv_tiles_f16(const ConvTilesArgs& args, hipStream_t stream);
 hipError_t launch_conv_tiles_bf16(const ConvTilesArgs& args, hipStream_t stream);
 hipError_t pack_conv_tiles_f16(const ConvTilesArgs& args, const void* w1, const void* w2, void* w1f, void* w2f, hipStream_t stream);
 hipError_t pack_conv_tiles_bf16(const ConvTilesArgs& args, const void* w1, const void* w2, void* w1f, void* w2f, hipStream_t stream);
+// depthwise 3x3 -> 1x1 on tiles of whole output rows (dw_tiles.h); mult 1 or 16
+hipError_t launch_dw_tiles_f16(int mult, const DwTilesArgs& args, hipStream_t stream);
+hipError_t launch_dw_tiles_bf16(int mult, const DwTilesArgs& args, hipStream_t stream);
 // depthwise first convolution (dw_conv_chain.h); c2_tiles in {1, 2, 4, 8}; mode 0 | 1: plain kernel,
 // vector-ALU depthwise stage (1: multiplier a multiple of 8); 2: persistent kernel, MFMA depthwise
 // stage (multiplier a multiple of 16); 3: persistent kernel, vector-ALU stage (3x3, multiplier 1, 2, 4, 8)

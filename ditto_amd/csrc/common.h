@@ -253,4 +253,9 @@ __device__ __forceinline__ unsigned xcd_remap(unsigned bid, unsigned nblk) {
   return (bid % NX) * (nblk / NX) + bid / NX;
 }
 
+// n / d for 0 <= n < 2^21 and inv = 1 / d: the half keeps the product inside the quotient's interval whatever its
+// rounding.  (An integer division by a run-time value is some thirty instructions, and a workgroup's start is a chain of
+// them.)
+__device__ __forceinline__ int div_by(int n, float inv) { return (int)(((float)n + 0.5f) * inv); }
+
 }  // namespace ditto

@@ -42,11 +42,6 @@ struct ConvTilesArgs {
   float inv_cg, inv_ng, inv_q;  // 1 / (c0p / 8), 1 / ceil(W / 8), 1 / Q
 };
 
-// n / d for 0 <= n < 2^21 and inv = 1 / d: the half keeps the product inside the quotient's interval whatever its
-// rounding.  (An integer division by a run-time value is some thirty instructions, and a workgroup's start is a chain of
-// them.)
-__device__ __forceinline__ int div_by(int n, float inv) { return (int)(((float)n + 0.5f) * inv); }
-
 template <int V>
 struct CtInt {
   static constexpr int value = V;

@@ -136,6 +136,7 @@ typedef struct ditto_conv_chain_desc {
                               3700 conv3x3 -> conv1x1 row pipeline        3800 conv1x1 -> conv3x3 row pipeline
                               4000 depthwise -> conv1x1, tile kernels (40xx = 4000 + 10 * output tiles + mode)
                               4024 / 4025 depthwise row-streaming kernels (multiplier 1 / 16)
+                              4100 depthwise 3x3 (multiplier 1 or 16) on tiles of whole output rows
                             DITTO_EINVAL if that kernel cannot run the chain; with a forced kernel a call
                             whose pointers or workspace the kernel cannot take fails instead of falling
                             back to the general kernel */

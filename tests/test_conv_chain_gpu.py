@@ -962,3 +962,47 @@ def test_conv_chain_on_row_tiles(oracle, case, dtype):
     chain.run_conv_chain(x, w1, w2, y, desc=desc, workspace=ws, prepared=True)
     torch.cuda.synchronize()
     assert np.array_equal(y.float().cpu().numpy(), got) and bool(torch.isnan(out[0]))
+
+
+CASES_DW_TILES = [
+    # N, C0, H, W, factor, stride, C2: depthwise 3x3 on tiles of whole output rows
+    (1, 8, 9, 8, 1, 1, 8),         # the narrowest image, a quarter of a channel chunk, half an output tile
+    (2, 40, 7, 9, 1, 1, 40),       # a row's last 8-pixel block starts at W - 8; a second chunk of 8 channels
+    (2, 64, 37, 37, 1, 1, 64),     # odd rows, two chunks
+    (3, 24, 13, 130, 1, 1, 33),    # two tiles per wave, an odd number of output channels
+    (1, 32, 21, 227, 1, 4, 16),    # stride 4, more blocks than a thread prefetches
+    (1, 2, 5, 23, 16, 1, 8),       # one channel pair
+    (2, 17, 11, 28, 16, 1, 24),    # an odd channel in a second chunk
+    (1, 48, 9, 256, 16, 1, 64),    # the longest output row
+    (5, 16, 31, 57, 16, 2, 32),    # stride 2 on odd rows
+    (1, 64, 6, 15, 16, 1, 40),     # four chunks, fewer rows than a tile takes
+]
+
+
+@pytest.mark.parametrize("case", CASES_DW_TILES)
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+def test_depthwise_chain_on_row_tiles(oracle, case, dtype):
+    N, C0, H, W, factor, stride, C2 = case
+    C1 = C0 * factor
+    rng = np.random.default_rng(C0 + C2 + W)
+    X = oracle.np_round_to(rng.standard_normal((N, C0, H, W)).astype(np.float32), dtype)
+    W1 = oracle.np_round_to(rng.standard_normal((C1, 1, 3, 3)).astype(np.float32) * 0.3, dtype)
+    W2 = oracle.np_round_to(rng.standard_normal((C2, C1, 1, 1)).astype(np.float32) * 0.02, dtype)
+    for relu in (False, True):
+        inter = "relu" if relu else "cast"
+        want = oracle.conv_chain_f32(X, W1, W2, 1, stride, 0, 1, relu_mid=relu, relu_out=relu, round_mid=dtype, groups1=C0)
+        got32 = run_conv(X, W1, W2, dtype, 1, stride, inter, relu, out_dtype="float32", groups1=C0, tile_variant=4100)
+        got = run_conv(X, W1, W2, dtype, 1, stride, inter, relu, groups1=C0, tile_variant=4100)
+        assert np.isfinite(got).all()
+        mx, rel = errors(got32, want)
+        assert mx <= MAX_ABS and rel <= REL_L2, (relu, mx, rel)
+        assert np.array_equal(got, oracle.np_round_to(got32, dtype)), relu
+    # tensors at any element's address
+    flat = to_dev(np.concatenate([np.zeros(1, np.float32), X.ravel()]), dtype)
+    x, w1, w2 = flat[1:].view(N, C0, H, W), to_dev(W1, dtype), to_dev(W2, dtype)
+    out = torch.full((got.size + 1,), float("nan"), device=x.device, dtype=x.dtype)
+    y = out[1:].view(got.shape)
+    desc = chain.conv_chain_desc(x, w1, w2, y, 1, stride, 0, 1, "relu", True, C0, tile_variant=4100)
+    chain.run_conv_chain(x, w1, w2, y, desc=desc)
+    torch.cuda.synchronize()
+    assert np.array_equal(y.float().cpu().numpy(), got) and bool(torch.isnan(out[0]))
