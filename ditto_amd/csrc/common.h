@@ -244,13 +244,13 @@ __device__ __forceinline__ void store_tile_rows(const char* tw, T* f0, long long
   }
 }
 
-// Workgroups are dealt round-robin to the 8 XCDs (each with a private L2) by
-// linear id.  Remap so that ids that are neighbours in the logical order (and
-// share operands) land on the same XCD.
+// Workgroups are dealt round-robin to the 8 XCDs (each with a private L2) by linear id.  Remap so that ids that are
+// neighbours in the logical order (and share operands) land on the same XCD; the first nblk % 8 XCDs take one more.
+// (Grids that are no multiple of 8 went round-robin before: 139 heads of 384 x 384 x 64 16.6 us against 10.7, 255 of 303 x 1910
+// 90 against 50, each key tile fetched from memory by as many XCDs as its head has row blocks.)
 __device__ __forceinline__ unsigned xcd_remap(unsigned bid, unsigned nblk) {
-  const unsigned NX = 8;
-  if (nblk % NX != 0) return bid;
-  return (bid % NX) * (nblk / NX) + bid / NX;
+  const unsigned x = bid & 7, r = nblk & 7;
+  return x * (nblk >> 3) + (x < r ? x : r) + (bid >> 3);
 }
 
 // n / d for 0 <= n < 2^21 and inv = 1 / d: the half keeps the product inside the quotient's interval whatever its
