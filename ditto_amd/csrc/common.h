@@ -239,7 +239,10 @@ __device__ __forceinline__ void store_tile_rows(const char* tw, T* f0, long long
     const V8 x = *reinterpret_cast<const V8*>(tw + r * tile_row_bytes<D>() + ch * 16);
     if (r < rows_valid && 8 * ch < N) {
       V8* const dst = reinterpret_cast<V8*>(f0 + (long long)r * f_rs + 8 * ch);
-      asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1" ::"v"(dst), "v"(x) : "memory");
+      // The store reads its four data registers after it has issued: the vector ALU may not write them for two wait states,
+      // which the compiler keeps behind its own stores but not behind one it cannot see into (a workgroup of the 80-column
+      // kernel, one instruction short, stored row numbers in place of two columns now and then).
+      asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1\n\ts_nop 1" ::"v"(dst), "v"(x) : "memory");
     }
   }
 }

@@ -351,6 +351,29 @@ def test_row_kernels_use_no_scratch_and_wait_for_lds_before_every_barrier(tmp_pa
     assert barriers_with_lds_in_flight(text) == []
 
 
+def hidden_stores_without_wait_states(asm_text):
+    """Stores of more than 64 bits in inline assembly without two wait states behind them in the same block.  The store
+    reads its data registers after issuing; the compiler keeps the vector ALU off them behind its own stores only."""
+    blocks = re.findall(r";;#ASMSTART\n(.*?);;#ASMEND", asm_text, re.S)
+    stores = [b for b in blocks if re.search(r"_store_dwordx[34]\b", b)]
+    return len(stores), [b for b in stores if not re.search(r"_store_dwordx[34]\b[^\n]*\n\s*s_nop [1-9]", b)]
+
+
+def test_wide_stores_in_inline_assembly_keep_their_data_registers(tmp_path):
+    planted = "\t;;#ASMSTART\n\tglobal_store_dwordx4 v[8:9], v[4:7], off\n%s\t;;#ASMEND\n\tv_or_b32_e32 v4, 16, v2\n"
+    assert hidden_stores_without_wait_states(planted % "")[1] and not hidden_stores_without_wait_states(planted % "\ts_nop 1\n")[1]
+    hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+    if not os.path.exists(hipcc):
+        pytest.skip("hipcc not available")
+    unit = [u for u in build_ext.UNITS if u[0] == "fp_f16_cast"][0]
+    out = tmp_path / "unit.s"
+    flags = [f for f in build_ext.HIPCC_FLAGS if f != "-fPIC"]
+    subprocess.run([hipcc, *flags, "--cuda-device-only", "-S", *unit[2], os.path.join(CSRC, unit[1]), "-o", str(out)], check=True,
+                   capture_output=True)
+    stores, bare = hidden_stores_without_wait_states(out.read_text())
+    assert stores > 0 and not bare
+
+
 @pytest.mark.parametrize("unit_name", ["gemm_chain_i8", "gemm_chain_f32"])
 def test_no_barrier_with_lds_accesses_in_flight(tmp_path, unit_name):
     hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
