@@ -15,6 +15,7 @@
 #include "bmm_chain_fp8.h"
 #include "bmm_chain_fp8m16.h"
 #include "bmm_chain_fp4m16.h"
+#include "bmm_chain_rows.h"
 #include "bmm_chain_split.h"
 #include "chain_kernels.h"
 
@@ -49,6 +50,7 @@ struct BmmPlan {
   int family;  // 0: fp16/bf16 register-resident chain, 1: fp32 chain, 2: int8 requant chain
   int d_pad, qt;  // fp chains: head pad and rows-per-wave code; int8 chain: row tiles and ring depth
   int split_dt = 0, split_rt = 0;  // fp chains on few rows: column tiles and row tiles of the key-splitting kernel (0: none)
+  int rows_nw = 0;  // fp chains of head size 65 to 80: waves of a workgroup of the kernel padded to 80 columns (0: none)
   int nb3 = 0, nb = 0;  // 16x16x32-MFMA kernel: row blocks of 384 rows / row blocks in all, per batch entry
   ditto_tile_param tile;
 };
@@ -216,23 +218,41 @@ int plan_bmm(const ditto_bmm_chain_desc* d, BmmPlan* plan, bool need_device) {
       // rounds.  Fitted to measurements at head sizes 64, 80 and 128 (us per launch, other kernel -> this one, LK):
       // 16 x 176 x 176 x 80 8.4 -> 4.9, 8 x 461 x 461 x 80 12.7 -> 5.9, 16 x 512 x 512 x 80 12.4 -> 7.3 (32 rows),
       // 2 x 2392 x 2392 x 80 38.5 -> 13.1, 2 x 4096 x 4096 x 128 60.9 -> 28.4, 8 x 512 x 2048 x 64 17.5 -> 8.8; but
-      // 40 x 300 x 300 x 80 10.1 against 11.2 and 60 x 58 x 58 x 64 3.7 against 4.1, which stay.
+      // 40 x 300 x 300 x 80 8.4 against 11.2 and 60 x 58 x 58 x 64 3.7 against 4.1, which stay.
       const int dt = dmax <= 64 ? 4 : dmax <= 80 ? 5 : 8;
       const bool kl_b = d->b_layout == DITTO_B_KL;
       int rt = 0;
-      if (d->tile_variant == 0 && (plan->qt == 1 || plan->qt == 4 || plan->qt == 5)) {
+      if (d->tile_variant == 0 && (dt == 5 || plan->qt == 1 || plan->qt == 4 || plan->qt == 5)) {
         const double start[2] = {dt == 4 ? 1.2 : dt == 5 ? 2.0 : 3.0, dt == 4 ? 2.7 : dt == 5 ? 2.9 : 4.5};
         const double per_key[2] = {dt == 4 ? 0.0022 : dt == 5 ? 0.0028 : 0.0044, dt == 4 ? 0.0029 : dt == 5 ? 0.0033 : 0.0053};
         const long long n64 = ((d->M + 63) / 64) * d->batch, n128 = ((d->M + 127) / 128) * d->batch;
         double best = dt == 4 ? (0.55 + 0.0065 * d->L) * (n64 <= cus ? 1.0 : 0.8 * ((n64 + cus - 1) / cus))
                               : (sm ? 3.6 + 0.0134 * d->L : 3.2 + 0.0099 * d->L) * ((n128 + cus - 1) / cus);
         best *= 0.95;
+        if (dt == 5) {
+          // Head sizes 65 to 80: the kernel padded to 80 columns (bmm_chain_rows.h), four waves with 128-row workgroups, two to a
+          // compute unit, or eight with 256 rows.  It replaces the kernels padded to 128 but for chains without softmax of one
+          // round of 128-row workgroups and more than about 500 keys, where one wave per SIMD of 32x32x16 MFMAs is ahead
+          // (12 x 1600 x 1600 20.8 against 22.8).  Fitted like the above, us per launch beyond 2.2, other kernel -> four | eight
+          // waves, LK with softmax: 160 x 197 x 197 18.2 -> 9.6 | 9.1, 640 x 49 x 49 22.9 -> 8.8 | 12.0, 80 x 400 x 400
+          // 23.2 -> 13.4 | 12.9, 160 x 577 x 577 44.0 -> 33.8 | 34.3, 80 x 1024 x 1024 60.8 -> 41.3 | 50.8,
+          // 32 x 4096 x 4096 206 -> 191 | 187; the key-splitting kernel stays at 12 x 400 x 400 (7.1 against 9.9).
+          if (sm || plan->qt != 1) best = 1e30;
+          const double key = (sm ? 1.0 : 0.9) * (kl_b ? 1.07 : 1.0) * d->L;
+          for (int nw = 4; nw <= 8; nw += 4) {
+            const long long rounds = (((d->M + 32 * nw - 1) / (32 * nw)) * d->batch + cus - 1) / cus;
+            const double cost = nw == 4 ? (rounds == 1 ? 2.3 + 0.0131 * key : 2.1 + rounds * (1.1 + 0.0114 * key))
+                                        : (rounds == 1 ? 2.9 + 0.0196 * key : 2.1 + rounds * (2.8 + 0.0226 * key));
+            if (cost < best) best = cost, plan->rows_nw = nw;
+          }
+        }
         for (int r = 1; r <= 2; ++r) {
           const long long rounds = (((d->M + 16 * r - 1) / (16 * r)) * d->batch + cus - 1) / cus;
           const double cost = rounds * (start[r - 1] + per_key[r - 1] * d->L) * (!kl_b ? 1.0 : dt == 8 ? 1.3 : 1.15);
           if (cost < best) best = cost, rt = r;
         }
       }
+      if (dmax <= 80 && (d->tile_variant == 2154 || d->tile_variant == 2158)) plan->rows_nw = d->tile_variant % 10;
       if (d->tile_variant == 2001 + 10 * dt || d->tile_variant == 2002 + 10 * dt) rt = d->tile_variant % 10;
       if (rt > 0) {
         plan->split_dt = dt, plan->split_rt = rt;
@@ -247,6 +267,20 @@ int plan_bmm(const ditto_bmm_chain_desc* d, BmmPlan* plan, bool need_device) {
         t.grid_x = (int)(plan->nb * d->batch);
         t.grid_y = t.grid_z = 1;
         t.variant = 2000 + 10 * dt + rt;
+        return DITTO_OK;
+      }
+      if (plan->rows_nw > 0) {
+        plan->nb = (int)((d->M + 32 * plan->rows_nw - 1) / (32 * plan->rows_nw));
+        ditto_tile_param& t = plan->tile;
+        t.block_threads = 64 * plan->rows_nw;
+        t.block_m = 32 * plan->rows_nw;
+        t.block_l = ditto::kBN;
+        t.block_n = (int)d->N;
+        t.head_pad = 80;
+        t.lds_bytes = kl_b ? ditto::bmm_chain_rows_lds<5, true, 4>() : ditto::bmm_chain_rows_lds<5, false, 4>();  // (the same for eight waves)
+        t.grid_x = (int)(plan->nb * d->batch);
+        t.grid_y = t.grid_z = 1;
+        t.variant = 2150 + plan->rows_nw;
         return DITTO_OK;
       }
     }
@@ -1239,6 +1273,9 @@ int ditto_bmm_chain_run(const ditto_bmm_chain_desc* d, const void* a, const void
     if (plan.split_rt > 0)
       e = d->in_dtype == DITTO_F16 ? ditto::launch_split_f16(plan.split_dt, plan.split_rt, sm, kl, args, st)
                                    : ditto::launch_split_bf16(plan.split_dt, plan.split_rt, sm, kl, args, st);
+    else if (plan.rows_nw > 0)
+      e = d->in_dtype == DITTO_F16 ? ditto::launch_rows_f16(plan.rows_nw, sm, kl, args, st)
+                                   : ditto::launch_rows_bf16(plan.rows_nw, sm, kl, args, st);
     else if (d->in_dtype == DITTO_F16)
       e = sm ? ditto::launch_f16_softmax(plan.d_pad, plan.qt, kl, args, st)
              : ditto::launch_f16_cast(plan.d_pad, plan.qt, kl, args, st);

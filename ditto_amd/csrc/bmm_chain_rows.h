@@ -1,0 +1,364 @@
+// Fused two-contraction chain  F = epilogue(inter(A.B).C)  for fp16 / bf16 with head sizes that fill neither 64 nor 128
+// columns: K and N are padded to 80.  (See bmm_chain_fp.h for the chain and the transposed formulation, bmm_chain_fp8m16.h for
+// the operand layouts of v_mfma_f32_16x16x32 and the hand-over between the contractions.)
+//
+// The kernels padded to 128 columns spend 1.6 times the matrix instructions, LDS traffic and LDS on a head of 80, and start
+// slowly: 197 keys were two to three of their steps of a pipeline several steps deep.  Here a wave owns 32 rows (every LDS
+// fragment feeds two MFMAs), four or eight waves share a ring of three 24 KB tiles of 64 keys, and two workgroups fit a compute
+// unit, one loading while the other computes.  A last tile of at most 32 keys costs half a step, a wave without rows only its
+// share of the loads.  Rows in LDS are padded to 13 and 10 16-byte chunks, which spreads both kinds of fragment reads over
+// all 64 banks without a swizzle (10-chunk rows: 16 lanes cover 4 rows x 32 bytes at banks 0, 40, 16, 56; 13-chunk rows:
+// strides of 52 banks), so all of a tile's fragment addresses are constants from two registers.
+//
+// Bound: matrix and vector pipes about evenly from a thousand keys on (32 x 4096 x 4096 187 us, 0.92 PFLOP/s counted without the
+// padding); below that the chain start -> first tile -> L / 64 steps of 0.85 us.  Measured, us per launch with softmax (2.4 of
+// them the launch), padded to 128 -> here, four | eight waves: 256 x 197 x 197 14.3 -> 10.6 | 10.3, 640 x 49 x 49
+// 22.9 -> 8.8 | 12.0, 80 x 400 x 400 23.2 -> 13.4 | 12.9, 96 x 700 x 700 44.8 -> 28.7 | 35.9, 32 x 4096 x 4096 206 -> 191 | 187.
+#pragma once
+#include "bmm_chain_fp8m16.h"
+#include "common.h"
+
+namespace ditto {
+
+constexpr int kRowsRing = 3;
+
+// One tile of 64 keys in LDS: B, then C, filled by direct loads of 64 16-byte chunks each that are dealt to the waves in
+// order; rows are padded to chunk counts that spread the reads of 16 lanes over all banks, no swizzle.
+// DT: column tiles of 16 that K and N are padded to; the contraction over K runs in steps of 32.
+template <int DT, bool B_KL>
+struct RowsTiles {
+  static constexpr int KS = (DT + 1) / 2;
+  static constexpr int B_CPR = B_KL ? 8 : 4 * KS + 1;  // [64 l][32 KS k], or [32 KS k][64 l] with swizzled 128-byte rows
+  static constexpr int B_ROWS = B_KL ? 32 * KS : kBN;
+  static constexpr int C_CPR = DT == 8 ? 18 : 10;
+  static constexpr int B_LOADS = (B_ROWS * B_CPR + 63) / 64, C_LOADS = (kBN * C_CPR + 63) / 64;
+  static constexpr int C_OFF = B_LOADS * 1024;
+};
+template <int DT, bool B_KL, int NW>
+__host__ __device__ constexpr int bmm_chain_rows_tile_bytes() {
+  return (RowsTiles<DT, B_KL>::B_LOADS + RowsTiles<DT, B_KL>::C_LOADS + NW - 1) / NW * NW * 1024;
+}
+template <int DT, bool B_KL, int NW>
+__host__ __device__ constexpr int bmm_chain_rows_lds() {
+  return kRowsRing * bmm_chain_rows_tile_bytes<DT, B_KL, NW>() + 64;  // the tiles and the flag of the optimistic walk
+}
+
+template <typename T, int DT, int NW, int INTER, bool B_KL>
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) void bmm_chain_rows_kernel(BmmChainArgs p) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  typedef typename Elem<T>::v8 V8;
+  typedef typename Elem<T>::v4 V4;
+  typedef typename Elem<T>::v2 V2;
+  typedef RowsTiles<DT, B_KL> S;
+  constexpr int RT = 2, KS = S::KS, NR = kRowsRing;
+  constexpr int TB = bmm_chain_rows_tile_bytes<DT, B_KL, NW>(), NLD = TB / 1024 / NW;
+  constexpr bool kSoftmax = INTER == kInterSoftmax;
+  // a row's partial sum above which its reference exponent is raised
+  constexpr float kLimit = Elem<T>::is_bf16 ? kSumLimitBf16 : kSumLimitF16;
+  extern __shared__ __attribute__((aligned(1024))) char smem_rw[];
+  const int tid = threadIdx.x, lane = tid & 63, c = lane & 15, q = lane >> 4;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const unsigned lid = xcd_remap(blockIdx.x, gridDim.x);
+  const int bz = lid / (unsigned)p.mblocks, m0 = (lid - bz * (unsigned)p.mblocks) * (16 * RT * NW) + 16 * RT * w;
+  const int zo = bz / (unsigned)p.batch_inner, zi = bz - zo * p.batch_inner;
+  const T* __restrict__ Ag = reinterpret_cast<const T*>(p.a) + zo * p.a_bs2 + zi * p.a_bs;
+  const T* const Bg = reinterpret_cast<const T*>(p.b) + zo * p.b_bs2 + zi * p.b_bs;
+  const T* const Cg = reinterpret_cast<const T*>(p.c) + zo * p.c_bs2 + zi * p.c_bs;
+  const int M = p.M, N = p.N, K = p.K, L = p.L;
+  const bool busy = m0 < M;  // a wave without rows loads its share of the tiles and keeps the barriers
+
+  // A fragments (operand column = row of A); with B stored [K][L] in the contraction order its transposing reads give.
+  // Rows past M repeat the last one, columns past K are loaded from column 0 and replaced by zeros.
+  V8 af[RT][KS];
+#pragma unroll
+  for (int j = 0; j < RT; ++j) {
+    const T* const row = Ag + (long long)min(m0 + 16 * j + c, M - 1) * p.a_rs;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      if constexpr (B_KL) {
+        const int k = 32 * s + 4 * q;
+        const V4 lo = *reinterpret_cast<const V4*>(row + (k < K ? k : 0)), hi = *reinterpret_cast<const V4*>(row + (k + 16 < K ? k + 16 : 0));
+        const V4 none = {0, 0, 0, 0};
+        af[j][s] = concat4<V4, V8>(k < K ? lo : none, k + 16 < K ? hi : none);
+      } else {
+        const int k = 32 * s + 8 * q;
+        const V8 v = *reinterpret_cast<const V8*>(row + (k < K ? k : 0)), none = {0, 0, 0, 0, 0, 0, 0, 0};
+        af[j][s] = k < K ? v : none;
+      }
+    }
+  }
+
+  // the wave's direct loads of a tile: source offset of the lane's chunk, its first key within the tile (a key past L, like a
+  // chunk past K or N, is asked for out of range and reads as zero)
+  const int b_bytes = (int)((B_KL ? (long long)(K - 1) * p.b_rs + L : (long long)(L - 1) * p.b_rs + K) * 2);
+  const int c_bytes = (int)(((long long)(L - 1) * p.c_rs + N) * 2);
+  const i32x4 b_rsrc = make_rsrc(Bg, (unsigned)b_bytes), c_rsrc = make_rsrc(Cg, (unsigned)c_bytes);
+  constexpr int kNever = 0x7fffffff;
+  int voff[NLD], key[NLD];
+#pragma unroll
+  for (int i = 0; i < NLD; ++i) {
+    const int ld = NLD * w + i;
+    if (ld < S::B_LOADS) {
+      const int ch = 64 * ld + lane, row = ch / S::B_CPR, pc = ch - row * S::B_CPR;
+      const int lc = B_KL ? pc ^ (2 * ((row >> 1) & 3)) : pc;
+      const bool in = B_KL ? row < K : row < kBN && 8 * lc < K;
+      key[i] = !in ? kNever : B_KL ? 8 * lc : row;
+      voff[i] = (row * p.b_rs + 8 * lc) * 2;
+    } else {
+      const int ch = 64 * (ld - S::B_LOADS) + lane, row = ch / S::C_CPR, lc = ch - row * S::C_CPR;
+      key[i] = row < kBN && 8 * lc < N ? row : kNever;
+      voff[i] = (row * p.c_rs + 8 * lc) * 2;
+    }
+  }
+  const unsigned lds_wave = (unsigned)(size_t)(DITTO_LDS char*)smem_rw + 1024 * NLD * w;
+  auto load_tile = [&](int tile, int slot) __attribute__((always_inline)) {
+    const int bo = tile * (kBN * 2) * (B_KL ? 1 : p.b_rs), co = tile * (kBN * 2) * p.c_rs, left = L - tile * kBN;
+#pragma unroll
+    for (int i = 0; i < NLD; ++i) {
+      const bool is_b = NLD * w + i < S::B_LOADS;
+      const int vo = key[i] < left ? voff[i] + (is_b ? bo : co) : kNever;
+      lds_dma_16_at(is_b ? b_rsrc : c_rsrc, (unsigned)vo, lds_wave + slot * TB, 1024 * i);
+    }
+  };
+
+  // LDS read addresses: B fragment of key tile kt (16 keys), k step s; C^T fragment of 32-key half h, column tile j
+  const int tr_row = 4 * q + (c >> 2), tr_half = (c & 3) >> 1, tr_byte = 8 * (c & 1);
+  constexpr int NBA = B_KL ? 4 : 1;
+  int b_ad[NBA];
+#pragma unroll
+  for (int kt = 0; kt < NBA; ++kt)
+    b_ad[kt] = B_KL ? tr_row * 128 + (((2 * kt + tr_half) ^ (2 * ((tr_row >> 1) & 3))) * 16) + tr_byte : c * (S::B_CPR * 16) + q * 16;
+  const int c_ad = tr_row * (S::C_CPR * 16) + tr_half * 16 + tr_byte + S::C_OFF;
+  auto b_frag = [&](const char* tile, int kt, int s) __attribute__((always_inline)) -> V8 {
+    if constexpr (B_KL) {
+      const char* const a = tile + b_ad[kt % NBA] + 32 * s * 128;
+      return concat4<V4, V8>(lds_read_tr4<T>(reinterpret_cast<const T*>(a)), lds_read_tr4<T>(reinterpret_cast<const T*>(a + 16 * 128)));
+    } else {
+      return *reinterpret_cast<const V8*>(tile + b_ad[0] + kt * 16 * (S::B_CPR * 16) + s * 64);
+    }
+  };
+  auto c_frag = [&](const char* tile, int h, int j) __attribute__((always_inline)) -> V8 {
+    const char* const a = tile + c_ad + 32 * h * (S::C_CPR * 16) + j * 32;
+    return concat4<V4, V8>(lds_read_tr4<T>(reinterpret_cast<const T*>(a)),
+                           lds_read_tr4<T>(reinterpret_cast<const T*>(a + 16 * (S::C_CPR * 16))));
+  };
+
+  // the first tile's loads go out before the wait for A, which falls between the first and the second tile's
+  load_tile(0, 0);
+#pragma unroll
+  for (int j = 0; j < RT; ++j)
+#pragma unroll
+    for (int s = 0; s < KS; ++s) asm volatile("" : "+v"(af[j][s]));
+  load_tile(1, 1);
+
+  // accumulators of F^T: o[j][t][r] = F^T[16 t + 4 q + r][16 j + c]; ls: the row sums, by the matrix pipe against ones
+  f32x4 o[RT][DT], ls[RT];
+  float ref[RT];  // reference exponent of the lane's row (exp2 domain)
+  V8 ones;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) ones[e] = (T)1.0f;
+  asm volatile("" : "+v"(ones));
+  const float c2 = p.scale_log2;
+  const int ntiles = (L + kBN - 1) / kBN;
+  int* const flag = reinterpret_cast<int*>(smem_rw + NR * TB);
+
+  // One tile, its first NH halves of 32 keys (a last tile of at most 32 keys has one).
+  auto tile_step = [&](int it, const char* tile, auto nh_c, auto safe_c) __attribute__((always_inline)) {
+    constexpr int NH = decltype(nh_c)::value;
+    constexpr bool SAFE = decltype(safe_c)::value;
+    f32x4 s[RT][2 * NH];
+#pragma unroll
+    for (int st = 0; st < KS; ++st)
+#pragma unroll
+      for (int kt = 0; kt < 2 * NH; ++kt) {
+        const V8 bf = b_frag(tile, kt, st);
+#pragma unroll
+        for (int j = 0; j < RT; ++j) s[j][kt] = Elem<T>::mfma16(bf, af[j][st], st == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : s[j][kt]);
+      }
+    if constexpr (kSoftmax) {
+      if (it * kBN + 32 * NH > L) {
+        const int left = L - it * kBN - 4 * q;  // keys left, counted from the lane's first
+#pragma unroll
+        for (int kt = 0; kt < 2 * NH; ++kt)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int gone = (left - (16 * kt + r) - 1) >> 31;
+#pragma unroll
+            for (int j = 0; j < RT; ++j) s[j][kt][r] = neg_inf_where(s[j][kt][r], gone);
+          }
+      }
+      if (SAFE || it == 0) {
+        float mx[RT];
+        bool raise = it == 0;
+#pragma unroll
+        for (int j = 0; j < RT; ++j) {
+          mx[j] = s[j][0][0];
+#pragma unroll
+          for (int kt = 0; kt < 2 * NH; ++kt)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) mx[j] = fmaxf(mx[j], s[j][kt][r]);
+          mx[j] *= c2;
+          raise = raise || mx[j] > ref[j] + kLazy;
+        }
+        if (__builtin_amdgcn_ballot_w64(raise) != 0) {
+          // the first tile sets the reference (nothing is accumulated yet); in the exact walk it then follows the running
+          // maximum, lazily
+#pragma unroll
+          for (int j = 0; j < RT; ++j) {
+            const float m = quad_max(mx[j]);
+            const float up = it == 0 ? m : fmaxf(ref[j], m);
+            const float alpha = it == 0 ? 1.f : __builtin_amdgcn_exp2f(ref[j] - up);
+            ref[j] = up;
+            ls[j] *= alpha;
+#pragma unroll
+            for (int t = 0; t < DT; ++t) o[j][t] *= alpha;
+          }
+        }
+      }
+    }
+#pragma unroll
+    for (int h = 0; h < NH; ++h) {
+      // element e of the operand is key 4 q + e of the half's first 16 (e < 4) or of its second; the sum is taken over the
+      // rounded values, exactly what enters the product
+      V8 pf[RT];
+#pragma unroll
+      for (int j = 0; j < RT; ++j) {
+#pragma unroll
+        for (int e = 0; e < 8; e += 2) {
+          float x = s[j][2 * h + (e >> 2)][e & 3], y = s[j][2 * h + (e >> 2)][(e & 3) + 1];
+          if constexpr (kSoftmax) {
+            x = __builtin_amdgcn_exp2f(__builtin_fmaf(x, c2, -ref[j]));
+            y = __builtin_amdgcn_exp2f(__builtin_fmaf(y, c2, -ref[j]));
+          } else if (p.relu) {
+            x = fmaxf(x, 0.f);
+            y = fmaxf(y, 0.f);
+          }
+          const V2 two = cvt2<T>(x, y);
+          pf[j][e] = two[0];
+          pf[j][e + 1] = two[1];
+        }
+        if constexpr (kSoftmax) ls[j] = Elem<T>::mfma16(ones, pf[j], ls[j]);
+      }
+#pragma unroll
+      for (int t = 0; t < DT; ++t) {
+        const V8 cf = c_frag(tile, h, t);
+#pragma unroll
+        for (int j = 0; j < RT; ++j) o[j][t] = Elem<T>::mfma16(cf, pf[j], o[j][t]);
+      }
+    }
+    if constexpr (kSoftmax && !SAFE) {
+      // optimistic walk: once per tile, lower the scale of a row whose sum has passed the limit (an infinite or NaN sum is
+      // left as it is: that is what the end of the walk looks for)
+      if (__builtin_amdgcn_ballot_w64(fmaxf(ls[0][0], ls[1][0]) > kLimit) != 0) {
+#pragma unroll
+        for (int j = 0; j < RT; ++j) {
+          const float sum = ls[j][0];
+          const int e = (sum > kLimit && sum < INFINITY) ? ((__builtin_bit_cast(int, sum) >> 23) & 255) - 127 : 0;
+          const float alpha = __builtin_bit_cast(float, (127 - e) << 23);  // 2^-e, exact
+          ref[j] += (float)e;
+          ls[j] *= alpha;
+#pragma unroll
+          for (int t = 0; t < DT; ++t) o[j][t] *= alpha;
+        }
+      }
+    }
+  };
+
+  // (tiles 0 and 1 are in flight: issued by the caller)
+  auto walk = [&](auto safe_c) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < RT; ++j) {
+      ref[j] = 0.f;
+      ls[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int t = 0; t < DT; ++t) o[j][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    int slot = 0;
+    for (int it = 0; it < ntiles; ++it) {
+      // tile `it` has landed (the next one's loads may stay in flight) and every wave is done with tile it - 1, whose slot
+      // the loads below fill
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NLD) : "memory");
+      wg_sync();
+      load_tile(it + 2, slot == 0 ? 2 : slot - 1);  // a tile past the last one: zeros
+      const char* const tile = smem_rw + slot * TB;
+      if (busy) {
+        if (it * kBN + 32 < L) tile_step(it, tile, IntC<2>{}, safe_c);
+        else tile_step(it, tile, IntC<1>{}, safe_c);
+      }
+      slot = slot == 2 ? 0 : slot + 1;
+    }
+    // no direct load still on its way into LDS, every wave done with the tiles
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if constexpr (kSoftmax && !decltype(safe_c)::value) {
+      // a sum that is not finite sends the workgroup through the exact walk (the tiles are its common property)
+      const bool bad = busy && (!(ls[0][0] < INFINITY) || !(ls[1][0] < INFINITY));
+      if (__builtin_amdgcn_ballot_w64(bad) != 0 && lane == 0) *flag = 1;
+    }
+    wg_sync();
+  };
+  if (tid == 0) *flag = 0;
+  walk(BoolC<false>{});
+  if constexpr (kSoftmax) {
+    if (__builtin_amdgcn_readfirstlane(*flag)) {
+      load_tile(0, 0);
+      load_tile(1, 1);
+      walk(BoolC<true>{});
+    }
+  }
+  if (!busy) return;
+
+  // ---- normalise (softmax), cast, store the wave's 32 rows: 16-bit rows of whole 16-byte vectors through LDS (see
+  // store_tile_rows), else 4 columns per lane from registers
+  const bool by_rows = !p.out_f32 && (N & 7) == 0 && (p.f_rs & 7) == 0 && (p.f_bs & 7) == 0 && (p.f_bs2 & 7) == 0 &&
+                       (reinterpret_cast<size_t>(p.f) & 15) == 0;  // wave-uniform
+  constexpr int D = 16 * DT, kRowBytes = tile_row_bytes<D>();
+  static_assert(NW * 16 * RT * kRowBytes <= NR * TB, "the parked rows need the staged tiles' LDS");
+  static_assert(16 * RT * D / 8 % 64 == 0, "whole waves of 16-byte stores");
+  char* const tw = smem_rw + w * (16 * RT * kRowBytes);
+  const long long f0 = zo * p.f_bs2 + zi * p.f_bs + (long long)m0 * p.f_rs;
+#pragma unroll
+  for (int j = 0; j < RT; ++j) {
+    const float inv = kSoftmax ? 1.f / ls[j][0] : 1.f;
+    if (!by_rows && m0 + 16 * j + c >= M) continue;
+#pragma unroll
+    for (int t = 0; t < DT; ++t) {
+      const int n = 16 * t + 4 * q;
+      f32x4 x = o[j][t] * inv;
+      if (!kSoftmax && p.relu_out)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) x[r] = fmaxf(x[r], 0.f);
+      const V2 lo = cvt2<T>(x[0], x[1]), hi = cvt2<T>(x[2], x[3]);
+      const V4 v = {lo[0], lo[1], hi[0], hi[1]};
+      if (by_rows) {
+        *reinterpret_cast<V4*>(tw + (16 * j + c) * kRowBytes + n * 2) = v;
+      } else if (n < N) {
+        const long long at = f0 + (long long)(16 * j + c) * p.f_rs + n;
+        if (p.out_f32) *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(p.f) + at) = x;
+        else *reinterpret_cast<V4*>(reinterpret_cast<T*>(p.f) + at) = v;
+      }
+    }
+  }
+  if (by_rows) store_tile_rows<T, D, 16 * RT>(tw, reinterpret_cast<T*>(p.f) + f0, p.f_rs, M - m0, N, lane);
+#else
+  (void)p;
+#endif
+}
+
+template <typename T, int DT, int NW, int INTER, bool B_KL>
+hipError_t launch_bmm_chain_rows(const BmmChainArgs& args, hipStream_t stream) {
+  constexpr int lds = bmm_chain_rows_lds<DT, B_KL, NW>();
+  auto kern = bmm_chain_rows_kernel<T, DT, NW, INTER, B_KL>;
+  static thread_local int configured_dev = -1;
+  int dev = 0;
+  hipError_t e = hipGetDevice(&dev);
+  if (e != hipSuccess) return e;
+  if (configured_dev != dev) {
+    e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    if (e != hipSuccess) return e;
+    configured_dev = dev;
+  }
+  hipLaunchKernelGGL(kern, dim3((unsigned)args.mblocks * (unsigned)args.batch), dim3(64 * NW), lds, stream, args);
+  return hipGetLastError();
+}
+
+}  // namespace ditto

@@ -26,6 +26,10 @@ hipError_t launch_bf16_softmax(int d_pad, int q, bool b_kl, const BmmChainArgs& 
 hipError_t launch_split_f16(int dt, int rt, bool softmax, bool b_kl, const BmmChainArgs& args, hipStream_t stream);
 hipError_t launch_split_bf16(int dt, int rt, bool softmax, bool b_kl, const BmmChainArgs& args, hipStream_t stream);
 
+// bmm_chain_rows_inst.hip, one object per element type: K and N padded to 80
+hipError_t launch_rows_f16(int nw, bool softmax, bool b_kl, const BmmChainArgs& args, hipStream_t stream);
+hipError_t launch_rows_bf16(int nw, bool softmax, bool b_kl, const BmmChainArgs& args, hipStream_t stream);
+
 // conv_chain_inst.hip, one object per element type; c1_tiles in {1, 2, 4, 8}
 // ch in {32, 16}: input channels per staged chunk
 hipError_t launch_conv_f16(int c1_tiles, int ch, const ConvChainArgs& args, hipStream_t stream);
