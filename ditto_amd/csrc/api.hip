@@ -453,6 +453,8 @@ struct ConvPlan {
   ditto::ConvRowsArgs cvargs;
   bool tiles;          // dense -> 1x1 on tiles of whole output rows (targs), both weights as fragments in the workspace
   ditto::ConvTilesArgs targs;
+  bool tiles13;        // 1x1 -> 3x3 with at most 64 channels on tiles of whole output rows (t13args), weights likewise
+  ditto::Conv13TilesArgs t13args;
   ditto::DwTilesArgs dwtargs;
   ditto_tile_param tile;
 };
@@ -477,6 +479,7 @@ struct ConvSteer {
   bool dw_rows = true;   // 4024
   bool dw16_rows = true; // 4025
   bool tiles = true;     // 3200: tiles of whole output rows
+  bool tiles13 = true;   // 3300: tiles of whole output rows, 1x1 -> 3x3
   bool dw_tiles = true;  // 4100: depthwise, tiles of whole output rows
   bool persist = false;  // 3900: the persistent 3x3 -> 1x1 kernel (switched off)
 };
@@ -489,11 +492,12 @@ int conv_steer(int tv, ConvSteer* st) {
   st->rows = fam == 3700 || fam == 3800;
   st->resident = fam == 3600;
   st->tiles = fam == 3200;
+  st->tiles13 = fam == 3300;
   st->dw_rows = tv == 4024;
   st->dw16_rows = tv == 4025;
   st->dw_tiles = fam == 4100;
   st->persist = fam == 3900;
-  if (!(fam == 3000 || fam == 3100 || fam == 3200 || fam == 3500 || fam == 3600 || fam == 3700 || fam == 3800 || fam == 3900 || fam == 4000 ||
+  if (!(fam == 3000 || fam == 3100 || fam == 3200 || fam == 3300 || fam == 3500 || fam == 3600 || fam == 3700 || fam == 3800 || fam == 3900 || fam == 4000 ||
         fam == 4100))
     return fail(DITTO_EINVAL, "tile_variant %d names no conv chain kernel family", tv);
   return DITTO_OK;
@@ -879,6 +883,58 @@ bool plan_conv_tiles(const ditto_conv_chain_desc* d, long long P, long long Q, b
   return true;
 }
 
+// 1x1 -> 3x3 with at most 64 channels on tiles of whole output rows (conv13_tiles.h), where that is the kernel for the shape
+// (`forced`: where it can run it at all).  The row pipeline comes before it (32 x 64 x 56 x 56 12.6 us against 14.3, 16 images
+// 8.6 / 8.9).  It is ahead of the persistent kernel with W2 in LDS on 16-bit outputs (8 x 64 x 112 x 112 20.3 -> 15.2,
+// 32 x 64 x 72 x 72 28.4 -> 21.6, 8 x 64 x 30 x 256 26.8 -> 11.8), which keeps the fp32 ones: here they leave in
+// pieces of 16 bytes.
+bool plan_conv13_tiles(const ditto_conv_chain_desc* d, bool forced, ConvPlan* plan, int cus) {
+  if (d->R1 != 1 || d->S1 != 1 || d->pad1 != 0 || d->stride1 != 1 || d->R2 != 3 || d->S2 != 3 || d->pad2 != 1 || d->stride2 != 1 ||
+      d->C0 > 64 || d->C1 > 64 || d->C2 > 64 || d->W < 8)
+    return false;
+  if (!forced && d->out_dtype == DITTO_F32 && d->C0 % 8 == 0 && d->W % 8 == 0) return false;
+  // Rows per workgroup, four waves (up to 128 pixels) or eight (256).  A workgroup alone on its compute unit takes a start, a
+  // share per halo pixel and one per pixel tile of a wave; a second and third beside it add two thirds of that with four
+  // waves, all of it with eight.  Fitted, us beyond the launch: one row of 56 pixels 3.0, of 112 5.7 (eight waves 5.0), two
+  // rows of 56 4.2, of 112 6.2 (eight waves).
+  int wp = 0, th = 0;
+  double best = 0;
+  for (int w = 2; w <= 4; w += 2)
+    for (int t = 1; t <= d->H && t * d->W <= ditto::conv13_tiles_slots(w); ++t) {
+      if (ditto::conv13_tiles_lds_bytes(t, (int)d->W, w) > 160 * 1024) break;
+      const long long wgs = d->N * ((d->H + t - 1) / t), rounds = (wgs + cus - 1) / cus, tiles = (t * d->W + 16 * w - 1) / (16 * w);
+      const double halo = (t + 2.0) * d->W;
+      const double one = w == 2 ? 1.7 + 0.3 * tiles + 0.0065 * halo : 2.6 + 0.45 * tiles + 0.004 * halo;
+      const double cost = one * (1.0 + (w == 2 ? 0.67 : 1.0) * (rounds - 1));
+      if (wp == 0 || cost < best) best = cost, wp = w, th = t;
+    }
+  if (wp == 0) return false;
+  ditto::Conv13TilesArgs& a = plan->t13args;
+  a.N = (int)d->N; a.C0 = (int)d->C0; a.H = (int)d->H; a.W = (int)d->W; a.C1 = (int)d->C1; a.C2 = (int)d->C2;
+  a.TH = th, a.wp = wp;
+  a.tiles_h = (int)((d->H + th - 1) / th);
+  a.c0p = d->C0 <= 32 ? 32 : 64;
+  a.relu_mid = d->inter_op == DITTO_INTER_RELU;
+  a.relu_out = d->relu_out != 0;
+  a.out_f32 = d->out_dtype == DITTO_F32;
+  a.inv_cg = 8.f / (float)a.c0p, a.inv_ng = 1.f / (float)((d->W + 7) / 8), a.inv_w = 1.f / (float)d->W;
+  plan->tiles13 = true;
+  plan->w1p_bytes = ditto::kC13W1Bytes;
+  plan->w2p_bytes = ditto::kC13W2Bytes;
+  ditto_tile_param& t = plan->tile;
+  t.block_threads = 128 * wp;
+  t.block_m = th * (int)d->W;
+  t.block_l = 64;
+  t.block_n = (int)d->C2;
+  t.head_pad = a.c0p;
+  t.lds_bytes = ditto::conv13_tiles_lds_bytes(th, (int)d->W, wp);
+  t.grid_x = a.N * a.tiles_h;
+  t.grid_y = th;
+  t.grid_z = (int)d->W;
+  t.variant = 3300 + (wp == 4 ? 50 : 0) + th;  // tiles of whole output rows, 1x1 -> 3x3; 50 more with eight waves; rows per workgroup
+  return true;
+}
+
 // allow_resident = false: the general kernels only (pointers the specialised ones cannot take);
 // allow_dw_rows: y takes 16-byte stores
 int plan_conv(const ditto_conv_chain_desc* d, ConvPlan* plan, bool need_device = false, int dw_vec_cap = 8,
@@ -1006,6 +1062,8 @@ int plan_conv_steered(const ditto_conv_chain_desc* d, const ConvSteer& steer, Co
         return DITTO_OK;
       }
     }
+    if (allow_resident && steer.tiles13 && plan_conv13_tiles(d, steer.tv / 100 == 33, plan, need_device ? device_cus() : 256))
+      return DITTO_OK;
     // 1x1 -> 3x3 (pad 1) with at most 64 channels everywhere and rows that are whole 16-byte vectors: the
     // persistent kernel that keeps W2 in LDS (conv_chain_resident.h), tiles of whole output rows
     if (allow_resident && steer.resident && s2 == 1 && d->R1 == 1 && d->S1 == 1 && d->pad1 == 0 && d->stride1 == 1 && d->R2 == 3 &&
@@ -1363,7 +1421,7 @@ size_t ditto_conv_chain_workspace_bytes(const ditto_conv_chain_desc* desc) {
   ConvPlan plan;
   if (plan_conv(desc, &plan, true) != DITTO_OK) return 0;
   size_t need = plan.w1p_bytes + plan.w2p_bytes;
-  if (plan.resident || plan.rows31 || plan.rows13 || plan.tiles) {
+  if (plan.resident || plan.rows31 || plan.rows13 || plan.tiles || plan.tiles13) {
     // a call with pointers these kernels cannot take falls back to the general one (tile_variant 0 only): the
     // larger of the two figures, whatever the device's compute-unit count makes of the choice
     ConvPlan general;
@@ -1462,7 +1520,7 @@ int conv_chain_call(int phase, const ditto_conv_chain_desc* d, const void* x, co
     if (e != hipSuccess) return fail(DITTO_EHIP, "kernel launch failed: %s", hipGetErrorString(e));
     return DITTO_OK;
   }
-  if (plan.tiles) {
+  if (plan.tiles || plan.tiles13) {
     // both weights as MFMA fragments in the workspace; x and y at any element
     const size_t need = plan.w1p_bytes + plan.w2p_bytes;
     const bool ok = workspace && workspace_bytes >= need && aligned(workspace, 16);
@@ -1491,6 +1549,24 @@ int conv_chain_call(int phase, const ditto_conv_chain_desc* d, const void* x, co
               : ditto::pack_conv_tiles_bf16(r, w1, w2, const_cast<void*>(r.w1f), const_cast<void*>(r.w2f), st);
     if (e == hipSuccess && (phase & kConvCompute))
       e = f16 ? ditto::launch_conv_tiles_f16(r, st) : ditto::launch_conv_tiles_bf16(r, st);
+    if (e != hipSuccess) return fail(DITTO_EHIP, "kernel launch failed: %s", hipGetErrorString(e));
+    return DITTO_OK;
+  }
+  if (plan.tiles13) {
+    ditto::Conv13TilesArgs r = plan.t13args;
+    if (!aligned(x, 2) || !aligned(y, r.out_f32 ? 4 : 2) || !aligned(w1, 2) || !aligned(w2, 2)) return fail(DITTO_EINVAL, "misaligned data pointer");
+    r.x = x;
+    r.w1f = workspace;
+    r.w2f = static_cast<char*>(workspace) + plan.w1p_bytes;
+    r.y = y;
+    hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+    const bool f16 = d->in_dtype == DITTO_F16;
+    hipError_t e = hipSuccess;
+    if (phase & kConvPrepare)
+      e = f16 ? ditto::pack_conv13_tiles_f16(r, w1, w2, const_cast<void*>(r.w1f), const_cast<void*>(r.w2f), st)
+              : ditto::pack_conv13_tiles_bf16(r, w1, w2, const_cast<void*>(r.w1f), const_cast<void*>(r.w2f), st);
+    if (e == hipSuccess && (phase & kConvCompute))
+      e = f16 ? ditto::launch_conv13_tiles_f16(r, st) : ditto::launch_conv13_tiles_bf16(r, st);
     if (e != hipSuccess) return fail(DITTO_EHIP, "kernel launch failed: %s", hipGetErrorString(e));
     return DITTO_OK;
   }

@@ -6,6 +6,7 @@
 #include "conv_chain.h"
 #include "conv_chain_resident.h"
 #include "conv_rows.h"
+#include "conv13_tiles.h"
 #include "conv_tiles.h"
 #include "dw_conv_chain.h"
 #include "dw_rows.h"
@@ -55,6 +56,11 @@ hipError_t launch_conv_tiles_f16(const ConvTilesArgs& args, hipStream_t stream);
 hipError_t launch_conv_tiles_bf16(const ConvTilesArgs& args, hipStream_t stream);
 hipError_t pack_conv_tiles_f16(const ConvTilesArgs& args, const void* w1, const void* w2, void* w1f, void* w2f, hipStream_t stream);
 hipError_t pack_conv_tiles_bf16(const ConvTilesArgs& args, const void* w1, const void* w2, void* w1f, void* w2f, hipStream_t stream);
+// conv 1x1 -> 3x3 with at most 64 channels on tiles of whole output rows (conv13_tiles.h)
+hipError_t launch_conv13_tiles_f16(const Conv13TilesArgs& args, hipStream_t stream);
+hipError_t launch_conv13_tiles_bf16(const Conv13TilesArgs& args, hipStream_t stream);
+hipError_t pack_conv13_tiles_f16(const Conv13TilesArgs& args, const void* w1, const void* w2, void* w1f, void* w2f, hipStream_t stream);
+hipError_t pack_conv13_tiles_bf16(const Conv13TilesArgs& args, const void* w1, const void* w2, void* w1f, void* w2f, hipStream_t stream);
 // depthwise 3x3 -> 1x1 on tiles of whole output rows (dw_tiles.h); mult 1 or 16
 hipError_t launch_dw_tiles_f16(int mult, const DwTilesArgs& args, hipStream_t stream);
 hipError_t launch_dw_tiles_bf16(int mult, const DwTilesArgs& args, hipStream_t stream);

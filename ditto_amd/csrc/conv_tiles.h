@@ -80,13 +80,70 @@ __global__ void pack_conv_fragments_kernel(ConvFragments w1, ConvFragments w2, u
       row < a.rows && col < a.cols ? static_cast<const T*>(a.w)[((long long)row * a.cols + col) * a.taps + tap] : (T)0.f;
 }
 
+// Halo rows of one image into LDS, channel fastest: [rows_in][cols_in][CHS], image column 0 at column `pad`.  A task is 8 pixels
+// x 8 channels of one image row: eight 16-byte loads (at element alignment: rows of any length), an 8x8 transposition in
+// registers, eight 16-byte writes.  The last group of a row starts at W - 8 and repeats pixels of the one before it.  Two
+// tasks of a thread are in flight together.  cg: groups of 8 channels staged; zg: groups zeroed in the columns left and right.
+template <int NT, typename T>
+__device__ __forceinline__ void stage_halo_rows(T* Xs, const T* Xg, int h0, int pad, int rows_in, int cols_in, int CHS, int cg, int zg,
+                                                int C0, int H, int W, float inv_cg, float inv_ng, int tid) {
+  typedef typename Elem<T>::v8 V8;
+  typedef __attribute__((ext_vector_type(8), aligned(2))) T V8u;  // 16 bytes at any element's address
+  const int row_step = cols_in * CHS, ng = (W + 7) / 8, tasks = rows_in * ng * cg;
+  const long long hw = (long long)H * W;
+  auto stage = [&](auto both, int t0) __attribute__((always_inline)) {
+    constexpr int U = decltype(both)::value;
+    i32x4 xr[U][8];
+    int col[U];
+    T* dst[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int t = t0 + u * NT, rest = div_by(t, inv_cg), ri = div_by(rest, inv_ng), chg = t - rest * cg;
+      const int w = min(8 * (rest - ri * ng), W - 8), h = h0 + ri;
+      col[u] = w + pad;
+      dst[u] = Xs + ri * row_step + (w + pad) * CHS + 8 * chg;
+      const bool live = t < tasks && h >= 0 && h < H;
+      const T* const src = Xg + (long long)(8 * chg) * hw + (long long)h * W + w;
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        i32x4 v = {0, 0, 0, 0};
+        if (live && 8 * chg + k < C0) v = __builtin_bit_cast(i32x4, (V8)*reinterpret_cast<const V8u*>(src + k * hw));
+        xr[u][k] = v;
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (t0 + u * NT >= tasks) break;
+#pragma unroll
+      for (int px = 0; px < 8; ++px) {
+        i32x4 o;
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+          o[k] = __builtin_amdgcn_perm(xr[u][2 * k + 1][px >> 1], xr[u][2 * k][px >> 1], (px & 1) ? 0x07060302 : 0x05040100);
+        if (col[u] + px < cols_in) *reinterpret_cast<i32x4*>(dst[u] + px * CHS) = o;
+      }
+    }
+  };
+  int t0 = tid;
+  for (; t0 - tid + NT < tasks; t0 += 2 * NT) stage(CtInt<2>(), t0);
+  if (t0 - tid < tasks) stage(CtInt<1>(), t0);
+  // the columns left and right of the image
+  const int right = max(0, cols_in - W - pad), nz = pad + right;
+  if (nz > 0) {
+    const float inv_nz = 1.f / (float)nz, inv_zg = zg == cg ? inv_cg : 1.f / (float)zg;
+    for (int t = tid; t < rows_in * nz * zg; t += NT) {
+      const int rest = div_by(t, inv_zg), chg = t - rest * zg, ri = div_by(rest, inv_nz), z = rest - ri * nz;
+      *reinterpret_cast<i32x4*>(Xs + ri * row_step + (z < pad ? z : W + z) * CHS + 8 * chg) = i32x4{0, 0, 0, 0};
+    }
+  }
+}
+
 // WC x WP waves: WC of them split the intermediate channels (MC tiles of 16 each), WP the pixels (PT tiles of 16 each).
 template <typename T, int WC, int WP, int MC, int PT>
 __global__ __launch_bounds__(64 * WC * WP) void conv_tiles_kernel(ConvTilesArgs p) {
 #if defined(__HIP_DEVICE_COMPILE__)
   typedef typename Elem<T>::v8 V8;
   typedef typename Elem<T>::v4 V4;
-  typedef __attribute__((ext_vector_type(8), aligned(2))) T V8u;  // 16 bytes at any element's address
   constexpr int NW = WC * WP, NT = 64 * NW, C1P = 16 * WC * MC, MS = conv_tiles_stride(C1P);
   constexpr int PO = WP * PT <= 2 ? 2 : WP * PT <= 4 ? 4 : 8;  // consecutive output pixels of a lane
   constexpr int D = NW == 8 ? 2 : 4;                 // W1 fragments in flight per tile
@@ -114,59 +171,9 @@ __global__ __launch_bounds__(64 * WC * WP) void conv_tiles_kernel(ConvTilesArgs 
 #pragma unroll
   for (int d = 0; d < D; ++d) load_w(d, d);
 
-  // ---- halo rows into LDS, channel fastest.  A task is 8 pixels x 8 channels of one image row: eight 16-byte loads (at
-  // element alignment: rows of any length), an 8x8 transposition in registers, eight 16-byte writes.  The last group of a
-  // row starts at W - 8 and repeats pixels of the one before it.  Two tasks of a thread are in flight together.
   const int row_step = p.cols_in * CHS;
-  {
-    const T* const Xg = reinterpret_cast<const T*>(p.x) + (long long)n * p.C0 * hw;
-    const int ng = (p.W + 7) / 8, tasks = p.rows_in * ng * cg;
-    auto stage = [&](auto both, int t0) __attribute__((always_inline)) {
-      constexpr int U = decltype(both)::value;
-      i32x4 xr[U][8];
-      int col[U];
-      T* dst[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int t = t0 + u * NT, rest = div_by(t, p.inv_cg), ri = div_by(rest, p.inv_ng), chg = t - rest * cg;
-        const int w = min(8 * (rest - ri * ng), p.W - 8), h = h0 + ri;
-        col[u] = w + p.pad;
-        dst[u] = Xs + ri * row_step + (w + p.pad) * CHS + 8 * chg;
-        const bool live = t < tasks && h >= 0 && h < p.H;
-        const T* const src = Xg + (long long)(8 * chg) * hw + (long long)h * p.W + w;
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {
-          i32x4 v = {0, 0, 0, 0};
-          if (live && 8 * chg + k < p.C0) v = __builtin_bit_cast(i32x4, (V8)*reinterpret_cast<const V8u*>(src + k * hw));
-          xr[u][k] = v;
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        if (t0 + u * NT >= tasks) break;
-#pragma unroll
-        for (int px = 0; px < 8; ++px) {
-          i32x4 o;
-#pragma unroll
-          for (int k = 0; k < 4; ++k)
-            o[k] = __builtin_amdgcn_perm(xr[u][2 * k + 1][px >> 1], xr[u][2 * k][px >> 1], (px & 1) ? 0x07060302 : 0x05040100);
-          if (col[u] + px < p.cols_in) *reinterpret_cast<i32x4*>(dst[u] + px * CHS) = o;
-        }
-      }
-    };
-    int t0 = tid;
-    for (; t0 - tid + NT < tasks; t0 += 2 * NT) stage(CtInt<2>(), t0);
-    if (t0 - tid < tasks) stage(CtInt<1>(), t0);
-    // the columns left and right of the image
-    const int right = max(0, p.cols_in - p.W - p.pad), nz = p.pad + right;
-    if (nz > 0) {
-      const float inv_nz = 1.f / (float)nz;
-      for (int t = tid; t < p.rows_in * nz * cg; t += NT) {
-        const int rest = div_by(t, p.inv_cg), chg = t - rest * cg, ri = div_by(rest, inv_nz), z = rest - ri * nz;
-        *reinterpret_cast<i32x4*>(Xs + ri * row_step + (z < p.pad ? z : p.W + z) * CHS + 8 * chg) = i32x4{0, 0, 0, 0};
-      }
-    }
-  }
+  stage_halo_rows<NT>(Xs, reinterpret_cast<const T*>(p.x) + (long long)n * p.C0 * hw, h0, p.pad, p.rows_in, p.cols_in, CHS, cg, cg, p.C0, p.H,
+                      p.W, p.inv_cg, p.inv_ng, tid);
 
   int xb[PT];  // element offset of this lane's pixel of tile t at tap (0, 0)
 #pragma unroll

@@ -131,6 +131,7 @@ typedef struct ditto_conv_chain_desc {
                             family id (a multiple of 100) that leaves the tile inside the family to the library:
                               3000 general kernel, 1x1 second convolution (31xx: 16-channel chunks)
                               3200 tiles of whole output rows, 1x1 second convolution
+                              3300 conv1x1 -> conv3x3 on tiles of whole output rows (33xx: rows, 50 more with eight waves)
                               3500 general kernel, second convolution up to 3x3 through LDS
                               3600 conv1x1 -> conv3x3, persistent workgroups, W2 resident in LDS
                               3700 conv3x3 -> conv1x1 row pipeline        3800 conv1x1 -> conv3x3 row pipeline

@@ -1006,3 +1006,40 @@ def test_depthwise_chain_on_row_tiles(oracle, case, dtype):
     chain.run_conv_chain(x, w1, w2, y, desc=desc)
     torch.cuda.synchronize()
     assert np.array_equal(y.float().cpu().numpy(), got) and bool(torch.isnan(out[0]))
+
+
+CASES_TILES13 = [
+    # N, C0, H, W, C1, C2: conv1x1 -> conv3x3 on tiles of whole output rows
+    (1, 8, 1, 8, 8, 8),        # a single image row of the narrowest image
+    (2, 24, 7, 9, 40, 33),     # a row's last 8-pixel group starts at W - 8; channels that fill no tile
+    (3, 64, 20, 20, 64, 64),   # several rows per workgroup, a ragged last tile
+    (1, 33, 11, 127, 56, 64),  # an odd number of input channels, one output row of 8 pixel tiles
+    (60, 16, 10, 50, 64, 16),  # more workgroups than compute units
+    (2, 64, 5, 255, 64, 64),   # eight waves, the widest ragged row
+]
+
+
+@pytest.mark.parametrize("case", CASES_TILES13)
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+def test_conv1x1_conv3x3_on_row_tiles(oracle, case, dtype):
+    N, C0, H, W, C1, C2 = case
+    X, W1, W2 = oracle.make_conv_chain_inputs(N, C0, H, W, C1, C2, 1, 3, dtype, seed=C0 + C2 + W, w_std=0.05)
+    for relu in (False, True):
+        inter = "relu" if relu else "cast"
+        want = oracle.conv_chain_f32(X, W1, W2, 0, 1, 1, 1, relu_mid=relu, relu_out=relu, round_mid=dtype)
+        got32 = run_conv(X, W1, W2, dtype, 0, 1, inter, relu, out_dtype="float32", pad2=1, tile_variant=3300)
+        got = run_conv(X, W1, W2, dtype, 0, 1, inter, relu, pad2=1, tile_variant=3300)
+        assert np.isfinite(got).all()
+        mx, rel = errors(got32, want)
+        assert mx <= MAX_ABS and rel <= REL_L2, (relu, mx, rel)
+        assert np.array_equal(got, oracle.np_round_to(got32, dtype)), relu
+    # tensors at any element's address, prepared weights
+    flat = to_dev(np.concatenate([np.zeros(1, np.float32), X.ravel()]), dtype)
+    x, w1, w2 = flat[1:].view(N, C0, H, W), to_dev(W1, dtype), to_dev(W2, dtype)
+    out = torch.full((got.size + 1,), float("nan"), device=x.device, dtype=x.dtype)
+    y = out[1:].view(got.shape)
+    desc = chain.conv_chain_desc(x, w1, w2, y, 0, 1, 1, 1, "relu", True, tile_variant=3300)
+    ws = chain.prepare_conv_chain(desc, w1, w2)
+    chain.run_conv_chain(x, w1, w2, y, desc=desc, workspace=ws, prepared=True)
+    torch.cuda.synchronize()
+    assert np.array_equal(y.float().cpu().numpy(), got) and bool(torch.isnan(out[0]))
