@@ -50,7 +50,7 @@ struct BmmPlan {
   int family;  // 0: fp16/bf16 register-resident chain, 1: fp32 chain, 2: int8 requant chain
   int d_pad, qt;  // fp chains: head pad and rows-per-wave code; int8 chain: row tiles and ring depth
   int split_dt = 0, split_rt = 0;  // fp chains on few rows: column tiles and row tiles of the key-splitting kernel (0: none)
-  int rows_nw = 0;  // fp chains of head size 65 to 80: waves of a workgroup of the kernel padded to 80 columns (0: none)
+  int rows_dt = 0, rows_nw = 0;  // fp chains: column tiles and waves of the kernel of 32 rows per wave and short tiles (0: none)
   int nb3 = 0, nb = 0;  // 16x16x32-MFMA kernel: row blocks of 384 rows / row blocks in all, per batch entry
   ditto_tile_param tile;
 };
@@ -243,7 +243,7 @@ int plan_bmm(const ditto_bmm_chain_desc* d, BmmPlan* plan, bool need_device) {
             const long long rounds = (((d->M + 32 * nw - 1) / (32 * nw)) * d->batch + cus - 1) / cus;
             const double cost = nw == 4 ? (rounds == 1 ? 2.3 + 0.0131 * key : 2.1 + rounds * (1.1 + 0.0114 * key))
                                         : (rounds == 1 ? 2.9 + 0.0196 * key : 2.1 + rounds * (2.8 + 0.0226 * key));
-            if (cost < best) best = cost, plan->rows_nw = nw;
+            if (cost < best) best = cost, plan->rows_dt = 5, plan->rows_nw = nw;
           }
         }
         for (int r = 1; r <= 2; ++r) {
@@ -252,7 +252,8 @@ int plan_bmm(const ditto_bmm_chain_desc* d, BmmPlan* plan, bool need_device) {
           if (cost < best) best = cost, rt = r;
         }
       }
-      if (dmax <= 80 && (d->tile_variant == 2154 || d->tile_variant == 2158)) plan->rows_nw = d->tile_variant % 10;
+      for (int id : {2144, 2148, 2154, 2158, 2188})
+        if (d->tile_variant == id && 16 * (id / 10 % 10) >= dmax) plan->rows_dt = id / 10 % 10, plan->rows_nw = id % 10;
       if (d->tile_variant == 2001 + 10 * dt || d->tile_variant == 2002 + 10 * dt) rt = d->tile_variant % 10;
       if (rt > 0) {
         plan->split_dt = dt, plan->split_rt = rt;
@@ -269,6 +270,30 @@ int plan_bmm(const ditto_bmm_chain_desc* d, BmmPlan* plan, bool need_device) {
         t.variant = 2000 + 10 * dt + rt;
         return DITTO_OK;
       }
+      // The same kernel at 64 and at 128 columns, where its short start and two workgroups on a compute unit tell.
+      if (d->tile_variant == 0 && dt == 8 && rt == 0) {
+        // Heads of 81 to 128, up to about 500 keys (600 with softmax), eight waves: against the pipelined 256-row kernel (9) at
+        // every size measured (128 x 400 x 400 20.8 -> 18.8 us, 320 x 197 x 197 28.9 -> 25.3; 160 x 577 x 577 46.6 -> 45.0, but
+        // 80 x 1024 x 1024 65.4 against 68.4), against 128-row workgroups where those take a second round and 256 rows do not
+        // (160 x 197 x 197 18.8 -> 12.0, 80 x 400 x 400 25.0 -> 17.5; in one round 80 x 257 x 257 11.1 against 13.9), and against the
+        // kernels of large grids unless those cover a head's rows in fewer blocks by taking 384 (512 x 197 x 197 33.2 -> 27.8,
+        // 256 x 400 x 400 39.1 -> 35.2; 256 x 257 x 257 25.2 against 28.4, 256 x 577 x 577 61.3 / 66.5).
+        const long long rows256 = (d->M + 255) / 256, n128 = ((d->M + 127) / 128) * d->batch;
+        bool take = d->L <= (sm ? 600 : 450);
+        if (plan->qt == 1) take = take && n128 > cus;
+        if (plan->qt == 6 || plan->qt == 2) {
+          const long long a384 = plan_rows_384(d->M, d->batch, cus), rest = d->M - 384 * a384;
+          take = d->L <= 512 && (plan->qt == 2 || a384 + (rest > 0 ? (rest + 255) / 256 : 0) >= rows256);
+        }
+        if (take) plan->rows_dt = 8, plan->rows_nw = 8;
+      }
+      if (d->tile_variant == 0 && dt == 4 && rt == 0 && !sm && n8 >= 2LL * cus && d->L <= 1024) {
+        // Heads of up to 64 without softmax from two 256-row workgroups per compute unit on, up to 1024 keys: 512 x 197 x 197 16.8 ->
+        // 12.2 us, 256 x 400 x 400 20.0 -> 16.6 (B [K][L] 22.3 -> 18.0), 256 x 577 x 577 35.0 -> 29.9, 128 x 1024 x 1024 35.3 -> 33.8;
+        // below that the 64-row kernel's grain is worth more (160 x 400 x 400 13.6 against 15.4), and so it is with softmax
+        // (256 x 400 x 400 21.0 against 22.8).
+        plan->rows_dt = 4, plan->rows_nw = d->M <= 128 ? 4 : 8;
+      }
       if (plan->rows_nw > 0) {
         plan->nb = (int)((d->M + 32 * plan->rows_nw - 1) / (32 * plan->rows_nw));
         ditto_tile_param& t = plan->tile;
@@ -276,11 +301,11 @@ int plan_bmm(const ditto_bmm_chain_desc* d, BmmPlan* plan, bool need_device) {
         t.block_m = 32 * plan->rows_nw;
         t.block_l = ditto::kBN;
         t.block_n = (int)d->N;
-        t.head_pad = 80;
-        t.lds_bytes = kl_b ? ditto::bmm_chain_rows_lds<5, true, 4>() : ditto::bmm_chain_rows_lds<5, false, 4>();  // (the same for eight waves)
+        t.head_pad = 16 * plan->rows_dt;
+        t.lds_bytes = ditto::bmm_chain_rows_lds(plan->rows_dt, plan->rows_nw, kl_b);
         t.grid_x = (int)(plan->nb * d->batch);
         t.grid_y = t.grid_z = 1;
-        t.variant = 2150 + plan->rows_nw;
+        t.variant = 2100 + 10 * plan->rows_dt + plan->rows_nw;
         return DITTO_OK;
       }
     }
@@ -1332,8 +1357,8 @@ int ditto_bmm_chain_run(const ditto_bmm_chain_desc* d, const void* a, const void
       e = d->in_dtype == DITTO_F16 ? ditto::launch_split_f16(plan.split_dt, plan.split_rt, sm, kl, args, st)
                                    : ditto::launch_split_bf16(plan.split_dt, plan.split_rt, sm, kl, args, st);
     else if (plan.rows_nw > 0)
-      e = d->in_dtype == DITTO_F16 ? ditto::launch_rows_f16(plan.rows_nw, sm, kl, args, st)
-                                   : ditto::launch_rows_bf16(plan.rows_nw, sm, kl, args, st);
+      e = d->in_dtype == DITTO_F16 ? ditto::launch_rows_f16(plan.rows_dt, plan.rows_nw, sm, kl, args, st)
+                                   : ditto::launch_rows_bf16(plan.rows_dt, plan.rows_nw, sm, kl, args, st);
     else if (d->in_dtype == DITTO_F16)
       e = sm ? ditto::launch_f16_softmax(plan.d_pad, plan.qt, kl, args, st)
              : ditto::launch_f16_cast(plan.d_pad, plan.qt, kl, args, st);

@@ -14,6 +14,8 @@
 // padding); below that the chain start -> first tile -> L / 64 steps of 0.85 us.  Measured, us per launch with softmax (2.4 of
 // them the launch), padded to 128 -> here, four | eight waves: 256 x 197 x 197 14.3 -> 10.6 | 10.3, 640 x 49 x 49
 // 22.9 -> 8.8 | 12.0, 80 x 400 x 400 23.2 -> 13.4 | 12.9, 96 x 700 x 700 44.8 -> 28.7 | 35.9, 32 x 4096 x 4096 206 -> 191 | 187.
+// The same kernel at 64 columns (without softmax, large grids) and at 128 (up to about 500 keys) is ahead of the others by its
+// start: 512 x 197 x 197 x 64 16.8 -> 12.2, x 128 with softmax 33.2 -> 27.8.
 #pragma once
 #include "bmm_chain_fp8m16.h"
 #include "common.h"
@@ -41,6 +43,13 @@ __host__ __device__ constexpr int bmm_chain_rows_tile_bytes() {
 template <int DT, bool B_KL, int NW>
 __host__ __device__ constexpr int bmm_chain_rows_lds() {
   return kRowsRing * bmm_chain_rows_tile_bytes<DT, B_KL, NW>() + 64;  // the tiles and the flag of the optimistic walk
+}
+
+inline int bmm_chain_rows_lds(int dt, int nw, bool kl) {
+  if (dt == 4 && nw == 4) return kl ? bmm_chain_rows_lds<4, true, 4>() : bmm_chain_rows_lds<4, false, 4>();
+  if (dt == 4) return kl ? bmm_chain_rows_lds<4, true, 8>() : bmm_chain_rows_lds<4, false, 8>();
+  if (dt == 5) return kl ? bmm_chain_rows_lds<5, true, 8>() : bmm_chain_rows_lds<5, false, 8>();  // (the same for four waves)
+  return kl ? bmm_chain_rows_lds<8, true, 8>() : bmm_chain_rows_lds<8, false, 8>();
 }
 
 template <typename T, int DT, int NW, int INTER, bool B_KL>

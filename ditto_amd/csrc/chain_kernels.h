@@ -28,8 +28,8 @@ hipError_t launch_split_f16(int dt, int rt, bool softmax, bool b_kl, const BmmCh
 hipError_t launch_split_bf16(int dt, int rt, bool softmax, bool b_kl, const BmmChainArgs& args, hipStream_t stream);
 
 // bmm_chain_rows_inst.hip, one object per element type: K and N padded to 80
-hipError_t launch_rows_f16(int nw, bool softmax, bool b_kl, const BmmChainArgs& args, hipStream_t stream);
-hipError_t launch_rows_bf16(int nw, bool softmax, bool b_kl, const BmmChainArgs& args, hipStream_t stream);
+hipError_t launch_rows_f16(int dt, int nw, bool softmax, bool b_kl, const BmmChainArgs& args, hipStream_t stream);
+hipError_t launch_rows_bf16(int dt, int nw, bool softmax, bool b_kl, const BmmChainArgs& args, hipStream_t stream);
 
 // conv_chain_inst.hip, one object per element type; c1_tiles in {1, 2, 4, 8}
 // ch in {32, 16}: input channels per staged chunk

@@ -164,8 +164,9 @@ typedef struct ditto_tile_param {
                              with 64-row workgroups (head_pad 64, either layout of B): q = 4 (a
                              wave owns 16 rows and all keys), q = 5 (32 rows and half the keys of
                              every tile); eight waves that split the keys: 2000 + 10 * (head size / 16 rounded
-                             up to 4, 5 or 8) + (row tiles of 16 per workgroup, 1 or 2); K and N padded to 80:
-                             2150 + (waves of 32 rows, 4 or 8); conv chains: the ids listed at
+                             up to 4, 5 or 8) + (row tiles of 16 per workgroup, 1 or 2); waves of 32 rows on
+                             short tiles: 2144, 2148, 2154, 2158, 2188 = 2100 + 10 * (head size / 16
+                             rounded up likewise) + (waves); conv chains: the ids listed at
                              ditto_conv_chain_desc.tile_variant; fp32 / fp64 1000 / 1001; int8
                              8000 + 10 * (row tiles of 32) + ring depth */
 } ditto_tile_param;

@@ -155,13 +155,14 @@ def test_key_splitting_kernel(oracle, shape, dtype, inter):
 
 
 @pytest.mark.parametrize("shape", [
-    # (batch, M, N, K, L) for the kernel padded to 80 columns: a last tile of one half and of two, one tile and more than the
+    # (batch, M, N, K, L) for the kernel of 32 rows per wave, padded to 64, 80 or 128 columns: a last tile of one half and of two, one tile and more than the
     # ring holds, waves without rows, column counts at and below the padding
     (1, 1, 80, 80, 8), (2, 129, 80, 80, 96), (3, 33, 72, 80, 520), (2, 257, 80, 72, 32), (1, 300, 80, 80, 200), (2, 40, 8, 16, 264),
+    (2, 260, 128, 104, 136),  # the 128-column form
 ])
 @pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
 @pytest.mark.parametrize("inter", ["relu", "softmax"])
-def test_kernel_padded_to_80_columns(oracle, shape, dtype, inter):
+def test_kernel_of_32_rows_per_wave(oracle, shape, dtype, inter):
     batch, M, N, K, L = shape
     std = 1.0 if inter == "softmax" else 0.25
     A, B, C = oracle.make_gemm_chain_inputs(batch, M, N, K, L, dtype, seed=900 + M + L, std=std)
@@ -169,15 +170,17 @@ def test_kernel_padded_to_80_columns(oracle, shape, dtype, inter):
     B = oracle.np_round_to(B * np.linspace(0.1, 6.0 if inter == "softmax" else 1.0, L, dtype=np.float32)[None, None, :], dtype)
     scale = 0.5 if inter == "softmax" else 1.0
     want = oracle.bmm_chain_f64(A, B, C, inter=inter, scale=scale, round_mid=None if inter == "softmax" else dtype)
-    for waves in (4, 8):
+    for variant in (2144, 2148, 2154, 2158, 2188):
+        if variant % 100 // 10 * 16 < max(K, N):
+            continue
         for b_layout in ("KL", "LK"):
-            got = run_chain(A, B, C, dtype, inter, scale, b_layout, "float32", 2150 + waves)
+            got = run_chain(A, B, C, dtype, inter, scale, b_layout, "float32", variant)
             assert np.isfinite(got).all()
             mx, rel = errors(got, want)
             bound = REL_L2 if inter != "softmax" or dtype == "float16" else 2.0e-3  # bf16: the probabilities' own rounding
-            assert rel <= bound and mx <= 4e-2, (waves, b_layout, mx, rel)
-            narrow = run_chain(A, B, C, dtype, inter, scale, b_layout, dtype, 2150 + waves)
-            assert np.array_equal(narrow, oracle.np_round_to(got, dtype)), (waves, b_layout)
+            assert rel <= bound and mx <= 4e-2, (variant, b_layout, mx, rel)
+            narrow = run_chain(A, B, C, dtype, inter, scale, b_layout, dtype, variant)
+            assert np.array_equal(narrow, oracle.np_round_to(got, dtype)), (variant, b_layout)
 
 
 @pytest.mark.parametrize("shape", [(1, 512, 64, 64, 64), (3, 100, 24, 40, 72), (2, 64, 128, 128, 200)])
