@@ -83,7 +83,9 @@ __global__ __launch_bounds__(64 * i8::NW) void gemm_chain_i8_kernel(I8ChainArgs 
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int ln = lane & 31, g = lane >> 5;
   const int i16 = lane & 15, h = (lane >> 4) & 1;
-  const unsigned lid = xcd_remap(blockIdx.x, gridDim.x);
+  // (One batch entry: all workgroups read the same B and C, there is nothing to group; ragged grids keep the round-robin order,
+  // 2000 x 144 x 128 x 848 8.2 us against 8.5.)
+  const unsigned lid = (gridDim.x & 7) && gridDim.x == (unsigned)p.mblocks ? blockIdx.x : xcd_remap(blockIdx.x, gridDim.x);
   const int mb = lid % p.mblocks, bz = lid / p.mblocks;
   const int m0 = mb * BM;
   const int M = p.M, N = p.N, K = p.K, L = p.L, Lp = p.Lp;
