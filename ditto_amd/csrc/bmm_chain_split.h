@@ -157,10 +157,11 @@ __global__ __launch_bounds__(64 * kSplitWaves) void bmm_chain_split_kernel(BmmCh
 #pragma unroll
     for (int j = 0; j < DT; ++j) o[rt][j] = f32x4{0.f, 0.f, 0.f, 0.f};
   // softmax in the exp2 domain: a row's reference exponent is its maximum over the wave's first keys, raised when a later
-  // score exceeds it by more than 2^kLazy
+  // score exceeds it by more than 2^kLazy; a wave whose keys so far all score minus infinity has none yet (it may be one of
+  // eight that has met any key of the row)
   float ref[RT], lsum[RT];
 #pragma unroll
-  for (int rt = 0; rt < RT; ++rt) ref[rt] = -INFINITY, lsum[rt] = 0.f;
+  for (int rt = 0; rt < RT; ++rt) ref[rt] = kNoKeyYet, lsum[rt] = 0.f;
   const float c2 = p.scale_log2;
 
   // the A fragments are named between the first direct loads: the compiler's wait for them then falls here, once, and not
@@ -280,7 +281,7 @@ __global__ __launch_bounds__(64 * kSplitWaves) void bmm_chain_split_kernel(BmmCh
     const int row = e / (4 * DT), n0 = 4 * (e - row * 4 * DT);
     float wt[kSplitWaves];
     if constexpr (kSoftmax) {
-      float mx = -INFINITY, s = 0.f;
+      float mx = kNoKeyYet, s = 0.f;
 #pragma unroll
       for (int i = 0; i < kSplitWaves; ++i) mx = fmaxf(mx, Ml[2 * (i * 16 * RT + row)]);
 #pragma unroll

@@ -125,6 +125,11 @@ __device__ __forceinline__ float neg_inf_where(float x, int gone) {
   return __builtin_bit_cast(float, (__builtin_bit_cast(int, x) & ~gone) | ((int)0xff800000 & gone));
 }
 
+// Reference exponent of a row that has met no key with a score above minus infinity.  Finite, so that a score of minus
+// infinity has weight 0 against it, where minus infinity less itself is NaN; any other score raises it, and the merge of
+// partial results gives it weight 0 beside a row that has one (a row with no such key at all ends as 0 / 0 = NaN).
+constexpr float kNoKeyYet = -3.402823466e+38f;
+
 template <typename V4, typename V8>
 __device__ __forceinline__ V8 concat4(V4 lo, V4 hi) {
   return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);

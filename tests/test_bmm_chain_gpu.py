@@ -154,6 +154,62 @@ def test_key_splitting_kernel(oracle, shape, dtype, inter):
             assert np.array_equal(narrow, oracle.np_round_to(got, dtype)), (variant, b_layout)
 
 
+def masked_scores(oracle, batch, M, N, K, L, dtype, masked, seed):
+    """Operands whose scores are minus infinity at the keys ``masked``: column 0 of the first operand is one, and the
+    keys hold minus infinity there (how a caller of a chain without a mask argument masks keys)."""
+    A, B, C = oracle.make_gemm_chain_inputs(batch, M, N, K, L, dtype, seed=seed)
+    A[:, :, 0] = 1.0
+    B[:, 0, :] = 0.0
+    B[:, 0, masked] = -np.inf
+    return A, B, C
+
+
+# whole groups of a wave's keys without a weight: behind key 100 (padding at the end), the first 96 (padding in front),
+# one aligned group alone, all but the last key
+MASKED_KEYS = {"end": lambda L: slice(100, L), "front": lambda L: slice(0, 96), "group": lambda L: slice(64, 96),
+               "all but one": lambda L: slice(0, L - 1)}
+
+@pytest.mark.parametrize("shape", [(1, 16, 64, 64, 176), (2, 40, 80, 80, 176), (1, 33, 128, 128, 528)])
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+@pytest.mark.parametrize("keys", sorted(MASKED_KEYS))
+def test_key_splitting_kernel_on_masked_keys(oracle, shape, dtype, keys):
+    """A wave whose keys all score minus infinity has no part in the row, whatever the other waves hold (it used to
+    make the row NaN: minus infinity less its own reference exponent of minus infinity)."""
+    batch, M, N, K, L = shape
+    A, B, C = masked_scores(oracle, batch, M, N, K, L, dtype, MASKED_KEYS[keys](L), seed=31 + L)
+    want = oracle.bmm_chain_f64(A, B, C, inter="softmax", scale=0.2)
+    width = 4 if max(K, N) <= 64 else 5 if max(K, N) <= 80 else 8
+    for rows in (1, 2):
+        for b_layout in ("KL", "LK"):
+            got = run_chain(A, B, C, dtype, "softmax", 0.2, b_layout, "float32", 2000 + 10 * width + rows)
+            assert np.isfinite(got).all(), (rows, b_layout)
+            mx, rel = errors(got, want)
+            # the probabilities' rounding, over as little as one key
+            assert mx <= 4e-2 and rel <= (REL_L2 if dtype == "float16" else 2.0e-3), (rows, b_layout, mx, rel)
+
+
+def test_key_splitting_kernel_masks_rows_one_by_one(oracle):
+    """Scores that overflow to minus infinity with the scale, in every other row: those rows' references stay where
+    they are while another row of the wave raises its own.  A row without any key is NaN, and only that row."""
+    batch, M, N, K, L = 1, 40, 80, 80, 176
+    A, B, C = oracle.make_gemm_chain_inputs(batch, M, N, K, L, "bfloat16", seed=5)
+    lowest = oracle.np_round_to(np.float32([-3.3e38]), "bfloat16")[0]
+    A[:, :, 0] = 0.0
+    A[:, ::2, 0] = 1.0
+    for masked, none in ((slice(32, L), False), (slice(0, 160), False), (slice(0, L), True)):
+        Bm = B.copy()
+        Bm[:, 0, :] = 0.0
+        Bm[:, 0, masked] = lowest
+        want = oracle.bmm_chain_f64(A, Bm, C, inter="softmax", scale=2.0)
+        for variant in (2051, 2052):
+            got = run_chain(A, Bm, C, "bfloat16", "softmax", 2.0, "LK", "float32", variant)
+            rows = slice(1, None, 2) if none else slice(None)
+            assert np.isfinite(got[:, rows]).all(), (variant, masked)
+            assert not none or np.isnan(got[:, ::2]).all()
+            mx, rel = errors(got[:, rows], want[:, rows])
+            assert mx <= 4e-2 and rel <= REL_L2_BF16_QUANT, (variant, masked, mx, rel)
+
+
 @pytest.mark.parametrize("shape", [
     # (batch, M, N, K, L) for the kernel of 32 rows per wave, padded to 64, 80 or 128 columns: a last tile of one half and of two, one tile and more than the
     # ring holds, waves without rows, column counts at and below the padding
