@@ -88,12 +88,13 @@ __global__ __launch_bounds__(64 * kWaves) void gemm_chain_f32_kernel(F32ChainArg
     for (int j = 0; j < DT; ++j) o[rt][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
   }
   // softmax in the exp2 domain: a row's reference exponent is its maximum over the wave's first keys, raised only when a
-  // later score exceeds it by 2^kSlack (a row sum stays below L 2^kSlack, far inside the fp32 range)
+  // later score exceeds it by 2^kSlack (a row sum stays below L 2^kSlack, far inside the fp32 range); none yet while the
+  // wave's keys all score minus infinity
   constexpr float kSlack = 20.f;
   const float c2 = p.softmax_scale * 1.4426950408889634f;
   float ref[RT], lsum[RT];
 #pragma unroll
-  for (int rt = 0; rt < RT; ++rt) ref[rt] = -INFINITY, lsum[rt] = 0.f;
+  for (int rt = 0; rt < RT; ++rt) ref[rt] = kNoKeyYet, lsum[rt] = 0.f;
 
   for (int step = w; step < nsteps; step += kWaves) {
     const int key0 = 16 * step;
@@ -198,7 +199,7 @@ __global__ __launch_bounds__(64 * kWaves) void gemm_chain_f32_kernel(F32ChainArg
     const int row = e / (4 * DT), n0 = 4 * (e - row * 4 * DT);
     float wt[kWaves];
     if constexpr (SM) {
-      float mx = -INFINITY, s = 0.f;
+      float mx = kNoKeyYet, s = 0.f;
 #pragma unroll
       for (int i = 0; i < kWaves; ++i) mx = fmaxf(mx, Ml[2 * (i * 16 * RT + row)]);
 #pragma unroll

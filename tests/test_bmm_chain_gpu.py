@@ -274,6 +274,26 @@ def test_fp32_chain_at_the_edges_of_its_tiles(oracle, shape, inter):
         assert np.isfinite(got).all() and rel <= 1e-5, (b_layout, mx, rel)
 
 
+@pytest.mark.parametrize("shape", [(1, 17, 64, 64, 100), (2, 40, 80, 80, 176), (9, 500, 80, 80, 176), (1, 20, 70, 66, 300), (1, 33, 128, 128, 528)])
+@pytest.mark.parametrize("keys", sorted(MASKED_KEYS))
+def test_fp32_chain_on_masked_keys(oracle, shape, keys):
+    """As above for the fp32 kernel, whose waves take 16 keys at a time."""
+    batch, M, N, K, L = shape
+    masked = slice(16, L) if keys == "end" and L == 100 else MASKED_KEYS[keys](L)
+    A, B, C = masked_scores(oracle, batch, M, N, K, L, "float32", masked, seed=31 + L)
+    want = oracle.bmm_chain_f64(A, B, C, inter="softmax", scale=0.2)
+    for b_layout in ("KL", "LK"):
+        got = run_chain(A, B, C, "float32", "softmax", 0.2, b_layout)
+        assert np.isfinite(got).all(), b_layout
+        mx, rel = errors(got, want)
+        assert rel <= 1e-5, (b_layout, mx, rel)  # fp32 sums, as in the tests above
+    # rows without any key are NaN, and only those
+    A[:, ::2, 0], A[:, 1::2, 0] = 1.0, 0.0
+    B[:, 0, :] = -3.3e38
+    got = run_chain(A, B, C, "float32", "softmax", 2.0, "LK")
+    assert np.isnan(got[:, ::2]).all() and np.isfinite(got[:, 1::2]).all()
+
+
 @pytest.mark.parametrize("shape", [(1, 512, 64, 64, 64), (3, 100, 24, 40, 72), (2, 64, 128, 128, 200)])
 @pytest.mark.parametrize("inter", ["cast", "relu", "softmax"])
 def test_fp64_chain_vs_oracle(oracle, shape, inter):
