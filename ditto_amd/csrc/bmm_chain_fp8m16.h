@@ -113,20 +113,6 @@ __device__ __forceinline__ void acc_scale(int i, float alpha, f32x4 (&o)[kMaxAcc
   acc_pin(i, o[i]);
 }
 
-// maximum over the four lanes c, c + 16, c + 32, c + 48 (every lane gets it).
-// v_permlane16_swap a, b swaps the odd rows of 16 lanes of a with the even rows of b; from a == b == x,
-// max(a, b) holds max(x[row 0], x[row 1]) in rows 0 and 1 and max(x[row 2], x[row 3]) in rows 2 and 3.
-__device__ __forceinline__ float quad_max(float x) {
-  float a = x, b = x;
-  asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(a), "+v"(b));
-  return pair_max(fmaxf(a, b));
-}
-__device__ __forceinline__ float quad_sum(float x) {
-  float a = x, b = x;
-  asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(a), "+v"(b));
-  return pair_sum(a + b);
-}
-
 // XOR applied to the 16-byte chunk index of a 128-byte row ([k][64 l] tiles of a B stored [K][L]) for the
 // transposing read with lanes (c, q) -> row 4 q + c / 4: 2.3 cycles per instruction with eight waves reading, against
 // 4 under the swizzle of the once-per-tile transposition passes

@@ -157,6 +157,20 @@ __device__ __forceinline__ float pair_sum(float x) {
   return a + b;
 }
 
+// maximum over the four lanes c, c + 16, c + 32, c + 48 (every lane gets it).
+// v_permlane16_swap a, b swaps the odd rows of 16 lanes of a with the even rows of b; from a == b == x,
+// max(a, b) holds max(x[row 0], x[row 1]) in rows 0 and 1 and max(x[row 2], x[row 3]) in rows 2 and 3.
+__device__ __forceinline__ float quad_max(float x) {
+  float a = x, b = x;
+  asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(a), "+v"(b));
+  return pair_max(fmaxf(a, b));
+}
+__device__ __forceinline__ float quad_sum(float x) {
+  float a = x, b = x;
+  asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(a), "+v"(b));
+  return pair_sum(a + b);
+}
+
 // Direct global -> LDS load of 16 bytes per lane (buffer_load_dwordx4 ... lds): lane l's data
 // lands at LDS byte address lds_base + 16*l; reads whose offset is at or past the resource's
 // num_records return zero.  Issued as inline asm so that the compiler does not track it: its

@@ -87,10 +87,12 @@ __global__ __launch_bounds__(64 * kWaves) void gemm_chain_f32_kernel(F32ChainArg
 #pragma unroll
     for (int j = 0; j < DT; ++j) o[rt][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
   }
-  // softmax in the exp2 domain: a row's reference exponent is its maximum over the wave's first keys, raised only when a
-  // later score exceeds it by 2^kSlack (a row sum stays below L 2^kSlack, far inside the fp32 range); none yet while the
-  // wave's keys all score minus infinity
-  constexpr float kSlack = 20.f;
+  // softmax in the exp2 domain: a row's reference exponent is no smaller than any score of the wave's keys so far, so no weight
+  // exceeds one and a result overflows only where the sum of its values does (a slack of 2^20 before a raise took that much
+  // off the range of C).  When a score exceeds the reference it is set kHeadroom above it: the few binary orders by which a
+  // later key usually exceeds the first sixteen then cost no second rescale, which waits for the accumulators (always to the
+  // maximum itself: 14.4 -> 14.8 us at 12 x 512 x 512 x 64, 4 % more at 1000 keys).  None yet while all score minus infinity.
+  constexpr float kHeadroom = 4.f;
   const float c2 = p.softmax_scale * 1.4426950408889634f;
   float ref[RT], lsum[RT];
 #pragma unroll
@@ -125,16 +127,15 @@ __global__ __launch_bounds__(64 * kWaves) void gemm_chain_f32_kernel(F32ChainArg
         for (int r = 0; r < 4; ++r) {
           st[rt][r] *= c2;
           if (tail && key0 + 4 * q + r >= L) st[rt][r] = -INFINITY;
-          raise |= st[rt][r] > ref[rt] + kSlack;
+          raise |= st[rt][r] > ref[rt];
         }
       }
       if (__any(raise)) {
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) {
           float mx = fmaxf(fmaxf(st[rt][0], st[rt][1]), fmaxf(st[rt][2], st[rt][3]));
-          mx = fmaxf(mx, __shfl_xor(mx, 16));
-          mx = fmaxf(mx, __shfl_xor(mx, 32));
-          const float up = fmaxf(ref[rt], mx), alpha = exp2f(ref[rt] - up);
+          mx = quad_max(mx);
+          const float up = mx > ref[rt] ? mx + kHeadroom : ref[rt], alpha = exp2f(ref[rt] - up);
           ref[rt] = up;
           lsum[rt] *= alpha;
 #pragma unroll

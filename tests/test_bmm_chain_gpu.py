@@ -294,6 +294,23 @@ def test_fp32_chain_on_masked_keys(oracle, shape, keys):
     assert np.isnan(got[:, ::2]).all() and np.isfinite(got[:, 1::2]).all()
 
 
+@pytest.mark.parametrize("shape", [(1, 40, 64, 64, 520), (9, 512, 64, 64, 520), (1, 20, 128, 128, 520)])
+def test_fp32_chain_on_large_values_and_climbing_scores(oracle, shape):
+    """Weights taken relative to a row's maximum are at most one, so a result that fp32 can hold comes out however the
+    scores climb: sums of 520 values of 1e34 stay below 1e38."""
+    batch, M, N, K, L = shape
+    A, B, C = oracle.make_gemm_chain_inputs(batch, M, N, K, L, "float32", seed=M + L)
+    B, C = B * np.float32(0.2), C * np.float32(1e34)
+    A[:, :, 0] = 1.0
+    B[:, 0, :] = 24.0 * (np.arange(L) // 128)  # every wave's next keys score 12 (seventeen binary orders) more
+    want = oracle.bmm_chain_f64(A, B, C, inter="softmax", scale=0.5)
+    for b_layout in ("KL", "LK"):
+        got = run_chain(A, B, C, "float32", "softmax", 0.5, b_layout)
+        assert np.isfinite(got).all(), b_layout
+        mx, rel = errors(got, want)
+        assert rel <= 1e-5, (b_layout, mx, rel)
+
+
 @pytest.mark.parametrize("shape", [(1, 512, 64, 64, 64), (3, 100, 24, 40, 72), (2, 64, 128, 128, 200)])
 @pytest.mark.parametrize("inter", ["cast", "relu", "softmax"])
 def test_fp64_chain_vs_oracle(oracle, shape, inter):
