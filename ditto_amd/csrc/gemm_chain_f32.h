@@ -20,6 +20,7 @@ struct F32ChainArgs {
   int softmax;   // inter path: softmax over L of scale * (A.B)
   float softmax_scale;
   int f64;       // elements are doubles
+  unsigned block0;  // fp32: workgroups in front of this launch's (filled by the launcher)
 };
 
 int f32_chain_lds_bytes_host(int K, int N, int f64, int row_tiles);

@@ -13,6 +13,7 @@ namespace ditto {
 namespace {
 constexpr int kMaxD = 128;
 constexpr int kWaves = 8;  // waves of an fp32 workgroup: they split the keys
+constexpr unsigned kLaunchBlocks = 1u << 22;  // most fp32 workgroups of one launch
 }
 
 // ---- fp32 ------------------------------------------------------------------------------------
@@ -45,7 +46,7 @@ __global__ __launch_bounds__(64 * kWaves) void gemm_chain_f32_kernel(F32ChainArg
   float* const Ml = smem_f32 + kWaves * 16 * RT * ORS;     // [wave][16 RT][reference exponent, sum]
   const int K = p.K, N = p.N, L = p.L, M = p.M;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, c = lane & 15, q = lane >> 4;
-  const unsigned bid = xcd_remap(blockIdx.x, gridDim.x);  // the row blocks of a batch entry read the same B and C
+  const unsigned bid = p.block0 + xcd_remap(blockIdx.x, gridDim.x);  // the row blocks of a batch entry read the same B and C
   const int bz = bid / (unsigned)p.mblocks, m0 = (bid - bz * (unsigned)p.mblocks) * 16 * RT;
   const float* const Ag = static_cast<const float*>(p.a) + (long long)bz * p.a_bs;
   const float* const Bg = static_cast<const float*>(p.b) + (long long)bz * p.b_bs;
@@ -376,8 +377,18 @@ static hipError_t launch_with_lds(Kernel kernel, unsigned threads, int lds, cons
     if (e != hipSuccess) return e;
     configured_dev = dev;
   }
-  hipLaunchKernelGGL(kernel, dim3((unsigned)args.mblocks * (unsigned)args.batch), dim3(threads), lds, stream, args);
-  return hipGetLastError();
+  // A launch holds fewer than 2^32 work items, which sixteen rows per 512 threads reach at 134 million rows: such a grid goes
+  // out in pieces (the fp64 kernel's 256 threads own 32 rows; it takes what one launch holds).
+  const unsigned long long blocks = (unsigned long long)args.mblocks * (unsigned long long)args.batch;
+  if (blocks > 0x7fffffffull) return hipErrorInvalidConfiguration;
+  const unsigned long long most = args.f64 ? blocks : kLaunchBlocks;
+  F32ChainArgs piece = args;
+  for (unsigned long long at = 0; at < blocks && e == hipSuccess; at += most) {
+    piece.block0 = (unsigned)at;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(blocks - at < most ? blocks - at : most)), dim3(threads), lds, stream, piece);
+    e = hipGetLastError();
+  }
+  return e;
 }
 
 template <int DT, int RT, bool EXACT, bool KL, bool SM>

@@ -311,6 +311,22 @@ def test_fp32_chain_on_large_values_and_climbing_scores(oracle, shape):
         assert rel <= 1e-5, (b_layout, mx, rel)
 
 
+def test_fp32_chain_beyond_the_work_items_of_one_launch():
+    """2^28 rows: 8.4 million workgroups of 512 threads, more than the 2^32 work items a launch holds."""
+    M, L, dev = (1 << 28) + 40, 3, "cuda:0"
+    gen = torch.Generator(device=dev).manual_seed(8)
+    a = torch.randn(1, M, 1, device=dev, generator=gen)
+    b, c = (torch.randn(*s, device=dev, generator=gen) for s in ((1, 1, L), (1, L, 1)))
+    f = torch.full((1, M, 1), float("nan"), device=dev)
+    tile = chain.select_tile(chain.bmm_chain_desc(a, b, c, f, "softmax"))
+    assert tile.grid_x * tile.block_threads > 1 << 32
+    chain.run_bmm_chain(a, b, c, f, "softmax")
+    for at in range(0, M, 1 << 25):
+        rows = slice(at, at + (1 << 25))
+        want = torch.softmax(a[0, rows] * b[0], -1) @ c[0]
+        assert float((f[0, rows] - want).abs().max()) <= 1e-5, at  # fp32 sums of three terms of order one
+
+
 @pytest.mark.parametrize("shape", [(1, 512, 64, 64, 64), (3, 100, 24, 40, 72), (2, 64, 128, 128, 200)])
 @pytest.mark.parametrize("inter", ["cast", "relu", "softmax"])
 def test_fp64_chain_vs_oracle(oracle, shape, inter):
