@@ -31,6 +31,10 @@ int fail(int code, const char* fmt, ...) {
   return code;
 }
 
+// What one launch holds: fewer than 2^32 work items.  The kernels that give few rows or pixels to many threads reach that
+// at sizes the general kernels still take, which keep them.
+bool launchable(long long workgroups, int threads) { return workgroups < (1LL << 32) / threads; }
+
 bool aligned(const void* p, size_t a) { return (reinterpret_cast<uintptr_t>(p) % a) == 0; }
 
 // Number of compute units of the current device (cached per thread).
@@ -240,14 +244,16 @@ int plan_bmm(const ditto_bmm_chain_desc* d, BmmPlan* plan, bool need_device) {
           if (sm || plan->qt != 1) best = 1e30;
           const double key = (sm ? 1.0 : 0.9) * (kl_b ? 1.07 : 1.0) * d->L;
           for (int nw = 4; nw <= 8; nw += 4) {
-            const long long rounds = (((d->M + 32 * nw - 1) / (32 * nw)) * d->batch + cus - 1) / cus;
+            const long long wgs = ((d->M + 32 * nw - 1) / (32 * nw)) * d->batch, rounds = (wgs + cus - 1) / cus;
+            if (!launchable(wgs, 64 * nw)) continue;
             const double cost = nw == 4 ? (rounds == 1 ? 2.3 + 0.0131 * key : 2.1 + rounds * (1.1 + 0.0114 * key))
                                         : (rounds == 1 ? 2.9 + 0.0196 * key : 2.1 + rounds * (2.8 + 0.0226 * key));
             if (cost < best) best = cost, plan->rows_dt = 5, plan->rows_nw = nw;
           }
         }
         for (int r = 1; r <= 2; ++r) {
-          const long long rounds = (((d->M + 16 * r - 1) / (16 * r)) * d->batch + cus - 1) / cus;
+          const long long wgs = ((d->M + 16 * r - 1) / (16 * r)) * d->batch, rounds = (wgs + cus - 1) / cus;
+          if (!launchable(wgs, 64 * ditto::kSplitWaves)) continue;
           const double cost = rounds * (start[r - 1] + per_key[r - 1] * d->L) * (!kl_b ? 1.0 : dt == 8 ? 1.3 : 1.15);
           if (cost < best) best = cost, rt = r;
         }
@@ -285,14 +291,15 @@ int plan_bmm(const ditto_bmm_chain_desc* d, BmmPlan* plan, bool need_device) {
           const long long a384 = plan_rows_384(d->M, d->batch, cus), rest = d->M - 384 * a384;
           take = d->L <= 512 && (plan->qt == 2 || a384 + (rest > 0 ? (rest + 255) / 256 : 0) >= rows256);
         }
-        if (take) plan->rows_dt = 8, plan->rows_nw = 8;
+        if (take && launchable(n8, 512)) plan->rows_dt = 8, plan->rows_nw = 8;
       }
       if (d->tile_variant == 0 && dt == 4 && rt == 0 && !sm && n8 >= 2LL * cus && d->L <= 1024) {
         // Heads of up to 64 without softmax from two 256-row workgroups per compute unit on, up to 1024 keys: 512 x 197 x 197 16.8 ->
         // 12.2 us, 256 x 400 x 400 20.0 -> 16.6 (B [K][L] 22.3 -> 18.0), 256 x 577 x 577 35.0 -> 29.9, 128 x 1024 x 1024 35.3 -> 33.8;
         // below that the 64-row kernel's grain is worth more (160 x 400 x 400 13.6 against 15.4), and so it is with softmax
         // (256 x 400 x 400 21.0 against 22.8).
-        plan->rows_dt = 4, plan->rows_nw = d->M <= 128 ? 4 : 8;
+        const int nw = d->M <= 128 ? 4 : 8;
+        if (launchable(((d->M + 32 * nw - 1) / (32 * nw)) * d->batch, 64 * nw)) plan->rows_dt = 4, plan->rows_nw = nw;
       }
       if (plan->rows_nw > 0) {
         plan->nb = (int)((d->M + 32 * plan->rows_nw - 1) / (32 * plan->rows_nw));
@@ -564,6 +571,7 @@ bool plan_dw_tiles(const ditto_conv_chain_desc* d, long long P, long long Q, Con
     const double cost = full * (per_round > cus ? pair : alone) + (rest > cus ? pair : rest > 0 ? alone : 0);
     if (t == 1 || cost < best) best = cost, th = t;
   }
+  if (!launchable(d->N * ((P + th - 1) / th), 64 * ditto::kDtWaves)) return false;
   ditto::DwTilesArgs& a = plan->dwtargs;
   a.N = (int)d->N; a.C0 = (int)d->C0; a.H = (int)d->H; a.W = (int)d->W; a.C2 = (int)d->C2;
   a.P = (int)P; a.Q = (int)Q; a.stride = (int)d->stride1;
@@ -876,6 +884,8 @@ bool plan_conv_tiles(const ditto_conv_chain_desc* d, long long P, long long Q, b
       break;
     }
   }
+  const ditto::ConvTilesSplit w = ditto::conv_tiles_split((int)d->C1, (int)(d->R1 * d->S1) * c0p / 32);
+  if (!launchable(d->N * ((P + th - 1) / th), 64 * w.wc * w.wp)) return false;
   ditto::ConvTilesArgs& a = plan->targs;
   a.N = (int)d->N; a.C0 = (int)d->C0; a.H = (int)d->H; a.W = (int)d->W; a.C1 = (int)d->C1; a.C2 = (int)d->C2;
   a.R = (int)d->R1; a.S = (int)d->S1; a.pad = (int)d->pad1; a.stride = (int)d->stride1;
@@ -894,7 +904,6 @@ bool plan_conv_tiles(const ditto_conv_chain_desc* d, long long P, long long Q, b
   plan->w1p_bytes = ditto::conv_tiles_w1_bytes((int)d->C1, c0p, (int)(d->R1 * d->S1));
   plan->w2p_bytes = ditto::conv_tiles_w2_bytes((int)d->C2, c1p);
   ditto_tile_param& t = plan->tile;
-  const ditto::ConvTilesSplit w = ditto::conv_tiles_split((int)d->C1, (int)(d->R1 * d->S1) * c0p / 32);
   t.block_threads = 64 * w.wc * w.wp;
   t.block_m = th * (int)Q;
   t.block_l = c1p;
@@ -927,7 +936,9 @@ bool plan_conv13_tiles(const ditto_conv_chain_desc* d, bool forced, ConvPlan* pl
   for (int w = 2; w <= 4; w += 2)
     for (int t = 1; t <= d->H && t * d->W <= ditto::conv13_tiles_slots(w); ++t) {
       if (ditto::conv13_tiles_lds_bytes(t, (int)d->W, w) > 160 * 1024) break;
-      const long long wgs = d->N * ((d->H + t - 1) / t), rounds = (wgs + cus - 1) / cus, tiles = (t * d->W + 16 * w - 1) / (16 * w);
+      const long long wgs = d->N * ((d->H + t - 1) / t);
+      if (!launchable(wgs, 128 * w)) continue;
+      const long long rounds = (wgs + cus - 1) / cus, tiles = (t * d->W + 16 * w - 1) / (16 * w);
       const double halo = (t + 2.0) * d->W;
       const double one = w == 2 ? 1.7 + 0.3 * tiles + 0.0065 * halo : 2.6 + 0.45 * tiles + 0.004 * halo;
       const double cost = one * (1.0 + (w == 2 ? 0.67 : 1.0) * (rounds - 1));

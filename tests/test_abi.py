@@ -201,6 +201,39 @@ def test_conv_tile_choice_without_gpu():
     assert tile.variant == 4043
 
 
+def test_grids_beyond_one_launch_stay_on_the_kernels_that_take_them():
+    """A launch holds fewer than 2^32 work items.  The kernels that give few rows or pixels to many threads reach that
+    where the general ones do not, and the general ones keep those sizes (plans only: nothing is launched)."""
+    lib = _lib.load()
+    tile = _lib.TileParam()
+
+    def bmm(batch, M, D, L, inter, b_layout):
+        d = _desc(batch=batch, M=M, N=D, K=D, L=L, inter_op=inter, b_layout=b_layout, a_batch_stride=M * D, a_row_stride=D,
+                  b_batch_stride=0, b_row_stride=L if b_layout == _lib.B_KL else D, c_batch_stride=0, c_row_stride=D,
+                  f_batch_stride=M * D, f_row_stride=D)
+        assert lib.ditto_bmm_chain_select_tile(ctypes.byref(d), ctypes.byref(tile)) == _lib.OK
+        return tile.variant, tile.grid_x * tile.block_threads
+
+    for M, D, L, inter, layout, near, far in (
+            (8, 8, 512, _lib.INTER_SOFTMAX, _lib.B_LK, 2041, 644),      # key-splitting kernel: 512 threads for 16 rows
+            (200, 8, 64, _lib.INTER_CAST, _lib.B_KL, 2148, 642),        # 32 rows per wave: eight waves for 200 rows
+            (256, 128, 64, _lib.INTER_CAST, _lib.B_KL, 2188, 1282)):
+        assert bmm((8 << 20) - 1, M, D, L, inter, layout)[0] == near, (M, D)
+        variant, items = bmm(8 << 20, M, D, L, inter, layout)
+        assert variant == far and items < 1 << 32, (M, D)
+
+    def conv(**kw):
+        assert lib.ditto_conv_chain_select_tile(ctypes.byref(_conv_desc(**kw)), ctypes.byref(tile)) == _lib.OK
+        return tile.variant // 100, tile.grid_x * tile.block_threads
+
+    # tiles of whole output rows: 256 or 512 threads for at most 128 or 256 pixels
+    for kw, near, far in ((dict(C0=1, C1=8), 32, 30), (dict(C0=1, C1=8, R1=1, S1=1, pad1=0, R2=3, S2=3, pad2=1), 33, 35),
+                          (dict(C0=2, C1=32, groups1=2), 41, 40)):
+        assert conv(N=64, H=1000, W=15, C2=1, **kw)[0] == near, kw
+        family, items = conv(N=65000, H=3000, W=15, C2=1, **kw)
+        assert family == far and items < 1 << 32, (kw, family, items)
+
+
 def test_run_rejects_bad_arguments_before_touching_the_device():
     lib = _lib.load()
     # null pointers are refused by validation, no launch happens
