@@ -232,6 +232,16 @@ __global__ __launch_bounds__(64 * WC * WP) void conv_tiles_kernel(ConvTilesArgs 
   };
   load_w2(wave);
   wg_sync();  // the halo rows are no longer read
+  // The channels that C1 is padded by are zero also under an infinite pixel, which meets zero weights there.  Where they are
+  // rare as one branch here; eight waves mask every store instead, which costs them less (one image of 128 x 28 x 28 -> 256 ->
+  // 128 8.9 us, 9.0 with the branch; masking stores costs the other splits up to 1 %).
+  constexpr bool kMaskStores = NW == 8;
+  if (!kMaskStores && p.C1 < C1P)
+#pragma unroll
+    for (int m = 0; m < MC; ++m)
+      if (16 * (wc * MC + m) + 4 * q >= p.C1)
+#pragma unroll
+        for (int t = 0; t < PT; ++t) acc[m][t] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int m = 0; m < MC; ++m)
 #pragma unroll
@@ -241,7 +251,10 @@ __global__ __launch_bounds__(64 * WC * WP) void conv_tiles_kernel(ConvTilesArgs 
 #pragma unroll
         for (int r = 0; r < 4; ++r) v[r] = fmaxf(v[r], 0.f);
       const typename Elem<T>::v2 lo = cvt2<T>(v[0], v[1]), hi = cvt2<T>(v[2], v[3]);
-      *reinterpret_cast<V4*>(Ms + (16 * (wp * PT + t) + c) * MS + 16 * (wc * MC + m) + 4 * q) = V4{lo[0], lo[1], hi[0], hi[1]};
+      const int c1 = 16 * (wc * MC + m) + 4 * q;
+      V4 x = {lo[0], lo[1], hi[0], hi[1]};
+      if (kMaskStores && c1 >= p.C1) x = V4{0, 0, 0, 0};
+      *reinterpret_cast<V4*>(Ms + (16 * (wp * PT + t) + c) * MS + c1) = x;
     }
   wg_sync();
   const T* const mb = Ms + PO * c * MS + 8 * q;

@@ -1043,3 +1043,33 @@ def test_conv1x1_conv3x3_on_row_tiles(oracle, case, dtype):
     chain.run_conv_chain(x, w1, w2, y, desc=desc, workspace=ws, prepared=True)
     torch.cuda.synchronize()
     assert np.array_equal(y.float().cpu().numpy(), got) and bool(torch.isnan(out[0]))
+
+
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+@pytest.mark.parametrize("case", [
+    # tile variant, C0, C1, first filter, second filter, groups: channel counts that fill no tile in every split of the waves
+    (3200, 16, 8, 3, 1, 1), (3200, 32, 32, 3, 1, 1), (3200, 64, 40, 3, 1, 1), (3200, 24, 72, 3, 1, 1), (3200, 40, 136, 1, 1, 1),
+    (3200, 16, 200, 3, 1, 1), (3300, 24, 40, 1, 3, 1), (4100, 24, 24, 3, 1, 24), (4100, 6, 96, 3, 1, 6),
+])
+def test_infinite_pixels_stay_where_the_filters_take_them(dtype, case):
+    """Padded channels take no part: with filters of one sign an infinite input pixel makes exactly the outputs infinite
+    that its two filters reach, and none NaN (zero times infinity in a padded channel)."""
+    tv, C0, C1, R1, R2, groups = case
+    H, W, C2 = 11, 13, 24
+    gen = torch.Generator().manual_seed(C1)
+    x = torch.randn(2, C0, H, W, generator=gen)
+    w1 = torch.rand(C1, C0 // groups, R1, R1, generator=gen) * 0.1 + 0.01
+    w2 = torch.rand(C2, C1, R2, R2, generator=gen) * 0.1 + 0.01
+    x[0, C0 // 2, 4, 5] = float("inf")
+    x[1, C0 - 1, H - 1, W - 1] = float("inf")
+    dt = TORCH_DTYPES[dtype]
+    x, w1, w2 = (t.to(dt) for t in (x, w1, w2))
+    mid = torch.nn.functional.conv2d(x.double(), w1.double(), padding=R1 // 2, groups=groups)
+    want = torch.nn.functional.conv2d(mid.to(dt).double(), w2.double(), padding=R2 // 2).float()
+    assert torch.isinf(want).any() and not torch.isnan(want).any()
+    y = torch.full((2, C2, H, W), float("nan"), device="cuda:0", dtype=dt)
+    chain.run_conv_chain(x.cuda(), w1.cuda(), w2.cuda(), y, R1 // 2, 1, R2 // 2, 1, groups1=groups, tile_variant=tv)
+    y = y.cpu()
+    assert torch.equal(torch.isinf(y), torch.isinf(want)) and not torch.isnan(y).any()
+    fin = torch.isfinite(want)
+    assert errors(y.float()[fin].numpy(), want.to(dt).float()[fin].numpy())[1] <= REL_L2
