@@ -1793,7 +1793,13 @@ extern "C" int ditto_conv_chain_run_static(const ditto_conv_chain_desc* d, const
   ConvPlan plan;
   int rc = plan_conv(d, &plan, true);
   if (rc != DITTO_OK) return rc;
-  const size_t need = plan.w1p_bytes + plan.w2p_bytes;
+  size_t need = plan.w1p_bytes + plan.w2p_bytes;
+  if (need > (size_t)DITTO_STATIC_WORKSPACE_BYTES && (plan.tiles || plan.tiles13) && d->tile_variant == 0) {
+    // the kernels on row tiles repack both weights, the general one (which the call then runs) W1 alone
+    rc = plan_conv(d, &plan, true, 4, false);
+    if (rc != DITTO_OK) return rc;
+    need = plan.w1p_bytes + plan.w2p_bytes;
+  }
   if (need > (size_t)DITTO_STATIC_WORKSPACE_BYTES)
     return fail(DITTO_EWORKSPACE, "the repacked weights take %zu bytes, the static workspace holds %zu", need,
                 (size_t)DITTO_STATIC_WORKSPACE_BYTES);

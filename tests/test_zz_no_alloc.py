@@ -92,3 +92,21 @@ def test_static_workspace_entry_under_graph_capture(oracle):
         assert torch.equal(y, want), it
         call()
         torch.cuda.synchronize()
+
+
+def test_static_workspace_entry_where_only_the_general_kernel_fits(oracle):
+    """Wide outputs on ragged rows run on row tiles, whose repacked weights (both tensors) can exceed the static array
+    where the general kernel's (W1 alone) do not: the call runs on the general kernel."""
+    N, C0, H, W, C1, C2 = 1, 512, 5, 9, 256, 4096
+    X, W1, W2 = oracle.make_conv_chain_inputs(N, C0, H, W, C1, C2, 3, 1, "float16", seed=4, w_std=0.05)
+    x, w1, w2 = to_dev(X, "float16"), to_dev(W1, "float16"), to_dev(W2, "float16")
+    want, got = (torch.full((N, C2, H, W), float("nan"), device=x.device, dtype=torch.float16) for _ in range(2))
+    desc = chain.conv_chain_desc(x, w1, w2, got)
+    assert chain.select_tile(desc).variant // 100 == 32 and chain.conv_chain_workspace_bytes(desc) > _lib.STATIC_WORKSPACE_BYTES
+    general = chain.conv_chain_desc(x, w1, w2, want, tile_variant=3000)
+    assert chain.conv_chain_workspace_bytes(general) <= _lib.STATIC_WORKSPACE_BYTES
+    chain.run_conv_chain(x, w1, w2, want, desc=general)
+    _lib.check(_lib.load().ditto_conv_chain_run_static(ctypes.byref(desc), x.data_ptr(), w1.data_ptr(), w2.data_ptr(),
+                                                       got.data_ptr(), torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    assert torch.isfinite(want).all() and torch.equal(got, want)
