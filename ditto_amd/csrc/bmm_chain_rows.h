@@ -211,11 +211,12 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
         }
         if (__builtin_amdgcn_ballot_w64(raise) != 0) {
           // the first tile sets the reference (nothing is accumulated yet); in the exact walk it then follows the running
-          // maximum, lazily
+          // maximum, lazily, and a first tile of scores of minus infinity alone leaves it at the lowest value (the optimistic
+          // walk ends with a NaN sum on such a row: the test there would cost it 1 % at 2000 keys)
 #pragma unroll
           for (int j = 0; j < RT; ++j) {
             const float m = quad_max(mx[j]);
-            const float up = it == 0 ? m : fmaxf(ref[j], m);
+            const float up = it > 0 ? fmaxf(ref[j], m) : SAFE ? fmaxf(kNoKeyYet, m) : m;
             const float alpha = it == 0 ? 1.f : __builtin_amdgcn_exp2f(ref[j] - up);
             ref[j] = up;
             ls[j] *= alpha;
@@ -300,7 +301,9 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     if constexpr (kSoftmax && !decltype(safe_c)::value) {
       // a sum that is not finite sends the workgroup through the exact walk (the tiles are its common property)
-      const bool bad = busy && (!(ls[0][0] < INFINITY) || !(ls[1][0] < INFINITY));
+      // (by its bits: a comparison may be compiled as if there were no NaN)
+      auto not_finite = [](float x) { return (__builtin_bit_cast(int, x) & 0x7f800000) == 0x7f800000; };
+      const bool bad = busy && (not_finite(ls[0][0]) || not_finite(ls[1][0]));
       if (__builtin_amdgcn_ballot_w64(bad) != 0 && lane == 0) *flag = 1;
     }
     wg_sync();

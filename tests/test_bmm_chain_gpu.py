@@ -239,6 +239,20 @@ def test_kernel_of_32_rows_per_wave(oracle, shape, dtype, inter):
             assert np.array_equal(narrow, oracle.np_round_to(got, dtype)), (variant, b_layout)
 
 
+@pytest.mark.parametrize("variant,D", [(2144, 64), (2148, 64), (2154, 80), (2158, 80), (2188, 128)])
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+@pytest.mark.parametrize("keys", sorted(MASKED_KEYS))
+def test_kernel_of_32_rows_per_wave_on_masked_keys(oracle, variant, D, dtype, keys):
+    batch, M, L = 2, 137, 280
+    A, B, C = masked_scores(oracle, batch, M, D, D, L, dtype, MASKED_KEYS[keys](L), seed=77 + D)
+    want = oracle.bmm_chain_f64(A, B, C, inter="softmax", scale=0.2)
+    for b_layout in ("KL", "LK"):
+        got = run_chain(A, B, C, dtype, "softmax", 0.2, b_layout, "float32", variant)
+        assert np.isfinite(got).all(), b_layout
+        mx, rel = errors(got, want)
+        assert mx <= 4e-2 and rel <= (REL_L2 if dtype == "float16" else 2.0e-3), (b_layout, mx, rel)
+
+
 @pytest.mark.parametrize("shape", [(1, 512, 64, 64, 64), (3, 100, 24, 40, 72), (2, 64, 128, 128, 200)])
 @pytest.mark.parametrize("inter", ["cast", "relu", "softmax"])
 def test_fp32_chain_vs_oracle(oracle, shape, inter):
