@@ -22,11 +22,20 @@ import os
 from ... import _lib, chain
 from ...hardware import query_hw_param
 
-# kernel codes of the fp16/bf16 chain: four waves x 32 | 64 rows, eight waves x 32 rows (staggered phases,
-# software pipelined, on the 16x16x32 MFMA with 256-row workgroups, the same with 384-row workgroups for the
-# first row blocks: the library refuses these two unless B is stored [L][K]), four waves with 64-row workgroups on
-# the 16x16x32 MFMA (a wave owns 16 rows and all keys | 32 rows and half the keys; head size up to 64)
-FP_VARIANT_CODES = (1, 2, 8, 9, 6, 7, 4, 5)
+# kernel codes of the fp16/bf16 chain: four waves with 64-row workgroups on the 16x16x32 MFMA (a wave owns 16 rows and
+# all keys | 32 rows and half the keys; head size up to 64), four waves x 32 | 64 rows, eight waves x 32 rows (staggered
+# phases, software pipelined, on the 16x16x32 MFMA with 256-row workgroups, the same with 384-row workgroups for the
+# first row blocks)
+FP_VARIANT_CODES = (4, 5, 1, 2, 8, 9, 6, 7)
+# by the head size's width class (column tiles of 16 that it is padded to): the kernel whose waves split the keys, with
+# workgroups of 16 | 32 rows, and the kernel of 32 rows per wave with four | eight waves
+FP_SPLIT_VARIANTS = {4: (2041, 2042), 5: (2051, 2052), 8: (2081, 2082)}
+FP_ROWS_VARIANTS = {4: (2144, 2148), 5: (2154, 2158), 8: (2188,)}
+# Beyond these the two were behind at every size measured and are left out: rounds of key-splitting workgroups over the
+# compute units (each pulls all keys for its 16 or 32 rows), keys for 32 rows per wave outside heads of 65 to 80 columns
+# (80 x 1024 x 1024 x 128 68.4 us against 65.4; with softmax at 64 columns at any number, 96 x 512 x 512 13.6 / 10.9)
+FP_SPLIT_ROUNDS = 4
+FP_ROWS_KEYS = 1024
 
 
 # int8 chain: 8000 + 10 * (row tiles of 32 per workgroup) + depth of the ring of staged weight chunks
@@ -44,38 +53,46 @@ class TuneEntry:
         return {"record": self.record, "value": self.value}
 
 
+def _fp_variants(desc, groups):
+    dmax = max(desc.K, desc.N)
+    width = 4 if dmax <= 64 else 5 if dmax <= 80 else 8
+    ids = [v for v in FP_SPLIT_VARIANTS[width]
+           if -(-desc.M // (16 * (v % 10))) * desc.batch <= FP_SPLIT_ROUNDS * groups]
+    if width == 5 or (desc.L <= FP_ROWS_KEYS and not (width == 4 and desc.inter_op == _lib.INTER_SOFTMAX)):
+        ids += FP_ROWS_VARIANTS[width]
+    return ids + [(64 if dmax <= 64 else 128) * 10 + q for q in FP_VARIANT_CODES]
+
+
 def make_tile_variant_space(desc):
     """Variants of the library that can run ``desc`` (capacity filter: the library rejects the
-    ones whose tile does not fit), as a list of tile descriptions."""
+    ones whose tile does not fit), as a list of tile descriptions: the library's own choice first."""
     lib = _lib.load()
     tile = _lib.TileParam()
     auto = copy.copy(desc)
     auto.tile_variant = 0
     _lib.check(lib.ditto_bmm_chain_select_tile(ctypes.byref(auto), ctypes.byref(tile)))
-    space = []
+    space = [tile.to_json()]
     if desc.in_dtype in (_lib.F16, _lib.BF16):
-        for q in FP_VARIANT_CODES:
-            d = copy.copy(desc)
-            d.tile_variant = tile.head_pad * 10 + q
-            t = _lib.TileParam()
-            if lib.ditto_bmm_chain_select_tile(ctypes.byref(d), ctypes.byref(t)) == _lib.OK:
-                space.append(t.to_json())
-    elif desc.in_dtype == _lib.I8:
-        for variant in I8_VARIANTS:
-            d = copy.copy(desc)
-            d.tile_variant = variant
-            t = _lib.TileParam()
-            if lib.ditto_bmm_chain_select_tile(ctypes.byref(d), ctypes.byref(t)) == _lib.OK:
-                space.append(t.to_json())
+        ids = _fp_variants(desc, int(query_hw_param("gpu.hip.MI355X").num_groups))
     else:
-        space.append(tile.to_json())
+        ids = I8_VARIANTS if desc.in_dtype == _lib.I8 else ()
+    for variant in ids:
+        d = copy.copy(desc)
+        d.tile_variant = variant
+        t = _lib.TileParam()
+        if variant != tile.variant and lib.ditto_bmm_chain_select_tile(ctypes.byref(d), ctypes.byref(t)) == _lib.OK:
+            space.append(t.to_json())
     return space
+
+
+# what one compute unit draws from its L2: 64 bytes per clock
+L2_BYTES_PER_S = 64 * 2.1e9
 
 
 def evaluate_param_hip(desc, tile, hw_param=None):
     """Analytic score of a tile (lower is better; 1e10 = over capacity), the shape of the
-    reference's filter: rounds of workgroups over the CUs x bytes each workgroup stages through
-    LDS / LDS bandwidth, plus the MFMA time of a round.  It ranks variants; it is not a time."""
+    reference's filter: rounds of workgroups over the CUs x the longest of the time its bytes take
+    through LDS, the time they take from L2 (what bounds workgroups of few rows) and the MFMA time of a round.  It ranks variants; it is not a time."""
     hw = hw_param or query_hw_param("gpu.hip.MI355X")
     if tile["lds_bytes"] > hw.shared_memory_per_group_kb * 1024:
         return 1e10
@@ -87,8 +104,9 @@ def evaluate_param_hip(desc, tile, hw_param=None):
     staged = desc.L * (desc.K + desc.N) * elem                     # B and C tiles of one workgroup
     flops = 2.0 * tile["block_m"] * desc.L * (desc.K + desc.N)     # of one workgroup
     lds_s = staged / (hw.shared_memory_bandwidth_gbs * 1e9 / groups)
+    l2_s = staged / L2_BYTES_PER_S
     mfma_s = flops * per_cu / (2.5e15 / groups)
-    return rounds * max(lds_s, mfma_s)
+    return rounds * max(lds_s, l2_s, mfma_s)
 
 
 def _log(log_file, wkl_key, entry):
@@ -98,12 +116,13 @@ def _log(log_file, wkl_key, entry):
 
 def select_tile_variant(wkl_key, log_file, A, B, C, F, inter_op="softmax", softmax_scale=1.0, top=3,
                         min_repeat_ms=50):
-    """Measure the ``top`` analytically best variants for these operands, append every measurement
-    to ``log_file`` and return the best ``TuneEntry``."""
+    """Measure the library's own choice and the analytically best other variants, ``top`` in all, for these
+    operands, append every measurement to ``log_file`` and return the best ``TuneEntry``."""
     import torch
 
     desc = chain.bmm_chain_desc(A, B, C, F, inter_op, softmax_scale)
-    space = sorted(make_tile_variant_space(desc), key=lambda t: evaluate_param_hip(desc, t))[:max(1, top)]
+    own, *others = make_tile_variant_space(desc)
+    space = [own] + sorted(others, key=lambda t: evaluate_param_hip(desc, t))[:max(0, top - 1)]
     best = None
     for tile in space:
         d = copy.copy(desc)

@@ -695,6 +695,25 @@ def test_tile_variant_tuning_round_trip(tmp_path, oracle):
     assert (f.float() - ref).abs().max().item() <= MAX_ABS
 
 
+def test_tuning_heads_of_80_columns(tmp_path, oracle):
+    # ViT-Huge attention: the kernels padded to 80 columns are measured, the library's own among them
+    from ditto_amd.auto_schedule.schedulers import chimera_integrate as ci
+
+    A, B, C = oracle.make_gemm_chain_inputs(16, 197, 80, 80, 197, "float16", seed=2)
+    q, k, v = to_dev(A, "float16"), to_dev(np.ascontiguousarray(B.transpose(0, 2, 1)), "float16"), to_dev(C, "float16")
+    f = torch.empty_like(q)
+    log = str(tmp_path / "chimera_80.log")
+    desc = chain.bmm_chain_desc(q, k.transpose(1, 2), v, f, "softmax", 80 ** -0.5)
+    key = ci.workload_key(desc)
+    variant = ci.auto_schedule_bmm_chain_hip(key, log, q, k.transpose(1, 2), v, f, "softmax", 80 ** -0.5)
+    lines = open(log).read().strip().splitlines()
+    assert len(lines) == 3 and '"variant": %d' % chain.select_tile(desc).variant in lines[0]
+    f.fill_(float("nan"))
+    chain.run_bmm_chain(q, k.transpose(1, 2), v, f, "softmax", 80 ** -0.5, tile_variant=variant)
+    want = oracle.bmm_chain_f64(A, B, C, inter="softmax", scale=80 ** -0.5)
+    assert errors(f.float().cpu().numpy(), want)[1] <= REL_L2
+
+
 def test_strided_views_and_errors():
     dev = "cuda:0"
     torch.manual_seed(0)

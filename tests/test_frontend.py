@@ -227,6 +227,40 @@ def test_tile_variant_space_and_analytic_filter():
     assert ci.workload_key(big) != ci.workload_key(small)
 
 
+@pytest.mark.parametrize("shape", [
+    # (batch, M, L, D, inter): ViT-Huge heads of 80 on few and on many rows, 128 columns on short sequences, few rows of 64,
+    # without softmax on a large grid, B stored [K][L]
+    (16, 197, 197, 80, "softmax", "LK"), (256, 197, 197, 80, "softmax", "LK"), (160, 197, 197, 128, "softmax", "LK"),
+    (8, 512, 2048, 64, "softmax", "LK"), (1, 512, 256, 64, "cast", "KL"), (512, 197, 197, 64, "cast", "LK"),
+    (64, 4096, 4096, 128, "softmax", "LK"), (12, 1600, 1600, 80, "relu", "KL"), (2, 4096, 4096, 128, "softmax", "KL"),
+])
+def test_tuning_measures_what_the_library_would_run(shape):
+    """The library's own kernel is a candidate at every size, and the first: tuning can confirm it, and never pins a call
+    to something slower because the faster kernel was not looked at.  Every candidate's id can be forced."""
+    from ditto_amd import _lib, chain
+    from ditto_amd.auto_schedule.schedulers import chimera_integrate as ci
+
+    batch, M, L, D, inter, layout = shape
+    d = _lib.BmmChainDesc()
+    d.abi_version = _lib.ABI_VERSION
+    d.in_dtype, d.acc_dtype, d.out_dtype = _lib.BF16, _lib.F32, _lib.BF16
+    d.inter_op = chain.INTER_OPS[inter]
+    d.batch, d.M, d.N, d.K, d.L = batch, M, D, D, L
+    d.b_layout, d.b_row_stride = (_lib.B_LK, D) if layout == "LK" else (_lib.B_KL, (L + 7) // 8 * 8)
+    if layout == "KL":
+        d.L = (L + 7) // 8 * 8
+    d.a_row_stride = d.c_row_stride = d.f_row_stride = D
+    d.a_batch_stride = d.f_batch_stride = M * D
+    d.b_batch_stride = d.c_batch_stride = d.L * D
+    d.softmax_scale = 0.125
+    own = chain.select_tile(d).variant
+    space = [t["variant"] for t in ci.make_tile_variant_space(d)]
+    assert space[0] == own and len(space) == len(set(space)) and len(space) >= 4
+    for v in space:
+        d.tile_variant = v
+        assert chain.select_tile(d).variant == v
+
+
 def test_conv_tile_variant_space():
     """Kernel families that can run a conv chain, as the tuner enumerates them (no device needed)."""
     import torch
