@@ -189,22 +189,45 @@ def auto_schedule_bmm_chain_hip(key, log_file, A, B, C, F, inter_op="softmax", s
 # ---- conv -> conv chains: the same measurement and log over the conv kernel families ------------
 # family ids of ``ditto_conv_chain_desc.tile_variant`` (include/ditto_chain.h): general kernel with a 1x1 second
 # convolution, general kernel with the second convolution through LDS, W2 resident in LDS, the two row pipelines;
-# depthwise: the tile kernels and the two row-streaming ones
+# depthwise: the persistent and plain kernels and the two row-streaming ones
 CONV_FAMILY_IDS = (3000, 3500, 3600, 3700, 3800, 4000, 4024, 4025)
+# tiles of whole output rows: dense -> 1x1, 1x1 -> 3x3, depthwise
+CONV_ROW_TILE_IDS = (3200, 3300, 4100)
+
+
+def _row_pipeline_ahead(desc, tile):
+    """Whether ``tile`` is a row pipeline's (or a depthwise row-streaming kernel's) at a size where the kernels on row
+    tiles are behind it (58 sizes measured; ahead on six of them, by up to 5 % of a 7 us call): channels that fill its
+    padding, and either bands of more than five rows over which its start is spread (32 x 64 x 56 x 56 1x1 -> 64 -> 3x3 64
+    12.3 us against 14.1; bands of five, 40 x 40, 10.1 against 8.8) or a wide output, whose stores only it overlaps
+    (16 x 64 x 40 x 40 3x3 -> 64 -> 256 10.5 against 12.1, -> 64 9.6 against 7.9)."""
+    variant, band = tile["variant"], tile["grid_y"]
+    if variant in (4024, 4025):
+        return desc.C0 > 16 and band > 5
+    if variant // 100 not in (37, 38) or desc.C0 <= 32 or desc.C1 <= 32:
+        return False
+    return band > 5 or (variant // 100 == 37 and desc.C2 >= 192)
 
 
 def make_conv_tile_variant_space(desc):
-    """Kernels of the library that can run the conv chain ``desc``: one tile description per family that accepts
-    it (the library refuses the others), each carrying the exact variant id the family resolves to."""
+    """Kernels of the library that can run the conv chain ``desc``: the library's own choice, then one tile description
+    per family that accepts it (the library refuses the others), each carrying the exact variant id the family resolves
+    to.  The kernels on row tiles are left out where a row pipeline is ahead of them (``_row_pipeline_ahead``)."""
     lib = _lib.load()
     space, seen = [], set()
-    for fam in (0,) + CONV_FAMILY_IDS:
-        d = copy.copy(desc)
-        d.tile_variant = fam
-        t = _lib.TileParam()
-        if lib.ditto_conv_chain_select_tile(ctypes.byref(d), ctypes.byref(t)) == _lib.OK and t.variant not in seen:
-            seen.add(t.variant)
-            space.append(t.to_json())
+
+    def add(families):
+        for fam in families:
+            d = copy.copy(desc)
+            d.tile_variant = fam
+            t = _lib.TileParam()
+            if lib.ditto_conv_chain_select_tile(ctypes.byref(d), ctypes.byref(t)) == _lib.OK and t.variant not in seen:
+                seen.add(t.variant)
+                space.append(t.to_json())
+
+    add((0,) + CONV_FAMILY_IDS)
+    if not any(_row_pipeline_ahead(desc, t) for t in space):
+        add(CONV_ROW_TILE_IDS)
     return space
 
 

@@ -286,6 +286,33 @@ def test_conv_tile_variant_space():
     assert ci.conv_workload_key(a) != ci.conv_workload_key(b)
 
 
+def test_conv_tuning_looks_at_the_kernels_on_row_tiles():
+    """Candidates wherever they can run, but for the sizes at which a row pipeline is ahead of them."""
+    import torch
+    from ditto_amd import chain
+    from ditto_amd.auto_schedule.schedulers import chimera_integrate as ci
+
+    def families(N, C0, H, C1, R1, C2, R2, groups=1, stride=1):
+        P = (H - 1) // stride + 1
+        x, w1 = torch.zeros(N, C0, H, H, dtype=torch.float16), torch.zeros(C1, C0 // groups, R1, R1, dtype=torch.float16)
+        w2, y = torch.zeros(C2, C1, R2, R2, dtype=torch.float16), torch.zeros(N, C2, P, P, dtype=torch.float16)
+        d = chain.conv_chain_desc(x, w1, w2, y, R1 // 2, stride, R2 // 2, 1, "cast", False, groups)
+        space = ci.make_conv_tile_variant_space(d)
+        assert space[0]["variant"] == chain.select_tile(d).variant
+        for t in space:  # every candidate's id can be forced
+            d.tile_variant = t["variant"]
+            assert chain.select_tile(d).variant == t["variant"]
+        return [t["variant"] // 100 for t in space]
+
+    assert families(2, 32, 147, 64, 3, 80, 1, stride=2) == [32, 30]    # the library's own choice, and the general kernel
+    assert 32 in families(32, 32, 56, 32, 3, 128, 1)                    # the general kernel is the own choice
+    assert 32 in families(16, 64, 40, 64, 3, 64, 1)                     # bands of three rows, a narrow output
+    assert families(16, 64, 40, 64, 3, 256, 1) == [37, 30]
+    assert 33 in families(32, 64, 40, 64, 1, 64, 3) and 33 in families(2, 64, 30, 64, 1, 64, 3)
+    assert 41 in families(4, 32, 56, 32, 3, 64, 1, groups=32) and 41 in families(4, 32, 56, 512, 3, 64, 1, groups=32)
+    assert 41 in families(32, 64, 56, 1024, 3, 64, 1, groups=64)
+
+
 def test_attention_layer_task_extraction_and_binding():
     """bert_inference.py:88-92 -- tasks keyed by layer fingerprint, attention layers bound to the
     chimera scheduler (chimera/task_binding.py:6-20), everything else to ansor."""
