@@ -41,7 +41,8 @@ def barriers_with_lds_in_flight(asm_text):
     """[(kernel, instruction index)] of every ``s_barrier`` that some path through the kernel reaches while an LDS
     access of the same wave may still be outstanding.  A forward may-analysis over the kernel's control-flow graph:
     the state is the sequence of LDS (and scalar-load) instructions issued since the counter last read zero,
-    ``s_waitcnt lgkmcnt(N)`` keeps the newest N of them, joins take the longer sequence."""
+    ``s_waitcnt lgkmcnt(N)`` keeps the newest N of them, joins take the longer sequence.  Lane shuffles
+    (``ds_bpermute`` and its like) count on the same counter but touch no LDS: in flight at a barrier they are harmless."""
     import collections
     found = []
     cur, body = None, []
@@ -97,9 +98,9 @@ def barriers_with_lds_in_flight(asm_text):
             i = work.popleft()
             s, t = state[i], ins[i]
             op = t.split()[0]
-            if op.startswith("ds_"):
+            if op.startswith("ds_") and not op.startswith(("ds_bpermute", "ds_permute", "ds_swizzle")):
                 s = (s + (1,))[-16:]
-            elif op.startswith(("s_load", "s_buffer_load")):
+            elif op.startswith(("s_load", "s_buffer_load", "ds_")):
                 s = (s + (2,))[-16:]
             elif op == "s_waitcnt":
                 m = re.search(r"lgkmcnt\((\d+)\)", t)
@@ -260,6 +261,8 @@ def test_bmm_chain_units_keep_their_counted_waits_exact(tmp_path, unit_name):
     assert untracked_memory_ops_in_direct_load_loops(text, loops) == []
     assert len({name for name, _, _ in loops}) == len(md)  # every kernel's tile loop was found and looked at
     assert barriers_with_lds_in_flight(text) == []
+    stores, bare = hidden_stores_without_wait_states(text)
+    assert stores > 0 and not bare
 
 
 def test_barrier_analysis_on_a_small_kernel():
@@ -279,6 +282,11 @@ _Z6kernelv:
 """
     # the first barrier is reachable over the branch with the write still in flight, the second is not
     assert barriers_with_lds_in_flight(text) == [("_Z6kernelv", 4)]
+    # a lane shuffle in flight touches no LDS; a write in front of it does, whatever the counter's newest entry is
+    shuffle = "_Z6kernelv:\n%s\tds_bpermute_b32 v2, v0, v1\n%s\ts_barrier\n\ts_endpgm\n.Lfunc_end0:\n"
+    assert barriers_with_lds_in_flight(shuffle % ("", "")) == []
+    assert barriers_with_lds_in_flight(shuffle % ("\tds_write_b32 v0, v1\n", "")) == [("_Z6kernelv", 2)]
+    assert barriers_with_lds_in_flight(shuffle % ("\tds_write_b32 v0, v1\n", "\ts_waitcnt lgkmcnt(1)\n")) == []
 
 
 def test_kernel_metadata_parser():
@@ -374,7 +382,32 @@ def test_wide_stores_in_inline_assembly_keep_their_data_registers(tmp_path):
     assert stores > 0 and not bare
 
 
-@pytest.mark.parametrize("unit_name", ["gemm_chain_i8", "gemm_chain_f32"])
+@pytest.mark.parametrize("unit_name,kernels", [("fp_split_f16", 24), ("fp_split_bf16", 24), ("fp_rows_f16", 20), ("fp_rows_bf16", 20)])
+def test_short_chain_units_keep_their_counted_waits_exact(tmp_path, unit_name, kernels):
+    """The same for the key-splitting kernel and the kernel of 32 rows per wave, which count their waits over untracked
+    direct loads too; and their output stores in inline assembly keep their data registers."""
+    hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+    if not os.path.exists(hipcc):
+        pytest.skip("hipcc not available")
+    unit = [u for u in build_ext.UNITS if u[0] == unit_name][0]
+    out = tmp_path / "unit.s"
+    flags = [f for f in build_ext.HIPCC_FLAGS if f != "-fPIC"]
+    cmd = [hipcc, *flags, "--cuda-device-only", "-S", *unit[2], os.path.join(CSRC, unit[1]), "-o", str(out)]
+    subprocess.run(cmd, check=True, capture_output=True)
+    text = out.read_text()
+    md = kernel_metadata(text)
+    assert len(md) == kernels  # widths and workgroup sizes x inter path x layout of B
+    for name, v in md.items():
+        assert v["vgpr_spill_count"] == 0, (name, v)
+    loops = []
+    assert untracked_memory_ops_in_direct_load_loops(text, loops) == []
+    assert len({name for name, _, _ in loops}) == kernels  # every kernel's walk was found and looked at
+    assert barriers_with_lds_in_flight(text) == []
+    stores, bare = hidden_stores_without_wait_states(text)
+    assert not bare and (stores > 0) == unit_name.startswith("fp_rows")
+
+
+@pytest.mark.parametrize("unit_name", ["gemm_chain_i8", "gemm_chain_f32", "conv_tiles_f16", "dw_tiles_f16"])
 def test_no_barrier_with_lds_accesses_in_flight(tmp_path, unit_name):
     hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
     if not os.path.exists(hipcc):
