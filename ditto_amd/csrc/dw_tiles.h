@@ -164,7 +164,9 @@ __global__ __launch_bounds__(64 * kDtWaves, MULT == 1 && RT == 2 ? 2 : 4) void d
       locate(b, off, drop);
       store_block(c0, b, load_block(c0, off), off, drop);
     }
+    // (filters behind the last one are zeros like their input channels: zero times an infinite weight is NaN)
     if constexpr (MULT == 16) {
+      if (c0 + CC > p.C0 && c0 * 144 + 8 * tid >= C1 * 9) w1v = V8{0, 0, 0, 0, 0, 0, 0, 0};
       if (tid < 256 * 9 / 8) reinterpret_cast<V8*>(w1_lds)[tid] = w1v;
       // lane q of a fragment holds outputs 4 q .. + 3 of the pair's first channel, then of its second
 #pragma unroll
@@ -176,6 +178,7 @@ __global__ __launch_bounds__(64 * kDtWaves, MULT == 1 && RT == 2 ? 2 : 4) void d
       }
     } else {
       if (tid < CC) {
+        if (c0 + tid >= C1) w1v = V8{0, 0, 0, 0, 0, 0, 0, 0}, w1last = 0;
         reinterpret_cast<V8*>(w1_lds)[2 * tid] = V8{w1v[0], w1v[1], w1v[2], 0, w1v[3], w1v[4], w1v[5], 0};
         reinterpret_cast<V8*>(w1_lds)[2 * tid + 1] = V8{w1v[6], w1v[7], w1last, 0, 0, 0, 0, 0};
       }

@@ -1073,3 +1073,20 @@ def test_infinite_pixels_stay_where_the_filters_take_them(dtype, case):
     assert torch.equal(torch.isinf(y), torch.isinf(want)) and not torch.isnan(y).any()
     fin = torch.isfinite(want)
     assert errors(y.float()[fin].numpy(), want.to(dt).float()[fin].numpy())[1] <= REL_L2
+
+
+@pytest.mark.parametrize("case", [(3200, 16, 40, 3, 1, 1), (3300, 24, 40, 1, 3, 1), (4100, 24, 24, 3, 1, 24), (4100, 6, 96, 3, 1, 6),
+                                  (4100, 17, 272, 3, 1, 17)])
+def test_infinite_filters_of_the_last_channel(case):
+    """An infinite filter makes its channel infinite where it lies in the image, and with it the outputs, but none NaN:
+    what fills a chunk of channels up behind the last one takes no part."""
+    tv, C0, C1, R1, R2, groups = case
+    gen = torch.Generator().manual_seed(C1)
+    x = torch.rand(1, C0, 11, 13, generator=gen) + 0.1
+    w1 = torch.rand(C1, C0 // groups, R1, R1, generator=gen) * 0.1 + 0.01
+    w2 = torch.rand(24, C1, R2, R2, generator=gen) * 0.1 + 0.01
+    w1[-1] = float("inf")
+    x, w1, w2 = (t.half().cuda() for t in (x, w1, w2))
+    y = torch.full((1, 24, 11, 13), float("nan"), device=x.device, dtype=torch.float16)
+    chain.run_conv_chain(x, w1, w2, y, R1 // 2, 1, R2 // 2, 1, groups1=groups, tile_variant=tv)
+    assert bool((y[:, :, 2:-2, 2:-2] == float("inf")).all())
