@@ -98,7 +98,7 @@ def conv_chain_desc(X, W1, W2, Y, pad1=1, stride1=1, pad2=0, stride2=1, inter_op
 
     ``groups1``: 1 (dense first convolution) or C0 (depthwise, C1 / C0 outputs per input channel).
     ``tile_variant``: 0 (the library's choice) or the kernel to force: a variant id ``select_tile`` reported or a
-    family id (3000, 3500, 3600, 3700, 3800, 4000; see ``include/ditto_chain.h``)."""
+    family id (3000, 3200, 3300, 3500, 3600, 3700, 3800, 4000, 4024, 4025, 4100; see ``include/ditto_chain.h``)."""
     for t, name in ((X, "X"), (W1, "W1"), (W2, "W2"), (Y, "Y")):
         if t.dim() != 4 or not t.is_contiguous():
             raise ValueError("%s must be a contiguous 4-D NCHW/KCRS tensor" % name)

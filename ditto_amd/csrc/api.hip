@@ -707,7 +707,8 @@ int plan_dw_conv(const ditto_conv_chain_desc* d, const ConvSteer& steer, long lo
     return DITTO_OK;
   }
   // Tiles of whole output rows: what the two row-streaming kernels do not take (they keep all weights in LDS: 8 x 32 x 56 x
-  // 56 times 16 7.6 us against 8.9, 32 x 32 x 56 x 56 times 1 7.8 / 12.5), 1.3 to 7 times the kernels below: 32 x 64 x 56 x 56
+  // 56 times 16 7.6 us against 8.9, 32 x 32 x 56 x 56 times 1 7.8 / 12.5; level or up to 9 % behind on one to four images,
+  // whose kernel alone takes less than the host's call), 1.3 to 7 times the kernels below: 32 x 64 x 56 x 56
   // times 16 -> 64 52.5 / 29.5 us, 8 x 32 x 37 x 37 times 16 25.6 / 9.1, 32 x 16 x 147 x 147 times 16 stride 2 127 / 19, 32 x
   // 64 x 112 x 112 times 1 73 / 48.  (The fp32 output of a shape the second one takes stays below, whose order of
   // accumulation is that kernel's.)
@@ -918,8 +919,10 @@ bool plan_conv_tiles(const ditto_conv_chain_desc* d, long long P, long long Q, b
 }
 
 // 1x1 -> 3x3 with at most 64 channels on tiles of whole output rows (conv13_tiles.h), where that is the kernel for the shape
-// (`forced`: where it can run it at all).  The row pipeline comes before it (32 x 64 x 56 x 56 12.6 us against 14.3, 16 images
-// 8.6 / 8.9).  It is ahead of the persistent kernel with W2 in LDS on 16-bit outputs (8 x 64 x 112 x 112 20.3 -> 15.2,
+// (`forced`: where it can run it at all).  The row pipeline comes before it: ahead on bands of six rows and more with all
+// channels filled (32 x 64 x 56 x 56 12.3 us against 14.1; 16 images, bands of four, 8.4 / 9.1).  On shorter bands and fewer
+// channels this kernel can be the faster one (32 x 64 x 40 x 40 10.1 / 8.8, 16 channels of 40 x 40 9.4 / 6.9, one image level):
+// such calls are left to tuning, which measures both.  It is ahead of the persistent kernel with W2 in LDS on 16-bit outputs (8 x 64 x 112 x 112 20.3 -> 15.2,
 // 32 x 64 x 72 x 72 28.4 -> 21.6, 8 x 64 x 30 x 256 26.8 -> 11.8), which keeps the fp32 ones: here they leave in
 // pieces of 16 bytes.
 bool plan_conv13_tiles(const ditto_conv_chain_desc* d, bool forced, ConvPlan* plan, int cus) {
@@ -1188,7 +1191,8 @@ int plan_conv_steered(const ditto_conv_chain_desc* d, const ConvSteer& steer, Co
       // where it pays (measured against the general kernel): the pipeline pads C0 and C1 to 64, and its gain is the
       // output stream under the compute - wide outputs - or, with few images, more workgroups than the general
       // kernel's tiles of 256 pixels (32 x 32 x 56 x 56 -> 32 -> 128: 16.4 against 12.3 us; 64 -> 64 -> 64: a tie;
-      // one image 64 -> 64 -> 256: 8.9 against 15.6 us)
+      // one image 64 -> 64 -> 256: 8.9 against 15.6 us).  Against the kernel on row tiles it is ahead on wide outputs
+      // (16 x 64 x 40 x 40 -> 64 -> 256 10.5 / 12.1) and behind on narrow ones (-> 64 -> 64 9.6 / 7.9), which tuning measures.
       (steer.tv / 100 == 37 ||
        ((d->C0 > 32 || d->C1 > 32) &&
       (d->C2 >= 192 || d->N * ((P + (256 / d->W > 0 ? 256 / d->W : 1) - 1) / (256 / d->W > 0 ? 256 / d->W : 1)) <

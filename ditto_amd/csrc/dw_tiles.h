@@ -58,9 +58,10 @@ __device__ __forceinline__ i32x4 drop_elements(i32x4 v, int s) {
 // C2 <= 16 NT output channels; pixel RT j + t of the wave's is column j of tile t, so a lane ends with RT consecutive pixels
 // of four channels of every output tile.  The depthwise results never leave the registers: in both forms a lane holds its
 // part of the 1x1 convolution's operand as it computes it.
-// What bounds it: on a full grid LDS reads and the vector ALU about evenly (32 x 64 x 56 x 56 times 16 -> 64: 29.5 us where
-// the matrix cores need 8 and the tensors 5; the general kernel, which walks padded rectangles one after another and waits
-// for each chunk, took 52.5); on small grids the chain of a chunk's load, barrier and products, 2 us per 16 channels (one
+// What bounds it: on a full grid, times 16, vector ALU (14 us), LDS reads (12) and matrix cores (9) of 33 us under the
+// tracer, taking turns more than overlapping (32 x 64 x 56 x 56 -> 64: 29.5 us untraced, the tensors need 5; the general
+// kernel, which walks padded rectangles one after another and waits for each chunk, took 52.5); times 1 the vector ALU (40 of
+// 54 us at 32 x 64 x 112 x 112); on small grids the chain of a chunk's load, barrier and products, 2 us per 16 channels (one
 // image of 32 x 37 x 37 times 16: 8.6 us, before 25.3; 32 x 16 x 147 x 147 times 16 stride 2: 19 us, before 127).
 // Eight waves of two tiles instead of four of four: half the blocks for a thread to stage, and two workgroups share a
 // compute unit (32.4 -> 29.5 us).  Filters are loaded as they lie in memory, by 16-byte blocks: one 18-byte filter per lane

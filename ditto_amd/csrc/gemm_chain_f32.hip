@@ -31,8 +31,10 @@ constexpr unsigned kLaunchBlocks = 1u << 22;  // most fp32 workgroups of one lau
 //
 // Bound: the fp32 matrix pipe (256 flop per cycle and compute unit) from a few rounds of workgroups on, the chain of
 // first loads, steps and merge below that.  12 x 512 x 512 x 64 (BERT-base, batch 1), softmax: 14.4 us per launch,
-// 56 TFLOP/s, where the plain fp32 FMAs over LDS tiles that this kernel replaced took 143 us (one row per eight threads,
-// an LDS read per operand of every FMA); 64 x 512 x 512 x 64: 52.7 us, 82 TFLOP/s; 4 x 1024 x 1024 x 128: 28.9 us, 74 TFLOP/s.
+// 56 TFLOP/s: 192 workgroups leave a quarter of the compute units idle, the others' matrix pipes are busy for 6.8 us of the
+// 12 beyond the launch, LDS hardly, and a third of the waves' time goes to waits for loads (56 MB out of L2).  The plain
+// fp32 FMAs over LDS tiles that this kernel replaced took 178 us (one row per eight threads, an LDS read per operand of
+// every FMA); 64 x 512 x 512 x 64: 52.7 us, 82 TFLOP/s; 4 x 1024 x 1024 x 128: 28.9 us, 74 TFLOP/s.
 //
 // DT: column tiles of 16 that K and N are padded to.  EXACT: K = N = 16 DT and every row starts on a 16-byte boundary;
 // otherwise elements are loaded one by one and columns past K or N are zeros.

@@ -216,7 +216,8 @@ int ditto_bmm_chain_run(const ditto_bmm_chain_desc* desc, const void* a, const v
 /* Run one fused conv->conv chain: replaces `func(Img, W1, W2, Out)`
  * (conv3x3_conv1x1_cuda.py:296-305).
  *   workspace : NULL, or ditto_conv_chain_workspace_bytes() bytes of device memory,
- *               16-byte aligned.  Given, a small kernel repacks w1 into it ahead of the
+ *               16-byte aligned.  Given, a small kernel repacks w1 (the kernels on row tiles: both
+ *               weights; the 1x1 -> 3x3 row pipeline and the resident kernel: w2) into it ahead of the
  *               fused kernel on `stream` (every call; calls that share a workspace must
  *               not overlap).  NULL: the fused kernel re-lays w1 out itself, slower.
  *               DITTO_EWORKSPACE if non-NULL and too small. */
