@@ -63,6 +63,7 @@ __global__ __launch_bounds__(128 * WP) void conv13_tiles_kernel(Conv13TilesArgs 
   const int n = lid / (unsigned)p.tiles_h, p0 = (lid - n * (unsigned)p.tiles_h) * p.TH;
   const int W = p.W, cols = W + 2, rows = p.TH + 2, npx = min(p.TH, p.H - p0) * W;
   const long long hw = (long long)p.H * W;
+  const int npm = rows * W, in0 = p0 == 0 ? W : 0, in1 = min(npm, (p.H - p0 + 1) * W);  // halo pixels, those inside the image
 
   V8 w1[2][4];
   const T* const w1f = reinterpret_cast<const T*>(p.w1f);
@@ -73,6 +74,11 @@ __global__ __launch_bounds__(128 * WP) void conv13_tiles_kernel(Conv13TilesArgs 
 
   stage_halo_rows<NT>(Xs, reinterpret_cast<const T*>(p.x) + (long long)n * p.C0 * hw, p0 - 1, 1, rows, cols, CS, p.c0p / 8, 8, p.C0, p.H, W,
                       p.inv_cg, p.inv_ng, tid);
+  if (p.c0p < 64)  // of the rows outside the image: the channels beyond the staged zeros
+    for (int t = tid; t < 4 * (in0 + npm - in1); t += NT) {
+      const int slot = t / 4 < in0 ? t / 4 : in1 - in0 + t / 4, ri = div_by(slot, p.inv_w);
+      *reinterpret_cast<i32x4*>(Xs + (ri * cols + slot - ri * W + 1) * CS + 32 + 8 * (t & 3)) = i32x4{0, 0, 0, 0};
+    }
   const T* const w2 = reinterpret_cast<const T*>(p.w2f) + (size_t)wc * (kC13Steps * 2 * 512) + lane * 8;
   V8 wf[D][2];
 #pragma unroll
@@ -81,11 +87,10 @@ __global__ __launch_bounds__(128 * WP) void conv13_tiles_kernel(Conv13TilesArgs 
     for (int m = 0; m < 2; ++m) wf[d][m] = *reinterpret_cast<const V8*>(w2 + (2 * d + m) * 512);
   wg_sync();
 
-  // ---- first convolution, in place: a wave turns the input channels of its 16 pixels into their 64 intermediate ones (a row
-  // outside the image is zero and stays so)
-  const int npm = rows * W;
-  for (int s0 = 16 * wave; s0 < npm; s0 += 16 * NW) {
-    const int slot = s0 + c < npm ? s0 + c : 0, ri = div_by(slot, p.inv_w);
+  // ---- first convolution, in place: a wave turns the input channels of its 16 pixels into their 64 intermediate ones.  A row
+  // outside the image stays zero whatever the weights: only the pixels of the rows inside are computed.
+  for (int s0 = in0 + 16 * wave; s0 < in1; s0 += 16 * NW) {
+    const int slot = s0 + c < in1 ? s0 + c : in0, ri = div_by(slot, p.inv_w);
     T* const px = Xs + (ri * cols + slot - ri * W + 1) * CS;
     f32x4 acc[4];
     const V8 x0 = *reinterpret_cast<const V8*>(px + 8 * q);
@@ -96,7 +101,7 @@ __global__ __launch_bounds__(128 * WP) void conv13_tiles_kernel(Conv13TilesArgs 
 #pragma unroll
       for (int m = 0; m < 4; ++m) acc[m] = Elem<T>::mfma16(w1[1][m], x1, acc[m]);
     }
-    if (s0 + c < npm) {
+    if (s0 + c < in1) {
 #pragma unroll
       for (int m = 0; m < 4; ++m) {
         if (p.relu_mid)
