@@ -369,7 +369,8 @@ int plan_bmm(const ditto_bmm_chain_desc* d, BmmPlan* plan, bool need_device) {
       return fail(DITTO_EINVAL, "the fp32 / fp64 chain accumulates and outputs its input type");
     if (d->inter_op != DITTO_INTER_CAST && d->inter_op != DITTO_INTER_RELU && d->inter_op != DITTO_INTER_SOFTMAX)
       return fail(DITTO_EUNSUPPORTED, "the fp32 chain takes inter_op cast, relu or softmax");
-    if (d->tile_variant != 0) return fail(DITTO_EINVAL, "the fp32 chain has a single variant (tile_variant must be 0)");
+    if (d->tile_variant != 0 && d->tile_variant != (in == DITTO_F64 ? 1001 : 1000))  // (the id that select_tile reports)
+      return fail(DITTO_EINVAL, "tile_variant %d: the fp32 chain has a single variant, 1000 (fp64: 1001)", d->tile_variant);
     if (d->K > ditto::f32_chain_max_dim() || d->N > ditto::f32_chain_max_dim())
       return fail(DITTO_EUNSUPPORTED, "the fp32 chain supports K, N up to %d", ditto::f32_chain_max_dim());
     if (d->a_row_stride < d->K || d->c_row_stride < d->N || d->f_row_stride < d->N ||

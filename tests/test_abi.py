@@ -115,6 +115,12 @@ def test_select_tile_and_validation_without_gpu():
         rc = lib.ditto_bmm_chain_select_tile(ctypes.byref(d), ctypes.byref(tile))
         return rc, _lib.last_error()
 
+    # fp32 and fp64 have one kernel each, whose id can be forced like any other that is reported
+    for dt, own, other in ((_lib.F32, 1000, 1001), (_lib.F64, 1001, 1000)):
+        types = dict(in_dtype=dt, acc_dtype=dt, out_dtype=dt)
+        assert rc_msg(_desc(**types))[0] == _lib.OK and tile.variant == own
+        assert rc_msg(_desc(tile_variant=own, **types))[0] == _lib.OK and tile.variant == own
+        assert rc_msg(_desc(tile_variant=other, **types))[0] == _lib.EINVAL
     assert rc_msg(_desc(abi_version=99))[0] == _lib.EINVAL
     rc, msg = rc_msg(_desc(K=60))
     assert rc == _lib.EINVAL and "multiples of 8" in msg

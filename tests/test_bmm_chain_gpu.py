@@ -706,6 +706,9 @@ def test_tuning_heads_of_80_columns(tmp_path, oracle):
     desc = chain.bmm_chain_desc(q, k.transpose(1, 2), v, f, "softmax", 80 ** -0.5)
     key = ci.workload_key(desc)
     variant = ci.auto_schedule_bmm_chain_hip(key, log, q, k.transpose(1, 2), v, f, "softmax", 80 ** -0.5)
+    # (fp32 has one kernel: tuning measures it)
+    q32, k32, v32, f32 = (t.float() for t in (q, k, v, f))
+    assert ci.auto_schedule_bmm_chain_hip("fp32", str(tmp_path / "f32.log"), q32, k32.transpose(1, 2), v32, f32) == 1000
     lines = open(log).read().strip().splitlines()
     assert len(lines) == 3 and '"variant": %d' % chain.select_tile(desc).variant in lines[0]
     f.fill_(float("nan"))
