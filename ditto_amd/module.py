@@ -31,7 +31,7 @@ class ChainFunction:
     and the call returns without synchronising.
 
     A call goes through native code (``csrc/host/host_call.cpp``) that checks the arguments, fills the C-ABI
-    descriptor and launches.  A conv chain that takes a workspace owns one per device, sized by
+    descriptor and launches.  A conv chain that takes a workspace owns one per device and output type, sized by
     ``ditto_conv_chain_workspace_bytes`` at its first call and never replaced, so a HIP graph that
     captured a call keeps a valid pointer; calls of ONE function object on two streams still race
     on it (use ``specialize`` for a second object).  ``specialize(W1, W2)`` returns a function bound
@@ -58,8 +58,8 @@ class ChainFunction:
         self.tile_variant = int(sch.tile_variant if tile_variant is None else tile_variant)
         self._native = None     # the native call, made at the first one
         self._descs = {}        # dtypes -> descriptor as filled for them first: what ran, for a caller that logs it
-        self._workspaces = {}   # device -> uint8 tensor (conv chains)
-        self._prepared = None   # (W1, W2, W1._version, W2._version): what the workspace holds the repacked form of
+        self._workspaces = {}   # (device, output dtype) -> uint8 tensor (conv chains)
+        self._prepared = None   # (W1, W2, W1._version, W2._version, output dtype): what its workspace holds the repacked form of
 
     def _make_native(self):
         host, s = _lib.host(), self.sch
@@ -122,11 +122,12 @@ class ChainFunction:
         f(x, w1, w2, y)
         layout.pack_output_into(y, out_p)
 
-    def _workspace(self, desc, dev):
-        ws = self._workspaces.get(dev)
+    def _workspace(self, desc, Y, dev):
+        # (the output's type is part of the kernel choice, and with it of the layout the weights are repacked in)
+        ws = self._workspaces.get((dev, Y.dtype))
         if ws is None:
             nbytes = chain.conv_chain_workspace_bytes(desc)
-            ws = self._workspaces[dev] = torch.empty(max(nbytes, 16), dtype=torch.uint8, device=dev) if nbytes else False
+            ws = self._workspaces[dev, Y.dtype] = torch.empty(max(nbytes, 16), dtype=torch.uint8, device=dev) if nbytes else False
         return ws
 
     def _conv_desc(self, X, W1, W2, Y):
@@ -154,16 +155,16 @@ class ChainFunction:
         X = torch.empty(tuple(xt.shape), device="meta", dtype=dt)
         Y = torch.empty(tuple(yt.shape), device="meta", dtype=_TORCH[yt.dtype])
         desc = self._conv_desc(X, W1, W2, Y)
-        ws = f._workspace(desc, W1.device)
+        ws = f._workspace(desc, Y, W1.device)
         if ws is not False:
             chain.prepare_conv_chain(desc, W1, W2, ws)
-            f._prepared = (W1, W2, W1._version, W2._version)
+            f._prepared = (W1, W2, W1._version, W2._version, Y.dtype)
             f._remember(desc, W1, W1, W2, Y, ws, True)
         return f
 
-    def _is_prepared(self, W1, W2):
+    def _is_prepared(self, W1, W2, out_dtype=None):
         p = self._prepared
-        if p is None:
+        if p is None or (out_dtype is not None and out_dtype != p[4]):
             return False
 
         def same(held, w):  # the held tensor itself, or another view of exactly its memory (views share the counter)
@@ -199,16 +200,16 @@ class ChainFunction:
         if X.dim() == 5:
             return self._call_packed(X, W1, W2, Y)
         desc = self._conv_desc(X, W1, W2, Y)
-        ws = self._workspace(desc, X.device)
-        prepared = ws is not False and self._is_prepared(W1, W2)
+        ws = self._workspace(desc, Y, X.device)
+        prepared = ws is not False and self._is_prepared(W1, W2, Y.dtype)
         if ws is not False and self._prepared is not None and not prepared:
-            # a specialised function handed other weights (or the bound ones after an in-place update):
-            # repack them now; they are the bound weights from here on
+            # a specialised function handed other weights (or the bound ones after an in-place update, or an output of
+            # another type): repack them now; they are the bound weights from here on
             self._prepared = None
             self._native.forget()
             try:
                 chain.prepare_conv_chain(desc, W1, W2, ws)
-                self._prepared = (W1, W2, W1._version, W2._version)
+                self._prepared = (W1, W2, W1._version, W2._version, Y.dtype)
                 prepared = True
             except ValueError:
                 pass  # pointers the prepared form cannot take: the one-call form below decides

@@ -306,3 +306,26 @@ def test_specialised_conv_chain_notices_other_and_updated_weights(oracle):
         eng.run()
         torch.cuda.synchronize()
         assert errors(eng.get_outputs()[0][:1].float().cpu().numpy(), want_b)[1] <= 1e-3, make.__name__
+
+
+def test_specialised_conv_chain_with_outputs_of_either_type(oracle):
+    """The output's type is part of the kernel choice (16 bits: the row pipeline; fp32: tiles of whole output rows), and
+    the kernels repack the weights in layouts and workspaces of their own."""
+    from ditto_amd.auto_compute.nn import functional as F
+    from tests.gpu_util import errors, to_dev
+
+    n, c0, hw_, c1, c2 = 2, 64, 56, 64, 256
+    cins, couts = F.Conv3x3Conv1x1(n, c0, hw_, hw_, c1, c2)
+    cl = ac.layer([couts[0].op], inputs=[cins[0]], weights=cins[1:], name="conv_chain")
+    func = ditto.build(common.describe_layer(cl), cl.schedule_tensors, "hip")
+    X, W1, W2 = oracle.make_conv_chain_inputs(n, c0, hw_, hw_, c1, c2, 3, 1, "float16", seed=12)
+    want = oracle.conv_chain_f32(X, W1, W2, 1, 1, 0, 1, round_mid="float16")
+    x, w1, w2 = (to_dev(t, "float16") for t in (X, W1, W2))
+    f = func.specialize(w1, w2)
+    for dt in (torch.float16, torch.float32, torch.float16, torch.float32, torch.float32):
+        y = torch.full((n, c2, hw_, hw_), float("nan"), device=x.device, dtype=dt)
+        f(x, w1, w2, y)
+        torch.cuda.synchronize()
+        mx, rel = errors(y.float().cpu().numpy(), want)
+        assert mx <= 1e-2 and rel <= 1e-3, (dt, mx, rel)
+        assert f._is_prepared(w1, w2, dt)
