@@ -46,6 +46,7 @@ __global__ __launch_bounds__(64 * kWaves) void gemm_chain_f32_kernel(F32ChainArg
   extern __shared__ __attribute__((aligned(16))) float smem_f32[];
   float* const Om = smem_f32;                              // [wave][16 RT][ORS]
   float* const Ml = smem_f32 + kWaves * 16 * RT * ORS;     // [wave][16 RT][reference exponent, sum]
+  int* const again = reinterpret_cast<int*>(Ml + kWaves * 16 * RT * 2);  // a result is not finite
   const int K = p.K, N = p.N, L = p.L, M = p.M;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, c = lane & 15, q = lane >> 4;
   const unsigned bid = p.block0 + xcd_remap(blockIdx.x, gridDim.x);  // the row blocks of a batch entry read the same B and C
@@ -87,157 +88,170 @@ __global__ __launch_bounds__(64 * kWaves) void gemm_chain_f32_kernel(F32ChainArg
     const float* const row = Ag + (long long)min(m0 + 16 * rt + c, M - 1) * p.a_rs;
 #pragma unroll
     for (int s = 0; s < DT; ++s) qf[rt][s] = load4(row, 16 * s + 4 * q, K);
-#pragma unroll
-    for (int j = 0; j < DT; ++j) o[rt][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
   }
-  // softmax in the exp2 domain: a row's reference exponent is no smaller than any score of the wave's keys so far, so no weight
-  // exceeds one and a result overflows only where the sum of its values does (a slack of 2^20 before a raise took that much
-  // off the range of C).  When a score exceeds the reference it is set kHeadroom above it: the few binary orders by which a
-  // later key usually exceeds the first sixteen then cost no second rescale, which waits for the accumulators (always to the
-  // maximum itself: 14.4 -> 14.8 us at 12 x 512 x 512 x 64, 4 % more at 1000 keys).  None yet while all score minus infinity.
-  constexpr float kHeadroom = 4.f;
+  // Softmax in the exp2 domain: a row's reference exponent is its maximum over the wave's first keys, raised only when a
+  // later score exceeds it by 2^slack; none yet while the wave's keys all score minus infinity.  Weights of up to 2^20 are
+  // no loss but at the end of the range of C: a workgroup with a result that is not finite walks the keys once more with
+  // weights of at most one (raising at any excess in the first place waits for the accumulators at every step: 14.4 -> 14.8 us
+  // at 12 x 512 x 512 x 64, 4 % at 1000 keys; a reference a few orders above the maximum costs 2 % of the accuracy).
   const float c2 = p.softmax_scale * 1.4426950408889634f;
-  float ref[RT], lsum[RT];
-#pragma unroll
-  for (int rt = 0; rt < RT; ++rt) ref[rt] = kNoKeyYet, lsum[rt] = 0.f;
+  float ref[RT], lsum[RT], slack = SM ? 20.f : 0.f;
+  if (SM && tid == 0) *again = 0;
 
-  for (int step = w; step < nsteps; step += kWaves) {
-    const int key0 = 16 * step;
+  for (;;) {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const float* const row = Cg + (long long)min(key0 + 4 * q + r, L - 1) * p.c_rs;
+    for (int rt = 0; rt < RT; ++rt) {
+      ref[rt] = kNoKeyYet, lsum[rt] = 0.f;
 #pragma unroll
-      for (int g = 0; g < G; ++g) vf[r][g] = load4(row, 64 * g + 4 * c, N);
-      if constexpr (REM > 0) vf[r][G][0] = EXACT || 64 * G + c < N ? row[64 * G + c] : 0.f;
+      for (int j = 0; j < DT; ++j) o[rt][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
     }
-    f32x4 st[RT];
+    for (int step = w; step < nsteps; step += kWaves) {
+      const int key0 = 16 * step;
 #pragma unroll
-    for (int rt = 0; rt < RT; ++rt) st[rt] = (f32x4){0.f, 0.f, 0.f, 0.f};
+      for (int r = 0; r < 4; ++r) {
+        const float* const row = Cg + (long long)min(key0 + 4 * q + r, L - 1) * p.c_rs;
 #pragma unroll
-    for (int s = 0; s < DT; ++s)
-#pragma unroll
-      for (int t = 0; t < 4; ++t)
-#pragma unroll
-        for (int rt = 0; rt < RT; ++rt)
-          st[rt] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[s][t], qf[rt][s][t], st[rt], 0, 0, 0);
-    if (step + kWaves < nsteps) load_k(step + kWaves);
-    const bool tail = key0 + 16 > L;
-    if constexpr (SM) {
-      bool raise = false;
-#pragma unroll
-      for (int rt = 0; rt < RT; ++rt) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          st[rt][r] *= c2;
-          if (tail && key0 + 4 * q + r >= L) st[rt][r] = -INFINITY;
-          raise |= st[rt][r] > ref[rt];
-        }
+        for (int g = 0; g < G; ++g) vf[r][g] = load4(row, 64 * g + 4 * c, N);
+        if constexpr (REM > 0) vf[r][G][0] = EXACT || 64 * G + c < N ? row[64 * G + c] : 0.f;
       }
-      if (__any(raise)) {
+      f32x4 st[RT];
 #pragma unroll
-        for (int rt = 0; rt < RT; ++rt) {
-          float mx = fmaxf(fmaxf(st[rt][0], st[rt][1]), fmaxf(st[rt][2], st[rt][3]));
-          mx = quad_max(mx);
-          const float up = mx > ref[rt] ? mx + kHeadroom : ref[rt], alpha = exp2f(ref[rt] - up);
-          ref[rt] = up;
-          lsum[rt] *= alpha;
+      for (int rt = 0; rt < RT; ++rt) st[rt] = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-          for (int j = 0; j < DT; ++j) o[rt][j] *= alpha;
-        }
-      }
-#pragma unroll
-      for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          st[rt][r] = __builtin_amdgcn_exp2f(st[rt][r] - ref[rt]);
-          lsum[rt] += st[rt][r];
-        }
-    } else {
-#pragma unroll
-      for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          if (p.relu) st[rt][r] = fmaxf(st[rt][r], 0.f);
-          if (tail && key0 + 4 * q + r >= L) st[rt][r] = 0.f;
-        }
-    }
-    if (tail) {  // the clamped rows stand for nothing, whatever the last row holds
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-#pragma unroll
-        for (int g = 0; g < G + REM; ++g)
-          if (key0 + 4 * q + r >= L) vf[r][g] = (f32x4){0.f, 0.f, 0.f, 0.f};
-    }
-#pragma unroll
-    for (int r = 0; r < 4; ++r)
-#pragma unroll
-      for (int j = 0; j < DT; ++j)
-#pragma unroll
-        for (int rt = 0; rt < RT; ++rt)
-          o[rt][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[r][j / 4][j % 4], st[rt][r], o[rt][j], 0, 0, 0);
-  }
-
-  // lane (c, q) holds of row c: columns 64 g + 16 q + 4 r + t in register r of tile 4 g + t, and 64 G + 4 q + r in the last
-#pragma unroll
-  for (int rt = 0; rt < RT; ++rt) {
-    float* const row = Om + (w * 16 * RT + 16 * rt + c) * ORS;
-#pragma unroll
-    for (int g = 0; g < G; ++g)
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        *reinterpret_cast<f32x4*>(row + 64 * g + 16 * q + 4 * r) =
-            (f32x4){o[rt][4 * g][r], o[rt][4 * g + 1][r], o[rt][4 * g + 2][r], o[rt][4 * g + 3][r]};
-    if constexpr (REM > 0) *reinterpret_cast<f32x4*>(row + 64 * G + 4 * q) = o[rt][4 * G];
-    if constexpr (SM) {
-      float s = lsum[rt];
-      s += __shfl_xor(s, 16);
-      s += __shfl_xor(s, 32);
-      if (q == 0) {
-        Ml[2 * (w * 16 * RT + 16 * rt + c)] = ref[rt];
-        Ml[2 * (w * 16 * RT + 16 * rt + c) + 1] = s;
-      }
-    }
-  }
-  wg_sync();
-  for (int e = tid; e < 16 * RT * 4 * DT; e += 64 * kWaves) {
-    const int row = e / (4 * DT), n0 = 4 * (e - row * 4 * DT);
-    float wt[kWaves];
-    if constexpr (SM) {
-      float mx = kNoKeyYet, s = 0.f;
-#pragma unroll
-      for (int i = 0; i < kWaves; ++i) mx = fmaxf(mx, Ml[2 * (i * 16 * RT + row)]);
-#pragma unroll
-      for (int i = 0; i < kWaves; ++i) {
-        wt[i] = exp2f(Ml[2 * (i * 16 * RT + row)] - mx);
-        s += wt[i] * Ml[2 * (i * 16 * RT + row) + 1];
-      }
-      const float inv = 1.f / s;
-#pragma unroll
-      for (int i = 0; i < kWaves; ++i) wt[i] *= inv;
-    } else {
-#pragma unroll
-      for (int i = 0; i < kWaves; ++i) wt[i] = 1.f;
-    }
-    f32x4 x = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int i = 0; i < kWaves; ++i) {
-      const f32x4 part = *reinterpret_cast<const f32x4*>(Om + (i * 16 * RT + row) * ORS + n0);
-#pragma unroll
-      for (int t = 0; t < 4; ++t) x[t] = __builtin_fmaf(wt[i], part[t], x[t]);
-    }
-    if (p.relu_out)
-#pragma unroll
-      for (int t = 0; t < 4; ++t) x[t] = fmaxf(x[t], 0.f);
-    if (m0 + row < M) {
-      float* const dst = Fg + (long long)(m0 + row) * p.f_rs + n0;
-      if constexpr (EXACT) {
-        *reinterpret_cast<f32x4*>(dst) = x;
-      } else {
+      for (int s = 0; s < DT; ++s)
 #pragma unroll
         for (int t = 0; t < 4; ++t)
-          if (n0 + t < N) dst[t] = x[t];
+#pragma unroll
+          for (int rt = 0; rt < RT; ++rt)
+            st[rt] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[s][t], qf[rt][s][t], st[rt], 0, 0, 0);
+      if (step + kWaves < nsteps) load_k(step + kWaves);
+      const bool tail = key0 + 16 > L;
+      if constexpr (SM) {
+        bool raise = false;
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            st[rt][r] *= c2;
+            if (tail && key0 + 4 * q + r >= L) st[rt][r] = -INFINITY;
+            raise |= st[rt][r] > ref[rt] + slack;
+          }
+        }
+        if (__any(raise)) {
+#pragma unroll
+          for (int rt = 0; rt < RT; ++rt) {
+            float mx = fmaxf(fmaxf(st[rt][0], st[rt][1]), fmaxf(st[rt][2], st[rt][3]));
+            mx = quad_max(mx);
+            const float up = fmaxf(ref[rt], mx), alpha = exp2f(ref[rt] - up);
+            ref[rt] = up;
+            lsum[rt] *= alpha;
+#pragma unroll
+            for (int j = 0; j < DT; ++j) o[rt][j] *= alpha;
+          }
+        }
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            st[rt][r] = __builtin_amdgcn_exp2f(st[rt][r] - ref[rt]);
+            lsum[rt] += st[rt][r];
+          }
+      } else {
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            if (p.relu) st[rt][r] = fmaxf(st[rt][r], 0.f);
+            if (tail && key0 + 4 * q + r >= L) st[rt][r] = 0.f;
+          }
+      }
+      if (tail) {  // the clamped rows stand for nothing, whatever the last row holds
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+          for (int g = 0; g < G + REM; ++g)
+            if (key0 + 4 * q + r >= L) vf[r][g] = (f32x4){0.f, 0.f, 0.f, 0.f};
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int j = 0; j < DT; ++j)
+#pragma unroll
+          for (int rt = 0; rt < RT; ++rt)
+            o[rt][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[r][j / 4][j % 4], st[rt][r], o[rt][j], 0, 0, 0);
+    }
+
+    // lane (c, q) holds of row c: columns 64 g + 16 q + 4 r + t in register r of tile 4 g + t, and 64 G + 4 q + r in the last
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) {
+      float* const row = Om + (w * 16 * RT + 16 * rt + c) * ORS;
+#pragma unroll
+      for (int g = 0; g < G; ++g)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          *reinterpret_cast<f32x4*>(row + 64 * g + 16 * q + 4 * r) =
+              (f32x4){o[rt][4 * g][r], o[rt][4 * g + 1][r], o[rt][4 * g + 2][r], o[rt][4 * g + 3][r]};
+      if constexpr (REM > 0) *reinterpret_cast<f32x4*>(row + 64 * G + 4 * q) = o[rt][4 * G];
+      if constexpr (SM) {
+        float s = lsum[rt];
+        s += __shfl_xor(s, 16);
+        s += __shfl_xor(s, 32);
+        if (q == 0) {
+          Ml[2 * (w * 16 * RT + 16 * rt + c)] = ref[rt];
+          Ml[2 * (w * 16 * RT + 16 * rt + c) + 1] = s;
+        }
       }
     }
+    wg_sync();
+    bool bad = false;
+    for (int e = tid; e < 16 * RT * 4 * DT; e += 64 * kWaves) {
+      const int row = e / (4 * DT), n0 = 4 * (e - row * 4 * DT);
+      float wt[kWaves];
+      if constexpr (SM) {
+        float mx = kNoKeyYet, s = 0.f;
+#pragma unroll
+        for (int i = 0; i < kWaves; ++i) mx = fmaxf(mx, Ml[2 * (i * 16 * RT + row)]);
+#pragma unroll
+        for (int i = 0; i < kWaves; ++i) {
+          wt[i] = exp2f(Ml[2 * (i * 16 * RT + row)] - mx);
+          s += wt[i] * Ml[2 * (i * 16 * RT + row) + 1];
+        }
+        const float inv = 1.f / s;
+#pragma unroll
+        for (int i = 0; i < kWaves; ++i) wt[i] *= inv;
+      } else {
+#pragma unroll
+        for (int i = 0; i < kWaves; ++i) wt[i] = 1.f;
+      }
+      f32x4 x = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int i = 0; i < kWaves; ++i) {
+        const f32x4 part = *reinterpret_cast<const f32x4*>(Om + (i * 16 * RT + row) * ORS + n0);
+#pragma unroll
+        for (int t = 0; t < 4; ++t) x[t] = __builtin_fmaf(wt[i], part[t], x[t]);
+      }
+      if (p.relu_out)
+#pragma unroll
+        for (int t = 0; t < 4; ++t) x[t] = fmaxf(x[t], 0.f);
+      if (m0 + row < M) {
+        float* const dst = Fg + (long long)(m0 + row) * p.f_rs + n0;
+        if constexpr (EXACT) {
+          *reinterpret_cast<f32x4*>(dst) = x;
+        } else {
+#pragma unroll
+          for (int t = 0; t < 4; ++t)
+            if (n0 + t < N) dst[t] = x[t];
+        }
+      }
+#pragma unroll
+      for (int t = 0; t < 4; ++t) bad |= (__builtin_bit_cast(int, x[t]) & 0x7f800000) == 0x7f800000;
+    }
+    if (!SM || slack == 0.f) return;
+    if (__any(bad) && lane == 0) *again = 1;
+    wg_sync();
+    if (*again == 0) return;
+    slack = 0.f;
+    if (w < nsteps) load_k(w);
   }
 }
 
@@ -365,7 +379,7 @@ static int f32_tiles(int K, int N) {  // column tiles of 16 the fp32 kernel is b
 }
 int f32_chain_lds_bytes_host(int K, int N, int f64, int rt) {
   if (f64) return f64_chain_lds_bytes(K, N);
-  return kWaves * 16 * rt * (16 * f32_tiles(K, N) + 4 + 2) * (int)sizeof(float);
+  return kWaves * 16 * rt * (16 * f32_tiles(K, N) + 4 + 2) * (int)sizeof(float) + 16;
 }
 
 template <typename Tag, typename Kernel>
