@@ -279,7 +279,7 @@ def test_fp32_chain_vs_oracle(oracle, shape, inter):
 def test_fp32_chain_at_the_edges_of_its_tiles(oracle, shape, inter):
     batch, M, N, K, L = shape
     A, B, C = oracle.make_gemm_chain_inputs(batch, M, N, K, L, "float32", seed=M + L, std=1.0 if inter == "softmax" else 0.25)
-    # scores that climb by far more than the headroom of the running reference as the keys go on
+    # scores that climb by far more than the slack of the running reference as the keys go on
     B = B * np.linspace(0.1, 8.0, L, dtype=np.float32)[None, None, :]
     want = oracle.bmm_chain_f64(A, B, C, inter=inter, scale=0.5 if inter == "softmax" else 1.0)
     for b_layout in ("KL", "LK"):
