@@ -104,6 +104,7 @@ class TileParam(ctypes.Structure):
 
 # Every symbol include/ditto_chain.h declares: (name, restype, argtypes)
 _P = ctypes.c_void_p
+_PP = ctypes.POINTER(ctypes.c_void_p)
 EXPORTS = [
     ("ditto_chain_abi_version", ctypes.c_int, []),
     ("ditto_last_error", ctypes.c_char_p, []),
@@ -113,6 +114,8 @@ EXPORTS = [
     ("ditto_conv_chain_workspace_bytes", ctypes.c_size_t, [ctypes.POINTER(ConvChainDesc)]),
     ("ditto_bmm_chain_run", ctypes.c_int,
      [ctypes.POINTER(BmmChainDesc), _P, _P, _P, _P, _P, _P, ctypes.c_size_t, _P]),
+    ("ditto_bmm_chain_run_sets", ctypes.c_int,
+     [ctypes.POINTER(BmmChainDesc), ctypes.c_int, _PP, _PP, _PP, _PP, _P]),
     ("ditto_conv_chain_run", ctypes.c_int,
      [ctypes.POINTER(ConvChainDesc), _P, _P, _P, _P, _P, ctypes.c_size_t, _P]),
     ("ditto_conv_chain_prepare", ctypes.c_int,

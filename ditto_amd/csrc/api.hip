@@ -1297,6 +1297,64 @@ int plan_conv_steered(const ditto_conv_chain_desc* d, const ConvSteer& steer, Co
   return DITTO_OK;
 }
 
+// The kernels that run several chains of one shape in one launch: those of 16 to 64 rows per workgroup or short tiles.  (They
+// find a row's first unmasked key wherever it lies, so a chain loses nothing by running with others.)
+bool plan_takes_sets(const BmmPlan& plan) { return plan.split_rt > 0 || plan.rows_nw > 0 || plan.qt == 4 || plan.qt == 5; }
+
+// The launch of a planned fp16 / bf16 chain; `sets`: where the tensors of the chains it is one of lie, or null.
+int launch_fp_chain(const ditto_bmm_chain_desc* d, const BmmPlan& plan, const void* a, const void* b, const void* c, void* f,
+                    const ditto::BmmSets* sets, hipStream_t st) {
+  ditto::BmmChainArgs args;
+  args.a = a;
+  args.b = b;
+  args.c = c;
+  args.f = f;
+  args.a_bs = d->a_batch_stride;
+  args.b_bs = d->b_batch_stride;
+  args.c_bs = d->c_batch_stride;
+  args.f_bs = d->f_batch_stride;
+  {
+    const bool two = d->batch_inner > 0 && d->batch_inner != d->batch;
+    args.batch_inner = two ? (int)d->batch_inner : (int)d->batch;
+    args.a_bs2 = two ? d->a_batch_stride_outer : 0;
+    args.b_bs2 = two ? d->b_batch_stride_outer : 0;
+    args.c_bs2 = two ? d->c_batch_stride_outer : 0;
+    args.f_bs2 = two ? d->f_batch_stride_outer : 0;
+  }
+  args.a_rs = (int)d->a_row_stride;
+  args.b_rs = (int)d->b_row_stride;
+  args.c_rs = (int)d->c_row_stride;
+  args.f_rs = (int)d->f_row_stride;
+  args.M = (int)d->M;
+  args.N = (int)d->N;
+  args.K = (int)d->K;
+  args.L = (int)d->L;
+  args.batch = (int)d->batch;
+  args.mblocks = plan.nb;
+  args.mblocks3 = plan.nb3;
+  args.scale_log2 = d->softmax_scale * 1.4426950408889634f;
+  args.relu = d->inter_op == DITTO_INTER_RELU;
+  args.relu_out = d->relu_out;
+  args.out_f32 = d->out_dtype == DITTO_F32;
+  const bool kl = d->b_layout == DITTO_B_KL;
+  const bool sm = d->inter_op == DITTO_INTER_SOFTMAX;
+  hipError_t e;
+  if (plan.split_rt > 0)
+    e = d->in_dtype == DITTO_F16 ? ditto::launch_split_f16(plan.split_dt, plan.split_rt, sm, kl, args, sets, st)
+                                 : ditto::launch_split_bf16(plan.split_dt, plan.split_rt, sm, kl, args, sets, st);
+  else if (plan.rows_nw > 0)
+    e = d->in_dtype == DITTO_F16 ? ditto::launch_rows_f16(plan.rows_dt, plan.rows_nw, sm, kl, args, sets, st)
+                                 : ditto::launch_rows_bf16(plan.rows_dt, plan.rows_nw, sm, kl, args, sets, st);
+  else if (d->in_dtype == DITTO_F16)
+    e = sm ? ditto::launch_f16_softmax(plan.d_pad, plan.qt, kl, args, sets, st)
+           : ditto::launch_f16_cast(plan.d_pad, plan.qt, kl, args, sets, st);
+  else
+    e = sm ? ditto::launch_bf16_softmax(plan.d_pad, plan.qt, kl, args, sets, st)
+           : ditto::launch_bf16_cast(plan.d_pad, plan.qt, kl, args, sets, st);
+  if (e != hipSuccess) return fail(DITTO_EHIP, "kernel launch failed: %s", hipGetErrorString(e));
+  return DITTO_OK;
+}
+
 }  // namespace
 
 extern "C" {
@@ -1333,57 +1391,7 @@ int ditto_bmm_chain_run(const ditto_bmm_chain_desc* d, const void* a, const void
     return fail(DITTO_EINVAL, "data pointers must be 16-byte aligned");
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
 
-  if (plan.family == 0) {
-    ditto::BmmChainArgs args;
-    args.a = a;
-    args.b = b;
-    args.c = c;
-    args.f = f;
-    args.a_bs = d->a_batch_stride;
-    args.b_bs = d->b_batch_stride;
-    args.c_bs = d->c_batch_stride;
-    args.f_bs = d->f_batch_stride;
-    {
-      const bool two = d->batch_inner > 0 && d->batch_inner != d->batch;
-      args.batch_inner = two ? (int)d->batch_inner : (int)d->batch;
-      args.a_bs2 = two ? d->a_batch_stride_outer : 0;
-      args.b_bs2 = two ? d->b_batch_stride_outer : 0;
-      args.c_bs2 = two ? d->c_batch_stride_outer : 0;
-      args.f_bs2 = two ? d->f_batch_stride_outer : 0;
-    }
-    args.a_rs = (int)d->a_row_stride;
-    args.b_rs = (int)d->b_row_stride;
-    args.c_rs = (int)d->c_row_stride;
-    args.f_rs = (int)d->f_row_stride;
-    args.M = (int)d->M;
-    args.N = (int)d->N;
-    args.K = (int)d->K;
-    args.L = (int)d->L;
-    args.batch = (int)d->batch;
-    args.mblocks = plan.nb;
-    args.mblocks3 = plan.nb3;
-    args.scale_log2 = d->softmax_scale * 1.4426950408889634f;
-    args.relu = d->inter_op == DITTO_INTER_RELU;
-    args.relu_out = d->relu_out;
-    args.out_f32 = d->out_dtype == DITTO_F32;
-    const bool kl = d->b_layout == DITTO_B_KL;
-    const bool sm = d->inter_op == DITTO_INTER_SOFTMAX;
-    hipError_t e;
-    if (plan.split_rt > 0)
-      e = d->in_dtype == DITTO_F16 ? ditto::launch_split_f16(plan.split_dt, plan.split_rt, sm, kl, args, st)
-                                   : ditto::launch_split_bf16(plan.split_dt, plan.split_rt, sm, kl, args, st);
-    else if (plan.rows_nw > 0)
-      e = d->in_dtype == DITTO_F16 ? ditto::launch_rows_f16(plan.rows_dt, plan.rows_nw, sm, kl, args, st)
-                                   : ditto::launch_rows_bf16(plan.rows_dt, plan.rows_nw, sm, kl, args, st);
-    else if (d->in_dtype == DITTO_F16)
-      e = sm ? ditto::launch_f16_softmax(plan.d_pad, plan.qt, kl, args, st)
-             : ditto::launch_f16_cast(plan.d_pad, plan.qt, kl, args, st);
-    else
-      e = sm ? ditto::launch_bf16_softmax(plan.d_pad, plan.qt, kl, args, st)
-             : ditto::launch_bf16_cast(plan.d_pad, plan.qt, kl, args, st);
-    if (e != hipSuccess) return fail(DITTO_EHIP, "kernel launch failed: %s", hipGetErrorString(e));
-    return DITTO_OK;
-  }
+  if (plan.family == 0) return launch_fp_chain(d, plan, a, b, c, f, nullptr, st);
   if (plan.family == 1) {
     ditto::F32ChainArgs args;
     args.a = a;
@@ -1447,6 +1455,52 @@ int ditto_bmm_chain_run(const ditto_bmm_chain_desc* d, const void* a, const void
     return DITTO_OK;
   }
   return fail(DITTO_EUNSUPPORTED, "no kernel family %d", plan.family);
+}
+
+int ditto_bmm_chain_run_sets(const ditto_bmm_chain_desc* d, int count, const void* const* a, const void* const* b,
+                             const void* const* c, void* const* f, void* stream) {
+  if (!d || count < 0 || (count > 0 && (!a || !b || !c || !f))) return fail(DITTO_EINVAL, "null argument or negative count");
+  const long long elem = 2, out_elem = d->out_dtype == DITTO_F32 ? 4 : 2;
+  for (int at = 0; at < count;) {
+    // the sets from `at` on that one launch takes: 16-bit chains whose A, B and C lie equally far from the first set's
+    int n = 1;
+    ditto::BmmSets sets = {};
+    if ((d->in_dtype == DITTO_F16 || d->in_dtype == DITTO_BF16) && d->inter_op == DITTO_INTER_SOFTMAX && d->b_layout == DITTO_B_LK) {
+      auto apart = [](const void* to, const void* from) {
+        return (long long)(reinterpret_cast<intptr_t>(to) - reinterpret_cast<intptr_t>(from));
+      };
+      for (; at + n < count && n < ditto::kMaxSets; ++n) {
+        const long long in = apart(a[at + n], a[at]);
+        if (!a[at + n] || !b[at + n] || !c[at + n] || !f[at + n] || !aligned(f[at + n], 16) || in % 16 != 0 ||
+            apart(b[at + n], b[at]) != in || apart(c[at + n], c[at]) != in)
+          break;
+        sets.in[n] = in / elem, sets.out[n] = apart(f[at + n], f[at]) / out_elem;
+      }
+    }
+    if (n > 1 && d->batch > 0 && d->batch <= 0x7fffffff / (2 * ditto::kMaxSets)) {
+      ditto_bmm_chain_desc all = *d;
+      all.batch = d->batch * n;
+      if (d->batch_inner == 0 || d->batch_inner == d->batch) {
+        all.batch_inner = d->batch;
+        all.a_batch_stride_outer = all.b_batch_stride_outer = all.c_batch_stride_outer = all.f_batch_stride_outer = 0;
+      }
+      BmmPlan plan;
+      if (plan_bmm(d, &plan, true) == DITTO_OK && plan_bmm(&all, &plan, true) == DITTO_OK && plan_takes_sets(plan)) {
+        if (!a[at] || !b[at] || !c[at] || !f[at]) return fail(DITTO_EINVAL, "null data pointer");
+        if (!aligned(a[at], 16) || !aligned(b[at], 16) || !aligned(c[at], 16) || !aligned(f[at], 16))
+          return fail(DITTO_EINVAL, "data pointers must be 16-byte aligned");
+        sets.count = n, sets.entries = (int)d->batch;
+        const int rc = launch_fp_chain(&all, plan, a[at], b[at], c[at], f[at], &sets, reinterpret_cast<hipStream_t>(stream));
+        if (rc != DITTO_OK) return rc;
+        at += n;
+        continue;
+      }
+    }
+    const int rc = ditto_bmm_chain_run(d, a[at], b[at], c[at], nullptr, f[at], nullptr, 0, stream);
+    if (rc != DITTO_OK) return rc;
+    ++at;
+  }
+  return DITTO_OK;
 }
 
 int ditto_conv_chain_select_tile(const ditto_conv_chain_desc* desc, ditto_tile_param* out) {

@@ -50,8 +50,8 @@ __host__ __device__ constexpr int bmm_chain4m16_lds_bytes() {
   return 2 * kRing4m16 * kBN * D * 2 + 64;  // the tiles and the flag of the optimistic walk
 }
 
-template <typename T, int D, int INTER, int KSPLIT, bool B_KL>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) void bmm_chain4m16_kernel(BmmChainArgs p) {
+template <typename T, int D, int INTER, int KSPLIT, bool B_KL, typename Args>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) void bmm_chain4m16_kernel(Args p) {
 #if defined(__HIP_DEVICE_COMPILE__)
   typedef typename Elem<T>::v8 V8;
   typedef typename Elem<T>::v4 V4;
@@ -85,10 +85,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
   const unsigned lid = xcd_remap(blockIdx.x, gridDim.x);
   const int mb = lid % p.mblocks;
   const int bz = lid / p.mblocks;
-  const int zo = bz / p.batch_inner, zi = bz - zo * p.batch_inner;
-  const T* __restrict__ Ag = reinterpret_cast<const T*>(p.a) + zo * p.a_bs2 + zi * p.a_bs;
-  const T* Bg = reinterpret_cast<const T*>(p.b) + zo * p.b_bs2 + zi * p.b_bs;
-  const T* Cg = reinterpret_cast<const T*>(p.c) + zo * p.c_bs2 + zi * p.c_bs;
+  const BatchEntry be = batch_entry(p, bz);
+  const T* __restrict__ Ag = reinterpret_cast<const T*>(p.a) + be.a;
+  const T* Bg = reinterpret_cast<const T*>(p.b) + be.b;
+  const T* Cg = reinterpret_cast<const T*>(p.c) + be.c;
   const int m_wave = mb * 64 + rh * (16 * RT);  // (either way 16 RT rows per unit of rh)
   const int M = p.M, N = p.N, K = p.K, L = p.L;
 
@@ -497,7 +497,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
       if (!by_rows && n >= N) continue;
       float v0 = oo[t][0] * inv, v1 = oo[t][1] * inv, v2 = oo[t][2] * inv, v3 = oo[t][3] * inv;
       if (!kSoftmax && p.relu_out) { v0 = fmaxf(v0, 0.f); v1 = fmaxf(v1, 0.f); v2 = fmaxf(v2, 0.f); v3 = fmaxf(v3, 0.f); }
-      const long long off = zo * p.f_bs2 + zi * p.f_bs + (long long)row * p.f_rs + n;
+      const long long off = be.f + (long long)row * p.f_rs + n;
       if (p.out_f32) {
         f32x4 w = {v0, v1, v2, v3};
         *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(p.f) + off) = w;
@@ -510,17 +510,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
     }
   }
   if (by_rows)
-    store_tile_rows<T, D, 16>(tw, reinterpret_cast<T*>(p.f) + zo * p.f_bs2 + zi * p.f_bs + (long long)m_tile * p.f_rs,
+    store_tile_rows<T, D, 16>(tw, reinterpret_cast<T*>(p.f) + be.f + (long long)m_tile * p.f_rs,
                                     p.f_rs, M - m_tile, N, lane);
 #else
   (void)p;
 #endif
 }
 
-template <typename T, int D, int INTER, int KSPLIT, bool B_KL>
-hipError_t launch_bmm_chain4m16(const BmmChainArgs& args, hipStream_t stream) {
+template <typename T, int D, int INTER, int KSPLIT, bool B_KL, typename Args>
+hipError_t launch_bmm_chain4m16_args(const Args& args, hipStream_t stream) {
   constexpr int lds = bmm_chain4m16_lds_bytes<D>();
-  auto kern = bmm_chain4m16_kernel<T, D, INTER, KSPLIT, B_KL>;
+  auto kern = bmm_chain4m16_kernel<T, D, INTER, KSPLIT, B_KL, Args>;
   static thread_local int configured_dev = -1;
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
@@ -533,6 +533,13 @@ hipError_t launch_bmm_chain4m16(const BmmChainArgs& args, hipStream_t stream) {
   const unsigned grid = (unsigned)args.mblocks * (unsigned)args.batch;
   hipLaunchKernelGGL(kern, dim3(grid), dim3(256), lds, stream, args);
   return hipGetLastError();
+}
+
+template <typename T, int D, int INTER, int KSPLIT, bool B_KL>
+hipError_t launch_bmm_chain4m16(const BmmChainArgs& args, const BmmSets* sets, hipStream_t stream) {
+  if constexpr (INTER == kInterSoftmax && !B_KL)
+    if (sets) return launch_bmm_chain4m16_args<T, D, INTER, KSPLIT, B_KL>(BmmSetsArgs{args, *sets}, stream);
+  return sets ? hipErrorInvalidValue : launch_bmm_chain4m16_args<T, D, INTER, KSPLIT, B_KL>(args, stream);
 }
 
 }  // namespace ditto

@@ -52,8 +52,8 @@ inline int bmm_chain_rows_lds(int dt, int nw, bool kl) {
   return kl ? bmm_chain_rows_lds<8, true, 8>() : bmm_chain_rows_lds<8, false, 8>();
 }
 
-template <typename T, int DT, int NW, int INTER, bool B_KL>
-__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) void bmm_chain_rows_kernel(BmmChainArgs p) {
+template <typename T, int DT, int NW, int INTER, bool B_KL, typename Args>
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) void bmm_chain_rows_kernel(Args p) {
 #if defined(__HIP_DEVICE_COMPILE__)
   typedef typename Elem<T>::v8 V8;
   typedef typename Elem<T>::v4 V4;
@@ -69,10 +69,10 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const unsigned lid = xcd_remap(blockIdx.x, gridDim.x);
   const int bz = lid / (unsigned)p.mblocks, m0 = (lid - bz * (unsigned)p.mblocks) * (16 * RT * NW) + 16 * RT * w;
-  const int zo = bz / (unsigned)p.batch_inner, zi = bz - zo * p.batch_inner;
-  const T* __restrict__ Ag = reinterpret_cast<const T*>(p.a) + zo * p.a_bs2 + zi * p.a_bs;
-  const T* const Bg = reinterpret_cast<const T*>(p.b) + zo * p.b_bs2 + zi * p.b_bs;
-  const T* const Cg = reinterpret_cast<const T*>(p.c) + zo * p.c_bs2 + zi * p.c_bs;
+  const BatchEntry be = batch_entry(p, bz);
+  const T* __restrict__ Ag = reinterpret_cast<const T*>(p.a) + be.a;
+  const T* const Bg = reinterpret_cast<const T*>(p.b) + be.b;
+  const T* const Cg = reinterpret_cast<const T*>(p.c) + be.c;
   const int M = p.M, N = p.N, K = p.K, L = p.L;
   const bool busy = m0 < M;  // a wave without rows loads its share of the tiles and keeps the barriers
 
@@ -327,7 +327,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
   static_assert(NW * 16 * RT * kRowBytes <= NR * TB, "the parked rows need the staged tiles' LDS");
   static_assert(16 * RT * D / 8 % 64 == 0, "whole waves of 16-byte stores");
   char* const tw = smem_rw + w * (16 * RT * kRowBytes);
-  const long long f0 = zo * p.f_bs2 + zi * p.f_bs + (long long)m0 * p.f_rs;
+  const long long f0 = be.f + (long long)m0 * p.f_rs;
 #pragma unroll
   for (int j = 0; j < RT; ++j) {
     const float inv = kSoftmax ? 1.f / ls[j][0] : 1.f;
@@ -356,10 +356,10 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
 #endif
 }
 
-template <typename T, int DT, int NW, int INTER, bool B_KL>
-hipError_t launch_bmm_chain_rows(const BmmChainArgs& args, hipStream_t stream) {
+template <typename T, int DT, int NW, int INTER, bool B_KL, typename Args>
+hipError_t launch_bmm_chain_rows_args(const Args& args, hipStream_t stream) {
   constexpr int lds = bmm_chain_rows_lds<DT, B_KL, NW>();
-  auto kern = bmm_chain_rows_kernel<T, DT, NW, INTER, B_KL>;
+  auto kern = bmm_chain_rows_kernel<T, DT, NW, INTER, B_KL, Args>;
   static thread_local int configured_dev = -1;
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
@@ -371,6 +371,13 @@ hipError_t launch_bmm_chain_rows(const BmmChainArgs& args, hipStream_t stream) {
   }
   hipLaunchKernelGGL(kern, dim3((unsigned)args.mblocks * (unsigned)args.batch), dim3(64 * NW), lds, stream, args);
   return hipGetLastError();
+}
+
+template <typename T, int DT, int NW, int INTER, bool B_KL>
+hipError_t launch_bmm_chain_rows(const BmmChainArgs& args, const BmmSets* sets, hipStream_t stream) {
+  if constexpr (INTER == kInterSoftmax && !B_KL)
+    if (sets) return launch_bmm_chain_rows_args<T, DT, NW, INTER, B_KL>(BmmSetsArgs{args, *sets}, stream);
+  return sets ? hipErrorInvalidValue : launch_bmm_chain_rows_args<T, DT, NW, INTER, B_KL>(args, stream);
 }
 
 }  // namespace ditto

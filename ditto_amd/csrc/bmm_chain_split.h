@@ -47,8 +47,8 @@ inline int bmm_chain_split_lds(int dt, int rt, bool kl) {
   return tiles > merge ? tiles : merge;
 }
 
-template <typename T, int DT, int RT, int INTER, bool B_KL>
-__global__ __launch_bounds__(64 * kSplitWaves) void bmm_chain_split_kernel(BmmChainArgs p) {
+template <typename T, int DT, int RT, int INTER, bool B_KL, typename Args>
+__global__ __launch_bounds__(64 * kSplitWaves) void bmm_chain_split_kernel(Args p) {
 #if defined(__HIP_DEVICE_COMPILE__)
   typedef typename Elem<T>::v8 V8;
   typedef typename Elem<T>::v4 V4;
@@ -64,10 +64,10 @@ __global__ __launch_bounds__(64 * kSplitWaves) void bmm_chain_split_kernel(BmmCh
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const unsigned lid = xcd_remap(blockIdx.x, gridDim.x);
   const int bz = lid / (unsigned)p.mblocks, m0 = (lid - bz * (unsigned)p.mblocks) * 16 * RT;
-  const int zo = bz / (unsigned)p.batch_inner, zi = bz - zo * p.batch_inner;
-  const T* __restrict__ Ag = reinterpret_cast<const T*>(p.a) + zo * p.a_bs2 + zi * p.a_bs;
-  const T* const Bg = reinterpret_cast<const T*>(p.b) + zo * p.b_bs2 + zi * p.b_bs;
-  const T* const Cg = reinterpret_cast<const T*>(p.c) + zo * p.c_bs2 + zi * p.c_bs;
+  const BatchEntry be = batch_entry(p, bz);
+  const T* __restrict__ Ag = reinterpret_cast<const T*>(p.a) + be.a;
+  const T* const Bg = reinterpret_cast<const T*>(p.b) + be.b;
+  const T* const Cg = reinterpret_cast<const T*>(p.c) + be.c;
   const int M = p.M, N = p.N, K = p.K, L = p.L;
 
   // A fragments (operand column = row of A); with B stored [K][L] in the contraction order its transposing reads give
@@ -276,7 +276,7 @@ __global__ __launch_bounds__(64 * kSplitWaves) void bmm_chain_split_kernel(BmmCh
     }
   }
   wg_sync();
-  const long long f0 = zo * p.f_bs2 + zi * p.f_bs;
+  const long long f0 = be.f;
   for (int e = tid; e < 16 * RT * 4 * DT; e += 64 * kSplitWaves) {
     const int row = e / (4 * DT), n0 = 4 * (e - row * 4 * DT);
     float wt[kSplitWaves];
@@ -318,10 +318,10 @@ __global__ __launch_bounds__(64 * kSplitWaves) void bmm_chain_split_kernel(BmmCh
 #endif
 }
 
-template <typename T, int DT, int RT, int INTER, bool B_KL>
-hipError_t launch_bmm_chain_split(const BmmChainArgs& args, hipStream_t stream) {
+template <typename T, int DT, int RT, int INTER, bool B_KL, typename Args>
+hipError_t launch_bmm_chain_split_args(const Args& args, hipStream_t stream) {
   const int lds = bmm_chain_split_lds(DT, RT, B_KL);
-  auto kern = bmm_chain_split_kernel<T, DT, RT, INTER, B_KL>;
+  auto kern = bmm_chain_split_kernel<T, DT, RT, INTER, B_KL, Args>;
   static thread_local int configured_dev = -1;
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
@@ -333,6 +333,13 @@ hipError_t launch_bmm_chain_split(const BmmChainArgs& args, hipStream_t stream) 
   }
   hipLaunchKernelGGL(kern, dim3((unsigned)args.mblocks * (unsigned)args.batch), dim3(64 * kSplitWaves), lds, stream, args);
   return hipGetLastError();
+}
+
+template <typename T, int DT, int RT, int INTER, bool B_KL>
+hipError_t launch_bmm_chain_split(const BmmChainArgs& args, const BmmSets* sets, hipStream_t stream) {
+  if constexpr (INTER == kInterSoftmax && !B_KL)
+    if (sets) return launch_bmm_chain_split_args<T, DT, RT, INTER, B_KL>(BmmSetsArgs{args, *sets}, stream);
+  return sets ? hipErrorInvalidValue : launch_bmm_chain_split_args<T, DT, RT, INTER, B_KL>(args, stream);
 }
 
 }  // namespace ditto

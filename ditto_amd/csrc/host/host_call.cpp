@@ -15,6 +15,7 @@
 
 #include <cstring>
 #include <string>
+#include <vector>
 
 #include "../../../include/ditto_chain.h"
 
@@ -258,35 +259,45 @@ PyObject* py_run_bmm_desc(PyObject*, PyObject* const* v, Py_ssize_t n) {
   });
 }
 
+// Attention over a packed projection x [batch, M, 3 * hidden] into out [batch, M, hidden]: the descriptor of the chain over
+// [batch, heads, M, d] views of the packed rows (keys as stored, one row of d per key); false where the tensors are not the
+// plain case (a 3-D projection with contiguous rows, a contiguous out).
+bool plain_projection(const at::Tensor& x, int64_t heads, int64_t hidden) {
+  return x.dim() == 3 && x.size(2) == 3 * hidden && x.stride(2) == 1 && x.device().type() == c10::kCUDA && x.size(0) > 0 &&
+         x.size(1) > 0 && hidden / heads > 1;
+}
+bool plain_output(const at::Tensor& o, const at::Tensor& x, int64_t hidden) {
+  return o.dim() == 3 && o.size(0) == x.size(0) && o.size(1) == x.size(1) && o.size(2) == hidden && o.is_contiguous() &&
+         o.device() == x.device();
+}
+void fill_attention(ditto_bmm_chain_desc* desc, const at::Tensor& x, at::ScalarType out, int64_t heads, int64_t hidden, float scale,
+                    int tile_variant) {
+  const int64_t batch = x.size(0), M = x.size(1), d = hidden / heads, s0 = x.stride(0), s1 = x.stride(1);
+  Operand Q, K, F;
+  Q.outer = batch, Q.outer_stride = s0, Q.batch = heads, Q.rows = M, Q.cols = d, Q.sb = d, Q.sr = s1, Q.sc = 1;
+  K = Q, K.rows = d, K.cols = M, K.sr = 1, K.sc = s1;
+  F = Q, F.outer_stride = M * hidden, F.sr = hidden;
+  fill_bmm(desc, Q, K, Q, F, x.scalar_type(), out, {DITTO_INTER_SOFTMAX, scale, 1.f, tile_variant, false});
+}
+
 // run_attention(query_key_value, out | None, heads, hidden, scale, tile_variant) -> (return code, out), or None where the
-// tensors are not the plain case (then the caller goes by views): a 3-D projection with contiguous rows, a contiguous out
+// tensors are not the plain case (then the caller goes by views)
 PyObject* py_run_attention(PyObject*, PyObject* const* v, Py_ssize_t n) {
   return guarded([&]() -> PyObject* {
     if (n != 6) fail(PyExc_TypeError, "run_attention takes 6 arguments");
     const at::Tensor& x = tensor_of(v[0]);
     const int64_t heads = integer(v[2]), hidden = integer(v[3]);
-    if (x.dim() != 3 || x.size(2) != 3 * hidden || x.stride(2) != 1 || x.device().type() != c10::kCUDA) Py_RETURN_NONE;
-    const int64_t batch = x.size(0), M = x.size(1), d = hidden / heads;
-    if (batch <= 0 || M <= 0 || d <= 1) Py_RETURN_NONE;
+    if (!plain_projection(x, heads, hidden)) Py_RETURN_NONE;
     at::Tensor made;
     PyObject* out_obj = v[1];
     if (out_obj != Py_None) {
-      const at::Tensor& o = tensor_of(out_obj);
-      if (o.dim() != 3 || o.size(0) != batch || o.size(1) != M || o.size(2) != hidden || !o.is_contiguous() || o.device() != x.device())
-        Py_RETURN_NONE;
+      if (!plain_output(tensor_of(out_obj), x, hidden)) Py_RETURN_NONE;
     } else {
-      made = at::empty({batch, M, hidden}, x.options().requires_grad(false));
+      made = at::empty({x.size(0), x.size(1), hidden}, x.options().requires_grad(false));
     }
     const at::Tensor& out = out_obj != Py_None ? tensor_of(out_obj) : made;
-    const int64_t s0 = x.stride(0), s1 = x.stride(1);
-    // [batch, heads, M, d] views of the packed rows; keys as stored, one row of d per key
-    Operand Q, K, F;
-    Q.outer = batch, Q.outer_stride = s0, Q.batch = heads, Q.rows = M, Q.cols = d, Q.sb = d, Q.sr = s1, Q.sc = 1;
-    K = Q, K.rows = d, K.cols = M, K.sr = 1, K.sc = s1;
-    F = Q, F.outer_stride = M * hidden, F.sr = hidden;
-    const BmmParams p = {DITTO_INTER_SOFTMAX, (float)number(v[4]), 1.f, (int)integer(v[5]), false};
     ditto_bmm_chain_desc desc;
-    fill_bmm(&desc, Q, K, Q, F, x.scalar_type(), out.scalar_type(), p);
+    fill_attention(&desc, x, out.scalar_type(), heads, hidden, (float)number(v[4]), (int)integer(v[5]));
     const int64_t step = hidden * x.element_size();
     const char* const base = static_cast<const char*>(x.data_ptr());
     void* const dst = out.data_ptr();
@@ -303,6 +314,48 @@ PyObject* py_run_attention(PyObject*, PyObject* const* v, Py_ssize_t n) {
       PyTuple_SET_ITEM(result, 1, THPVariable_Wrap(std::move(made)));
     }
     return result;
+  });
+}
+
+// run_attention_sets(projections, outs, heads, hidden, scale, tile_variant): run_attention on several projections of one
+// shape, in as few launches as hold them -> return code, or None where that does not do: tensors that are not the plain
+// case or not alike, or an output that shares memory with another set's tensors (then the caller runs them in order)
+PyObject* py_run_attention_sets(PyObject*, PyObject* const* v, Py_ssize_t n) {
+  return guarded([&]() -> PyObject* {
+    if (n != 6 || !PyList_Check(v[0]) || !PyList_Check(v[1]) || PyList_GET_SIZE(v[0]) != PyList_GET_SIZE(v[1]) ||
+        PyList_GET_SIZE(v[0]) == 0)
+      fail(PyExc_TypeError, "run_attention_sets takes two lists of tensors, equally long, and 4 numbers");
+    const int64_t heads = integer(v[2]), hidden = integer(v[3]);
+    const Py_ssize_t sets = PyList_GET_SIZE(v[0]);
+    struct Span {
+      uintptr_t begin, end;
+      bool meets(const Span& o) const { return begin < o.end && o.begin < end; }
+    };
+    std::vector<Span> in(sets), out(sets);
+    std::vector<const void*> q(sets), k(sets), c(sets);
+    std::vector<void*> f(sets);
+    const at::Tensor &x0 = tensor_of(PyList_GET_ITEM(v[0], 0)), &o0 = tensor_of(PyList_GET_ITEM(v[1], 0));
+    const int64_t step = hidden * (int64_t)x0.element_size();
+    for (Py_ssize_t i = 0; i < sets; ++i) {
+      const at::Tensor &x = tensor_of(PyList_GET_ITEM(v[0], i)), &o = tensor_of(PyList_GET_ITEM(v[1], i));
+      if (!plain_projection(x, heads, hidden) || !plain_output(o, x, hidden) || x.sizes() != x0.sizes() ||
+          x.strides() != x0.strides() || x.scalar_type() != x0.scalar_type() || o.scalar_type() != o0.scalar_type() ||
+          x.device() != x0.device())
+        Py_RETURN_NONE;
+      const char* const base = static_cast<const char*>(x.data_ptr());
+      q[i] = base, k[i] = base + step, c[i] = base + 2 * step, f[i] = o.data_ptr();
+      const int64_t last = (x.size(0) - 1) * x.stride(0) + (x.size(1) - 1) * x.stride(1) + x.size(2);
+      in[i] = {reinterpret_cast<uintptr_t>(base), reinterpret_cast<uintptr_t>(base) + last * x.element_size()};
+      out[i] = {reinterpret_cast<uintptr_t>(f[i]), reinterpret_cast<uintptr_t>(f[i]) + o.numel() * o.element_size()};
+    }
+    for (Py_ssize_t i = 0; i < sets; ++i)
+      for (Py_ssize_t j = 0; j < sets; ++j)
+        if (i != j && (out[i].meets(in[j]) || out[i].meets(out[j]))) Py_RETURN_NONE;
+    ditto_bmm_chain_desc desc;
+    fill_attention(&desc, x0, o0.scalar_type(), heads, hidden, (float)number(v[4]), (int)integer(v[5]));
+    return PyLong_FromLong(on_current_stream(x0.device(), [&](void* stream) {
+      return ditto_bmm_chain_run_sets(&desc, (int)sets, q.data(), k.data(), c.data(), f.data(), stream);
+    }));
   });
 }
 
@@ -508,6 +561,7 @@ PyTypeObject conv_call_type = {PyVarObject_HEAD_INIT(nullptr, 0)};
 #define FAST(name, fn) {name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)(void)>(fn)), METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {FAST("fill_bmm_desc", py_fill_bmm_desc), FAST("run_bmm", py_run_bmm),
                          FAST("run_bmm_desc", py_run_bmm_desc), FAST("run_attention", py_run_attention),
+                         FAST("run_attention_sets", py_run_attention_sets),
                          {nullptr, nullptr, 0, nullptr}};
 #undef FAST
 

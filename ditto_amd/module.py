@@ -376,11 +376,28 @@ class AttentionFunction:
         self.sch = sch
         self.tensors = list(tensors) if tensors is not None else sch.layer.schedule_tensors
 
-    def __call__(self, query_key_value, out):
+    def _check(self, query_key_value, out):
         for a, t in zip((query_key_value, out), self.tensors):
             if tuple(a.shape) != tuple(t.shape):
                 raise ValueError("argument for %s has shape %s, expected %s" % (t.name, tuple(a.shape), t.shape))
+
+    def __call__(self, query_key_value, out):
+        self._check(query_key_value, out)
         self.sch.module.forward(query_key_value, out, tile_variant=self.sch.tile_variant)
+
+    def run_sets(self, calls):
+        """What calling the function with each ``(query_key_value, out)`` of ``calls`` in order does.  Calls that do not
+        read or write what another of them writes share launches (``ditto_bmm_chain_run_sets``); else they run one by one."""
+        for args in calls:
+            self._check(*args)
+        m = self.sch.module
+        rc = _lib.host().run_attention_sets([x for x, _ in calls], [o for _, o in calls], m.num_heads, m.hidden_size, m.scale,
+                                            self.sch.tile_variant)
+        if rc is None:
+            for args in calls:
+                self(*args)
+        elif rc:
+            _lib.check(rc)
 
 
 def build(sch, tensors=None, target="hip", name="default_function", tile_variant=None):

@@ -329,3 +329,84 @@ def test_specialised_conv_chain_with_outputs_of_either_type(oracle):
         mx, rel = errors(y.float().cpu().numpy(), want)
         assert mx <= 1e-2 and rel <= 1e-3, (dt, mx, rel)
         assert f._is_prepared(w1, w2, dt)
+
+def _attention_layers(heads, d, batch, M, dtype, count):
+    from ditto_amd import auto_schedule, chimera
+
+    mha = ac.nn.module.MultiHeadAttentionMMA(heads, heads * d, dtype, "float32", scale=None)
+    graph = runtime.Graph([mha.layer(batch, M) for _ in range(count)], outputs=[(i, 0) for i in range(count)])
+    bound = chimera.task_binding(auto_schedule.extract_tasks_from_graph(graph))
+    opt = auto_schedule.ScheduleOption("hip", log_file="untuned.log", dtype=dtype)
+    mods = {k: ditto.build(s, a, "hip") for k, (s, a) in auto_schedule.retrieve_schedule_bound_tasks(bound, opt).items()}
+    return graph, mods
+
+# layers x heads x rows on either side of what one launch takes and of the lines between the kernels (key-splitting, 64-row,
+# 32 rows per wave, the large ones that take no sets), ragged rows among them
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+@pytest.mark.parametrize("heads,d,batch,M,count", [(2, 64, 1, 49, 2), (12, 64, 1, 99, 12), (8, 64, 2, 257, 17), (3, 80, 1, 130, 5),
+                                                   (2, 128, 1, 65, 3), (12, 64, 8, 512, 3), (4, 64, 1, 2100, 33)])
+def test_layers_that_share_a_launch_match_layers_run_one_by_one(heads, d, batch, M, count, dtype):
+    graph, mods = _attention_layers(heads, d, batch, M, dtype, count)
+    (func,) = mods.values()
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    ins = [torch.empty(batch, M, 3 * heads * d, dtype=getattr(torch, dtype), device="cuda").normal_(generator=gen)
+           for _ in range(count)]
+    alone = [torch.empty(batch, M, heads * d, dtype=x.dtype, device="cuda") for x in ins]
+    for x, o in zip(ins, alone):
+        func(x, o)
+    # both are within the 16-bit chain's bound of the closed form (another kernel may be chosen for all of them together)
+    bound = 1e-3 if dtype == "float16" else 2 * 2.6e-3
+    for make in (runtime.create_graph_engine, runtime.create_hip_graph_engine):
+        eng = make(graph, mods, "cuda:0")
+        eng.set_inputs(ins)
+        eng.compile()
+        for _ in range(3):  # replays with eager work and synchronisations in between
+            for o in eng.get_outputs():
+                o.zero_()
+            torch.cuda.synchronize()
+            eng.run()
+            torch.cuda.synchronize()
+            for got, want in zip(eng.get_outputs(), alone):
+                assert (got.float() - want.float()).norm() <= bound * want.float().norm()
+            func(ins[0], alone[0])
+
+def test_calls_that_share_memory_run_in_order():
+    """An output that is part of the next call's input: the calls are not independent and must not share a launch."""
+    heads, d, M = 2, 64, 64
+    graph, mods = _attention_layers(heads, d, 1, M, "float16", 2)
+    (func,) = mods.values()
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    x0 = torch.empty(1, M, 3 * heads * d, dtype=torch.float16, device="cuda").normal_(generator=gen)
+    x1 = torch.empty_like(x0).normal_(generator=gen)
+    o0 = x1.view(-1)[: M * heads * d].view(1, M, heads * d)
+    o1 = torch.empty(1, M, heads * d, dtype=torch.float16, device="cuda")
+    a0, a1 = x0.clone(), x1.clone()
+    b0, b1 = a1.view(-1)[: M * heads * d].view(1, M, heads * d), torch.empty_like(o1)
+    func.run_sets([(x0, o0), (x1, o1)])
+    func(a0, b0)
+    func(a1, b1)
+    assert torch.equal(o0, b0) and torch.equal(o1, b1)
+    with pytest.raises(ValueError):
+        func.run_sets([(x0, o0), (x1[:, :32], o1)])
+
+def test_run_sets_through_the_c_abi_matches_single_calls():
+    """Sets whose A, B and C are not equally far from the first's are launched by themselves, others together."""
+    import ctypes
+
+    from ditto_amd import _lib, chain
+
+    gen = torch.Generator(device="cuda").manual_seed(7)
+    shape, n = (3, 65, 64), 4
+    rows = [torch.empty(shape, dtype=torch.float16, device="cuda").normal_(generator=gen) for _ in range(3 * n)]
+    outs = [torch.empty(shape, dtype=torch.float16, device="cuda") for _ in range(n)]
+    want = torch.empty_like(outs[0])
+    q, k, v = rows[:n], rows[n:2 * n], rows[2 * n:]
+    desc = chain.bmm_chain_desc(q[0], k[0].transpose(1, 2), v[0], outs[0], "softmax", 0.125, 1.0, 0, False)
+    arrays = [(ctypes.c_void_p * n)(*(t.data_ptr() for t in ts)) for ts in (q, k, v, outs)]
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    assert _lib.load().ditto_bmm_chain_run_sets(ctypes.byref(desc), n, *arrays, stream) == 0
+    for i in range(n):
+        chain.run_bmm_chain(q[i], k[i].transpose(1, 2), v[i], want, inter_op="softmax", softmax_scale=0.125)
+        assert (outs[i].float() - want.float()).norm() <= 1e-3 * want.float().norm()
+    assert _lib.load().ditto_bmm_chain_run_sets(ctypes.byref(desc), -1, *arrays, stream) == -1
+    assert _lib.load().ditto_bmm_chain_run_sets(ctypes.byref(desc), 0, *arrays, stream) == 0
