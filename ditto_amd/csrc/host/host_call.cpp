@@ -317,14 +317,14 @@ PyObject* py_run_attention(PyObject*, PyObject* const* v, Py_ssize_t n) {
   });
 }
 
-// run_attention_sets(projections, outs, heads, hidden, scale, tile_variant): run_attention on several projections of one
-// shape, in as few launches as hold them -> return code, or None where that does not do: tensors that are not the plain
-// case or not alike, or an output that shares memory with another set's tensors (then the caller runs them in order)
+// run_attention_sets(projections, outs, heads, hidden, scale, tile_variant, batch, rows): run_attention on several projections
+// [batch, rows, 3 * hidden], in as few launches as hold them -> return code, or None where that does not do: tensors that are
+// not the plain case, not of that shape or not alike, or an output that shares memory with another set's tensors (then the caller runs them in order)
 PyObject* py_run_attention_sets(PyObject*, PyObject* const* v, Py_ssize_t n) {
   return guarded([&]() -> PyObject* {
-    if (n != 6 || !PyList_Check(v[0]) || !PyList_Check(v[1]) || PyList_GET_SIZE(v[0]) != PyList_GET_SIZE(v[1]) ||
+    if (n != 8 || !PyList_Check(v[0]) || !PyList_Check(v[1]) || PyList_GET_SIZE(v[0]) != PyList_GET_SIZE(v[1]) ||
         PyList_GET_SIZE(v[0]) == 0)
-      fail(PyExc_TypeError, "run_attention_sets takes two lists of tensors, equally long, and 4 numbers");
+      fail(PyExc_TypeError, "run_attention_sets takes two lists of tensors, equally long, and 6 numbers");
     const int64_t heads = integer(v[2]), hidden = integer(v[3]);
     const Py_ssize_t sets = PyList_GET_SIZE(v[0]);
     struct Span {
@@ -334,11 +334,12 @@ PyObject* py_run_attention_sets(PyObject*, PyObject* const* v, Py_ssize_t n) {
     std::vector<Span> in(sets), out(sets);
     std::vector<const void*> q(sets), k(sets), c(sets);
     std::vector<void*> f(sets);
+    const int64_t batch = integer(v[6]), rows = integer(v[7]);
     const at::Tensor &x0 = tensor_of(PyList_GET_ITEM(v[0], 0)), &o0 = tensor_of(PyList_GET_ITEM(v[1], 0));
     const int64_t step = hidden * (int64_t)x0.element_size();
     for (Py_ssize_t i = 0; i < sets; ++i) {
       const at::Tensor &x = tensor_of(PyList_GET_ITEM(v[0], i)), &o = tensor_of(PyList_GET_ITEM(v[1], i));
-      if (!plain_projection(x, heads, hidden) || !plain_output(o, x, hidden) || x.sizes() != x0.sizes() ||
+      if (!plain_projection(x, heads, hidden) || !plain_output(o, x, hidden) || x.size(0) != batch || x.size(1) != rows ||
           x.strides() != x0.strides() || x.scalar_type() != x0.scalar_type() || o.scalar_type() != o0.scalar_type() ||
           x.device() != x0.device())
         Py_RETURN_NONE;

@@ -385,19 +385,23 @@ class AttentionFunction:
         self._check(query_key_value, out)
         self.sch.module.forward(query_key_value, out, tile_variant=self.sch.tile_variant)
 
-    def run_sets(self, calls):
-        """What calling the function with each ``(query_key_value, out)`` of ``calls`` in order does.  Calls that do not
-        read or write what another of them writes share launches (``ditto_bmm_chain_run_sets``); else they run one by one."""
-        for args in calls:
-            self._check(*args)
-        m = self.sch.module
-        rc = _lib.host().run_attention_sets([x for x, _ in calls], [o for _, o in calls], m.num_heads, m.hidden_size, m.scale,
-                                            self.sch.tile_variant)
-        if rc is None:
-            for args in calls:
-                self(*args)
-        elif rc:
-            _lib.check(rc)
+    def sets(self, calls):
+        """A callable that does what calling the function with each ``(query_key_value, out)`` of ``calls`` in order does.
+        Calls that do not read or write what another of them writes share launches (``ditto_bmm_chain_run_sets``); else they
+        run one by one."""
+        m, host = self.sch.module, _lib.host()
+        xs, outs = [x for x, _ in calls], [o for _, o in calls]
+        batch, rows = self.tensors[0].shape[:2]
+
+        def run():
+            rc = host.run_attention_sets(xs, outs, m.num_heads, m.hidden_size, m.scale, self.sch.tile_variant, batch, rows)
+            if rc is None:
+                for args in calls:
+                    self(*args)
+            elif rc:
+                _lib.check(rc)
+
+        return run
 
 
 def build(sch, tensors=None, target="hip", name="default_function", tile_variant=None):

@@ -8,6 +8,7 @@ device; every layer's function is called as ``f(*inputs, *weights, *outputs)``
 the whole sequence once into a HIP graph and replays it, the counterpart of the reference's
 CUDA-graph engine.
 """
+import functools
 import time
 
 import torch
@@ -116,29 +117,36 @@ class GraphEngine:
                 func = func.specialize(*self.weight_buffer[li])
             args = [*self.input_buffer[li], *self.weight_buffer[li], *self.output_buffer[li]]
             self._to_exe.append((func, args))
+        self._steps = self._make_steps()
+        self._weights = [w for li in sorted(self.weight_buffer) for w in self.weight_buffer[li]]
         self._weight_versions = self._versions()
 
     def _versions(self):
-        return [w._version for li in sorted(self.weight_buffer) for w in self.weight_buffer[li]]
+        return [w._version for w in self._weights]
 
     def run(self):
         if not self._to_exe:
             self.compile()
-        # Consecutive layers of one function that takes several calls at once (attention blocks) go to it together, up to a
-        # layer that reads what one of them makes.  Twelve such layers in a launch of their own each are twelve starts and
-        # twelve tails: 12 x [8 heads, 236 rows of 64] 54 -> 5.5 us, 12 x [96 heads, 512 rows of 64] 176 -> 128 us.
-        li = 0
+        for step in self._steps:
+            step()
+
+    def _make_steps(self):
+        """The calls of one run.  Consecutive layers of one function that takes several calls at once (attention blocks) make
+        one step, up to a layer that reads what one of them makes: twelve such layers in a launch of their own each are twelve
+        starts and twelve tails (12 x [96 heads, 512 rows of 64] 171 -> 131 us, 12 x [12 heads, 99 rows of 64] 50 -> 18)."""
+        steps, li = [], 0
         while li < len(self._to_exe):
             func, args = self._to_exe[li]
             end = li + 1
-            if hasattr(func, "run_sets"):
+            if hasattr(func, "sets"):
                 while end < len(self._to_exe) and self._to_exe[end][0] is func and not self._reads(end, li):
                     end += 1
             if end - li > 1:
-                func.run_sets([tuple(a) for _, a in self._to_exe[li:end]])
+                steps.append(func.sets([tuple(a) for _, a in self._to_exe[li:end]]))
             else:
-                func(*args)
+                steps.append(functools.partial(func, *args))
             li = end
+        return steps
 
     def _reads(self, li, first):
         """Whether layer ``li`` has an edge from layer ``first`` or a later one."""
@@ -159,13 +167,20 @@ class GraphEngine:
 
 
 class HipGraphEngine(GraphEngine):
-    """Records the layer sequence into a HIP graph at compile time and replays it on run."""
+    """Records the layer sequence into a HIP graph at compile time and replays it on run.
+
+    A replay costs the host 17 us however little the graph holds, a step by itself 3 - 4 us: up to four steps (attention
+    layers that share a launch are one) are not recorded but called."""
+
+    MOST_CALLED = 4
 
     def compile(self):
         super().compile()
         self._graph = None
         GraphEngine.run(self)  # warm-up outside the capture (first-call set-up, cached workspaces)
         torch.cuda.synchronize(self.dev)
+        if len(self._steps) <= self.MOST_CALLED:
+            return
         g = torch.cuda.CUDAGraph()
         with torch.cuda.graph(g):
             GraphEngine.run(self)
@@ -174,9 +189,12 @@ class HipGraphEngine(GraphEngine):
     def run(self):
         # (a recorded graph holds the repacked weights of compile time: weights updated in place since then
         # need the repacking, and with it the recording, done again)
-        if not self._to_exe or getattr(self, "_graph", None) is None or self._versions() != self._weight_versions:
+        if not self._to_exe or self._versions() != self._weight_versions:
             self.compile()
-        self._graph.replay()
+        if self._graph is None:
+            GraphEngine.run(self)
+        else:
+            self._graph.replay()
 
 
 def create_graph_engine(graph, built_mods, dev="cuda:0"):

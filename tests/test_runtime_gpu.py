@@ -356,10 +356,14 @@ def test_layers_that_share_a_launch_match_layers_run_one_by_one(heads, d, batch,
         func(x, o)
     # both are within the 16-bit chain's bound of the closed form (another kernel may be chosen for all of them together)
     bound = 1e-3 if dtype == "float16" else 2 * 2.6e-3
-    for make in (runtime.create_graph_engine, runtime.create_hip_graph_engine):
+    for make, recorded in ((runtime.create_graph_engine, None), (runtime.create_hip_graph_engine, False),
+                           (runtime.create_hip_graph_engine, True)):
         eng = make(graph, mods, "cuda:0")
+        if recorded:
+            eng.MOST_CALLED = 0
         eng.set_inputs(ins)
         eng.compile()
+        assert recorded is None or (eng._graph is not None) == recorded
         for _ in range(3):  # replays with eager work and synchronisations in between
             for o in eng.get_outputs():
                 o.zero_()
@@ -382,12 +386,12 @@ def test_calls_that_share_memory_run_in_order():
     o1 = torch.empty(1, M, heads * d, dtype=torch.float16, device="cuda")
     a0, a1 = x0.clone(), x1.clone()
     b0, b1 = a1.view(-1)[: M * heads * d].view(1, M, heads * d), torch.empty_like(o1)
-    func.run_sets([(x0, o0), (x1, o1)])
+    func.sets([(x0, o0), (x1, o1)])()
     func(a0, b0)
     func(a1, b1)
     assert torch.equal(o0, b0) and torch.equal(o1, b1)
     with pytest.raises(ValueError):
-        func.run_sets([(x0, o0), (x1[:, :32], o1)])
+        func.sets([(x0, o0), (x1[:, :32], o1)])()
 
 def test_run_sets_through_the_c_abi_matches_single_calls():
     """Sets whose A, B and C are not equally far from the first's are launched by themselves, others together."""
