@@ -97,7 +97,95 @@ int plan_rows_384(long long M, long long batch, int cus) {
   return best_a;
 }
 
+// What a kernel takes, in us per launch: start + (first + per_key L) for every round of workgroups over the compute units; a
+// kernel of several workgroups to a compute unit has a pair for each number of them, the last one for full rounds.
+struct BmmPrice {
+  int variant, rows, threads, resident;
+  float start, first[3], per_key[3];
+};
+// Least squares over 3300 random shapes (batch 1 - 160, 32 - 4096 rows and keys, fp16 and bf16), root mean square error
+// 4 - 12 %; the columns: head sizes up to 64 | 128, without | with softmax, B [L][K] | [K][L].
+constexpr BmmPrice kPrices64[2][8] = {
+    {{641, 128, 256, 1, 0.71f, {3.38f}, {.0074f}}, {644, 64, 256, 3, 2.64f, {1.30f, 1.81f, 2.36f}, {.0049f, .0079f, .0121f}},
+     {645, 64, 256, 2, 2.98f, {1.34f, 2.09f}, {.0042f, .0070f}}, {649, 256, 512, 1, 0, {5.03f}, {.0118f}},
+     {2144, 128, 256, 2, 1.51f, {2.68f, 3.41f}, {.0091f, .0155f}}, {2148, 256, 512, 1, 2.23f, {2.31f}, {.0124f}}},
+    {{641, 128, 256, 1, 0.68f, {3.38f}, {.0077f}}, {644, 64, 256, 3, 2.75f, {1.33f, 1.93f, 2.79f}, {.0060f, .0092f, .0128f}},
+     {645, 64, 256, 2, 3.05f, {1.53f, 2.74f}, {.0049f, .0074f}}, {649, 256, 512, 1, 0, {5.14f}, {.0117f}},
+     {2144, 128, 256, 2, 1.67f, {2.89f, 4.04f}, {.0097f, .0158f}}, {2148, 256, 512, 1, 1.81f, {3.20f}, {.0116f}},
+     {2041, 16, 512, 1, 2.89f, {1.35f}, {.0025f}}, {2042, 32, 512, 1, 2.78f, {2.37f}, {.0027f}}}};
+constexpr BmmPrice kPrices128[2][2][7] = {
+    {{{1281, 128, 256, 1, 0, {5.79f}, {.0113f}}, {1282, 256, 256, 1, 0, {8.95f}, {.0223f}}, {1286, 256, 512, 1, 0, {7.95f}, {.0277f}},
+      {1289, 256, 512, 1, 0, {6.92f}, {.0227f}}, {2188, 256, 512, 1, 0, {5.55f}, {.0230f}},
+      {2081, 16, 512, 1, 1.70f, {2.93f}, {.0043f}}, {2082, 32, 512, 1, 1.19f, {4.82f}, {.0044f}}},
+     {{1281, 128, 256, 1, 0, {5.79f}, {.0116f}}, {1282, 256, 256, 1, 0, {8.58f}, {.0228f}},
+      {1289, 256, 512, 1, 0, {7.35f}, {.0245f}}, {2188, 256, 512, 1, 0, {6.83f}, {.0226f}},
+      {2081, 16, 512, 1, 1.38f, {3.82f}, {.0059f}}, {2082, 32, 512, 1, 0.64f, {6.61f}, {.0061f}}}},
+    {{{1281, 128, 256, 1, 0, {6.58f}, {.0149f}}, {1289, 256, 512, 1, 0, {8.03f}, {.0242f}}, {1286, 256, 512, 1, 0, {8.67f}, {.0244f}},
+      {2188, 256, 512, 1, 0, {5.57f}, {.0269f}}, {2081, 16, 512, 1, 1.54f, {3.70f}, {.0043f}},
+      {2082, 32, 512, 1, 1.09f, {6.13f}, {.0049f}}},
+     {{1281, 128, 256, 1, 0, {6.67f}, {.0154f}}, {1289, 256, 512, 1, 0, {8.50f}, {.0256f}}, {1286, 256, 512, 1, 0, {9.59f}, {.0266f}},
+      {2188, 256, 512, 1, 0, {7.13f}, {.0244f}}, {2081, 16, 512, 1, 1.15f, {4.61f}, {.0063f}},
+      {2082, 32, 512, 1, 1.43f, {7.09f}, {.0068f}}}}};
+
+// The kernel that is priced at least 7 % below `own`, the one the rules of plan_bmm name, or 0.  The rules draw their lines
+// along one size at a time and miss where the rounds of two kernels fall differently: one round of 256-row workgroups against
+// two of 128 rows (40 x 809 x 1608 x 128 softmax 59.2 -> 44.2 us), 1.2 rounds of 256 against 2.2 of 128 (30 x 2080 x 2032 x 128
+// 122 -> 79), without softmax 50 x 1520 x 576 x 64 24.7 -> 19.1, 5 x 432 x 144 x 128 7.6 -> 6.0.  Over 400 - 700 random shapes
+// a class the mean is 0.8 to 3.6 % lower, the best 0.50 of the time, the worst 1.06 - 1.11 of it.
+int cheaper_variant(const ditto_bmm_chain_desc* d, int own, int cus) {
+  const long long dmax = d->K > d->N ? d->K : d->N;
+  const bool sm = d->inter_op == DITTO_INTER_SOFTMAX, kl = d->b_layout == DITTO_B_KL;
+  // with softmax the kernels that find a row's first unmasked key wherever it lies (20xx, 21xx, 644, 645) keep what they have
+  if (dmax <= 64 ? sm : dmax <= 80 || (sm && own >= 2000)) return 0;
+  const BmmPrice* const prices = dmax <= 64 ? kPrices64[kl] : kPrices128[sm][kl];
+  const int count = dmax <= 64 ? 8 : 7;
+  int best = 0;
+  float own_price = 0, best_price = 0;
+  for (int i = 0; i < count && prices[i].variant != 0; ++i) {
+    const BmmPrice& p = prices[i];
+    const long long wgs = ((d->M + p.rows - 1) / p.rows) * d->batch, full = wgs / (p.resident * cus);
+    const int left = (int)((wgs - full * p.resident * cus + cus - 1) / cus), r = p.resident - 1;
+    const float L = (float)d->L, price = p.start + full * (p.first[r] + p.per_key[r] * L) +
+                                         (left > 0 ? p.first[left - 1] + p.per_key[left - 1] * L : 0.f);
+    if (p.variant == own) own_price = price;
+    if (p.variant == 2188 && (d->L < 64 || d->L > 700)) continue;  // (beyond the lines its price fits, by 4 - 9 %)
+    if ((best == 0 || price < best_price) && launchable(wgs, p.threads)) best = p.variant, best_price = price;
+  }
+  return best != own && own_price > 0 && best_price < 0.93f * own_price ? best : 0;
+}
+
+int plan_bmm_rules(const ditto_bmm_chain_desc* d, BmmPlan* plan, int cus);
+
 int plan_bmm(const ditto_bmm_chain_desc* d, BmmPlan* plan, bool need_device) {
+  // A plan depends on the descriptor and the number of compute units alone: the last few are kept, so that a
+  // repeated call pays for a comparison and not for the pricing.
+  struct Kept {
+    ditto_bmm_chain_desc desc;
+    int cus;
+    BmmPlan plan;
+  };
+  constexpr int kKept = 4;
+  static thread_local Kept kept[kKept] = {};  // (an all-zero descriptor is refused: abi_version)
+  static thread_local int next = 0;
+  const int cus = need_device ? device_cus() : 256;
+  if (d)
+    for (const Kept& k : kept)
+      if (k.cus == cus && memcmp(&k.desc, d, sizeof(*d)) == 0) return *plan = k.plan, DITTO_OK;
+  int rc = plan_bmm_rules(d, plan, cus);
+  if (rc != DITTO_OK) return rc;
+  if (plan->family == 0 && d->tile_variant == 0) {
+    ditto_bmm_chain_desc forced = *d;
+    forced.tile_variant = cheaper_variant(d, plan->tile.variant, cus);
+    if (forced.tile_variant != 0) rc = plan_bmm_rules(&forced, plan, cus);
+  }
+  if (rc == DITTO_OK) {
+    kept[next] = {*d, cus, *plan};
+    next = (next + 1) % kKept;
+  }
+  return rc;
+}
+
+int plan_bmm_rules(const ditto_bmm_chain_desc* d, BmmPlan* plan, int cus) {
   if (!d) return fail(DITTO_EINVAL, "null descriptor");
   if (d->abi_version != DITTO_CHAIN_ABI_VERSION)
     return fail(DITTO_EINVAL, "descriptor abi_version %d, library %d", d->abi_version,
@@ -165,7 +253,6 @@ int plan_bmm(const ditto_bmm_chain_desc* d, BmmPlan* plan, bool need_device) {
       return fail(DITTO_EUNSUPPORTED, "max(K,N)=%lld: register-resident chain supports up to 128", dmax);
     plan->family = 0;
     plan->d_pad = dmax <= 64 ? 64 : 128;
-    const int cus = need_device ? device_cus() : 256;
     // Variant table (measured on MI355X, fp16 and bf16, head_pad 64 and 128).  n8 = number of 256-row
     // workgroups.  Below 3/4 of the CUs the four-wave kernel with 128-row workgroups spreads over more
     // CUs.  From there on eight waves (two per SIMD) win, in their software-pipelined form (9) at every
@@ -293,6 +380,14 @@ int plan_bmm(const ditto_bmm_chain_desc* d, BmmPlan* plan, bool need_device) {
         }
         if (take && launchable(n8, 512)) plan->rows_dt = 8, plan->rows_nw = 8;
       }
+      if (d->tile_variant == 0 && dt == 4 && rt == 0 && sm && plan->qt != 6) {
+        // Heads of up to 64 with softmax where the 64-row kernel, three workgroups to a compute unit, needs a second round and this
+        // one in its four-wave form, two of 128 rows to a compute unit, does not: on 250 shapes 0.74 - 0.86 of the time at 64 keys,
+        // 0.83 - 0.96 at 200, 0.87 - 1.02 at 600, 1.06 at 1000 (256 x 197 x 197 10.9 -> 9.3 us, 512 x 100 x 100 9.6 -> 8.2).  With more
+        // rounds than that the two are level.  (Without softmax cheaper_variant sees to it.)
+        const long long n64 = ((d->M + 63) / 64) * d->batch, n128 = ((d->M + 127) / 128) * d->batch;
+        if (n64 > 3LL * cus && n128 <= 2LL * cus && d->L <= 600 && launchable(n128, 256)) plan->rows_dt = 4, plan->rows_nw = 4;
+      }
       if (d->tile_variant == 0 && dt == 4 && rt == 0 && !sm && n8 >= 2LL * cus && d->L <= 1024) {
         // Heads of up to 64 without softmax from two 256-row workgroups per compute unit on, up to 1024 keys: 512 x 197 x 197 16.8 ->
         // 12.2 us, 256 x 400 x 400 20.0 -> 16.6 (B [K][L] 22.3 -> 18.0), 256 x 577 x 577 35.0 -> 29.9, 128 x 1024 x 1024 35.3 -> 33.8;
@@ -386,7 +481,6 @@ int plan_bmm(const ditto_bmm_chain_desc* d, BmmPlan* plan, bool need_device) {
     // Measured, us per launch, 16 / 32 rows: 12 x 512 x 512 x 64 16.0 / 14.4, 1 x 512 x 512 x 64 8.8 / 13.9,
     // 16 x 700 x 700 x 64 28.2 / 33.4, 64 x 512 x 512 x 64 51.6 / 52.7 (B [K][L]: 62.6 / 57.1).  Beyond 80 columns two row
     // tiles do not fit the registers.
-    const int cus = need_device ? device_cus() : 256;
     auto rounds = [&](int rows) { return (((d->M + rows - 1) / rows) * d->batch + cus - 1) / cus; };
     plan->qt = !f64 && (d->K > 80 || d->N > 80 || (double)rounds(16) < 1.8 * (double)rounds(32)) ? 1 : 2;
     ditto_tile_param& t = plan->tile;
@@ -424,7 +518,6 @@ int plan_bmm(const ditto_bmm_chain_desc* d, BmmPlan* plan, bool need_device) {
       return fail(DITTO_EUNSUPPORTED, "a batch entry of A, B or C exceeds 2 GiB");
     // 64-row workgroups halve the weight traffic per row but need twice as many rows to fill the
     // chip; the ring of staged chunks is as deep as LDS allows (four or three stages, else two)
-    const int cus = need_device ? device_cus() : 256;
     int mt = ((d->M + 63) / 64) * d->batch >= 2LL * cus ? 2 : 1;
     auto fits = [&](int m, int n) { return ditto::i8_chain_lds_bytes_host((int)Lp, m, n) <= 160 * 1024; };
     int nst = mt == 2 ? 3 : 4;

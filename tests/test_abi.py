@@ -207,6 +207,35 @@ def test_conv_tile_choice_without_gpu():
     assert tile.variant == 4043
 
 
+def test_kernels_are_priced_against_each_other():
+    """Where the rounds of two kernels fall differently the cheaper one is planned; a forced kernel stays, and softmax chains
+    keep a kernel that finds a row's first unmasked key wherever it lies."""
+    lib = _lib.load()
+    tile = _lib.TileParam()
+
+    def plan(batch, M, L, D, inter, layout, variant=0):
+        d = _desc(batch=batch, M=M, N=D, K=D, L=L, inter_op=inter, b_layout=layout, a_batch_stride=M * D, a_row_stride=D,
+                  b_batch_stride=L * D, b_row_stride=L if layout == _lib.B_KL else D, c_batch_stride=L * D, c_row_stride=D,
+                  f_batch_stride=M * D, f_row_stride=D, tile_variant=variant)
+        for _ in range(2):  # planned, and kept
+            assert lib.ditto_bmm_chain_select_tile(ctypes.byref(d), ctypes.byref(tile)) == _lib.OK
+        return tile.variant
+
+    SM, CAST, LK, KL = _lib.INTER_SOFTMAX, _lib.INTER_CAST, _lib.B_LK, _lib.B_KL
+    assert plan(40, 809, 1608, 128, SM, LK) == 1289   # 160 workgroups of 256 rows, 280 of 128
+    assert plan(30, 2080, 2032, 128, SM, KL) == 1281  # 270 and 510
+    assert plan(40, 809, 1608, 128, SM, LK, 1281) == 1281
+    assert plan(5, 432, 144, 128, CAST, KL) == 2081
+    assert plan(65, 416, 416, 64, CAST, KL) == 644
+    assert plan(160, 300, 296, 64, CAST, KL) == 2144
+    assert plan(256, 197, 197, 64, SM, LK) == 2144 and plan(256, 197, 640, 64, SM, LK) == 644
+    for M in (100, 300, 1000):
+        for L in (64, 500, 1500):
+            for batch in (1, 20, 200):
+                if ((M + 255) // 256) * batch < 512:
+                    assert plan(batch, M, L, 64, SM, LK) in (644, 645, 2041, 2042, 2144, 2148)
+
+
 def test_grids_beyond_one_launch_stay_on_the_kernels_that_take_them():
     """A launch holds fewer than 2^32 work items.  The kernels that give few rows or pixels to many threads reach that
     where the general ones do not, and the general ones keep those sizes (plans only: nothing is launched)."""

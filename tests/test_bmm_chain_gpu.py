@@ -154,6 +154,23 @@ def test_key_splitting_kernel(oracle, shape, dtype, inter):
             assert np.array_equal(narrow, oracle.np_round_to(got, dtype)), (variant, b_layout)
 
 
+@pytest.mark.parametrize("batch,M,L,D,inter,b_layout", [
+    # shapes whose kernel is named by its price, on either side of a round of workgroups, ragged rows among them
+    (40, 809, 408, 128, "softmax", "LK"), (130, 129, 200, 128, "softmax", "KL"), (5, 432, 144, 128, "relu", "KL"),
+    (13, 2049, 200, 128, "cast", "LK"), (65, 416, 416, 64, "relu", "KL"), (160, 300, 296, 64, "cast", "KL"),
+    (257, 197, 197, 64, "softmax", "LK"), (3, 49, 176, 64, "cast", "KL"),
+])
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+def test_kernels_named_by_their_price(oracle, batch, M, L, D, inter, b_layout, dtype):
+    std, scale = (1.0, D ** -0.5) if inter == "softmax" else (0.25, 1.0)
+    A, B, C = oracle.make_gemm_chain_inputs(batch, M, D, D, L, dtype, seed=M + L, std=std)
+    want = oracle.bmm_chain_f64(A, B, C, inter=inter, scale=scale, round_mid=None if inter == "softmax" else dtype)
+    got = run_chain(A, B, C, dtype, inter, scale, b_layout, "float32")
+    mx, rel = errors(got, want)
+    assert np.isfinite(got).all() and mx <= 4e-2, mx
+    assert rel <= (REL_L2 if inter != "softmax" or dtype == "float16" else REL_L2_BF16_P_ONLY), rel
+
+
 def masked_scores(oracle, batch, M, N, K, L, dtype, masked, seed):
     """Operands whose scores are minus infinity at the keys ``masked``: column 0 of the first operand is one, and the
     keys hold minus infinity there (how a caller of a chain without a mask argument masks keys)."""
