@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <vector>
 
 #include <cstdarg>
@@ -55,6 +56,7 @@ struct BmmPlan {
   int d_pad, qt;  // fp chains: head pad and rows-per-wave code; int8 chain: row tiles and ring depth
   int split_dt = 0, split_rt = 0;  // fp chains on few rows: column tiles and row tiles of the key-splitting kernel (0: none)
   int rows_dt = 0, rows_nw = 0;  // fp chains: column tiles and waves of the kernel of 32 rows per wave and short tiles (0: none)
+  int units_rt = 0, slices = 0, slice_blocks = 0;  // int8 chain on few rows: row tiles, slices of the columns, blocks of 64 of each (0: none)
   int nb3 = 0, nb = 0;  // 16x16x32-MFMA kernel: row blocks of 384 rows / row blocks in all, per batch entry
   ditto_tile_param tile;
 };
@@ -516,6 +518,49 @@ int plan_bmm_rules(const ditto_bmm_chain_desc* d, BmmPlan* plan, int cus) {
     if ((d->M + 64) * d->a_row_stride >= 0x7fffffffLL || d->K * d->b_row_stride >= 0x7fffffffLL ||
         Lp * d->c_row_stride >= 0x7fffffffLL)
       return fail(DITTO_EUNSUPPORTED, "a batch entry of A, B or C exceeds 2 GiB");
+    // Few rows: the kernel whose waves take units of 64 x 64 weights, with as many workgroups to a row block (slices of its
+    // columns) as pay.  Prices in us per launch, least squares over 300 random shapes (64 - 8192 rows, K and N 16 - 1024, L 16 -
+    // 512) with 1 - 6 slices, root mean square error 5 %, up to one round of the other kernel's workgroups; where this one is
+    // priced 3 % lower it takes 0.79 of the time in the mean (224 x 48 x 208 x 928 7.8 -> 4.8 us, 256 x 912 x 96 x 800 10.4 ->
+    // 6.2, 1120 x 32 x 48 x 16 4.8 -> 3.8), the worst of 244 1.26.
+    {
+      const double nl = (double)((d->L + 63) / 64), units1 = nl * (double)((d->K + 63) / 64) / 8;
+      const long long nbt = (d->N + 63) / 64, rows32 = ((d->M + 31) / 32) * d->batch, Lc = Lp / 256;
+      const long long chunks = Lc * ((d->K + 127) / 128) + 2 * Lc * ((d->N + 255) / 256);
+      double best = 0.97 * (3.61 + 0.413 * chunks + 0.444e-6 * (double)(d->batch * d->M) * (double)d->N);
+      if (d->tile_variant == 8101 || d->tile_variant == 8102) best = 1e30;
+      for (int rt = 1; rt <= 2; ++rt) {
+        if (d->tile_variant == 0 ? rows32 > cus : d->tile_variant != 8100 + rt) continue;
+        const long long wgs = ((d->M + 16 * rt - 1) / (16 * rt)) * d->batch;
+        for (long long s = 1; s <= nbt && s <= 16; ++s) {
+          const long long blocks = (nbt + s - 1) / s;
+          if ((nbt + blocks - 1) / blocks != s || ditto::i8_units_lds_bytes_host(d->L, rt, (int)std::min(blocks, 1LL << 20)) > 160 * 1024) continue;
+          if (!launchable(wgs * s, 512)) break;
+          const double rounds = (double)((wgs * s + cus - 1) / cus), units2 = nl * (double)blocks / 8, grid = (double)(wgs * s) / cus;
+          const double price = rt == 1 ? 3.17 + rounds * (0.07 + 0.155 * nl + 0.158 * blocks + 0.417 * units1 + 0.206 * units2 +
+                                                           0.056 * ceil(units1) + 0.183 * ceil(units2)) + 0.472 * grid
+                                       : 3.5 + rounds * (0.375 * nl + 0.306 * blocks + 0.582 * units1 + 0.474 * units2) + 0.568 * grid;
+          if (price < best) best = price, plan->units_rt = rt, plan->slices = (int)s, plan->slice_blocks = (int)blocks;
+        }
+      }
+      if (plan->units_rt > 0) {
+        plan->family = 2;
+        const int rt = plan->units_rt;
+        ditto_tile_param& t = plan->tile;
+        t.block_threads = 512;
+        t.block_m = 16 * rt;
+        t.block_l = 64;
+        t.block_n = 64 * plan->slice_blocks;
+        t.head_pad = 0;
+        t.lds_bytes = (int)ditto::i8_units_lds_bytes_host(d->L, rt, plan->slice_blocks);
+        t.grid_x = (int)(((d->M + 16 * rt - 1) / (16 * rt)) * d->batch * plan->slices);
+        t.grid_y = t.grid_z = 1;
+        t.variant = 8100 + rt;  // units of 64 x 64 weights; row tiles of 16
+        return DITTO_OK;
+      }
+      if (d->tile_variant == 8101 || d->tile_variant == 8102)
+        return fail(DITTO_EINVAL, "tile_variant %d cannot run this int8 chain (LDS or grid)", d->tile_variant);
+    }
     // 64-row workgroups halve the weight traffic per row but need twice as many rows to fill the
     // chip; the ring of staged chunks is as deep as LDS allows (four or three stages, else two)
     int mt = ((d->M + 63) / 64) * d->batch >= 2LL * cus ? 2 : 1;
@@ -529,7 +574,7 @@ int plan_bmm_rules(const ditto_bmm_chain_desc* d, BmmPlan* plan, int cus) {
       const int fm = (d->tile_variant - 8000) / 10, fn = d->tile_variant % 10;
       const bool built = (fm == 1 && (fn == 2 || fn == 4)) || (fm == 2 && (fn == 2 || fn == 3));
       if (d->tile_variant < 8000 || !built || !fits(fm, fn))
-        return fail(DITTO_EINVAL, "tile_variant %d cannot run this int8 chain (8012, 8014, 8022 or 8023, within LDS)",
+        return fail(DITTO_EINVAL, "tile_variant %d cannot run this int8 chain (8012, 8014, 8022, 8023, 8101 or 8102, within LDS)",
                     d->tile_variant);
       mt = fm, nst = fn;
     }
@@ -1543,7 +1588,10 @@ int ditto_bmm_chain_run(const ditto_bmm_chain_desc* d, const void* a, const void
     args.batch = (int)d->batch;
     args.mblocks = (int)((d->M + plan.tile.block_m - 1) / plan.tile.block_m);
     args.Lp = plan.tile.block_l;
-    hipError_t e = ditto::launch_gemm_chain_i8(args, plan.d_pad, plan.qt, st);
+    args.slices = plan.slices;
+    args.slice_blocks = plan.slice_blocks;
+    hipError_t e = plan.units_rt > 0 ? ditto::launch_gemm_chain_i8_units(args, plan.units_rt, st)
+                                     : ditto::launch_gemm_chain_i8(args, plan.d_pad, plan.qt, st);
     if (e != hipSuccess) return fail(DITTO_EHIP, "kernel launch failed: %s", hipGetErrorString(e));
     return DITTO_OK;
   }

@@ -20,6 +20,7 @@ struct I8ChainArgs {
   int M, N, K, L, batch;
   int mblocks;
   int Lp;  // L rounded up to the weight-chunk width
+  int slices, slice_blocks;  // unit kernel: workgroups that share a row block's columns of the result, blocks of 64 columns of each
 };
 
 // dynamic LDS bytes of the kernel for a padded L, mt = 1|2 row tiles of 32 per workgroup and a
@@ -28,5 +29,9 @@ int i8_chain_lds_bytes_host(int Lp, int mt, int nst);
 // threads per workgroup of the kernel
 int i8_chain_threads();
 hipError_t launch_gemm_chain_i8(const I8ChainArgs& args, int mt, int nst, hipStream_t stream);
+
+// The kernel of 16 * rt rows per workgroup whose waves take units of 64 x 64 weights (rt = 1 | 2)
+long long i8_units_lds_bytes_host(long long L, int rt, int slice_blocks);
+hipError_t launch_gemm_chain_i8_units(const I8ChainArgs& args, int rt, hipStream_t stream);
 
 }  // namespace ditto

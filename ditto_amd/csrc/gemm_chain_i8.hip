@@ -355,6 +355,242 @@ __global__ __launch_bounds__(64 * i8::NW) void gemm_chain_i8_kernel(I8ChainArgs 
 #endif
 }
 
+// ---- few rows: units ---------------------------------------------------------------------------
+// A workgroup owns 16 RT rows and a slice of the result's columns (the middle result is made anew for every slice), and its
+// eight waves take UNITS of 64 contraction rows x 64 columns of B, then of D, in equal shares whatever the shape: a unit's
+// four column tiles are accumulated in registers and added to an int32 block in LDS where a wave's share ends (integer sums
+// are exact in any order).  The kernel above moves 128 x 256 chunks through one ring in lock step, at least two for the
+// first product and two for the second with a barrier each, all padded; here nothing is padded beyond 64, a wave waits for
+// its own loads only, and there are four barriers.
+//
+// B and D hold the contraction index in their rows.  A lane loads a dword, four neighbouring columns, of each of 16 rows (16
+// lanes: 64 contiguous bytes) and transposes 16 x 4 bytes in registers; column 4 c + t is row c of tile t, so what a lane
+// ends with, acc[t][r], is the 16 neighbouring columns 16 q + 4 r + t of one row of A.
+//
+// Bound: a unit's 17 vector loads and 32 byte permutations (0.4 us for the eight waves' units, about what their issue takes),
+// the LDS additions, and a few round trips to L2.  Measured, us per launch, the kernel above -> this one: 224 x 48 x 208 x 928
+// (M, K, L, N) 7.8 -> 4.8, 256 x 912 x 96 x 800 10.4 -> 6.2, 1120 x 32 x 48 x 16 4.8 -> 3.8, 544 x 144 x 240 x 128 4.8 against 5.1.
+// Tried and slower: tiles through direct loads to LDS and its transposing reads (+2 us, their issue), eight columns to a lane
+// (128-column units), four units in flight instead of two, a block of columns to a wave with the partial sums written to LDS.
+template <int RT>
+__global__ __launch_bounds__(512) void gemm_chain_i8_units_kernel(I8ChainArgs p) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  extern __shared__ __attribute__((aligned(16))) char smem_un[];
+  constexpr int ROWS = 16 * RT;
+  constexpr int kOut = -16;  // as an unsigned offset beyond any range: reads zero
+  const int tid = threadIdx.x, lane = tid & 63, c = lane & 15, q = lane >> 4;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int M = p.M, N = p.N, K = p.K, L = p.L;
+  const unsigned lid = xcd_remap(blockIdx.x, gridDim.x);
+  const int sl = lid % (unsigned)p.slices, rest = lid / (unsigned)p.slices;
+  const int mb = rest % (unsigned)p.mblocks, bz = rest / (unsigned)p.mblocks;
+  const int m0 = mb * ROWS, n0 = 64 * sl * p.slice_blocks;
+  const int8_t* const Ag = p.a + (long long)bz * p.a_bs;
+  const int8_t* const Bg = p.b + (long long)bz * p.b_bs;
+  const int8_t* const Dg = p.d + (long long)bz * p.d_bs;
+  const int nk = (K + 63) / 64, nl = (L + 63) / 64, nb = min(p.slice_blocks, (N - n0 + 63) / 64);
+  const int S1 = 64 * nl + 1, S2 = 64 * nb + 1;  // odd row strides: the 64 lanes' additions fall on 64 banks
+  int* const acc1 = reinterpret_cast<int*>(smem_un);  // [ROWS][S1] middle result
+  int* const acc2 = acc1 + ROWS * S1;                 // [ROWS][S2] result
+  const int MS = 64 * nl + 16;
+  int8_t* const mid = reinterpret_cast<int8_t*>(acc2 + (ROWS * (S1 + S2) + 3) / 4 * 4 - ROWS * S1);  // [ROWS][MS], 16-byte aligned
+  float* const sc = reinterpret_cast<float*>(mid + ROWS * MS);                                       // [64 nl]
+
+  const long long b_bytes = (long long)(K - 1) * p.b_rs + L, d_bytes = (long long)(L - 1) * p.d_rs + N;
+  const long long a_bytes = (long long)(M - 1) * p.a_rs + K;
+  auto rsrc = [](const int8_t* base, long long at, long long bytes) __attribute__((always_inline)) {
+    const i32x4 r = make_rsrc_uniform(base + at, at < bytes ? (unsigned)(bytes - at) : 0u);
+    return __builtin_amdgcn_make_buffer_rsrc(
+        reinterpret_cast<void*>((unsigned long long)(unsigned)r[0] | ((unsigned long long)(unsigned)r[1] << 32)), 0, r[2], 0x00020000);
+  };
+  int vb[16], vd[16], va[RT];
+#pragma unroll
+  for (int i = 0; i < 16; ++i) vb[i] = (16 * q + i) * p.b_rs + 4 * c, vd[i] = (16 * q + i) * p.d_rs + 4 * c;
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt) va[rt] = (m0 + 16 * rt + c) * p.a_rs + 16 * q;
+
+  struct Unit {
+    int w[16];
+  };
+  auto load_b = [&](Unit& u, int lb, int ks) __attribute__((always_inline)) {
+    const auto r = rsrc(Bg, (long long)(64 * ks) * p.b_rs + 64 * lb, b_bytes);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) u.w[i] = __builtin_amdgcn_raw_buffer_load_b32(r, vb[i], 0, 0);
+  };
+  auto load_a = [&](i32x4 (&a)[RT], int ks) __attribute__((always_inline)) {
+    const auto r = rsrc(Ag, 64 * ks, a_bytes);
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt)
+      a[rt] = __builtin_bit_cast(i32x4, __builtin_amdgcn_raw_buffer_load_b128(r, 64 * ks + 16 * q < K ? va[rt] : kOut, 0, 0));
+  };
+  auto load_d = [&](Unit& u, int nbk, int ls) __attribute__((always_inline)) {
+    const auto r = rsrc(Dg, (long long)(64 * ls) * p.d_rs + n0 + 64 * nbk, d_bytes);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) u.w[i] = __builtin_amdgcn_raw_buffer_load_b32(r, vd[i], 0, 0);
+  };
+  // 16 rows x 4 columns of bytes -> four vectors of 16 rows
+  auto transpose = [](const Unit& u, i32x4 (&t)[4]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const unsigned r0 = u.w[4 * j], r1 = u.w[4 * j + 1], r2 = u.w[4 * j + 2], r3 = u.w[4 * j + 3];
+      const unsigned a = __builtin_amdgcn_perm(r1, r0, 0x05010400), b = __builtin_amdgcn_perm(r1, r0, 0x07030602);
+      const unsigned d = __builtin_amdgcn_perm(r3, r2, 0x05010400), e = __builtin_amdgcn_perm(r3, r2, 0x07030602);
+      t[0][j] = __builtin_amdgcn_perm(d, a, 0x05040100), t[1][j] = __builtin_amdgcn_perm(d, a, 0x07060302);
+      t[2][j] = __builtin_amdgcn_perm(e, b, 0x05040100), t[3][j] = __builtin_amdgcn_perm(e, b, 0x07060302);
+    }
+  };
+  i32x4 acc[RT][4];
+  auto zero_acc = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+      for (int t = 0; t < 4; ++t) acc[rt][t] = i32x4{0, 0, 0, 0};
+  };
+  auto multiply = [&](const Unit& u, const i32x4 (&a)[RT]) __attribute__((always_inline)) {
+    i32x4 t[4];
+    transpose(u, t);
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt) acc[rt][k] = __builtin_amdgcn_mfma_i32_16x16x64_i8(t[k], a[rt], acc[rt][k], 0, 0, 0);
+  };
+  auto flush = [&](int* to, int S, int block) __attribute__((always_inline)) {
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+          __hip_atomic_fetch_add(to + (16 * rt + c) * S + 64 * block + 16 * q + 4 * r + t, acc[rt][t][r], __ATOMIC_RELAXED,
+                                 __HIP_MEMORY_SCOPE_WORKGROUP);
+    zero_acc();
+  };
+
+  const float scale0 = p.scale ? p.scale[min(tid, L - 1)] : p.scale_uniform;  // (asked for before the units are)
+
+  // a wave's share of the units, contraction steps of one block of 64 columns after another
+  const int n1 = nl * nk, s1 = (n1 + 7) / 8, u1 = min(n1, (w + 1) * s1);
+  const int n2 = nb * nl, s2 = (n2 + 7) / 8, u2 = min(n2, (w + 1) * s2);
+  Unit ub[2];
+  i32x4 af[2][RT];
+  int lb = (w * s1) / nk, ks = w * s1 - lb * nk;  // of the next unit to fetch
+  auto fetch1 = [&](int b) __attribute__((always_inline)) {
+    load_b(ub[b], lb, ks);
+    load_a(af[b], ks);
+    if (++ks == nk) ks = 0, ++lb;
+  };
+  int u = w * s1;
+  if (u < u1) fetch1(0);
+  if (u + 1 < u1) fetch1(1);
+  for (int i = tid; i < ROWS * (S1 + S2); i += 512) acc1[i] = 0;
+  if (tid < 64 * nl) sc[tid] = scale0;
+  for (int l = 512 + tid; l < 64 * nl; l += 512) sc[l] = p.scale ? p.scale[min(l, L - 1)] : p.scale_uniform;
+  zero_acc();
+  wg_sync();
+  {
+    int blk = u / nk, left = (blk + 1) * nk - u;  // block of the unit in hand, units of it from here on
+    for (; u < u1; u += 2) {
+#pragma unroll
+      for (int b = 0; b < 2; ++b) {
+        if (u + b >= u1) break;
+        multiply(ub[b], af[b]);
+        if (u + b + 2 < u1) fetch1(b);
+        if (--left == 0 || u + b + 1 == u1) {
+          flush(acc1, S1, blk);
+          ++blk, left = nk;
+        }
+      }
+    }
+  }
+  // the second product's first units do not wait for the middle result
+  u = w * s2;
+  int nbk = u / nl, ls = u - nbk * nl;
+  auto fetch2 = [&](int b) __attribute__((always_inline)) {
+    load_d(ub[b], nbk, ls);
+    if (++ls == nl) ls = 0, ++nbk;
+  };
+  int cls = ls;  // contraction step of the unit in hand
+  int blk2 = nbk;
+  if (u < u2) fetch2(0);
+  if (u + 1 < u2) fetch2(1);
+  wg_sync();
+  const float inv_l = 1.f / (float)(16 * nl);
+  for (int i = tid; i < ROWS * 16 * nl; i += 512) {
+    const int row = div_by(i, inv_l), l = 4 * (i - row * 16 * nl);
+    int packed = 0;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      int v = acc1[row * S1 + l + t];
+      if (p.wrap) v = p.relu ? max(v, 0) : v;
+      else v = requant_i8(v, sc[l + t]);
+      packed |= (v & 0xff) << (8 * t);
+    }
+    *reinterpret_cast<int*>(mid + row * MS + l) = packed;
+  }
+  wg_sync();
+  for (; u < u2; u += 2) {
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      if (u + b >= u2) break;
+      i32x4 a[RT];
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt) a[rt] = *reinterpret_cast<const i32x4*>(mid + (16 * rt + c) * MS + 64 * cls + 16 * q);
+      multiply(ub[b], a);
+      if (u + b + 2 < u2) fetch2(b);
+      if (++cls == nl || u + b + 1 == u2) {
+        flush(acc2, S2, blk2);
+        ++blk2, cls = 0;
+      }
+    }
+  }
+  wg_sync();
+  const int quads = min(16 * nb, (N - n0) / 4);  // columns in fours
+  const float inv_n = 1.f / (float)quads;
+  typedef __attribute__((ext_vector_type(4), aligned(4))) int Row4;  // (rows of the result need no alignment of their own)
+  typedef __attribute__((aligned(1))) int Row4b;
+  for (int i = tid; i < ROWS * quads; i += 512) {
+    const int row = div_by(i, inv_n), n = 4 * (i - row * quads);
+    if (m0 + row >= M) break;
+    const int* const v = acc2 + row * S2 + n;
+    const long long at = (long long)bz * p.e_bs + (long long)(m0 + row) * p.e_rs + n0 + n;
+    if (p.out_i8)
+      *reinterpret_cast<Row4b*>(reinterpret_cast<int8_t*>(p.e) + at) =
+          (v[0] & 0xff) | ((v[1] & 0xff) << 8) | ((v[2] & 0xff) << 16) | ((unsigned)v[3] << 24);
+    else
+      *reinterpret_cast<Row4*>(p.e + at) = Row4{v[0], v[1], v[2], v[3]};
+  }
+#else
+  (void)p;
+#endif
+}
+
+long long i8_units_lds_bytes_host(long long L, int rt, int slice_blocks) {
+  const long long nl = (L + 63) / 64;
+  return (16LL * rt * (64 * nl + 1 + 64 * slice_blocks + 1) + 3) / 4 * 16 + 16LL * rt * (64 * nl + 16) + 256 * nl;
+}
+
+template <int RT>
+static hipError_t launch_i8_units(const I8ChainArgs& args, hipStream_t stream) {
+  const int lds = (int)i8_units_lds_bytes_host(args.L, RT, args.slice_blocks);
+  auto kern = gemm_chain_i8_units_kernel<RT>;
+  static thread_local int configured_dev = -1;
+  int dev = 0;
+  hipError_t e = hipGetDevice(&dev);
+  if (e != hipSuccess) return e;
+  if (configured_dev != dev) {
+    e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    if (e != hipSuccess) return e;
+    configured_dev = dev;
+  }
+  const unsigned grid = (unsigned)args.mblocks * (unsigned)args.batch * (unsigned)args.slices;
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(512), lds, stream, args);
+  return hipGetLastError();
+}
+
+hipError_t launch_gemm_chain_i8_units(const I8ChainArgs& args, int rt, hipStream_t stream) {
+  return rt == 1 ? launch_i8_units<1>(args, stream) : rt == 2 ? launch_i8_units<2>(args, stream) : hipErrorInvalidValue;
+}
+
 int i8_chain_threads() { return 64 * i8::NW; }
 int i8_chain_lds_bytes_host(int Lp, int mt, int nst) { return i8_chain_lds_bytes(Lp, mt, nst); }
 

@@ -79,6 +79,43 @@ def test_i8_chain_variants_agree(oracle):
             chain.bmm_chain_desc(a, b, d, e, "requant", tile_variant=8013))
 
 
+@pytest.mark.parametrize("variant", [8101, 8102])
+@pytest.mark.parametrize("M,K,L,N", [
+    # one unit, one more row / column / contraction group than a unit or a row tile holds, equal and unequal shares of eight waves
+    (1, 16, 16, 16), (16, 64, 64, 64), (17, 80, 80, 80), (33, 48, 144, 528), (31, 1024, 16, 1024), (100, 272, 512, 208), (65, 592, 464, 16),
+])
+@pytest.mark.parametrize("inter", ["requant", "cast", "relu"])
+def test_i8_chain_in_units(oracle, M, K, L, N, inter, variant):
+    A, B, D, scale = oracle.make_i8_chain_inputs(M, K, L, N, seed=M + K)
+    want = oracle.gemm_chain_i8(A, B, D, scale)[0] if inter == "requant" else oracle.gemm_chain_i8_wrap(A, B, D, inter == "relu")[0]
+    dev = "cuda:0"
+    a, b, d = (torch.from_numpy(np.ascontiguousarray(x)).to(dev) for x in (A, B, D))
+    aux = torch.from_numpy(scale).to(dev) if inter == "requant" else None
+    # result rows at any distance: the columns behind them stay as they are
+    for dtype, pad in ((torch.int32, 0), (torch.int32, 3), (torch.int8, 5)):
+        if dtype == torch.int8 and inter == "requant":
+            continue
+        e = torch.full((M, N + pad), -7, dtype=dtype, device=dev)
+        chain.run_bmm_chain(a, b, d, e[:, :N], inter, aux=aux, tile_variant=variant)
+        torch.cuda.synchronize()
+        got = e.cpu().numpy()
+        assert np.array_equal(got[:, :N], want.astype(got.dtype)) and (got[:, N:] == -7).all()
+
+
+def test_i8_units_are_planned_on_few_rows_and_agree_over_a_batch(oracle):
+    batch, M, K, L, N = 3, 70, 144, 80, 272
+    A, B, D, scale = oracle.make_i8_chain_inputs(M, K, L, N, seed=3)
+    dev = "cuda:0"
+    ops = [torch.from_numpy(np.stack([np.roll(x, i, 0) for i in range(batch)])).to(dev) for x in (A, B, D)]
+    aux = torch.from_numpy(scale).to(dev)
+    e = {v: torch.full((batch, M, N), -7, dtype=torch.int32, device=dev) for v in (0, 8014, 8102)}
+    assert chain.select_tile(chain.bmm_chain_desc(*ops, e[0], "requant")).variant in (8101, 8102)
+    for v, out in e.items():
+        chain.run_bmm_chain(*ops, out, "requant", aux=aux, tile_variant=v)
+    torch.cuda.synchronize()
+    assert torch.equal(e[0], e[8014]) and torch.equal(e[0], e[8102])
+
+
 def test_i8_chain_per_column_scales_and_saturation(oracle):
     M, K, L, N = 96, 256, 64, 48
     A, B, D, _ = oracle.make_i8_chain_inputs(M, K, L, N, seed=5)
