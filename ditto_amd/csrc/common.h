@@ -275,6 +275,23 @@ __device__ __forceinline__ unsigned xcd_remap(unsigned bid, unsigned nblk) {
   return x * (nblk >> 3) + (x < r ? x : r) + (bid >> 3);
 }
 
+// The first n of the values of v, 0 < n < their number (2, 4 or 8), to consecutive elements at any element's address, in
+// pieces of 4, 2 and 1.  (Element by element a wave issues up to seven stores for its one ragged lane, each with a test of its
+// own: at 16 bytes a lane and 95 pixels a row that was two thirds of conv_tiles_kernel's vector memory instructions.)
+template <typename T, typename V>
+__device__ __forceinline__ void store_some(T* dst, V v, int n) {
+  constexpr int D = sizeof(V) / 4;
+  typedef __attribute__((ext_vector_type(2), aligned(2))) unsigned U2;
+  typedef __attribute__((aligned(2))) unsigned U1;
+  unsigned d[D < 4 ? 4 : D];
+  __builtin_memcpy(d, &v, sizeof(V));
+  if (D == 4 && (n & 4)) *reinterpret_cast<U2*>(dst) = U2{d[0], d[1]};
+  const unsigned two = D == 4 && (n & 4) ? d[2] : d[0];
+  if (D >= 2 && (n & 2)) *reinterpret_cast<U1*>(dst + (n & 4)) = two;
+  const unsigned one = D >= 2 && (n & 2) ? (D == 4 && (n & 4) ? d[3] : d[1]) : two;
+  if (n & 1) *reinterpret_cast<unsigned short*>(dst + (n & 6)) = (unsigned short)one;
+}
+
 // n / d for 0 <= n < 2^21 and inv = 1 / d: the half keeps the product inside the quotient's interval whatever its
 // rounding.  (An integer division by a run-time value is some thirty instructions, and a workgroup's start is a chain of
 // them.)

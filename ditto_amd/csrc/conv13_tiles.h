@@ -185,13 +185,8 @@ __global__ __launch_bounds__(128 * WP) void conv13_tiles_kernel(Conv13TilesArgs 
     const T* const src = Xs + c2 * OS + v;
     T* const dst = yt + c2 * hw + v;
     const V8 o = *reinterpret_cast<const V8*>(src);
-    if (v + 8 <= npx) {
-      *reinterpret_cast<V8u*>(dst) = o;
-    } else {
-#pragma unroll
-      for (int e = 0; e < 7; ++e)
-        if (v + e < npx) dst[e] = o[e];
-    }
+    if (v + 8 <= npx) *reinterpret_cast<V8u*>(dst) = o;
+    else store_some(dst, o, npx - v);
   }
 #else
   (void)p;

@@ -303,13 +303,8 @@ __global__ __launch_bounds__(64 * WC * WP) void conv_tiles_kernel(ConvTilesArgs 
         v[t] = two[0], v[t + 1] = two[1];
       }
       T* const dst = reinterpret_cast<T*>(p.y) + at;
-      if (valid >= PO) {
-        *reinterpret_cast<VPu*>(dst) = v;
-      } else {
-#pragma unroll
-        for (int t = 0; t < PO; ++t)
-          if (t < valid) dst[t] = v[t];
-      }
+      if (valid >= PO) *reinterpret_cast<VPu*>(dst) = v;
+      else if (valid > 0) store_some(dst, v, valid);
     }
   }
 #else
