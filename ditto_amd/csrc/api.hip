@@ -385,10 +385,17 @@ int plan_bmm_rules(const ditto_bmm_chain_desc* d, BmmPlan* plan, int cus) {
       if (d->tile_variant == 0 && dt == 4 && rt == 0 && sm && plan->qt != 6) {
         // Heads of up to 64 with softmax where the 64-row kernel, three workgroups to a compute unit, needs a second round and this
         // one in its four-wave form, two of 128 rows to a compute unit, does not: on 250 shapes 0.74 - 0.86 of the time at 64 keys,
-        // 0.83 - 0.96 at 200, 0.87 - 1.02 at 600, 1.06 at 1000 (256 x 197 x 197 10.9 -> 9.3 us, 512 x 100 x 100 9.6 -> 8.2).  With more
-        // rounds than that the two are level.  (Without softmax cheaper_variant sees to it.)
+        // 0.83 - 0.96 at 200, 0.87 - 1.02 at 600, 1.06 at 1000 (256 x 197 x 197 10.9 -> 9.3 us, 512 x 100 x 100 9.6 -> 8.2).  With a
+        // few rounds more the two are level or this one is behind by its part of a round (300 x 512 x 512 30.6 / 33.8).
+        // Many rounds hide that, and a wave of 32 rows reads half as much LDS a row: from eight rounds on 0.95 - 1.00 of the time
+        // where 128-row blocks waste no more rows than 64-row ones (1152 x 512 x 512 122 -> 115, 2097 x 384 x 512 170 -> 164,
+        // 1249 x 256 x 256 level).  Where a last block has 65 to 96 rows one of its four waves has nothing to do, against a
+        // quarter of two 64-row blocks: 0.90 - 1.00 from four rounds on (2339 x 96 x 96 27.6 -> 24.9, 3268 x 197 x 197 111 -> 102).
+        // (Without softmax cheaper_variant sees to it.)
         const long long n64 = ((d->M + 63) / 64) * d->batch, n128 = ((d->M + 127) / 128) * d->batch;
-        if (n64 > 3LL * cus && n128 <= 2LL * cus && d->L <= 600 && launchable(n128, 256)) plan->rows_dt = 4, plan->rows_nw = 4;
+        const long long last = (d->M - 1) % 128 + 1, rounds = n128 / (2LL * cus);
+        const bool many = last > 64 && rounds >= (last <= 96 ? 4 : 8);
+        if (n64 > 3LL * cus && (n128 <= 2LL * cus || many) && d->L <= 600 && launchable(n128, 256)) plan->rows_dt = 4, plan->rows_nw = 4;
       }
       if (d->tile_variant == 0 && dt == 4 && rt == 0 && !sm && n8 >= 2LL * cus && d->L <= 1024) {
         // Heads of up to 64 without softmax from two 256-row workgroups per compute unit on, up to 1024 keys: 512 x 197 x 197 16.8 ->

@@ -158,7 +158,7 @@ def test_key_splitting_kernel(oracle, shape, dtype, inter):
     # shapes whose kernel is named by its price, on either side of a round of workgroups, ragged rows among them
     (40, 809, 408, 128, "softmax", "LK"), (130, 129, 200, 128, "softmax", "KL"), (5, 432, 144, 128, "relu", "KL"),
     (13, 2049, 200, 128, "cast", "LK"), (65, 416, 416, 64, "relu", "KL"), (160, 300, 296, 64, "cast", "KL"),
-    (257, 197, 197, 64, "softmax", "LK"), (3, 49, 176, 64, "cast", "KL"),
+    (257, 197, 197, 64, "softmax", "LK"), (3, 49, 176, 64, "cast", "KL"), (2100, 96, 96, 64, "softmax", "LK"),
 ])
 @pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
 def test_kernels_named_by_their_price(oracle, batch, M, L, D, inter, b_layout, dtype):
