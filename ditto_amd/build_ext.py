@@ -75,6 +75,8 @@ UNITS = [
     ("fp_split_bf16", "bmm_chain_split_inst.hip", ["-DDITTO_INST_T=bf16", "-DDITTO_SPLIT_NAME=launch_split_bf16", *FP_CHAIN_FLAGS]),
     ("fp_rows_f16", "bmm_chain_rows_inst.hip", ["-DDITTO_INST_T=f16", "-DDITTO_ROWS_NAME=launch_rows_f16", *FP_CHAIN_FLAGS]),
     ("fp_rows_bf16", "bmm_chain_rows_inst.hip", ["-DDITTO_INST_T=bf16", "-DDITTO_ROWS_NAME=launch_rows_bf16", *FP_CHAIN_FLAGS]),
+    ("fp_sets_f16", "bmm_chain_sets_inst.hip", ["-DDITTO_INST_T=f16", "-DDITTO_SETS_NAME=launch_sets_f16", *FP_CHAIN_FLAGS]),
+    ("fp_sets_bf16", "bmm_chain_sets_inst.hip", ["-DDITTO_INST_T=bf16", "-DDITTO_SETS_NAME=launch_sets_bf16", *FP_CHAIN_FLAGS]),
 ]
 
 

@@ -1484,18 +1484,26 @@ int launch_fp_chain(const ditto_bmm_chain_desc* d, const BmmPlan& plan, const vo
   const bool kl = d->b_layout == DITTO_B_KL;
   const bool sm = d->inter_op == DITTO_INTER_SOFTMAX;
   hipError_t e;
-  if (plan.split_rt > 0)
-    e = d->in_dtype == DITTO_F16 ? ditto::launch_split_f16(plan.split_dt, plan.split_rt, sm, kl, args, sets, st)
-                                 : ditto::launch_split_bf16(plan.split_dt, plan.split_rt, sm, kl, args, sets, st);
+  if (sets) {
+    const ditto::BmmSetsKernel k = plan.split_rt > 0 ? ditto::BmmSetsKernel::split
+                                   : plan.rows_nw > 0 ? ditto::BmmSetsKernel::rows
+                                                      : ditto::BmmSetsKernel::rows64;
+    const int dt = plan.split_rt > 0 ? plan.split_dt : plan.rows_dt;
+    const int q = plan.split_rt > 0 ? plan.split_rt : plan.rows_nw > 0 ? plan.rows_nw : plan.qt;
+    const ditto::BmmSetsArgs all{args, *sets};
+    e = d->in_dtype == DITTO_F16 ? ditto::launch_sets_f16(k, dt, q, all, st) : ditto::launch_sets_bf16(k, dt, q, all, st);
+  } else if (plan.split_rt > 0)
+    e = d->in_dtype == DITTO_F16 ? ditto::launch_split_f16(plan.split_dt, plan.split_rt, sm, kl, args, st)
+                                 : ditto::launch_split_bf16(plan.split_dt, plan.split_rt, sm, kl, args, st);
   else if (plan.rows_nw > 0)
-    e = d->in_dtype == DITTO_F16 ? ditto::launch_rows_f16(plan.rows_dt, plan.rows_nw, sm, kl, args, sets, st)
-                                 : ditto::launch_rows_bf16(plan.rows_dt, plan.rows_nw, sm, kl, args, sets, st);
+    e = d->in_dtype == DITTO_F16 ? ditto::launch_rows_f16(plan.rows_dt, plan.rows_nw, sm, kl, args, st)
+                                 : ditto::launch_rows_bf16(plan.rows_dt, plan.rows_nw, sm, kl, args, st);
   else if (d->in_dtype == DITTO_F16)
-    e = sm ? ditto::launch_f16_softmax(plan.d_pad, plan.qt, kl, args, sets, st)
-           : ditto::launch_f16_cast(plan.d_pad, plan.qt, kl, args, sets, st);
+    e = sm ? ditto::launch_f16_softmax(plan.d_pad, plan.qt, kl, args, st)
+           : ditto::launch_f16_cast(plan.d_pad, plan.qt, kl, args, st);
   else
-    e = sm ? ditto::launch_bf16_softmax(plan.d_pad, plan.qt, kl, args, sets, st)
-           : ditto::launch_bf16_cast(plan.d_pad, plan.qt, kl, args, sets, st);
+    e = sm ? ditto::launch_bf16_softmax(plan.d_pad, plan.qt, kl, args, st)
+           : ditto::launch_bf16_cast(plan.d_pad, plan.qt, kl, args, st);
   if (e != hipSuccess) return fail(DITTO_EHIP, "kernel launch failed: %s", hipGetErrorString(e));
   return DITTO_OK;
 }

@@ -58,6 +58,7 @@ struct BmmSets {
 struct BmmSetsArgs : BmmChainArgs {
   BmmSets sets;
 };
+enum class BmmSetsKernel { split, rows, rows64 };  // those that take them
 
 // Where batch entry bz = zo * batch_inner + zi has its operands and its result, in elements from a, b, c, f.
 struct BatchEntry {

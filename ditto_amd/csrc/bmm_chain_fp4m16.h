@@ -518,7 +518,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
 }
 
 template <typename T, int D, int INTER, int KSPLIT, bool B_KL, typename Args>
-hipError_t launch_bmm_chain4m16_args(const Args& args, hipStream_t stream) {
+hipError_t launch_bmm_chain4m16(const Args& args, hipStream_t stream) {
   constexpr int lds = bmm_chain4m16_lds_bytes<D>();
   auto kern = bmm_chain4m16_kernel<T, D, INTER, KSPLIT, B_KL, Args>;
   static thread_local int configured_dev = -1;
@@ -533,13 +533,6 @@ hipError_t launch_bmm_chain4m16_args(const Args& args, hipStream_t stream) {
   const unsigned grid = (unsigned)args.mblocks * (unsigned)args.batch;
   hipLaunchKernelGGL(kern, dim3(grid), dim3(256), lds, stream, args);
   return hipGetLastError();
-}
-
-template <typename T, int D, int INTER, int KSPLIT, bool B_KL>
-hipError_t launch_bmm_chain4m16(const BmmChainArgs& args, const BmmSets* sets, hipStream_t stream) {
-  if constexpr (INTER == kInterSoftmax && !B_KL)
-    if (sets) return launch_bmm_chain4m16_args<T, D, INTER, KSPLIT, B_KL>(BmmSetsArgs{args, *sets}, stream);
-  return sets ? hipErrorInvalidValue : launch_bmm_chain4m16_args<T, D, INTER, KSPLIT, B_KL>(args, stream);
 }
 
 }  // namespace ditto

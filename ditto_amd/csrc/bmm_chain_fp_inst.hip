@@ -11,7 +11,7 @@ namespace ditto {
 // software pipelined; q = 6 | 7: eight-wave kernel on the 16x16x32 MFMA (7: args.mblocks3 of a
 // batch entry's row blocks have 384 rows); q = 4 | 5: four-wave kernel on the 16x16x32 MFMA, 64-row workgroups (head_pad 64;
 // 5: the waves split the keys of a tile as well as the rows)
-hipError_t DITTO_INST_NAME(int d_pad, int q, bool b_kl, const BmmChainArgs& args, const BmmSets* sets, hipStream_t stream) {
+hipError_t DITTO_INST_NAME(int d_pad, int q, bool b_kl, const BmmChainArgs& args, hipStream_t stream) {
   typedef DITTO_INST_T T;
   constexpr int I = DITTO_INST_INTER;
 #define DITTO_CASE(DP, Q)                                                  \
@@ -30,10 +30,9 @@ hipError_t DITTO_INST_NAME(int d_pad, int q, bool b_kl, const BmmChainArgs& args
   if (d_pad == DP && (q == 6 || q == 7))                                   \
     return b_kl ? launch_bmm_chain8m16<T, DP, I, true>(args, stream) : launch_bmm_chain8m16<T, DP, I, false>(args, stream);
   if (d_pad == 64 && q == 4)
-    return b_kl ? launch_bmm_chain4m16<T, 64, I, 1, true>(args, sets, stream) : launch_bmm_chain4m16<T, 64, I, 1, false>(args, sets, stream);
+    return b_kl ? launch_bmm_chain4m16<T, 64, I, 1, true>(args, stream) : launch_bmm_chain4m16<T, 64, I, 1, false>(args, stream);
   if (d_pad == 64 && q == 5)
-    return b_kl ? launch_bmm_chain4m16<T, 64, I, 2, true>(args, sets, stream) : launch_bmm_chain4m16<T, 64, I, 2, false>(args, sets, stream);
-  if (sets) return hipErrorInvalidValue;  // (the 64-row kernels alone take several chains)
+    return b_kl ? launch_bmm_chain4m16<T, 64, I, 2, true>(args, stream) : launch_bmm_chain4m16<T, 64, I, 2, false>(args, stream);
   DITTO_CASE(64, 1)
   DITTO_CASE(64, 2)
   DITTO_CASE(128, 1)

@@ -357,7 +357,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
 }
 
 template <typename T, int DT, int NW, int INTER, bool B_KL, typename Args>
-hipError_t launch_bmm_chain_rows_args(const Args& args, hipStream_t stream) {
+hipError_t launch_bmm_chain_rows(const Args& args, hipStream_t stream) {
   constexpr int lds = bmm_chain_rows_lds<DT, B_KL, NW>();
   auto kern = bmm_chain_rows_kernel<T, DT, NW, INTER, B_KL, Args>;
   static thread_local int configured_dev = -1;
@@ -371,13 +371,6 @@ hipError_t launch_bmm_chain_rows_args(const Args& args, hipStream_t stream) {
   }
   hipLaunchKernelGGL(kern, dim3((unsigned)args.mblocks * (unsigned)args.batch), dim3(64 * NW), lds, stream, args);
   return hipGetLastError();
-}
-
-template <typename T, int DT, int NW, int INTER, bool B_KL>
-hipError_t launch_bmm_chain_rows(const BmmChainArgs& args, const BmmSets* sets, hipStream_t stream) {
-  if constexpr (INTER == kInterSoftmax && !B_KL)
-    if (sets) return launch_bmm_chain_rows_args<T, DT, NW, INTER, B_KL>(BmmSetsArgs{args, *sets}, stream);
-  return sets ? hipErrorInvalidValue : launch_bmm_chain_rows_args<T, DT, NW, INTER, B_KL>(args, stream);
 }
 
 }  // namespace ditto

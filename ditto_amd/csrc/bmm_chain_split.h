@@ -319,7 +319,7 @@ __global__ __launch_bounds__(64 * kSplitWaves) void bmm_chain_split_kernel(Args 
 }
 
 template <typename T, int DT, int RT, int INTER, bool B_KL, typename Args>
-hipError_t launch_bmm_chain_split_args(const Args& args, hipStream_t stream) {
+hipError_t launch_bmm_chain_split(const Args& args, hipStream_t stream) {
   const int lds = bmm_chain_split_lds(DT, RT, B_KL);
   auto kern = bmm_chain_split_kernel<T, DT, RT, INTER, B_KL, Args>;
   static thread_local int configured_dev = -1;
@@ -333,13 +333,6 @@ hipError_t launch_bmm_chain_split_args(const Args& args, hipStream_t stream) {
   }
   hipLaunchKernelGGL(kern, dim3((unsigned)args.mblocks * (unsigned)args.batch), dim3(64 * kSplitWaves), lds, stream, args);
   return hipGetLastError();
-}
-
-template <typename T, int DT, int RT, int INTER, bool B_KL>
-hipError_t launch_bmm_chain_split(const BmmChainArgs& args, const BmmSets* sets, hipStream_t stream) {
-  if constexpr (INTER == kInterSoftmax && !B_KL)
-    if (sets) return launch_bmm_chain_split_args<T, DT, RT, INTER, B_KL>(BmmSetsArgs{args, *sets}, stream);
-  return sets ? hipErrorInvalidValue : launch_bmm_chain_split_args<T, DT, RT, INTER, B_KL>(args, stream);
 }
 
 }  // namespace ditto

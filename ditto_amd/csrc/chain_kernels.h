@@ -18,18 +18,22 @@
 namespace ditto {
 
 // bmm_chain_fp_inst.hip, one object per (element type, inter-op)
-hipError_t launch_f16_cast(int d_pad, int q, bool b_kl, const BmmChainArgs& args, const BmmSets* sets, hipStream_t stream);
-hipError_t launch_f16_softmax(int d_pad, int q, bool b_kl, const BmmChainArgs& args, const BmmSets* sets, hipStream_t stream);
-hipError_t launch_bf16_cast(int d_pad, int q, bool b_kl, const BmmChainArgs& args, const BmmSets* sets, hipStream_t stream);
-hipError_t launch_bf16_softmax(int d_pad, int q, bool b_kl, const BmmChainArgs& args, const BmmSets* sets, hipStream_t stream);
+hipError_t launch_f16_cast(int d_pad, int q, bool b_kl, const BmmChainArgs& args, hipStream_t stream);
+hipError_t launch_f16_softmax(int d_pad, int q, bool b_kl, const BmmChainArgs& args, hipStream_t stream);
+hipError_t launch_bf16_cast(int d_pad, int q, bool b_kl, const BmmChainArgs& args, hipStream_t stream);
+hipError_t launch_bf16_softmax(int d_pad, int q, bool b_kl, const BmmChainArgs& args, hipStream_t stream);
 
 // bmm_chain_split_inst.hip, one object per element type: few rows, the waves split the keys
-hipError_t launch_split_f16(int dt, int rt, bool softmax, bool b_kl, const BmmChainArgs& args, const BmmSets* sets, hipStream_t stream);
-hipError_t launch_split_bf16(int dt, int rt, bool softmax, bool b_kl, const BmmChainArgs& args, const BmmSets* sets, hipStream_t stream);
+hipError_t launch_split_f16(int dt, int rt, bool softmax, bool b_kl, const BmmChainArgs& args, hipStream_t stream);
+hipError_t launch_split_bf16(int dt, int rt, bool softmax, bool b_kl, const BmmChainArgs& args, hipStream_t stream);
 
 // bmm_chain_rows_inst.hip, one object per element type: K and N padded to 80
-hipError_t launch_rows_f16(int dt, int nw, bool softmax, bool b_kl, const BmmChainArgs& args, const BmmSets* sets, hipStream_t stream);
-hipError_t launch_rows_bf16(int dt, int nw, bool softmax, bool b_kl, const BmmChainArgs& args, const BmmSets* sets, hipStream_t stream);
+hipError_t launch_rows_f16(int dt, int nw, bool softmax, bool b_kl, const BmmChainArgs& args, hipStream_t stream);
+hipError_t launch_rows_bf16(int dt, int nw, bool softmax, bool b_kl, const BmmChainArgs& args, hipStream_t stream);
+
+// softmax chains of one shape, several to a launch (bmm_chain_sets_inst.hip); q: split: row tiles of 16, rows: waves, rows64: 4 | 5
+hipError_t launch_sets_f16(BmmSetsKernel kernel, int dt, int q, const BmmSetsArgs& args, hipStream_t stream);
+hipError_t launch_sets_bf16(BmmSetsKernel kernel, int dt, int q, const BmmSetsArgs& args, hipStream_t stream);
 
 // conv_chain_inst.hip, one object per element type; c1_tiles in {1, 2, 4, 8}
 // ch in {32, 16}: input channels per staged chunk

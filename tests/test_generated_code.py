@@ -407,6 +407,27 @@ def test_short_chain_units_keep_their_counted_waits_exact(tmp_path, unit_name, k
     assert not bare and (stores > 0) == unit_name.startswith("fp_rows")
 
 
+@pytest.mark.parametrize("unit_name", ["fp_sets_f16", "fp_sets_bf16"])
+def test_units_of_several_chains_a_launch_keep_their_counted_waits_exact(tmp_path, unit_name):
+    """The same for the kernels compiled again with a table of chains in their arguments."""
+    hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+    if not os.path.exists(hipcc):
+        pytest.skip("hipcc not available")
+    unit = [u for u in build_ext.UNITS if u[0] == unit_name][0]
+    out = tmp_path / "unit.s"
+    flags = [f for f in build_ext.HIPCC_FLAGS if f != "-fPIC"]
+    subprocess.run([hipcc, *flags, "--cuda-device-only", "-S", *unit[2], os.path.join(CSRC, unit[1]), "-o", str(out)], check=True,
+                   capture_output=True)
+    text = out.read_text()
+    md = kernel_metadata(text)
+    assert len(md) == 6 + 5 + 2  # split, rows, 64 rows
+    assert all(v["vgpr_spill_count"] == 0 for v in md.values())
+    loops = []
+    assert untracked_memory_ops_in_direct_load_loops(text, loops) == []
+    assert len({name for name, _, _ in loops}) == len(md)
+    assert barriers_with_lds_in_flight(text) == []
+
+
 @pytest.mark.parametrize("unit_name", ["gemm_chain_i8", "gemm_chain_f32", "conv_tiles_f16", "dw_tiles_f16"])
 def test_no_barrier_with_lds_accesses_in_flight(tmp_path, unit_name):
     hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
