@@ -107,14 +107,20 @@ struct BmmPrice {
 };
 // Least squares over 3300 random shapes (batch 1 - 160, 32 - 4096 rows and keys, fp16 and bf16), root mean square error
 // 4 - 12 %; the columns: head sizes up to 64 | 128, without | with softmax, B [L][K] | [K][L].
-constexpr BmmPrice kPrices64[2][8] = {
-    {{641, 128, 256, 1, 0.71f, {3.38f}, {.0074f}}, {644, 64, 256, 3, 2.64f, {1.30f, 1.81f, 2.36f}, {.0049f, .0079f, .0121f}},
-     {645, 64, 256, 2, 2.98f, {1.34f, 2.09f}, {.0042f, .0070f}}, {649, 256, 512, 1, 0, {5.03f}, {.0118f}},
-     {2144, 128, 256, 2, 1.51f, {2.68f, 3.41f}, {.0091f, .0155f}}, {2148, 256, 512, 1, 2.23f, {2.31f}, {.0124f}}},
-    {{641, 128, 256, 1, 0.68f, {3.38f}, {.0077f}}, {644, 64, 256, 3, 2.75f, {1.33f, 1.93f, 2.79f}, {.0060f, .0092f, .0128f}},
-     {645, 64, 256, 2, 3.05f, {1.53f, 2.74f}, {.0049f, .0074f}}, {649, 256, 512, 1, 0, {5.14f}, {.0117f}},
-     {2144, 128, 256, 2, 1.67f, {2.89f, 4.04f}, {.0097f, .0158f}}, {2148, 256, 512, 1, 1.81f, {3.20f}, {.0116f}},
-     {2041, 16, 512, 1, 2.89f, {1.35f}, {.0025f}}, {2042, 32, 512, 1, 2.78f, {2.37f}, {.0027f}}}};
+constexpr BmmPrice kPrices64[2][2][8] = {
+    {{{641, 128, 256, 1, 0.71f, {3.38f}, {.0074f}}, {644, 64, 256, 3, 2.64f, {1.30f, 1.81f, 2.36f}, {.0049f, .0079f, .0121f}},
+      {645, 64, 256, 2, 2.98f, {1.34f, 2.09f}, {.0042f, .0070f}}, {649, 256, 512, 1, 0, {5.03f}, {.0118f}},
+      {2144, 128, 256, 3, 2.40f, {1.77f, 2.36f, 3.74f}, {.0091f, .0156f, .0208f}}, {2148, 256, 512, 1, 2.23f, {2.31f}, {.0124f}}},
+     {{641, 128, 256, 1, 0.68f, {3.38f}, {.0077f}}, {644, 64, 256, 3, 2.75f, {1.33f, 1.93f, 2.79f}, {.0060f, .0092f, .0128f}},
+      {645, 64, 256, 2, 3.05f, {1.53f, 2.74f}, {.0049f, .0074f}}, {649, 256, 512, 1, 0, {5.14f}, {.0117f}},
+      {2144, 128, 256, 3, 2.11f, {2.30f, 3.42f, 4.75f}, {.0102f, .0154f, .0209f}}, {2148, 256, 512, 1, 1.81f, {3.20f}, {.0116f}},
+      {2041, 16, 512, 1, 2.89f, {1.35f}, {.0025f}}, {2042, 32, 512, 1, 2.78f, {2.37f}, {.0027f}}}},
+    {{{644, 64, 256, 3, 2.64f, {1.38f, 1.90f, 2.65f}, {.0057f, .0096f, .0132f}}, {645, 64, 256, 2, 3.38f, {1.16f, 2.21f}, {.0054f, .0083f}},
+      {646, 256, 512, 1, 0, {6.41f}, {.0170f}}, {649, 256, 512, 1, 0, {5.96f}, {.0159f}},
+      {2144, 128, 256, 3, 2.77f, {1.45f, 2.35f, 3.81f}, {.0118f, .0183f, .0242f}}},
+     {{644, 64, 256, 3, 2.74f, {1.40f, 2.10f, 3.04f}, {.0062f, .0100f, .0138f}}, {645, 64, 256, 2, 3.54f, {1.34f, 2.81f}, {.0057f, .0085f}},
+      {649, 256, 512, 1, 0, {6.02f}, {.0162f}},
+      {2144, 128, 256, 3, 2.94f, {1.55f, 2.95f, 4.34f}, {.0119f, .0177f, .0243f}}}}};
 constexpr BmmPrice kPrices128[2][2][7] = {
     {{{1281, 128, 256, 1, 0, {5.79f}, {.0113f}}, {1282, 256, 256, 1, 0, {8.95f}, {.0223f}}, {1286, 256, 512, 1, 0, {7.95f}, {.0277f}},
       {1289, 256, 512, 1, 0, {6.92f}, {.0227f}}, {2188, 256, 512, 1, 0, {5.55f}, {.0230f}},
@@ -133,13 +139,16 @@ constexpr BmmPrice kPrices128[2][2][7] = {
 // along one size at a time and miss where the rounds of two kernels fall differently: one round of 256-row workgroups against
 // two of 128 rows (40 x 809 x 1608 x 128 softmax 59.2 -> 44.2 us), 1.2 rounds of 256 against 2.2 of 128 (30 x 2080 x 2032 x 128
 // 122 -> 79), without softmax 50 x 1520 x 576 x 64 24.7 -> 19.1, 5 x 432 x 144 x 128 7.6 -> 6.0.  Over 400 - 700 random shapes
-// a class the mean is 0.8 to 3.6 % lower, the best 0.50 of the time, the worst 1.06 - 1.11 of it.
+// a class the mean is 0.8 to 3.6 % lower, the best 0.50 of the time, the worst 1.06 - 1.11 of it.  Softmax chains of up to 64
+// columns have one other kernel to go to, 32 rows a wave, from 5 % on: of 1800 + 900 random shapes with B [L][K] | [K][L] it
+// takes 150 + 100 there, at 0.90 | 0.88 of the time, the worst 1.01 (1152 x 512 x 512 122 -> 107 us, 3268 x 197 x 197 110 -> 84,
+// 830 x 1024 x 1024 295 -> 258; long keys on few rows stay: 830 x 192 x 2048 114 against 136).
 int cheaper_variant(const ditto_bmm_chain_desc* d, int own, int cus) {
   const long long dmax = d->K > d->N ? d->K : d->N;
   const bool sm = d->inter_op == DITTO_INTER_SOFTMAX, kl = d->b_layout == DITTO_B_KL;
   // with softmax the kernels that find a row's first unmasked key wherever it lies (20xx, 21xx, 644, 645) keep what they have
-  if (dmax <= 64 ? sm : dmax <= 80 || (sm && own >= 2000)) return 0;
-  const BmmPrice* const prices = dmax <= 64 ? kPrices64[kl] : kPrices128[sm][kl];
+  if (dmax > 64 && (dmax <= 80 || (sm && own >= 2000))) return 0;
+  const BmmPrice* const prices = dmax <= 64 ? kPrices64[sm][kl] : kPrices128[sm][kl];
   const int count = dmax <= 64 ? 8 : 7;
   int best = 0;
   float own_price = 0, best_price = 0;
@@ -150,10 +159,12 @@ int cheaper_variant(const ditto_bmm_chain_desc* d, int own, int cus) {
     const float L = (float)d->L, price = p.start + full * (p.first[r] + p.per_key[r] * L) +
                                          (left > 0 ? p.first[left - 1] + p.per_key[left - 1] * L : 0.f);
     if (p.variant == own) own_price = price;
-    if (p.variant == 2188 && (d->L < 64 || d->L > 700)) continue;  // (beyond the lines its price fits, by 4 - 9 %)
+    // (beyond the lines their prices fit, by 4 - 9 %)
+    if ((p.variant == 2188 && (d->L < 64 || d->L > 700)) || (p.variant == 2144 && d->L <= 64 && !(sm && full > 0))) continue;
+    if (sm && dmax <= 64 && p.variant != 2144) continue;
     if ((best == 0 || price < best_price) && launchable(wgs, p.threads)) best = p.variant, best_price = price;
   }
-  return best != own && own_price > 0 && best_price < 0.93f * own_price ? best : 0;
+  return best != own && own_price > 0 && best_price < (sm && dmax <= 64 ? 0.95f : 0.93f) * own_price ? best : 0;
 }
 
 int plan_bmm_rules(const ditto_bmm_chain_desc* d, BmmPlan* plan, int cus);
@@ -384,18 +395,11 @@ int plan_bmm_rules(const ditto_bmm_chain_desc* d, BmmPlan* plan, int cus) {
       }
       if (d->tile_variant == 0 && dt == 4 && rt == 0 && sm && plan->qt != 6) {
         // Heads of up to 64 with softmax where the 64-row kernel, three workgroups to a compute unit, needs a second round and this
-        // one in its four-wave form, two of 128 rows to a compute unit, does not: on 250 shapes 0.74 - 0.86 of the time at 64 keys,
-        // 0.83 - 0.96 at 200, 0.87 - 1.02 at 600, 1.06 at 1000 (256 x 197 x 197 10.9 -> 9.3 us, 512 x 100 x 100 9.6 -> 8.2).  With a
-        // few rounds more the two are level or this one is behind by its part of a round (300 x 512 x 512 30.6 / 33.8).
-        // Many rounds hide that, and a wave of 32 rows reads half as much LDS a row: from eight rounds on 0.95 - 1.00 of the time
-        // where 128-row blocks waste no more rows than 64-row ones (1152 x 512 x 512 122 -> 115, 2097 x 384 x 512 170 -> 164,
-        // 1249 x 256 x 256 level).  Where a last block has 65 to 96 rows one of its four waves has nothing to do, against a
-        // quarter of two 64-row blocks: 0.90 - 1.00 from four rounds on (2339 x 96 x 96 27.6 -> 24.9, 3268 x 197 x 197 111 -> 102).
-        // (Without softmax cheaper_variant sees to it.)
+        // one in its four-wave form, of 128 rows, does not: on 250 shapes 0.74 - 0.86 of the time at 64 keys,
+        // 0.83 - 0.96 at 200, 0.87 - 1.02 at 600 (256 x 197 x 197 10.9 -> 9.0 us, 512 x 100 x 100 9.6 -> 8.2).  Other sizes go by
+        // their price.
         const long long n64 = ((d->M + 63) / 64) * d->batch, n128 = ((d->M + 127) / 128) * d->batch;
-        const long long last = (d->M - 1) % 128 + 1, rounds = n128 / (2LL * cus);
-        const bool many = last > 64 && rounds >= (last <= 96 ? 4 : 8);
-        if (n64 > 3LL * cus && (n128 <= 2LL * cus || many) && d->L <= 600 && launchable(n128, 256)) plan->rows_dt = 4, plan->rows_nw = 4;
+        if (n64 > 3LL * cus && n128 <= 2LL * cus && d->L <= 600 && launchable(n128, 256)) plan->rows_dt = 4, plan->rows_nw = 4;
       }
       if (d->tile_variant == 0 && dt == 4 && rt == 0 && !sm && n8 >= 2LL * cus && d->L <= 1024) {
         // Heads of up to 64 without softmax from two 256-row workgroups per compute unit on, up to 1024 keys: 512 x 197 x 197 16.8 ->

@@ -16,7 +16,14 @@
 // 22.9 -> 8.8 | 12.0, 80 x 400 x 400 23.2 -> 13.4 | 12.9, 96 x 700 x 700 44.8 -> 28.7 | 35.9, 32 x 4096 x 4096 206 -> 191 | 187.
 // The same kernel at 64 columns (without softmax, large grids) and at 128 (up to about 500 keys) is ahead of the others by its
 // start: 512 x 197 x 197 x 64 16.8 -> 12.2, x 128 with softmax 33.2 -> 27.8.
+//
+// At 64 columns a row of B or C is 128 bytes and needs no padding if it is swizzled: tiles of 16 KB instead of 20, four direct
+// loads a wave and tile instead of five, and three workgroups of four waves to a compute unit instead of two.  With two waves on
+// a SIMD its pipes were 72 % busy (vector ALU 41, of which v_exp_f32 two thirds, matrix 30); the third takes the waits of the
+// other two: 1152 x 512 x 512 with softmax 115 -> 107 us, 830 x 1024 x 1024 291 -> 258, 1249 x 256 x 256 41.6 -> 36.2, and one
+// round more of workgroups fits (329 x 197 x 128 9.6 -> 7.8).
 #pragma once
+#include "bmm_chain_fp4m16.h"
 #include "bmm_chain_fp8m16.h"
 #include "common.h"
 
@@ -25,14 +32,16 @@ namespace ditto {
 constexpr int kRowsRing = 3;
 
 // One tile of 64 keys in LDS: B, then C, filled by direct loads of 64 16-byte chunks each that are dealt to the waves in
-// order; rows are padded to chunk counts that spread the reads of 16 lanes over all banks, no swizzle.
+// order; rows are padded to chunk counts that spread the reads of 16 lanes over all banks, no swizzle.  Heads of 64 columns
+// fill 128-byte rows: those are swizzled (see swz4m16_rows), a tile is 16 KB and three workgroups of four waves fit a compute unit.
 // DT: column tiles of 16 that K and N are padded to; the contraction over K runs in steps of 32.
 template <int DT, bool B_KL>
 struct RowsTiles {
   static constexpr int KS = (DT + 1) / 2;
-  static constexpr int B_CPR = B_KL ? 8 : 4 * KS + 1;  // [64 l][32 KS k], or [32 KS k][64 l] with swizzled 128-byte rows
+  static constexpr bool SWZ = DT == 4;
+  static constexpr int B_CPR = B_KL || SWZ ? 8 : 4 * KS + 1;  // [64 l][32 KS k], or [32 KS k][64 l] with swizzled 128-byte rows
   static constexpr int B_ROWS = B_KL ? 32 * KS : kBN;
-  static constexpr int C_CPR = DT == 8 ? 18 : 10;
+  static constexpr int C_CPR = SWZ ? 8 : DT == 8 ? 18 : 10;
   static constexpr int B_LOADS = (B_ROWS * B_CPR + 63) / 64, C_LOADS = (kBN * C_CPR + 63) / 64;
   static constexpr int C_OFF = B_LOADS * 1024;
 };
@@ -53,7 +62,7 @@ inline int bmm_chain_rows_lds(int dt, int nw, bool kl) {
 }
 
 template <typename T, int DT, int NW, int INTER, bool B_KL, typename Args>
-__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) void bmm_chain_rows_kernel(Args p) {
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(DT == 4 && NW == 4 ? 3 : 2))) void bmm_chain_rows_kernel(Args p) {
 #if defined(__HIP_DEVICE_COMPILE__)
   typedef typename Elem<T>::v8 V8;
   typedef typename Elem<T>::v4 V4;
@@ -109,12 +118,13 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
     const int ld = NLD * w + i;
     if (ld < S::B_LOADS) {
       const int ch = 64 * ld + lane, row = ch / S::B_CPR, pc = ch - row * S::B_CPR;
-      const int lc = B_KL ? pc ^ (2 * ((row >> 1) & 3)) : pc;
+      const int lc = B_KL ? pc ^ swz4m16_tr(row) : S::SWZ ? pc ^ swz4m16_rows(row) : pc;
       const bool in = B_KL ? row < K : row < kBN && 8 * lc < K;
       key[i] = !in ? kNever : B_KL ? 8 * lc : row;
       voff[i] = (row * p.b_rs + 8 * lc) * 2;
     } else {
-      const int ch = 64 * (ld - S::B_LOADS) + lane, row = ch / S::C_CPR, lc = ch - row * S::C_CPR;
+      const int ch = 64 * (ld - S::B_LOADS) + lane, row = ch / S::C_CPR, pc = ch - row * S::C_CPR;
+      const int lc = S::SWZ ? pc ^ swz4m16_tr(row) : pc;
       key[i] = row < kBN && 8 * lc < N ? row : kNever;
       voff[i] = (row * p.c_rs + 8 * lc) * 2;
     }
@@ -132,22 +142,26 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
 
   // LDS read addresses: B fragment of key tile kt (16 keys), k step s; C^T fragment of 32-key half h, column tile j
   const int tr_row = 4 * q + (c >> 2), tr_half = (c & 3) >> 1, tr_byte = 8 * (c & 1);
-  constexpr int NBA = B_KL ? 4 : 1;
-  int b_ad[NBA];
+  constexpr int NBA = B_KL ? 4 : S::SWZ ? KS : 1, NCA = S::SWZ ? DT : 1;
+  int b_ad[NBA], c_ad[NCA];
 #pragma unroll
-  for (int kt = 0; kt < NBA; ++kt)
-    b_ad[kt] = B_KL ? tr_row * 128 + (((2 * kt + tr_half) ^ (2 * ((tr_row >> 1) & 3))) * 16) + tr_byte : c * (S::B_CPR * 16) + q * 16;
-  const int c_ad = tr_row * (S::C_CPR * 16) + tr_half * 16 + tr_byte + S::C_OFF;
+  for (int i = 0; i < NBA; ++i)
+    b_ad[i] = B_KL     ? tr_row * 128 + (((2 * i + tr_half) ^ swz4m16_tr(tr_row)) * 16) + tr_byte
+              : S::SWZ ? c * 128 + (((4 * i + q) ^ swz4m16_rows(c)) * 16)
+                       : c * (S::B_CPR * 16) + q * 16;
+#pragma unroll
+  for (int j = 0; j < NCA; ++j)
+    c_ad[j] = tr_row * (S::C_CPR * 16) + (S::SWZ ? (2 * j + tr_half) ^ swz4m16_tr(tr_row) : tr_half) * 16 + tr_byte + S::C_OFF;
   auto b_frag = [&](const char* tile, int kt, int s) __attribute__((always_inline)) -> V8 {
     if constexpr (B_KL) {
       const char* const a = tile + b_ad[kt % NBA] + 32 * s * 128;
       return concat4<V4, V8>(lds_read_tr4<T>(reinterpret_cast<const T*>(a)), lds_read_tr4<T>(reinterpret_cast<const T*>(a + 16 * 128)));
     } else {
-      return *reinterpret_cast<const V8*>(tile + b_ad[0] + kt * 16 * (S::B_CPR * 16) + s * 64);
+      return *reinterpret_cast<const V8*>(tile + b_ad[s % NBA] + kt * 16 * (S::B_CPR * 16) + (S::SWZ ? 0 : s * 64));
     }
   };
   auto c_frag = [&](const char* tile, int h, int j) __attribute__((always_inline)) -> V8 {
-    const char* const a = tile + c_ad + 32 * h * (S::C_CPR * 16) + j * 32;
+    const char* const a = tile + c_ad[j % NCA] + 32 * h * (S::C_CPR * 16) + (S::SWZ ? 0 : j * 32);
     return concat4<V4, V8>(lds_read_tr4<T>(reinterpret_cast<const T*>(a)),
                            lds_read_tr4<T>(reinterpret_cast<const T*>(a + 16 * (S::C_CPR * 16))));
   };

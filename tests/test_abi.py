@@ -228,11 +228,10 @@ def test_kernels_are_priced_against_each_other():
     assert plan(5, 432, 144, 128, CAST, KL) == 2081
     assert plan(65, 416, 416, 64, CAST, KL) == 644
     assert plan(160, 300, 296, 64, CAST, KL) == 2144
-    assert plan(256, 197, 197, 64, SM, LK) == 2144 and plan(256, 197, 640, 64, SM, LK) == 644
-    # rounds of 128-row workgroups: 2 and a bit, 9; a last block of 96 rows: 4 and a bit, 3 and a bit; of 32 rows: 17
-    assert plan(300, 512, 512, 64, SM, LK) == 644 and plan(1152, 512, 512, 64, SM, LK) == 2144
-    assert plan(2100, 96, 96, 64, SM, LK) == 2144 and plan(1600, 96, 96, 64, SM, LK) == 644
-    assert plan(4520, 160, 160, 64, SM, LK) == 644
+    assert plan(256, 197, 197, 64, SM, LK) == 2144 and plan(256, 197, 640, 64, SM, LK) == 2144
+    # one round of 128-row workgroups, several; not: 64 rows, long keys on few rows, a last block of 32 rows in 5 / 4 of a round
+    assert plan(329, 197, 128, 64, SM, LK) == 2144 and plan(1152, 512, 512, 64, SM, KL) == 2144 and plan(2100, 96, 96, 64, SM, LK) == 2144
+    assert plan(2202, 64, 64, 64, SM, LK) == 644 and plan(830, 192, 2048, 64, SM, LK) == 645 and plan(493, 160, 160, 64, SM, LK) == 644
     for M in (100, 300, 1000):
         for L in (64, 500, 1500):
             for batch in (1, 20, 200):
