@@ -705,17 +705,24 @@ bool plan_dw_tiles(const ditto_conv_chain_desc* d, long long P, long long Q, Con
       (mult == 1 && d->C0 % 8) || d->C0 * d->H * d->W > 0x3fffffff)
     return false;
   auto rows_in = [&](int th) { return (int)((th - 1) * d->stride1 + 3); };
-  auto lds_of = [&](int th) { return ditto::dw_tiles_lds_bytes(mult, rows_in(th), (int)d->W, d->C2 <= 32 ? 2 : 4); };
+  // A workgroup has eight waves and a tile of 16 pixels needs one: where half or three quarters of them would have none, two or
+  // four waves share out the channels of a tile.
+  auto groups_of = [&](int th) { return th * Q <= 4 * ditto::kDtWaves ? 4 : th * Q <= 8 * ditto::kDtWaves ? 2 : 1; };
+  auto lds_of = [&](int th) {
+    return ditto::dw_tiles_lds_bytes(mult, rows_in(th), (int)d->W, d->C2 <= 32 ? 2 : 4, groups_of(th));
+  };
   if (lds_of(1) > 160 * 1024) return false;
   // Rows per workgroup.  A workgroup of one pixel tile per wave takes two units alone on a compute unit and three (multiplier
-  // 1: 2.6) beside another, one of two tiles 3 and 4.6 (5.2); a compute unit holds two.  The height with the fewest units on
-  // the busiest compute unit wins, the smaller one on ties (32 x 64 x 56 x 56 times 16: one row 63 us, two 38, four 29.5;
-  // times 1: 22, 16.2, 18.3).
+  // 1: 2.6) beside another, one of two tiles 3 and 4.6 (5.2), with two waves to a tile 1.5 and 2.4 (1.9 and 2.3), with four 1.25
+  // and 2 (1.65 and 2); a compute unit holds two.  The height with the fewest units on the busiest compute unit wins, the smaller
+  // one on ties (32 x 64 x 56 x 56 times 16: one row 63 us, two 38, four 29.5; times 1: 22, 16.2, 18.3; 11 x 64 x 28 x 28 times
+  // 16: one row 13.1, two 10.6, four 13.7; times 1: 7.2, 6.3, 6.7).
   int th = 1;
   double best = 0;
   for (int t = 1; t <= P && t * Q <= slots && lds_of(t) <= 160 * 1024; ++t) {
-    const bool two = t * Q > 16 * ditto::kDtWaves;
-    const double alone = two ? 3 : 2, pair = mult == 16 ? (two ? 4.6 : 3) : (two ? 5.2 : 2.6);
+    const int k = t * Q > 16 * ditto::kDtWaves ? 0 : groups_of(t) == 1 ? 1 : groups_of(t) == 2 ? 2 : 3;
+    static constexpr double kAlone[2][4] = {{3, 2, 1.9, 1.65}, {3, 2, 1.5, 1.25}}, kPair[2][4] = {{5.2, 2.6, 2.3, 2}, {4.6, 3, 2.4, 2}};
+    const double alone = kAlone[mult == 16][k], pair = kPair[mult == 16][k];
     const long long wgs = d->N * ((P + t - 1) / t), per_round = 2LL * lds_of(t) <= 160 * 1024 ? 2 * cus : cus;
     const long long full = wgs / per_round, rest = wgs % per_round;
     const double cost = full * (per_round > cus ? pair : alone) + (rest > cus ? pair : rest > 0 ? alone : 0);
@@ -728,6 +735,7 @@ bool plan_dw_tiles(const ditto_conv_chain_desc* d, long long P, long long Q, Con
   a.TH = th;
   a.tiles_h = (int)((P + th - 1) / th);
   a.rows_in = rows_in(th);
+  a.groups = groups_of(th);
   a.relu_mid = d->inter_op == DITTO_INTER_RELU;
   a.relu_out = d->relu_out != 0;
   a.out_f32 = d->out_dtype == DITTO_F32;

@@ -17,6 +17,7 @@ struct DwTilesArgs {
   int relu_mid, relu_out, out_f32;
   float inv_blocks, inv_rows, inv_q;  // 1 / (16-byte blocks per row), 1 / rows_in, 1 / Q
   float inv_group;                    // 1 / (blocks of eight channels and their padding)
+  int groups;                         // of waves that share out a chunk's channels: 1, or 2 or 4 with one tile a wave
 };
 
 constexpr int kDtWaves = 8;
@@ -28,9 +29,11 @@ __host__ __device__ constexpr int dw_tiles_chunk(int mult) { return mult == 16 ?
 // that read channels 8 q .. + 7 (one output per channel) then start in four different quarters of the banks.
 __host__ __device__ inline int dw_tiles_row_blocks(int W) { return 1 + (W + 7) / 8; }
 __host__ __device__ inline int dw_tiles_group_blocks(int rows_in, int W) { return 8 * rows_in * dw_tiles_row_blocks(W) + 4; }
-__host__ __device__ inline int dw_tiles_lds_bytes(int mult, int rows_in, int W, int nt) {
+__host__ __device__ inline int dw_tiles_lds_bytes(int mult, int rows_in, int W, int nt, int groups) {
   const int x = dw_tiles_chunk(mult) / 8 * dw_tiles_group_blocks(rows_in, W) * 16;
-  return x + (mult == 16 ? 256 * 18 + 8 * nt * 1024 : 32 * 32 + nt * 1024);
+  const int chunk = x + (mult == 16 ? 256 * 18 + 8 * nt * 1024 : 32 * 32 + nt * 1024);
+  const int sums = (kDtWaves - kDtWaves / groups) * nt * 1024;  // of all groups of waves but the first
+  return chunk > sums ? chunk : sums;
 }
 
 template <typename T>
@@ -63,20 +66,25 @@ __device__ __forceinline__ i32x4 drop_elements(i32x4 v, int s) {
 // kernel, which walks padded rectangles one after another and waits for each chunk, took 52.5); times 1 the vector ALU (40 of
 // 54 us at 32 x 64 x 112 x 112); on small grids the chain of a chunk's load, barrier and products, 2 us per 16 channels (one
 // image of 32 x 37 x 37 times 16: 8.6 us, before 25.3; 32 x 16 x 147 x 147 times 16 stride 2: 19 us, before 127).
+// Rows of at most 64 pixels on few images leave waves without a tile, and the chain above is theirs who have one: two or four
+// waves share out the channels of a chunk then (G) and their sums meet at the end (4 x 64 x 28 x 28 times 16: 13.6 -> 9.1 us,
+// 3 x 64 x 62 x 62 13.3 -> 10.7, 4 x 32 x 57 x 57 9.6 -> 7.9; times 1, whose sums are shorter: 4 x 64 x 28 x 28 6.5 -> 5.8).
 // Eight waves of two tiles instead of four of four: half the blocks for a thread to stage, and two workgroups share a
 // compute unit (32.4 -> 29.5 us).  Filters are loaded as they lie in memory, by 16-byte blocks: one 18-byte filter per lane
 // cost 0.4 us per chunk in misaligned loads.
-template <typename T, int MULT, int RT, int NT>
+template <typename T, int MULT, int RT, int NT, int G>
 __global__ __launch_bounds__(64 * kDtWaves, MULT == 1 && RT == 2 ? 2 : 4) void dw_tiles_kernel(DwTilesArgs p) {
 #if defined(__HIP_DEVICE_COMPILE__)
   typedef typename Elem<T>::v8 V8;
   typedef typename Elem<T>::v4 V4;
   typedef typename Elem<T>::v2 V2;
   typedef __attribute__((ext_vector_type(8), aligned(2))) T V8u;
-  constexpr int CC = dw_tiles_chunk(MULT), THREADS = 64 * kDtWaves;
+  constexpr int CC = dw_tiles_chunk(MULT), THREADS = 64 * kDtWaves, WP = kDtWaves / G;
+  static_assert(G == 1 || RT == 1, "");
   extern __shared__ __attribute__((aligned(16))) char smem_dt[];
   const int tid = threadIdx.x, lane = tid & 63, c = lane & 15, q = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wp = wave % WP, wg = wave / WP;  // its pixel tiles, its share of the channels
   const unsigned lid = xcd_remap(blockIdx.x, gridDim.x);
   const int n = lid / (unsigned)p.tiles_h, p0 = (lid - n * (unsigned)p.tiles_h) * p.TH;
   const int npx = min(p.TH, p.P - p0) * p.Q, h0 = p0 * p.stride - 1;
@@ -99,7 +107,7 @@ __global__ __launch_bounds__(64 * kDtWaves, MULT == 1 && RT == 2 ? 2 : 4) void d
   int xd[RT], sh[RT];
 #pragma unroll
   for (int t = 0; t < RT; ++t) {
-    int slot = 16 * RT * wave + RT * c + t;
+    int slot = 16 * RT * wp + RT * c + t;
     slot = slot < npx ? slot : 0;
     const int ph = div_by(slot, p.inv_q), pw = slot - ph * p.Q;
     const int e = 7 + pw * p.stride;
@@ -197,7 +205,7 @@ __global__ __launch_bounds__(64 * kDtWaves, MULT == 1 && RT == 2 ? 2 : 4) void d
       const int o1 = 9 * c + 3 * min(q, 2), w1d = o1 >> 1, w1sh = (o1 & 1) * 16;
       const unsigned keep = q < 3 ? 0xffffffffu : 0u;
 #pragma unroll 2
-      for (int pr = 0; pr < 8; ++pr) {
+      for (int pr = wg; pr < 8; pr += G) {
         i32x2 a[2];
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
@@ -235,13 +243,18 @@ __global__ __launch_bounds__(64 * kDtWaves, MULT == 1 && RT == 2 ? 2 : 4) void d
     } else {
       // One output per channel: lane (c, q) computes channels 8 q .. + 7 of pixel c, its share of the 1x1 convolution's
       // operand, as six two-element dot products per channel (three taps of a row: a pair, and one against zero)
+      // (with several groups of waves: 8 / G of them, the rest of the operand zeros)
+      constexpr int KG = 8 / G;
+      const int k0 = KG * wg;
       V8 pf[RT];
 #pragma unroll
-      for (int k = 0; k < 8; k += 2) {
+      for (int t = 0; t < RT; ++t) pf[t] = V8{0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+      for (int k = 0; k < KG; k += 2) {
         float m[RT][2];
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
-          const i32x2* const w = reinterpret_cast<const i32x2*>(w1_lds) + (8 * q + k + u) * 4;
+          const i32x2* const w = reinterpret_cast<const i32x2*>(w1_lds) + (8 * q + k0 + k + u) * 4;
 #pragma unroll
           for (int t = 0; t < RT; ++t) m[t][u] = 0.f;
 #pragma unroll
@@ -250,7 +263,7 @@ __global__ __launch_bounds__(64 * kDtWaves, MULT == 1 && RT == 2 ? 2 : 4) void d
             const int taps01 = taps[0], tap2 = taps[1];  // (a bit cast of a vector's element takes element 0)
 #pragma unroll
             for (int t = 0; t < RT; ++t) {
-              const unsigned* const x = Xs + q * group * 4 + (k + u) * plane + r * blocks * 4 + xd[t];
+              const unsigned* const x = Xs + q * group * 4 + (k0 + k + u) * plane + r * blocks * 4 + xd[t];
               const unsigned lo = x[0], hi = x[1];
               m[t][u] = Elem<T>::dot2(__builtin_bit_cast(V2, __builtin_amdgcn_alignbit(hi, lo, sh[t])), __builtin_bit_cast(V2, taps01), m[t][u]);
               m[t][u] = Elem<T>::dot2(__builtin_bit_cast(V2, __builtin_amdgcn_ubfe(hi, sh[t], 16)), __builtin_bit_cast(V2, tap2), m[t][u]);
@@ -268,14 +281,38 @@ __global__ __launch_bounds__(64 * kDtWaves, MULT == 1 && RT == 2 ? 2 : 4) void d
       for (int t = 0; t < RT; ++t) pf[t] = relu_packed(pf[t], thr);
 #pragma unroll
       for (int j = 0; j < NT; ++j) {
-        const V8 w2 = reinterpret_cast<const V8*>(W2s)[j * 64 + lane];
+        V8 w2;
+        if constexpr (G == 1) {
+          w2 = reinterpret_cast<const V8*>(W2s)[j * 64 + lane];
+        } else {
+          typedef __attribute__((ext_vector_type(KG))) T VG;
+          const VG own = *reinterpret_cast<const VG*>(W2s + (j * 64 + lane) * 8 + k0);
+          w2 = V8{0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+          for (int e = 0; e < KG; ++e) w2[e] = own[e];
+        }
 #pragma unroll
         for (int t = 0; t < RT; ++t) acc[t][j] = Elem<T>::mfma16(w2, pf[t], acc[t][j]);
       }
     }
   }
 
-  const int first = 16 * RT * wave + RT * c, valid = npx - first;  // of this lane's pixels
+  if constexpr (G > 1) {
+    // the groups' sums meet in LDS, which nobody needs any more, and are added in the order of the groups
+    f32x4* const sums = reinterpret_cast<f32x4*>(smem_dt) + wp * NT * 64 + lane;
+    wg_sync();
+    if (wg > 0)
+#pragma unroll
+      for (int j = 0; j < NT; ++j) sums[((wg - 1) * WP * NT + j) * 64] = acc[0][j];
+    wg_sync();
+    if (wg > 0) return;
+#pragma unroll
+    for (int g = 1; g < G; ++g)
+#pragma unroll
+      for (int j = 0; j < NT; ++j) acc[0][j] += sums[((g - 1) * WP * NT + j) * 64];
+  }
+
+  const int first = 16 * RT * wp + RT * c, valid = npx - first;  // of this lane's pixels
   const long long out_plane = (long long)p.P * p.Q;
 #pragma unroll
   for (int j = 0; j < NT; ++j)
@@ -319,9 +356,9 @@ __global__ __launch_bounds__(64 * kDtWaves, MULT == 1 && RT == 2 ? 2 : 4) void d
 #endif
 }
 
-template <typename T, int MULT, int RT, int NT>
+template <typename T, int MULT, int RT, int NT, int G = 1>
 hipError_t launch_dw_tiles_as(const DwTilesArgs& a, hipStream_t stream) {
-  auto kern = dw_tiles_kernel<T, MULT, RT, NT>;
+  auto kern = dw_tiles_kernel<T, MULT, RT, NT, G>;
   static thread_local int configured_dev = -1;
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
@@ -331,7 +368,7 @@ hipError_t launch_dw_tiles_as(const DwTilesArgs& a, hipStream_t stream) {
     if (e != hipSuccess) return e;
     configured_dev = dev;
   }
-  const int lds = dw_tiles_lds_bytes(MULT, a.rows_in, a.W, NT);
+  const int lds = dw_tiles_lds_bytes(MULT, a.rows_in, a.W, NT, a.groups);
   hipLaunchKernelGGL(kern, dim3((unsigned)a.N * (unsigned)a.tiles_h), dim3(64 * kDtWaves), lds, stream, a);
   return hipGetLastError();
 }
@@ -340,6 +377,9 @@ hipError_t launch_dw_tiles_mult(const DwTilesArgs& a, hipStream_t stream) {
   const int tiles = (a.TH * a.Q + 15) / 16;
   if (tiles > kDtMaxTiles || a.C2 > 64) return hipErrorInvalidValue;
   const bool one = tiles <= kDtWaves;
+  if (a.groups > 1 && tiles * a.groups > kDtWaves) return hipErrorInvalidValue;
+  if (a.groups == 2) return a.C2 <= 32 ? launch_dw_tiles_as<T, MULT, 1, 2, 2>(a, stream) : launch_dw_tiles_as<T, MULT, 1, 4, 2>(a, stream);
+  if (a.groups == 4) return a.C2 <= 32 ? launch_dw_tiles_as<T, MULT, 1, 2, 4>(a, stream) : launch_dw_tiles_as<T, MULT, 1, 4, 4>(a, stream);
   if (a.C2 <= 32)
     return one ? launch_dw_tiles_as<T, MULT, 1, 2>(a, stream) : launch_dw_tiles_as<T, MULT, 2, 2>(a, stream);
   return one ? launch_dw_tiles_as<T, MULT, 1, 4>(a, stream) : launch_dw_tiles_as<T, MULT, 2, 4>(a, stream);

@@ -1008,6 +1008,26 @@ def test_depthwise_chain_on_row_tiles(oracle, case, dtype):
     assert np.array_equal(y.float().cpu().numpy(), got) and bool(torch.isnan(out[0]))
 
 
+@pytest.mark.parametrize("case,waves", [
+    # waves to a tile of 16 pixels: where a workgroup has at most 64 pixels, 32
+    ((1, 24, 3, 32, 16, 1, 64), 4),   # all of 32 pixels; half of the second chunk's channels
+    ((2, 17, 5, 33, 16, 1, 33), 2),   # one pixel in the third tile, one channel in the second chunk
+    ((1, 16, 4, 64, 16, 1, 32), 2),
+    ((1, 3, 9, 62, 16, 2, 8), 4),     # stride 2, fewer channels than the waves share out
+    ((1, 40, 2, 31, 1, 1, 40), 4),    # a second chunk of 8 channels
+    ((2, 8, 3, 61, 1, 1, 64), 2),
+    ((1, 64, 1, 16, 1, 1, 20), 4),    # sums that need more LDS than a chunk
+])
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+def test_depthwise_chain_on_row_tiles_with_channels_shared_out(oracle, case, waves, dtype):
+    N, C0, H, W, factor, stride, C2 = case
+    x, w1, w2 = (torch.empty(s, dtype=TORCH_DTYPES[dtype], device="cuda") for s in ((N, C0, H, W), (factor * C0, 1, 3, 3), (C2, factor * C0, 1, 1)))
+    y = torch.empty((N, C2, (H - 1) // stride + 1, (W - 1) // stride + 1), dtype=x.dtype, device="cuda")
+    tile = chain.select_tile(chain.conv_chain_desc(x, w1, w2, y, 1, stride, 0, 1, "cast", False, C0, tile_variant=4100))
+    assert 128 // (2 * waves) < tile.block_m <= 128 // waves or (waves == 4 and tile.block_m <= 32)
+    test_depthwise_chain_on_row_tiles(oracle, case, dtype)
+
+
 CASES_TILES13 = [
     # N, C0, H, W, C1, C2: conv1x1 -> conv3x3 on tiles of whole output rows
     (1, 8, 1, 8, 8, 8),        # a single image row of the narrowest image
