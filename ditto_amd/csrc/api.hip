@@ -57,6 +57,7 @@ struct BmmPlan {
   int split_dt = 0, split_rt = 0;  // fp chains on few rows: column tiles and row tiles of the key-splitting kernel (0: none)
   int rows_dt = 0, rows_nw = 0;  // fp chains: column tiles and waves of the kernel of 32 rows per wave and short tiles (0: none)
   int units_rt = 0, slices = 0, slice_blocks = 0;  // int8 chain on few rows: row tiles, slices of the columns, blocks of 64 of each (0: none)
+  int f32_width = 0, f32_cols = 1;  // fp32 chain on few rows: columns of a workgroup (0: all), workgroups that share them out
   int nb3 = 0, nb = 0;  // 16x16x32-MFMA kernel: row blocks of 384 rows / row blocks in all, per batch entry
   ditto_tile_param tile;
 };
@@ -496,14 +497,16 @@ int plan_bmm_rules(const ditto_bmm_chain_desc* d, BmmPlan* plan, int cus) {
     // tiles do not fit the registers.
     auto rounds = [&](int rows) { return (((d->M + rows - 1) / rows) * d->batch + cus - 1) / cus; };
     plan->qt = !f64 && (d->K > 80 || d->N > 80 || (double)rounds(16) < 1.8 * (double)rounds(32)) ? 1 : 2;
+    plan->f32_width = f64 || plan->qt != 1 ? 0 : ditto::f32_chain_width((int)d->K, (int)d->N, ((d->M + 15) / 16) * d->batch, cus);
+    plan->f32_cols = plan->f32_width ? (int)((d->N + plan->f32_width - 1) / plan->f32_width) : 1;
     ditto_tile_param& t = plan->tile;
     t.block_threads = f64 ? 256 : 512;
     t.block_m = 16 * plan->qt;
-    t.block_n = (int)d->N;
+    t.block_n = plan->f32_width ? plan->f32_width : (int)d->N;
     t.head_pad = 0;
     t.block_l = f64 ? 32 : 128;
-    t.lds_bytes = ditto::f32_chain_lds_bytes_host((int)d->K, (int)d->N, f64, plan->qt);
-    t.grid_x = (int)(((d->M + t.block_m - 1) / t.block_m) * d->batch);
+    t.lds_bytes = ditto::f32_chain_lds_bytes_host((int)d->K, (int)d->N, f64, plan->qt, plan->f32_width);
+    t.grid_x = (int)(((d->M + t.block_m - 1) / t.block_m) * d->batch * plan->f32_cols);
     t.grid_y = t.grid_z = 1;
     t.variant = f64 ? 1001 : 1000;  // fp32 (MFMA) / fp64 (FMA) chain
     return DITTO_OK;
@@ -1579,6 +1582,8 @@ int ditto_bmm_chain_run(const ditto_bmm_chain_desc* d, const void* a, const void
     args.batch = (int)d->batch;
     args.mblocks = (int)((d->M + plan.tile.block_m - 1) / plan.tile.block_m);
     args.row_tiles = plan.qt;
+    args.width = plan.f32_width;
+    args.col_blocks = plan.f32_cols;
     args.b_lk = d->b_layout == DITTO_B_LK;
     args.relu = d->inter_op == DITTO_INTER_RELU;
     args.relu_out = d->relu_out;

@@ -14,6 +14,8 @@ struct F32ChainArgs {
   int M, N, K, L, batch;
   int mblocks;    // workgroups per batch entry
   int row_tiles;  // fp32: rows of a workgroup / 16 (1 or 2); fp64: workgroups own 32 rows
+  int width;      // fp32: columns of F a workgroup owns: 0 (all), 64, 32 or 16
+  int col_blocks; // fp32: workgroups that share out the columns of a block of rows
   int b_lk;     // B stored [L][K]
   int relu;
   int relu_out;  // ReLU on the output
@@ -23,7 +25,8 @@ struct F32ChainArgs {
   unsigned block0;  // fp32: workgroups in front of this launch's (filled by the launcher)
 };
 
-int f32_chain_lds_bytes_host(int K, int N, int f64, int row_tiles);
+int f32_chain_lds_bytes_host(int K, int N, int f64, int row_tiles, int width);
+int f32_chain_width(int K, int N, long long row_blocks, int cus);
 int f32_chain_max_dim();  // largest K and N the kernels take
 hipError_t launch_gemm_chain_f32(const F32ChainArgs& args, hipStream_t stream);
 

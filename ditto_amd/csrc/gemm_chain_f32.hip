@@ -36,12 +36,19 @@ constexpr unsigned kLaunchBlocks = 1u << 22;  // most fp32 workgroups of one lau
 // fp32 FMAs over LDS tiles that this kernel replaced took 178 us (one row per eight threads, an LDS read per operand of
 // every FMA); 64 x 512 x 512 x 64: 52.7 us, 82 TFLOP/s; 4 x 1024 x 1024 x 128: 28.9 us, 74 TFLOP/s.
 //
+// With few rows the matrix pipes of a few compute units are the bound and the others idle: workgroups then own W = 64, 32 or 16
+// of the columns of F as well (0: all), computing the first product once each, 8 DT MFMAs a step down to 4 DT + W / 4: softmax
+// 3 x 132 x 756 x 80 13.5 -> 9.8 us, 11 x 79 x 609 x 128 19.5 -> 15.7, 1 x 180 x 387 x 80 8.9 -> 7.0.  As narrow as leaves every
+// workgroup a compute unit: beyond that the repeated first products cost what the others save.
 // DT: column tiles of 16 that K and N are padded to.  EXACT: K = N = 16 DT and every row starts on a 16-byte boundary;
 // otherwise elements are loaded one by one and columns past K or N are zeros.
-template <int DT, int RT, bool EXACT, bool KL, bool SM>
+template <int DT, int RT, bool EXACT, bool KL, bool SM, int W>
 __global__ __launch_bounds__(64 * kWaves) void gemm_chain_f32_kernel(F32ChainArgs p) {
-  constexpr int G = DT / 4, REM = DT % 4;  // column groups of 64 (16-byte pieces), column tiles beyond them
-  constexpr int ORS = 16 * DT + 4;         // row stride of a parked partial result, floats
+  constexpr int PW = W == 0 || W == 64 ? 4 : W / 16;                   // columns of a lane's piece of a row
+  constexpr int G = W == 0 ? DT / 4 : 1, REM = W == 0 ? DT % 4 : 0;  // column groups of 16 PW, column tiles beyond them
+  constexpr int NT = PW * G + REM;                                     // column tiles of the workgroup
+  constexpr int ORS = 16 * NT + 4;         // row stride of a parked partial result, floats
+  typedef __attribute__((ext_vector_type(PW == 1 ? 2 : PW))) float Piece;
   static_assert(REM <= 1, "columns beyond the groups of 64: at most one tile of 16");
   extern __shared__ __attribute__((aligned(16))) float smem_f32[];
   float* const Om = smem_f32;                              // [wave][16 RT][ORS]
@@ -49,7 +56,13 @@ __global__ __launch_bounds__(64 * kWaves) void gemm_chain_f32_kernel(F32ChainArg
   int* const again = reinterpret_cast<int*>(Ml + kWaves * 16 * RT * 2);  // a result is not finite
   const int K = p.K, N = p.N, L = p.L, M = p.M;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, c = lane & 15, q = lane >> 4;
-  const unsigned bid = p.block0 + xcd_remap(blockIdx.x, gridDim.x);  // the row blocks of a batch entry read the same B and C
+  unsigned bid = p.block0 + xcd_remap(blockIdx.x, gridDim.x);  // the row blocks of a batch entry read the same B and C
+  int col0 = 0;  // the workgroup's first column
+  if constexpr (W > 0) {
+    const unsigned rows = bid / (unsigned)p.col_blocks;
+    col0 = W * (int)(bid - rows * (unsigned)p.col_blocks);
+    bid = rows;
+  }
   const int bz = bid / (unsigned)p.mblocks, m0 = (bid - bz * (unsigned)p.mblocks) * 16 * RT;
   const float* const Ag = static_cast<const float*>(p.a) + (long long)bz * p.a_bs;
   const float* const Bg = static_cast<const float*>(p.b) + (long long)bz * p.b_bs;
@@ -66,7 +79,7 @@ __global__ __launch_bounds__(64 * kWaves) void gemm_chain_f32_kernel(F32ChainArg
   };
 
   const int nsteps = (L + 15) / 16;
-  f32x4 kf[DT], qf[RT][DT], vf[4][G + REM], o[RT][DT];
+  f32x4 kf[DT], qf[RT][DT], vf[4][G + REM], o[RT][NT];
   auto load_k = [&](int step) __attribute__((always_inline)) {
     const int key = min(16 * step + c, L - 1);  // keys past the last are masked below
 #pragma unroll
@@ -103,7 +116,7 @@ __global__ __launch_bounds__(64 * kWaves) void gemm_chain_f32_kernel(F32ChainArg
     for (int rt = 0; rt < RT; ++rt) {
       ref[rt] = kNoKeyYet, lsum[rt] = 0.f;
 #pragma unroll
-      for (int j = 0; j < DT; ++j) o[rt][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+      for (int j = 0; j < NT; ++j) o[rt][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
     }
     for (int step = w; step < nsteps; step += kWaves) {
       const int key0 = 16 * step;
@@ -111,7 +124,18 @@ __global__ __launch_bounds__(64 * kWaves) void gemm_chain_f32_kernel(F32ChainArg
       for (int r = 0; r < 4; ++r) {
         const float* const row = Cg + (long long)min(key0 + 4 * q + r, L - 1) * p.c_rs;
 #pragma unroll
-        for (int g = 0; g < G; ++g) vf[r][g] = load4(row, 64 * g + 4 * c, N);
+        for (int g = 0; g < G; ++g) {
+          const int n = col0 + 16 * PW * g + PW * c;
+          if constexpr (PW == 4) {
+            vf[r][g] = load4(row, n, N);
+          } else if constexpr (PW == 2 && EXACT) {
+            const Piece two = *reinterpret_cast<const Piece*>(row + n);
+            vf[r][g][0] = two[0], vf[r][g][1] = two[1];
+          } else {
+#pragma unroll
+            for (int t = 0; t < PW; ++t) vf[r][g][t] = EXACT || n + t < N ? row[n + t] : 0.f;
+          }
+        }
         if constexpr (REM > 0) vf[r][G][0] = EXACT || 64 * G + c < N ? row[64 * G + c] : 0.f;
       }
       f32x4 st[RT];
@@ -146,7 +170,7 @@ __global__ __launch_bounds__(64 * kWaves) void gemm_chain_f32_kernel(F32ChainArg
             ref[rt] = up;
             lsum[rt] *= alpha;
 #pragma unroll
-            for (int j = 0; j < DT; ++j) o[rt][j] *= alpha;
+            for (int j = 0; j < NT; ++j) o[rt][j] *= alpha;
           }
         }
 #pragma unroll
@@ -175,22 +199,30 @@ __global__ __launch_bounds__(64 * kWaves) void gemm_chain_f32_kernel(F32ChainArg
 #pragma unroll
       for (int r = 0; r < 4; ++r)
 #pragma unroll
-        for (int j = 0; j < DT; ++j)
+        for (int j = 0; j < NT; ++j)
 #pragma unroll
           for (int rt = 0; rt < RT; ++rt)
-            o[rt][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[r][j / 4][j % 4], st[rt][r], o[rt][j], 0, 0, 0);
+            o[rt][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[r][j / PW][j % PW], st[rt][r], o[rt][j], 0, 0, 0);
     }
 
-    // lane (c, q) holds of row c: columns 64 g + 16 q + 4 r + t in register r of tile 4 g + t, and 64 G + 4 q + r in the last
+    // lane (c, q) holds of row c: columns PW (16 g + 4 q + r) + t in register r of tile PW g + t, and 64 G + 4 q + r in the last
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
       float* const row = Om + (w * 16 * RT + 16 * rt + c) * ORS;
 #pragma unroll
-      for (int g = 0; g < G; ++g)
+      for (int g = 0; g < G; ++g) {
+        if constexpr (PW == 1) {
+          *reinterpret_cast<f32x4*>(row + 16 * g + 4 * q) = o[rt][g];
+        } else {
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-          *reinterpret_cast<f32x4*>(row + 64 * g + 16 * q + 4 * r) =
-              (f32x4){o[rt][4 * g][r], o[rt][4 * g + 1][r], o[rt][4 * g + 2][r], o[rt][4 * g + 3][r]};
+          for (int r = 0; r < 4; ++r) {
+            Piece piece;
+#pragma unroll
+            for (int t = 0; t < PW; ++t) piece[t] = o[rt][PW * g + t][r];
+            *reinterpret_cast<Piece*>(row + PW * (16 * g + 4 * q + r)) = piece;
+          }
+        }
+      }
       if constexpr (REM > 0) *reinterpret_cast<f32x4*>(row + 64 * G + 4 * q) = o[rt][4 * G];
       if constexpr (SM) {
         float s = lsum[rt];
@@ -204,8 +236,8 @@ __global__ __launch_bounds__(64 * kWaves) void gemm_chain_f32_kernel(F32ChainArg
     }
     wg_sync();
     bool bad = false;
-    for (int e = tid; e < 16 * RT * 4 * DT; e += 64 * kWaves) {
-      const int row = e / (4 * DT), n0 = 4 * (e - row * 4 * DT);
+    for (int e = tid; e < 16 * RT * 4 * NT; e += 64 * kWaves) {
+      const int row = e / (4 * NT), n0 = 4 * (e - row * 4 * NT);
       float wt[kWaves];
       if constexpr (SM) {
         float mx = kNoKeyYet, s = 0.f;
@@ -234,13 +266,13 @@ __global__ __launch_bounds__(64 * kWaves) void gemm_chain_f32_kernel(F32ChainArg
 #pragma unroll
         for (int t = 0; t < 4; ++t) x[t] = fmaxf(x[t], 0.f);
       if (m0 + row < M) {
-        float* const dst = Fg + (long long)(m0 + row) * p.f_rs + n0;
+        float* const dst = Fg + (long long)(m0 + row) * p.f_rs + col0 + n0;
         if constexpr (EXACT) {
           *reinterpret_cast<f32x4*>(dst) = x;
         } else {
 #pragma unroll
           for (int t = 0; t < 4; ++t)
-            if (n0 + t < N) dst[t] = x[t];
+            if (col0 + n0 + t < N) dst[t] = x[t];
         }
       }
 #pragma unroll
@@ -377,9 +409,16 @@ static int f32_tiles(int K, int N) {  // column tiles of 16 the fp32 kernel is b
   const int d = K > N ? K : N;
   return d <= 64 ? 4 : d <= 80 ? 5 : 8;
 }
-int f32_chain_lds_bytes_host(int K, int N, int f64, int rt) {
+int f32_chain_lds_bytes_host(int K, int N, int f64, int rt, int width) {
   if (f64) return f64_chain_lds_bytes(K, N);
-  return kWaves * 16 * rt * (16 * f32_tiles(K, N) + 4 + 2) * (int)sizeof(float) + 16;
+  return kWaves * 16 * rt * ((width ? width : 16 * f32_tiles(K, N)) + 4 + 2) * (int)sizeof(float) + 16;
+}
+// The columns a workgroup owns, 0 for all: the fewest that leave every workgroup a compute unit of its own.
+int f32_chain_width(int K, int N, long long row_blocks, int cus) {
+  const int dt = f32_tiles(K, N);
+  for (int w = 16; w <= 64; w *= 2)
+    if (w < 16 * dt && (dt != 5 || w == 16) && row_blocks * ((N + w - 1) / w) <= cus) return w;
+  return 0;
 }
 
 template <typename Tag, typename Kernel>
@@ -395,7 +434,7 @@ static hipError_t launch_with_lds(Kernel kernel, unsigned threads, int lds, cons
   }
   // A launch holds fewer than 2^32 work items, which sixteen rows per 512 threads reach at 134 million rows: such a grid goes
   // out in pieces (the fp64 kernel's 256 threads own 32 rows; it takes what one launch holds).
-  const unsigned long long blocks = (unsigned long long)args.mblocks * (unsigned long long)args.batch;
+  const unsigned long long blocks = (unsigned long long)args.mblocks * (unsigned long long)args.batch * (unsigned)(args.f64 ? 1 : args.col_blocks);
   if (blocks > 0x7fffffffull) return hipErrorInvalidConfiguration;
   const unsigned long long most = args.f64 ? blocks : kLaunchBlocks;
   F32ChainArgs piece = args;
@@ -407,25 +446,36 @@ static hipError_t launch_with_lds(Kernel kernel, unsigned threads, int lds, cons
   return e;
 }
 
-template <int DT, int RT, bool EXACT, bool KL, bool SM>
+template <int DT, int RT, bool EXACT, bool KL, bool SM, int W>
 struct F32Tag {};
 
-template <int DT, int RT, bool EXACT>
+template <int DT, int RT, bool EXACT, int W>
 static hipError_t launch_f32(const F32ChainArgs& a, hipStream_t stream) {
-  const int lds = f32_chain_lds_bytes_host(a.K, a.N, 0, RT), threads = 64 * kWaves;
+  const int lds = f32_chain_lds_bytes_host(a.K, a.N, 0, RT, W), threads = 64 * kWaves;
   if (a.softmax)
-    return a.b_lk ? launch_with_lds<F32Tag<DT, RT, EXACT, false, true>>(gemm_chain_f32_kernel<DT, RT, EXACT, false, true>, threads, lds, a, stream)
-                  : launch_with_lds<F32Tag<DT, RT, EXACT, true, true>>(gemm_chain_f32_kernel<DT, RT, EXACT, true, true>, threads, lds, a, stream);
-  return a.b_lk ? launch_with_lds<F32Tag<DT, RT, EXACT, false, false>>(gemm_chain_f32_kernel<DT, RT, EXACT, false, false>, threads, lds, a, stream)
-                : launch_with_lds<F32Tag<DT, RT, EXACT, true, false>>(gemm_chain_f32_kernel<DT, RT, EXACT, true, false>, threads, lds, a, stream);
+    return a.b_lk ? launch_with_lds<F32Tag<DT, RT, EXACT, false, true, W>>(gemm_chain_f32_kernel<DT, RT, EXACT, false, true, W>, threads, lds, a, stream)
+                  : launch_with_lds<F32Tag<DT, RT, EXACT, true, true, W>>(gemm_chain_f32_kernel<DT, RT, EXACT, true, true, W>, threads, lds, a, stream);
+  return a.b_lk ? launch_with_lds<F32Tag<DT, RT, EXACT, false, false, W>>(gemm_chain_f32_kernel<DT, RT, EXACT, false, false, W>, threads, lds, a, stream)
+                : launch_with_lds<F32Tag<DT, RT, EXACT, true, false, W>>(gemm_chain_f32_kernel<DT, RT, EXACT, true, false, W>, threads, lds, a, stream);
+}
+
+template <int DT, bool EXACT>
+static hipError_t launch_f32_rows(const F32ChainArgs& a, hipStream_t stream) {
+  if constexpr (DT <= 5)
+    if (a.row_tiles == 2 && a.width == 0) return launch_f32<DT, 2, EXACT, 0>(a, stream);
+  if (a.row_tiles != 1) return hipErrorInvalidValue;
+  if (a.width == 0) return launch_f32<DT, 1, EXACT, 0>(a, stream);
+  if (a.width == 16) return launch_f32<DT, 1, EXACT, 16>(a, stream);
+  if constexpr (DT != 5)
+    if (a.width == 32) return launch_f32<DT, 1, EXACT, 32>(a, stream);
+  if constexpr (DT == 8)
+    if (a.width == 64) return launch_f32<DT, 1, EXACT, 64>(a, stream);
+  return hipErrorInvalidValue;
 }
 
 template <int DT>
 static hipError_t launch_f32_rows(const F32ChainArgs& a, bool exact, hipStream_t stream) {
-  if constexpr (DT <= 5)
-    if (a.row_tiles == 2) return exact ? launch_f32<DT, 2, true>(a, stream) : launch_f32<DT, 2, false>(a, stream);
-  if (a.row_tiles != 1) return hipErrorInvalidValue;
-  return exact ? launch_f32<DT, 1, true>(a, stream) : launch_f32<DT, 1, false>(a, stream);
+  return exact ? launch_f32_rows<DT, true>(a, stream) : launch_f32_rows<DT, false>(a, stream);
 }
 
 hipError_t launch_gemm_chain_f32(const F32ChainArgs& a, hipStream_t stream) {

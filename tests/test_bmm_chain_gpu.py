@@ -305,6 +305,20 @@ def test_fp32_chain_at_the_edges_of_its_tiles(oracle, shape, inter):
         assert np.isfinite(got).all() and rel <= 1e-5, (b_layout, mx, rel)
 
 
+@pytest.mark.parametrize("shape,width", [
+    # (batch, M, N, K, L) and the columns of a workgroup: few rows, more of them, whole rows and ragged ones
+    ((1, 33, 64, 64, 40), 16), ((5, 225, 64, 64, 40), 32), ((9, 230, 64, 64, 40), 64), ((5, 225, 50, 60, 40), 32), ((2, 300, 72, 80, 40), 16),
+    ((2, 130, 80, 24, 300), 16), ((2, 250, 128, 128, 40), 16), ((3, 250, 128, 128, 40), 32), ((5, 250, 128, 128, 50), 64),
+    ((5, 250, 100, 120, 50), 64), ((5, 250, 20, 128, 50), 16),
+])
+@pytest.mark.parametrize("inter", ["relu", "softmax"])
+def test_fp32_chain_with_columns_shared_out(oracle, shape, width, inter):
+    batch, M, N, K, L = shape
+    d = chain.bmm_chain_desc(*(torch.empty(batch, *s, device="cuda") for s in ((M, K), (K, L), (L, N), (M, N))), inter, 0.5, 1.0, 0, False)
+    assert chain.select_tile(d).block_n == width
+    test_fp32_chain_at_the_edges_of_its_tiles(oracle, shape, inter)
+
+
 @pytest.mark.parametrize("shape", [(1, 17, 64, 64, 100), (2, 40, 80, 80, 176), (9, 500, 80, 80, 176), (1, 20, 70, 66, 300), (1, 33, 128, 128, 528)])
 @pytest.mark.parametrize("keys", sorted(MASKED_KEYS))
 def test_fp32_chain_on_masked_keys(oracle, shape, keys):
