@@ -33,13 +33,15 @@ FP_SPLIT_VARIANTS = {4: (2041, 2042), 5: (2051, 2052), 8: (2081, 2082)}
 FP_ROWS_VARIANTS = {4: (2144, 2148), 5: (2154, 2158), 8: (2188,)}
 # Beyond these the two were behind at every size measured and are left out: rounds of key-splitting workgroups over the
 # compute units (each pulls all keys for its 16 or 32 rows), keys for 32 rows per wave outside heads of 65 to 80 columns
-# (80 x 1024 x 1024 x 128 68.4 us against 65.4; with softmax at 64 columns at any number, 96 x 512 x 512 13.6 / 10.9)
+# (80 x 1024 x 1024 x 128 68.4 us against 65.4; with softmax at 64 columns the eight-wave form at any number, 1152 x 512 x 512
+# 128 against 107 with four)
 FP_SPLIT_ROUNDS = 4
 FP_ROWS_KEYS = 1024
 
 
-# int8 chain: 8000 + 10 * (row tiles of 32 per workgroup) + depth of the ring of staged weight chunks
-I8_VARIANTS = (8012, 8014, 8022, 8023)
+# int8 chain: 8000 + 10 * (row tiles of 32 per workgroup) + depth of the ring of staged weight chunks; 8100 + row tiles of 16 per
+# workgroup of the kernel for few rows (the library refuses it where the rows are many)
+I8_VARIANTS = (8012, 8014, 8022, 8023, 8101, 8102)
 
 
 class TuneEntry:
@@ -58,7 +60,9 @@ def _fp_variants(desc, groups):
     width = 4 if dmax <= 64 else 5 if dmax <= 80 else 8
     ids = [v for v in FP_SPLIT_VARIANTS[width]
            if -(-desc.M // (16 * (v % 10))) * desc.batch <= FP_SPLIT_ROUNDS * groups]
-    if width == 5 or (desc.L <= FP_ROWS_KEYS and not (width == 4 and desc.inter_op == _lib.INTER_SOFTMAX)):
+    if width == 4 and desc.inter_op == _lib.INTER_SOFTMAX:
+        ids += FP_ROWS_VARIANTS[width][:1]
+    elif width == 5 or desc.L <= FP_ROWS_KEYS:
         ids += FP_ROWS_VARIANTS[width]
     return ids + [(64 if dmax <= 64 else 128) * 10 + q for q in FP_VARIANT_CODES]
 

@@ -227,6 +227,24 @@ def test_tile_variant_space_and_analytic_filter():
     assert ci.workload_key(big) != ci.workload_key(small)
 
 
+def test_tile_variant_space_of_the_kernels_for_many_rows_of_64_columns_and_few_int8_rows():
+    import torch
+    from ditto_amd import chain
+    from ditto_amd.auto_schedule.schedulers import chimera_integrate as ci
+
+    q = torch.zeros(30, 512, 64, dtype=torch.float16)
+    ids = [t["variant"] for t in ci.make_tile_variant_space(chain.bmm_chain_desc(q, q.transpose(1, 2), q, q, "softmax", 0.1))]
+    assert 2144 in ids and 2148 not in ids
+
+    def i8(M):
+        z = lambda *s: torch.zeros(1, *s, dtype=torch.int8)
+        return chain.bmm_chain_desc(z(M, 240), z(240, 112), z(112, 928), torch.zeros(1, M, 928, dtype=torch.int32), "requant", 1.0, 0.5)
+
+    few = ci.make_tile_variant_space(i8(688))
+    assert {8101, 8102} <= {t["variant"] for t in few}
+    assert all(0 < ci.evaluate_param_hip(i8(688), t) < 1e10 for t in few)
+
+
 @pytest.mark.parametrize("shape", [
     # (batch, M, L, D, inter): ViT-Huge heads of 80 on few and on many rows, 128 columns on short sequences, few rows of 64,
     # without softmax on a large grid, B stored [K][L]
