@@ -532,16 +532,23 @@ int plan_bmm_rules(const ditto_bmm_chain_desc* d, BmmPlan* plan, int cus) {
     if ((d->M + 64) * d->a_row_stride >= 0x7fffffffLL || d->K * d->b_row_stride >= 0x7fffffffLL ||
         Lp * d->c_row_stride >= 0x7fffffffLL)
       return fail(DITTO_EUNSUPPORTED, "a batch entry of A, B or C exceeds 2 GiB");
+    // Compute units that would be idle take a share of the columns of the result, in blocks of 256: their workgroups repeat the
+    // first product (2014 x 96 x 192 x 624 7.8 -> 5.9 us with three to a row block, 680 x 736 x 384 x 1024 15.9 -> 12.4).  Beyond a
+    // workgroup to a compute unit that costs more than it saves (5020 x 352 x 224 x 448 7.2, 10.7 with two).
+    const long long blocks256 = (d->N + 255) / 256;
+    const long long rows32 = ((d->M + 31) / 32) * d->batch, most_slices = std::min(blocks256, std::max(1LL, cus / rows32));
+    const long long blocks_per_slice = (blocks256 + most_slices - 1) / most_slices;
     // Few rows: the kernel whose waves take units of 64 x 64 weights, with as many workgroups to a row block (slices of its
     // columns) as pay.  Prices in us per launch, least squares over 300 random shapes (64 - 8192 rows, K and N 16 - 1024, L 16 -
-    // 512) with 1 - 6 slices, root mean square error 5 %, up to one round of the other kernel's workgroups; where this one is
-    // priced 3 % lower it takes 0.79 of the time in the mean (224 x 48 x 208 x 928 7.8 -> 4.8 us, 256 x 912 x 96 x 800 10.4 ->
-    // 6.2, 1120 x 32 x 48 x 16 4.8 -> 3.8), the worst of 244 1.26.
+    // 512) with 1 - 6 slices, root mean square error 5 %, the other kernel's over 800, 4 %, up to one round of its workgroups; by
+    // these prices the faster of the two is missed by 0.2 % in the mean, the worst of 640 1.11 (224 x 48 x 208 x 928 7.8 -> 4.8 us,
+    // 256 x 912 x 96 x 800 10.4 -> 6.2, 1120 x 32 x 48 x 16 4.8 -> 3.8).
     {
       const double nl = (double)((d->L + 63) / 64), units1 = nl * (double)((d->K + 63) / 64) / 8;
-      const long long nbt = (d->N + 63) / 64, rows32 = ((d->M + 31) / 32) * d->batch, Lc = Lp / 256;
-      const long long chunks = Lc * ((d->K + 127) / 128) + 2 * Lc * ((d->N + 255) / 256);
-      double best = 0.97 * (3.61 + 0.413 * chunks + 0.444e-6 * (double)(d->batch * d->M) * (double)d->N);
+      const long long nbt = (d->N + 63) / 64;
+      const double chunks1 = (double)(Lp / 256 * ((d->K + 127) / 128)), chunks2 = (double)((d->L + 127) / 128 * blocks_per_slice);
+      double best = 0.98 * (3.90 + 0.355 * chunks1 + 0.474 * chunks2 + 0.357e-6 * (double)(d->batch * d->M) * (double)d->N +
+                            0.289 * (double)(rows32 * ((blocks256 + blocks_per_slice - 1) / blocks_per_slice)) / cus);
       if (d->tile_variant == 8101 || d->tile_variant == 8102) best = 1e30;
       for (int rt = 1; rt <= 2; ++rt) {
         if (d->tile_variant == 0 ? rows32 > cus : d->tile_variant != 8100 + rt) continue;
@@ -592,6 +599,8 @@ int plan_bmm_rules(const ditto_bmm_chain_desc* d, BmmPlan* plan, int cus) {
                     d->tile_variant);
       mt = fm, nst = fn;
     }
+    plan->slice_blocks = (int)(mt == 1 ? blocks_per_slice : blocks256);
+    plan->slices = (int)((blocks256 + plan->slice_blocks - 1) / plan->slice_blocks);
     const int lds = ditto::i8_chain_lds_bytes_host((int)Lp, mt, nst);
     if (lds > 160 * 1024)
       return fail(DITTO_EUNSUPPORTED, "L=%lld: the requantised row block does not fit in LDS", (long long)d->L);
@@ -602,10 +611,10 @@ int plan_bmm_rules(const ditto_bmm_chain_desc* d, BmmPlan* plan, int cus) {
     t.block_threads = ditto::i8_chain_threads();
     t.block_m = 32 * mt;
     t.block_l = (int)Lp;
-    t.block_n = 256;
+    t.block_n = 256 * plan->slice_blocks;
     t.head_pad = 0;
     t.lds_bytes = lds;
-    t.grid_x = (int)(((d->M + 32 * mt - 1) / (32 * mt)) * d->batch);
+    t.grid_x = (int)(((d->M + 32 * mt - 1) / (32 * mt)) * d->batch * plan->slices);
     t.grid_y = t.grid_z = 1;
     t.variant = 8000 + 10 * mt + nst;  // int8 chain: 8000 + 10 * (row tiles of 32) + ring depth
     return DITTO_OK;

@@ -20,7 +20,7 @@ struct I8ChainArgs {
   int M, N, K, L, batch;
   int mblocks;
   int Lp;  // L rounded up to the weight-chunk width
-  int slices, slice_blocks;  // unit kernel: workgroups that share a row block's columns of the result, blocks of 64 columns of each
+  int slices, slice_blocks;  // workgroups that share a row block's columns of the result, blocks of 64 (chunk kernel: 256) columns of each
 };
 
 // dynamic LDS bytes of the kernel for a padded L, mt = 1|2 row tiles of 32 per workgroup and a

@@ -30,6 +30,11 @@
 // compute waves: barrier, consume chunk c).  Tiles are stored unpadded; 32-byte column groups (weights)
 // and 16-byte chunks (A) are XOR-swizzled by row on the global-address side so that the
 // transposing reads and the 16-byte row reads are bank-conflict free.
+//
+// Few rows leave compute units idle: workgroups then share out the 256-column blocks of D of a row block (slices) and each
+// repeats phase 1.  Rows of D past L, which is padded to whole blocks of B's columns in LDS, are walked only to the end of a
+// chunk: 2192 x 448 x 48 x 80 and 280 x 160 x 48 x 976 take one chunk a block instead of two (8.4 -> 7.9 us the latter, and 5.7
+// with four workgroups to a row block).
 #include "common.h"
 #include "gemm_chain_i8.h"
 
@@ -67,7 +72,8 @@ __device__ __forceinline__ int requant_i8(int acc, float s) {
   return (int)v;
 }
 
-template <int MT, int NST>
+// (SLICED: the workgroups of a row block share out its columns; a run-time switch cost the others 0.1 - 0.4 us)
+template <int MT, int NST, bool SLICED>
 __global__ __launch_bounds__(64 * i8::NW) void gemm_chain_i8_kernel(I8ChainArgs p) {
 #if defined(__HIP_DEVICE_COMPILE__)
   using namespace i8;
@@ -85,8 +91,10 @@ __global__ __launch_bounds__(64 * i8::NW) void gemm_chain_i8_kernel(I8ChainArgs 
   const int i16 = lane & 15, h = (lane >> 4) & 1;
   // (One batch entry: all workgroups read the same B and C, there is nothing to group; ragged grids keep the round-robin order,
   // 2000 x 144 x 128 x 848 8.2 us against 8.5.)
-  const unsigned lid = (gridDim.x & 7) && gridDim.x == (unsigned)p.mblocks ? blockIdx.x : xcd_remap(blockIdx.x, gridDim.x);
-  const int mb = lid % p.mblocks, bz = lid / p.mblocks;
+  const unsigned lid = (gridDim.x & 7) && p.batch == 1 ? blockIdx.x : xcd_remap(blockIdx.x, gridDim.x);
+  const unsigned rb = SLICED ? lid / (unsigned)p.slices : lid;
+  const int slice = SLICED ? (int)(lid - rb * (unsigned)p.slices) : 0;
+  const int mb = rb % p.mblocks, bz = rb / p.mblocks;
   const int m0 = mb * BM;
   const int M = p.M, N = p.N, K = p.K, L = p.L, Lp = p.Lp;
   const int8_t* Ag = p.a + (long long)bz * p.a_bs;
@@ -99,16 +107,18 @@ __global__ __launch_bounds__(64 * i8::NW) void gemm_chain_i8_kernel(I8ChainArgs 
   const unsigned lds0 = (unsigned)(size_t)(DITTO_LDS char*)smem_raw;
 
   const int nk = (K + KC - 1) / KC;  // chunks per 256-column block of B
-  const int nl = Lp / KC;            // chunks per 256-column block of D
-  const int nlc = Lp / WC, nnc = (N + WC - 1) / WC;
+  const int nl = (L + KC - 1) / KC;  // chunks per 256-column block of D
+  const int nc0 = SLICED ? slice * p.slice_blocks : 0;  // the workgroup's first 256-column block of D
+  const int nlc = Lp / WC, nnc = SLICED ? min((N + WC - 1) / WC - nc0, p.slice_blocks) : (N + WC - 1) / WC;
   const int NC1 = nlc * nk;
   const int NC = NC1 + nnc * nl;
   // All workgroups walk the same B and D.  Started together on the same chunk they would all hit
   // the same few L2 channels at the same time, so each workgroup starts its walk at a different
   // chunk: the contraction order and the column-block order are rotated by the workgroup index
   // (integer accumulation is exact in any order).
-  const int rot_k = mb % nk, rot_lc = (mb / nk) % nlc;
-  const int rot_l = mb % nl, rot_nc = (mb / nl) % nnc;
+  const int turn = SLICED ? mb * p.slices + slice : mb;
+  const int rot_k = turn % nk, rot_lc = (turn / nk) % nlc;
+  const int rot_l = turn % nl, rot_nc = (turn / nl) % nnc;
   auto rot = [](int i, int r, int n) __attribute__((always_inline)) { return i + r >= n ? i + r - n : i + r; };
 
   if (wave >= NCW) {
@@ -162,10 +172,9 @@ __global__ __launch_bounds__(64 * i8::NW) void gemm_chain_i8_kernel(I8ChainArgs 
           if (NAI * pw + q < 4 * MT)
             lds_dma_16(ra, kb * KC + KC > K ? av_m[q] : av[q], lds0 + i_stage * STAGE + WBYTES + 1024 * (NAI * pw + q));
       } else {
-        const int lb = rot(i_inner, rot_l, nl), cb = rot(i_outer, rot_nc, nnc);
+        const int lb = rot(i_inner, rot_l, nl), cb = nc0 + rot(i_outer, rot_nc, nnc);
         const unsigned off = (unsigned)(lb * KC) * (unsigned)p.d_rs + cb * WC;
-        // row blocks past L (L is padded to a multiple of 256 here) lie entirely out of range
-        const i32x4 rs = make_rsrc_uniform(Dg + off, off < d_bytes ? d_bytes - off : 0u);
+        const i32x4 rs = make_rsrc_uniform(Dg + off, d_bytes - off);
         const bool edge = cb * WC + WC > N;
 #pragma unroll
         for (int q = 0; q < NWI; ++q) lds_dma_16(rs, edge ? wv_dm[q] : wv_d[q], sbase + 1024 * q);
@@ -305,7 +314,7 @@ __global__ __launch_bounds__(64 * i8::NW) void gemm_chain_i8_kernel(I8ChainArgs 
       }
       // acc[nt][mt][r] = E[m][n], m = m0 + 32mt + 8(r/4) + 4g + r%4, n = nc + 32(CTW*wave + nt) + ln:
       // the 32 lanes of a half-wave write 128 contiguous bytes of one output row
-      const int nc = rot(ob, rot_nc, nnc) * WC;
+      const int nc = (nc0 + rot(ob, rot_nc, nnc)) * WC;
       if (p.out_i8) {
         // one byte per result: the 32 lanes of a half-wave write 32 contiguous bytes of one output row
         int8_t* const E8 = reinterpret_cast<int8_t*>(p.e) + (long long)bz * p.e_bs;
@@ -594,10 +603,10 @@ hipError_t launch_gemm_chain_i8_units(const I8ChainArgs& args, int rt, hipStream
 int i8_chain_threads() { return 64 * i8::NW; }
 int i8_chain_lds_bytes_host(int Lp, int mt, int nst) { return i8_chain_lds_bytes(Lp, mt, nst); }
 
-template <int MT, int NST>
+template <int MT, int NST, bool SLICED = false>
 static hipError_t launch_i8(const I8ChainArgs& args, hipStream_t stream) {
   const int lds = i8_chain_lds_bytes(args.Lp, MT, NST);
-  auto kern = gemm_chain_i8_kernel<MT, NST>;
+  auto kern = gemm_chain_i8_kernel<MT, NST, SLICED>;
   static thread_local int configured_dev = -1;
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
@@ -607,14 +616,15 @@ static hipError_t launch_i8(const I8ChainArgs& args, hipStream_t stream) {
     if (e != hipSuccess) return e;
     configured_dev = dev;
   }
-  const unsigned grid = (unsigned)args.mblocks * (unsigned)args.batch;
+  const unsigned grid = (unsigned)args.mblocks * (unsigned)args.batch * (SLICED ? (unsigned)args.slices : 1u);
   hipLaunchKernelGGL(kern, dim3(grid), dim3(64 * i8::NW), lds, stream, args);
   return hipGetLastError();
 }
 
 hipError_t launch_gemm_chain_i8(const I8ChainArgs& args, int mt, int nst, hipStream_t stream) {
-  if (mt == 1 && nst == 4) return launch_i8<1, 4>(args, stream);
-  if (mt == 1 && nst == 2) return launch_i8<1, 2>(args, stream);
+  if (args.slices > 1 && mt != 1) return hipErrorInvalidValue;
+  if (mt == 1 && nst == 4) return args.slices > 1 ? launch_i8<1, 4, true>(args, stream) : launch_i8<1, 4>(args, stream);
+  if (mt == 1 && nst == 2) return args.slices > 1 ? launch_i8<1, 2, true>(args, stream) : launch_i8<1, 2>(args, stream);
   if (mt == 2 && nst == 3) return launch_i8<2, 3>(args, stream);
   if (mt == 2 && nst == 2) return launch_i8<2, 2>(args, stream);
   return hipErrorInvalidValue;

@@ -102,6 +102,31 @@ def test_i8_chain_in_units(oracle, M, K, L, N, inter, variant):
         assert np.array_equal(got[:, :N], want.astype(got.dtype)) and (got[:, N:] == -7).all()
 
 
+@pytest.mark.parametrize("batch,M,K,L,N,slices", [
+    # blocks of 256 columns shared out: one each, two and the rest, none to share; rows of D that end in the first, second, third and
+    # fourth chunk of 128
+    (1, 33, 160, 16, 1040, 5), (1, 3200, 48, 144, 528, 2), (2, 70, 144, 272, 800, 4), (1, 8192, 16, 400, 512, 1), (3, 40, 272, 128, 272, 2),
+])
+def test_i8_chain_with_columns_shared_out(oracle, batch, M, K, L, N, slices):
+    A, B, D, scale = oracle.make_i8_chain_inputs(M, K, L, N, seed=M + L)
+    want = oracle.gemm_chain_i8(A, B, D, scale)[0]
+    dev = "cuda:0"
+    ops = [torch.from_numpy(np.stack([x] * batch)).to(dev) for x in (A, B, D)]
+    aux = torch.from_numpy(scale).to(dev)
+    for variant in (8012, 8014, 8022, 8023):
+        e = torch.full((batch, M, N), -7, dtype=torch.int32, device=dev)
+        desc = chain.bmm_chain_desc(*ops, e, "requant", tile_variant=variant)
+        try:
+            tile = chain.select_tile(desc)
+        except ValueError:
+            continue  # (the row block and a ring of that depth do not fit LDS)
+        if variant < 8020:
+            assert tile.grid_x == -(-M // 32) * batch * slices
+        chain.run_bmm_chain(*ops, e, aux=aux, desc=desc)
+        torch.cuda.synchronize()
+        assert all(np.array_equal(e[i].cpu().numpy(), want) for i in range(batch)), variant
+
+
 def test_i8_units_are_planned_on_few_rows_and_agree_over_a_batch(oracle):
     batch, M, K, L, N = 3, 70, 144, 80, 272
     A, B, D, scale = oracle.make_i8_chain_inputs(M, K, L, N, seed=3)
