@@ -73,6 +73,8 @@ UNITS = [
      ["-DDITTO_INST_T=bf16", "-DDITTO_INST_INTER=2", "-DDITTO_INST_NAME=launch_bf16_softmax", *FP_CHAIN_FLAGS]),
     ("fp_split_f16", "bmm_chain_split_inst.hip", ["-DDITTO_INST_T=f16", "-DDITTO_SPLIT_NAME=launch_split_f16", *FP_CHAIN_FLAGS]),
     ("fp_split_bf16", "bmm_chain_split_inst.hip", ["-DDITTO_INST_T=bf16", "-DDITTO_SPLIT_NAME=launch_split_bf16", *FP_CHAIN_FLAGS]),
+    ("fp_split_cols_f16", "bmm_chain_split_cols_inst.hip", ["-DDITTO_INST_T=f16", "-DDITTO_SPLITCOLS_NAME=launch_split_cols_f16", *FP_CHAIN_FLAGS]),
+    ("fp_split_cols_bf16", "bmm_chain_split_cols_inst.hip", ["-DDITTO_INST_T=bf16", "-DDITTO_SPLITCOLS_NAME=launch_split_cols_bf16", *FP_CHAIN_FLAGS]),
     ("fp_rows_f16", "bmm_chain_rows_inst.hip", ["-DDITTO_INST_T=f16", "-DDITTO_ROWS_NAME=launch_rows_f16", *FP_CHAIN_FLAGS]),
     ("fp_rows_bf16", "bmm_chain_rows_inst.hip", ["-DDITTO_INST_T=bf16", "-DDITTO_ROWS_NAME=launch_rows_bf16", *FP_CHAIN_FLAGS]),
     ("fp_sets_f16", "bmm_chain_sets_inst.hip", ["-DDITTO_INST_T=f16", "-DDITTO_SETS_NAME=launch_sets_f16", *FP_CHAIN_FLAGS]),

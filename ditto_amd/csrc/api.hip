@@ -54,7 +54,8 @@ int device_cus() {
 struct BmmPlan {
   int family;  // 0: fp16/bf16 register-resident chain, 1: fp32 chain, 2: int8 requant chain
   int d_pad, qt;  // fp chains: head pad and rows-per-wave code; int8 chain: row tiles and ring depth
-  int split_dt = 0, split_rt = 0;  // fp chains on few rows: column tiles and row tiles of the key-splitting kernel (0: none)
+  // fp chains on few rows: column tiles and row tiles of the key-splitting kernel (0: none), column tiles of a workgroup if not all
+  int split_dt = 0, split_rt = 0, split_ct = 0;
   int rows_dt = 0, rows_nw = 0;  // fp chains: column tiles and waves of the kernel of 32 rows per wave and short tiles (0: none)
   int units_rt = 0, slices = 0, slice_blocks = 0;  // int8 chain on few rows: row tiles, slices of the columns, blocks of 64 of each (0: none)
   int f32_width = 0, f32_cols = 1;  // fp32 chain on few rows: columns of a workgroup (0: all), workgroups that share them out
@@ -365,14 +366,25 @@ int plan_bmm_rules(const ditto_bmm_chain_desc* d, BmmPlan* plan, int cus) {
       if (rt > 0) {
         plan->split_dt = dt, plan->split_rt = rt;
         plan->nb = (int)((d->M + 16 * rt - 1) / (16 * rt));
+        // Half of the columns to a workgroup (32 of 80), or a quarter of 128, where every workgroup still has a compute unit: 0.80 -
+        // 0.97 of the time in 105 of 112 random shapes, two workgroups to one 1.1 - 2.2 times as long.  With B as [K][L], whose
+        // rows of 32 keys are read in pieces of 64 bytes, more than 150 workgroups on long keys wait for L2: 1 x 1399 x 2056 x 64
+        // 7.8 against 9.2 us, 9 x 143 x 1848 x 128 13.0 / 14.0, while 32 x 22 x 1616 x 128 gains (11.2 -> 10.5); and a quarter of
+        // 128 columns is level with half (2 x 224 x 1808 x 128 11.0 / 10.2; B [L][K] 21 x 25 x 944 x 128 7.0 / 7.6).
+        const long long wgs = plan->nb * d->batch;
+        auto blocks = [&](int ct) { return (d->N + 16 * ct - 1) / (16 * ct); };
+        const int half = dt == 8 ? 4 : 2;
+        if (rt == 1 && blocks(half) > 1 && wgs * blocks(half) <= cus && !(kl_b && d->L > 1000 && 5 * wgs * blocks(half) > 3LL * cus))
+          plan->split_ct = dt == 8 && blocks(2) > blocks(4) && wgs * blocks(2) <= cus && (!kl_b || d->L <= 500) ? 2 : half;
+        const int ct = plan->split_ct ? plan->split_ct : dt;
         ditto_tile_param& t = plan->tile;
         t.block_threads = 64 * ditto::kSplitWaves;
         t.block_m = 16 * rt;
         t.block_l = 32 * ditto::kSplitWaves;
-        t.block_n = (int)d->N;
+        t.block_n = plan->split_ct ? 16 * ct : (int)d->N;
         t.head_pad = 16 * dt;
-        t.lds_bytes = ditto::bmm_chain_split_lds(dt, rt, kl_b);
-        t.grid_x = (int)(plan->nb * d->batch);
+        t.lds_bytes = ditto::bmm_chain_split_lds(dt, ct, rt, kl_b);
+        t.grid_x = (int)(wgs * (plan->split_ct ? blocks(ct) : 1));
         t.grid_y = t.grid_z = 1;
         t.variant = 2000 + 10 * dt + rt;
         return DITTO_OK;
@@ -1516,7 +1528,10 @@ int launch_fp_chain(const ditto_bmm_chain_desc* d, const BmmPlan& plan, const vo
     const int q = plan.split_rt > 0 ? plan.split_rt : plan.rows_nw > 0 ? plan.rows_nw : plan.qt;
     const ditto::BmmSetsArgs all{args, *sets};
     e = d->in_dtype == DITTO_F16 ? ditto::launch_sets_f16(k, dt, q, all, st) : ditto::launch_sets_bf16(k, dt, q, all, st);
-  } else if (plan.split_rt > 0)
+  } else if (plan.split_ct > 0)
+    e = d->in_dtype == DITTO_F16 ? ditto::launch_split_cols_f16(plan.split_dt, plan.split_ct, sm, kl, args, st)
+                                 : ditto::launch_split_cols_bf16(plan.split_dt, plan.split_ct, sm, kl, args, st);
+  else if (plan.split_rt > 0)
     e = d->in_dtype == DITTO_F16 ? ditto::launch_split_f16(plan.split_dt, plan.split_rt, sm, kl, args, st)
                                  : ditto::launch_split_bf16(plan.split_dt, plan.split_rt, sm, kl, args, st);
   else if (plan.rows_nw > 0)

@@ -14,6 +14,10 @@
 // Measured, us per launch (2.4 of them the launch), other kernel -> this one: 16 x 176 x 176 x 80 8.4 -> 4.9,
 // 8 x 461 x 461 x 80 12.7 -> 5.9, 2 x 2392 x 2392 x 80 38.5 -> 13.1, 2 x 4096 x 4096 x 128 60.9 -> 28.4,
 // 8 x 512 x 2048 x 64 17.5 -> 8.8, the chain 1 x 512 x 256 x 64 without softmax 4.7 -> 4.05.
+//
+// Where two or more workgroups to a row block still leave each a compute unit, they share out the columns of F (CT of the DT
+// tiles each) and repeat the first product: a workgroup then pulls all of B and its columns of C.  21 x 25 x 944 x 128 with softmax
+// 8.8 -> 7.0 us, 1 x 1463 x 2296 x 128 13.1 -> 10.5, 1 x 710 x 1408 x 80 8.2 -> 7.2, 11 x 67 x 2128 x 64 7.05 -> 5.97.
 #pragma once
 #include "bmm_chain_fp.h"
 #include "common.h"
@@ -24,11 +28,12 @@ constexpr int kSplitWaves = 8;
 
 // LDS of one wave: a tile of 32 rows of C and one of B (32 keys), filled by direct loads of 64 16-byte chunks each.
 // DT: column tiles of 16 that K and N are padded to; the contraction over K runs in steps of 32.
-template <int DT, bool B_KL>
+// CT: column tiles of C that the workgroup owns.
+template <int DT, bool B_KL, int CT = DT>
 struct SplitTiles {
   static constexpr int KS = (DT + 1) / 2;
   static constexpr bool POW2 = DT == 4 || DT == 8;
-  static constexpr int C_CPR = 2 * DT;                       // chunks per row of the C tile
+  static constexpr int C_CPR = 2 * CT;                       // chunks per row of the C tile
   static constexpr int C_LOADS = 32 * C_CPR / 64;
   // B stored [L][K]: rows of keys, KS * 32 columns; an odd number of chunks per row where the swizzle has no power of two
   // to work in.  B stored [K][L]: KS * 32 rows of 32 keys.
@@ -38,31 +43,37 @@ struct SplitTiles {
   static constexpr int C_OFF = B_LOADS * 1024;
   static constexpr int BYTES = C_OFF + C_LOADS * 1024;       // per wave
 };
-// LDS of a workgroup: its waves' tiles, or the merge's partial results and their exponents and sums
-inline int bmm_chain_split_lds(int dt, int rt, bool kl) {
-  const int tiles = kSplitWaves * (dt == 4   ? (kl ? SplitTiles<4, true>::BYTES : SplitTiles<4, false>::BYTES)
+// LDS of a workgroup of ct of the column tiles of C: its waves' tiles, or the merge's partial results and their exponents and sums
+inline int bmm_chain_split_lds(int dt, int ct, int rt, bool kl) {
+  const int whole = (dt == 4   ? (kl ? SplitTiles<4, true>::BYTES : SplitTiles<4, false>::BYTES)
                                    : dt == 5 ? (kl ? SplitTiles<5, true>::BYTES : SplitTiles<5, false>::BYTES)
                                              : (kl ? SplitTiles<8, true>::BYTES : SplitTiles<8, false>::BYTES));
-  const int merge = kSplitWaves * 16 * rt * (16 * dt + 4 + 2) * 4;
+  const int tiles = kSplitWaves * (whole - 1024 * (dt - ct)), merge = kSplitWaves * 16 * rt * (16 * ct + 4 + 2) * 4;
   return tiles > merge ? tiles : merge;
 }
 
-template <typename T, int DT, int RT, int INTER, bool B_KL, typename Args>
+template <typename T, int DT, int RT, int INTER, bool B_KL, typename Args, int CT = DT>
 __global__ __launch_bounds__(64 * kSplitWaves) void bmm_chain_split_kernel(Args p) {
 #if defined(__HIP_DEVICE_COMPILE__)
   typedef typename Elem<T>::v8 V8;
   typedef typename Elem<T>::v4 V4;
   typedef typename Elem<T>::v2 V2;
-  typedef SplitTiles<DT, B_KL> S;
-  constexpr int KS = S::KS, ORS = 16 * DT + 4;
+  typedef SplitTiles<DT, B_KL, CT> S;
+  constexpr int KS = S::KS, ORS = 16 * CT + 4;
   constexpr bool kSoftmax = INTER == kInterSoftmax;
   // swizzles of the 16-byte chunks of a row: plain row reads (lanes = 16 rows), transposing reads (lanes = 4 rows x 32 bytes)
   auto swz_rows = [](int row) { return DT == 4 ? (row >> 1) & 7 : DT == 8 ? row & 15 : 0; };
-  auto swz_tr = [](int row) { return DT == 4 ? 2 * ((row >> 1) & 3) : DT == 8 ? 2 * (row & 7) : 0; };
+  auto swz_tr = [](int row) { return CT == 2 ? 2 * ((row >> 2) & 1) : CT == 4 ? 2 * ((row >> 1) & 3) : CT == 8 ? 2 * (row & 7) : 0; };
   extern __shared__ __attribute__((aligned(1024))) char smem_sp[];
   const int tid = threadIdx.x, lane = tid & 63, c = lane & 15, q = lane >> 4;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const unsigned lid = xcd_remap(blockIdx.x, gridDim.x);
+  unsigned lid = xcd_remap(blockIdx.x, gridDim.x);
+  int col0 = 0;  // the workgroup's first column of F
+  if constexpr (CT < DT) {
+    const unsigned rows = lid / ((unsigned)(p.N + 16 * CT - 1) / (16u * CT));
+    col0 = 16 * CT * (int)(lid - rows * ((unsigned)(p.N + 16 * CT - 1) / (16u * CT)));
+    lid = rows;
+  }
   const int bz = lid / (unsigned)p.mblocks, m0 = (lid - bz * (unsigned)p.mblocks) * 16 * RT;
   const BatchEntry be = batch_entry(p, bz);
   const T* __restrict__ Ag = reinterpret_cast<const T*>(p.a) + be.a;
@@ -112,7 +123,7 @@ __global__ __launch_bounds__(64 * kSplitWaves) void bmm_chain_split_kernel(Args 
 #pragma unroll
   for (int i = 0; i < S::C_LOADS; ++i) {
     const int ch = 64 * i + lane, row = ch / S::C_CPR, lc = (ch - row * S::C_CPR) ^ swz_tr(row);
-    c_voff[i] = 8 * lc < N ? (row * p.c_rs + 8 * lc) * 2 : kNone;
+    c_voff[i] = col0 + 8 * lc < N ? (row * p.c_rs + col0 + 8 * lc) * 2 : kNone;
   }
   char* const tile = smem_sp + w * S::BYTES;
   const unsigned lds = (unsigned)(size_t)(DITTO_LDS char*)smem_sp + w * S::BYTES;
@@ -151,11 +162,11 @@ __global__ __launch_bounds__(64 * kSplitWaves) void bmm_chain_split_kernel(Args 
                            lds_read_tr4<T>(reinterpret_cast<const T*>(a + 16 * 16 * S::C_CPR)));
   };
 
-  f32x4 o[RT][DT];
+  f32x4 o[RT][CT];
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-    for (int j = 0; j < DT; ++j) o[rt][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < CT; ++j) o[rt][j] = f32x4{0.f, 0.f, 0.f, 0.f};
   // softmax in the exp2 domain: a row's reference exponent is its maximum over the wave's first keys, raised when a later
   // score exceeds it by more than 2^kLazy; a wave whose keys so far all score minus infinity has none yet (it may be one of
   // eight that has met any key of the row)
@@ -218,7 +229,7 @@ __global__ __launch_bounds__(64 * kSplitWaves) void bmm_chain_split_kernel(Args 
           ref[rt] = up;
           lsum[rt] *= alpha;
 #pragma unroll
-          for (int j = 0; j < DT; ++j) o[rt][j] *= alpha;
+          for (int j = 0; j < CT; ++j) o[rt][j] *= alpha;
         }
       }
     }
@@ -244,13 +255,13 @@ __global__ __launch_bounds__(64 * kSplitWaves) void bmm_chain_split_kernel(Args 
           pf[rt][4 * kt + r + 1] = two[1];
         }
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(S::B_LOADS) : "memory");  // this step's C tile, not the next B tile
-    V8 cf[DT];
+    V8 cf[CT];
 #pragma unroll
-    for (int j = 0; j < DT; ++j) cf[j] = c_frag(j);
+    for (int j = 0; j < CT; ++j) cf[j] = c_frag(j);
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     load_c(step + kSplitWaves);
 #pragma unroll
-    for (int j = 0; j < DT; ++j)
+    for (int j = 0; j < CT; ++j)
 #pragma unroll
       for (int rt = 0; rt < RT; ++rt) o[rt][j] = Elem<T>::mfma16(cf[j], pf[rt], o[rt][j]);
   }
@@ -264,7 +275,7 @@ __global__ __launch_bounds__(64 * kSplitWaves) void bmm_chain_split_kernel(Args 
   for (int rt = 0; rt < RT; ++rt) {
     float* const row = Om + (w * 16 * RT + 16 * rt + c) * ORS + 4 * q;
 #pragma unroll
-    for (int j = 0; j < DT; ++j) *reinterpret_cast<f32x4*>(row + 16 * j) = o[rt][j];
+    for (int j = 0; j < CT; ++j) *reinterpret_cast<f32x4*>(row + 16 * j) = o[rt][j];
     if constexpr (kSoftmax) {
       float s = lsum[rt];
       s += __shfl_xor(s, 16);
@@ -277,8 +288,8 @@ __global__ __launch_bounds__(64 * kSplitWaves) void bmm_chain_split_kernel(Args 
   }
   wg_sync();
   const long long f0 = be.f;
-  for (int e = tid; e < 16 * RT * 4 * DT; e += 64 * kSplitWaves) {
-    const int row = e / (4 * DT), n0 = 4 * (e - row * 4 * DT);
+  for (int e = tid; e < 16 * RT * 4 * CT; e += 64 * kSplitWaves) {
+    const int row = e / (4 * CT), n0 = 4 * (e - row * 4 * CT);
     float wt[kSplitWaves];
     if constexpr (kSoftmax) {
       float mx = kNoKeyYet, s = 0.f;
@@ -303,8 +314,8 @@ __global__ __launch_bounds__(64 * kSplitWaves) void bmm_chain_split_kernel(Args 
     if (p.relu_out)
 #pragma unroll
       for (int t = 0; t < 4; ++t) x[t] = fmaxf(x[t], 0.f);
-    if (m0 + row < M && n0 < N) {  // N is a multiple of 8
-      const long long at = f0 + (long long)(m0 + row) * p.f_rs + n0;
+    if (m0 + row < M && col0 + n0 < N) {  // N is a multiple of 8
+      const long long at = f0 + (long long)(m0 + row) * p.f_rs + col0 + n0;
       if (p.out_f32) {
         *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(p.f) + at) = x;
       } else {
@@ -318,10 +329,10 @@ __global__ __launch_bounds__(64 * kSplitWaves) void bmm_chain_split_kernel(Args 
 #endif
 }
 
-template <typename T, int DT, int RT, int INTER, bool B_KL, typename Args>
+template <typename T, int DT, int RT, int INTER, bool B_KL, int CT = DT, typename Args>
 hipError_t launch_bmm_chain_split(const Args& args, hipStream_t stream) {
-  const int lds = bmm_chain_split_lds(DT, RT, B_KL);
-  auto kern = bmm_chain_split_kernel<T, DT, RT, INTER, B_KL, Args>;
+  const int lds = bmm_chain_split_lds(DT, CT, RT, B_KL);
+  auto kern = bmm_chain_split_kernel<T, DT, RT, INTER, B_KL, Args, CT>;
   static thread_local int configured_dev = -1;
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
@@ -331,7 +342,8 @@ hipError_t launch_bmm_chain_split(const Args& args, hipStream_t stream) {
     if (e != hipSuccess) return e;
     configured_dev = dev;
   }
-  hipLaunchKernelGGL(kern, dim3((unsigned)args.mblocks * (unsigned)args.batch), dim3(64 * kSplitWaves), lds, stream, args);
+  const unsigned cols = CT == DT ? 1u : (unsigned)(args.N + 16 * CT - 1) / (16u * CT);
+  hipLaunchKernelGGL(kern, dim3((unsigned)args.mblocks * (unsigned)args.batch * cols), dim3(64 * kSplitWaves), lds, stream, args);
   return hipGetLastError();
 }
 

@@ -26,6 +26,9 @@ hipError_t launch_bf16_softmax(int d_pad, int q, bool b_kl, const BmmChainArgs& 
 // bmm_chain_split_inst.hip, one object per element type: few rows, the waves split the keys
 hipError_t launch_split_f16(int dt, int rt, bool softmax, bool b_kl, const BmmChainArgs& args, hipStream_t stream);
 hipError_t launch_split_bf16(int dt, int rt, bool softmax, bool b_kl, const BmmChainArgs& args, hipStream_t stream);
+// the same on few rows, 16 to a workgroup, of whose columns a workgroup owns 16 ct
+hipError_t launch_split_cols_f16(int dt, int ct, bool softmax, bool b_kl, const BmmChainArgs& args, hipStream_t stream);
+hipError_t launch_split_cols_bf16(int dt, int ct, bool softmax, bool b_kl, const BmmChainArgs& args, hipStream_t stream);
 
 // bmm_chain_rows_inst.hip, one object per element type: K and N padded to 80
 hipError_t launch_rows_f16(int dt, int nw, bool softmax, bool b_kl, const BmmChainArgs& args, hipStream_t stream);

@@ -171,6 +171,31 @@ def test_kernels_named_by_their_price(oracle, batch, M, L, D, inter, b_layout, d
     assert rel <= (REL_L2 if inter != "softmax" or dtype == "float16" else REL_L2_BF16_P_ONLY), rel
 
 
+@pytest.mark.parametrize("batch,M,L,K,N,b_layout,columns", [
+    # columns of a workgroup: half, a quarter, a last block of 16, of 8, whole rows where there is nothing to gain or no compute unit left
+    (2, 40, 136, 64, 64, "LK", 32), (1, 100, 1112, 64, 64, "KL", 32), (3, 33, 176, 80, 80, "LK", 32), (2, 17, 72, 72, 72, "KL", 32),
+    (2, 50, 200, 128, 128, "LK", 32), (5, 200, 264, 128, 128, "LK", 64), (2, 50, 520, 128, 128, "KL", 64), (2, 50, 200, 128, 104, "KL", 32),
+    (3, 40, 96, 64, 24, "LK", 24), (9, 300, 64, 64, 64, "LK", 64),
+])
+@pytest.mark.parametrize("inter", ["softmax", "relu"])
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+def test_key_splitting_kernel_with_columns_shared_out(oracle, batch, M, L, K, N, b_layout, columns, inter, dtype):
+    std, scale = (1.0, K ** -0.5) if inter == "softmax" else (0.25, 1.0)
+    A, B, C = oracle.make_gemm_chain_inputs(batch, M, N, K, L, dtype, seed=M + L, std=std)
+    want = oracle.bmm_chain_f64(A, B, C, inter=inter, scale=scale, round_mid=None if inter == "softmax" else dtype)
+    width = 4 if max(K, N) <= 64 else 5 if max(K, N) <= 80 else 8
+    t = lambda *s: torch.empty(batch, *s, dtype=TORCH_DTYPES[dtype], device="cuda")
+    b = t(K, L) if b_layout == "KL" else t(L, K).transpose(1, 2)
+    tile = chain.select_tile(chain.bmm_chain_desc(t(M, K), b, t(L, N), t(M, N), inter, scale, 1.0, 2001 + 10 * width, False))
+    assert (tile.variant, tile.block_n) == (2001 + 10 * width, columns)
+    got = run_chain(A, B, C, dtype, inter, scale, b_layout, "float32", 2001 + 10 * width)
+    mx, rel = errors(got, want)
+    assert np.isfinite(got).all() and mx <= 4e-2, mx
+    assert rel <= (REL_L2 if inter != "softmax" or dtype == "float16" else REL_L2_BF16_P_ONLY), rel
+    narrow = run_chain(A, B, C, dtype, inter, scale, b_layout, dtype, 2001 + 10 * width)
+    assert np.array_equal(narrow, oracle.np_round_to(got, dtype))
+
+
 def masked_scores(oracle, batch, M, N, K, L, dtype, masked, seed):
     """Operands whose scores are minus infinity at the keys ``masked``: column 0 of the first operand is one, and the
     keys hold minus infinity there (how a caller of a chain without a mask argument masks keys)."""

@@ -407,9 +407,10 @@ def test_short_chain_units_keep_their_counted_waits_exact(tmp_path, unit_name, k
     assert not bare and (stores > 0) == unit_name.startswith("fp_rows")
 
 
-@pytest.mark.parametrize("unit_name", ["fp_sets_f16", "fp_sets_bf16"])
-def test_units_of_several_chains_a_launch_keep_their_counted_waits_exact(tmp_path, unit_name):
-    """The same for the kernels compiled again with a table of chains in their arguments."""
+@pytest.mark.parametrize("unit_name,kernels", [("fp_sets_f16", 6 + 5 + 2), ("fp_sets_bf16", 6 + 5 + 2), ("fp_split_cols_f16", 16)])
+def test_units_of_kernels_compiled_again_keep_their_counted_waits_exact(tmp_path, unit_name, kernels):
+    """The same for the kernels compiled again with a table of chains in their arguments (split, rows, 64 rows), and for a few of
+    the columns."""
     hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
     if not os.path.exists(hipcc):
         pytest.skip("hipcc not available")
@@ -420,7 +421,7 @@ def test_units_of_several_chains_a_launch_keep_their_counted_waits_exact(tmp_pat
                    capture_output=True)
     text = out.read_text()
     md = kernel_metadata(text)
-    assert len(md) == 6 + 5 + 2  # split, rows, 64 rows
+    assert len(md) == kernels
     assert all(v["vgpr_spill_count"] == 0 for v in md.values())
     loops = []
     assert untracked_memory_ops_in_direct_load_loops(text, loops) == []
