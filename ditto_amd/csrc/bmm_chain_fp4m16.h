@@ -28,8 +28,8 @@
 // first keys; the lane's partial row SUM is watched once per tile and the reference raised by whole binary orders
 // when it passes a limit; a sum that ends up infinite or NaN sends the workgroup through the exact walk), for bf16
 // and for fp16: an fp16 probability overflows at 2^16, so the limit is 2^8 there and a row whose scores climb by
-// more than 2^8 within one tile takes the second walk.  fp16 also uses the pre-scaled form of the pipelined
-// eight-wave kernel: A is multiplied by scale * log2(e) once and every score tile starts from minus the reference
+// more than 2^8 within one tile takes the second walk.  fp16 also uses (one chain to a launch) the pre-scaled form of the
+// pipelined eight-wave kernel: A is multiplied by scale * log2(e) once and every score tile starts from minus the reference
 // exponent, so a score costs its v_exp_f32 and nothing else.
 #pragma once
 #include "bmm_chain_fp8m16.h"
@@ -71,7 +71,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
   constexpr int NLD = TB / 1024 / NW;    // direct loads per wave per tile
   constexpr int B_OFF = 0, C_OFF = NR * TB;
   constexpr bool kSoftmax = INTER == kInterSoftmax;
-  constexpr bool PRE = kSoftmax && !Elem<T>::is_bf16;
+  // (Not with several chains in a launch: A times scale is rounded to 16 bits again, which the key-splitting and the 32-row
+  // kernels don't do that the same chains may be launched on one by one.)
+  constexpr bool PRE = kSoftmax && !Elem<T>::is_bf16 && std::is_same<Args, BmmChainArgs>::value;
   // a lane's partial row sum above which the reference exponent is raised
   constexpr float kLimit = Elem<T>::is_bf16 ? kSumLimitBf16 : kSumLimitF16;
 

@@ -330,10 +330,10 @@ def test_specialised_conv_chain_with_outputs_of_either_type(oracle):
         assert mx <= 1e-2 and rel <= 1e-3, (dt, mx, rel)
         assert f._is_prepared(w1, w2, dt)
 
-def _attention_layers(heads, d, batch, M, dtype, count):
+def _attention_layers(heads, d, batch, M, dtype, count, scale=None):
     from ditto_amd import auto_schedule, chimera
 
-    mha = ac.nn.module.MultiHeadAttentionMMA(heads, heads * d, dtype, "float32", scale=None)
+    mha = ac.nn.module.MultiHeadAttentionMMA(heads, heads * d, dtype, "float32", scale=scale)
     graph = runtime.Graph([mha.layer(batch, M) for _ in range(count)], outputs=[(i, 0) for i in range(count)])
     bound = chimera.task_binding(auto_schedule.extract_tasks_from_graph(graph))
     opt = auto_schedule.ScheduleOption("hip", log_file="untuned.log", dtype=dtype)
@@ -414,3 +414,40 @@ def test_run_sets_through_the_c_abi_matches_single_calls():
         assert (outs[i].float() - want.float()).norm() <= 1e-3 * want.float().norm()
     assert _lib.load().ditto_bmm_chain_run_sets(ctypes.byref(desc), -1, *arrays, stream) == -1
     assert _lib.load().ditto_bmm_chain_run_sets(ctypes.byref(desc), 0, *arrays, stream) == 0
+
+def _attention_f64(x, heads, scale):
+    b, m, w = x.shape
+    q, k, v = x.double().cpu().view(b, m, 3, heads, w // 3 // heads).permute(2, 0, 3, 1, 4).unbind(0)
+    return (torch.softmax(scale * (q @ k.transpose(-1, -2)), -1) @ v).permute(0, 2, 1, 3).reshape(b, m, w // 3)
+
+# (8 heads of 172 rows alone are a key-splitting chain, twelve layers together 64-row workgroups; 2100 rows: their form of two
+# key halves)
+@pytest.mark.parametrize("heads,M,count", [(8, 172, 12), (2, 2100, 12)])
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+def test_layers_that_share_a_launch_are_as_exact_as_alone(heads, M, count, dtype):
+    """No operand is rounded that a layer by itself does not round: queries that leave the 16-bit range once they are scaled
+    come out, and the error against 64 bits is no larger than one layer's."""
+    d, scale = 64, 1.0
+    graph, mods = _attention_layers(heads, d, 1, M, dtype, count, scale)
+    (func,) = mods.values()
+    gen = torch.Generator(device="cuda").manual_seed(9)
+    dt = getattr(torch, dtype)
+    for large in (False, True):
+        ins = [torch.empty(1, M, 3 * heads * d, dtype=dt, device="cuda").normal_(0.0, 0.35, generator=gen) for _ in range(count)]
+        for x in ins if large else ():
+            q, k, _ = x.view(1, M, 3, heads, d).unbind(2)
+            q[..., 0] = 60000.0  # times log2(e) beyond the largest fp16; against keys small enough for scores of a few units
+            k[..., 0] = 2.0 ** -14 * torch.randint(-2, 3, (1, M, heads), device="cuda", generator=gen)
+        outs = [torch.empty(1, M, heads * d, dtype=dt, device="cuda") for _ in ins]
+        func.sets(list(zip(ins, outs)))()
+        alone = torch.empty_like(outs[0])
+        for x, o in list(zip(ins, outs))[::5]:
+            func(x, alone)
+            want = _attention_f64(x, heads, scale)
+            rel = [float((t.double().cpu() - want).norm() / want.norm()) for t in (o, alone)]
+            # both round every probability and every result once, at most u = 2^-11 | 2^-9 of it each
+            assert max(rel) <= (2 * 2 ** -11 if dtype == "float16" else 2 * 2 ** -9), rel
+            # and the same number of times.  The two roundings are of one size, so that the error is sqrt(2) times the result's own
+            # rounding; where a row's largest probabilities are exact, because they are the references of the keys' parts that a
+            # kernel walks apart, it is less, and no less than that one.
+            assert large or rel[0] <= 2 ** 0.5 * rel[1], rel
