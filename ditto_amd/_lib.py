@@ -116,6 +116,7 @@ EXPORTS = [
      [ctypes.POINTER(BmmChainDesc), _P, _P, _P, _P, _P, _P, ctypes.c_size_t, _P]),
     ("ditto_bmm_chain_run_sets", ctypes.c_int,
      [ctypes.POINTER(BmmChainDesc), ctypes.c_int, _PP, _PP, _PP, _PP, _P]),
+    ("ditto_bmm_chain_sets_launches", ctypes.c_int, [ctypes.POINTER(BmmChainDesc), ctypes.c_int, _PP, _PP, _PP, _PP]),
     ("ditto_conv_chain_run", ctypes.c_int,
      [ctypes.POINTER(ConvChainDesc), _P, _P, _P, _P, _P, ctypes.c_size_t, _P]),
     ("ditto_conv_chain_prepare", ctypes.c_int,

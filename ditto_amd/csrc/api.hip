@@ -179,7 +179,7 @@ int plan_bmm(const ditto_bmm_chain_desc* d, BmmPlan* plan, bool need_device) {
     int cus;
     BmmPlan plan;
   };
-  constexpr int kKept = 4;
+  constexpr int kKept = 8;
   static thread_local Kept kept[kKept] = {};  // (an all-zero descriptor is refused: abi_version)
   static thread_local int next = 0;
   const int cus = need_device ? device_cus() : 256;
@@ -1482,6 +1482,65 @@ int plan_conv_steered(const ditto_conv_chain_desc* d, const ConvSteer& steer, Co
 // find a row's first unmasked key wherever it lies, so a chain loses nothing by running with others.)
 bool plan_takes_sets(const BmmPlan& plan) { return plan.split_rt > 0 || plan.rows_nw > 0 || plan.qt == 4 || plan.qt == 5; }
 
+// The launch of n chains of one descriptor together, if there is one.
+struct SetsPlan {
+  ditto_bmm_chain_desc desc;
+  BmmPlan plan;
+};
+bool plan_sets(const ditto_bmm_chain_desc* d, int n, SetsPlan* out) {
+  BmmPlan alone;
+  if (d->batch <= 0 || d->batch > 0x7fffffff / (2 * ditto::kMaxSets) || plan_bmm(d, &alone, true) != DITTO_OK) return false;
+  ditto_bmm_chain_desc& all = out->desc;
+  all = *d;
+  all.batch = d->batch * n;
+  if (d->batch_inner == 0 || d->batch_inner == d->batch) {
+    all.batch_inner = d->batch;
+    all.a_batch_stride_outer = all.b_batch_stride_outer = all.c_batch_stride_outer = all.f_batch_stride_outer = 0;
+  }
+  if (plan_bmm(&all, &out->plan, true) != DITTO_OK || !plan_takes_sets(out->plan)) return false;
+  out->plan.split_ct = 0;  // (the key-splitting kernel for several chains has workgroups of all columns only)
+  return true;
+}
+
+// Calls launch(first chain, plan, where the chains lie) for every launch that `count` chains go out in, until one returns an
+// error; the plan is null for a chain by itself.
+template <typename Launch>
+int for_sets_launches(const ditto_bmm_chain_desc* d, int count, const void* const* a, const void* const* b, const void* const* c,
+                      void* const* f, Launch&& launch) {
+  const long long elem = 2, out_elem = d->out_dtype == DITTO_F32 ? 4 : 2;
+  unsigned refused = 0;  // bit n: no kernel takes n of the chains together
+  int alone = 0;         // chains from `at` on that are known to go out by themselves
+  for (int at = 0; at < count;) {
+    // the chains from `at` on that may share a launch: 16-bit ones whose A, B and C lie equally far from the first one's
+    int n = 1;
+    ditto::BmmSets sets = {};
+    if (alone == 0 && (d->in_dtype == DITTO_F16 || d->in_dtype == DITTO_BF16) && d->inter_op == DITTO_INTER_SOFTMAX &&
+        d->b_layout == DITTO_B_LK) {
+      auto apart = [](const void* to, const void* from) {
+        return (long long)(reinterpret_cast<intptr_t>(to) - reinterpret_cast<intptr_t>(from));
+      };
+      for (; at + n < count && n < ditto::kMaxSets; ++n) {
+        const long long in = apart(a[at + n], a[at]);
+        if (!a[at + n] || !b[at + n] || !c[at + n] || !f[at + n] || !aligned(f[at + n], 16) || in % 16 != 0 ||
+            apart(b[at + n], b[at]) != in || apart(c[at + n], c[at]) != in)
+          break;
+        sets.in[n] = in / elem, sets.out[n] = apart(f[at + n], f[at]) / out_elem;
+      }
+    }
+    // as many of them as a kernel takes, by halves: all together may be so large that one is chosen which takes no sets
+    SetsPlan together;
+    int take = n;
+    while (take > 1 && ((refused >> take & 1) != 0 || !plan_sets(d, take, &together))) refused |= 1u << take, take = (take + 1) / 2;
+    if (take == 1 && n > 1) alone = n;
+    sets.count = take, sets.entries = (int)d->batch;
+    const int rc = launch(at, take > 1 ? &together : nullptr, sets);
+    if (rc != DITTO_OK) return rc;
+    at += take;
+    if (alone > 0) --alone;
+  }
+  return DITTO_OK;
+}
+
 // The launch of a planned fp16 / bf16 chain; `sets`: where the tensors of the chains it is one of lie, or null.
 int launch_fp_chain(const ditto_bmm_chain_desc* d, const BmmPlan& plan, const void* a, const void* b, const void* c, void* f,
                     const ditto::BmmSets* sets, hipStream_t st) {
@@ -1657,47 +1716,21 @@ int ditto_bmm_chain_run(const ditto_bmm_chain_desc* d, const void* a, const void
 int ditto_bmm_chain_run_sets(const ditto_bmm_chain_desc* d, int count, const void* const* a, const void* const* b,
                              const void* const* c, void* const* f, void* stream) {
   if (!d || count < 0 || (count > 0 && (!a || !b || !c || !f))) return fail(DITTO_EINVAL, "null argument or negative count");
-  const long long elem = 2, out_elem = d->out_dtype == DITTO_F32 ? 4 : 2;
-  for (int at = 0; at < count;) {
-    // the sets from `at` on that one launch takes: 16-bit chains whose A, B and C lie equally far from the first set's
-    int n = 1;
-    ditto::BmmSets sets = {};
-    if ((d->in_dtype == DITTO_F16 || d->in_dtype == DITTO_BF16) && d->inter_op == DITTO_INTER_SOFTMAX && d->b_layout == DITTO_B_LK) {
-      auto apart = [](const void* to, const void* from) {
-        return (long long)(reinterpret_cast<intptr_t>(to) - reinterpret_cast<intptr_t>(from));
-      };
-      for (; at + n < count && n < ditto::kMaxSets; ++n) {
-        const long long in = apart(a[at + n], a[at]);
-        if (!a[at + n] || !b[at + n] || !c[at + n] || !f[at + n] || !aligned(f[at + n], 16) || in % 16 != 0 ||
-            apart(b[at + n], b[at]) != in || apart(c[at + n], c[at]) != in)
-          break;
-        sets.in[n] = in / elem, sets.out[n] = apart(f[at + n], f[at]) / out_elem;
-      }
-    }
-    if (n > 1 && d->batch > 0 && d->batch <= 0x7fffffff / (2 * ditto::kMaxSets)) {
-      ditto_bmm_chain_desc all = *d;
-      all.batch = d->batch * n;
-      if (d->batch_inner == 0 || d->batch_inner == d->batch) {
-        all.batch_inner = d->batch;
-        all.a_batch_stride_outer = all.b_batch_stride_outer = all.c_batch_stride_outer = all.f_batch_stride_outer = 0;
-      }
-      BmmPlan plan;
-      if (plan_bmm(d, &plan, true) == DITTO_OK && plan_bmm(&all, &plan, true) == DITTO_OK && plan_takes_sets(plan)) {
-        if (!a[at] || !b[at] || !c[at] || !f[at]) return fail(DITTO_EINVAL, "null data pointer");
-        if (!aligned(a[at], 16) || !aligned(b[at], 16) || !aligned(c[at], 16) || !aligned(f[at], 16))
-          return fail(DITTO_EINVAL, "data pointers must be 16-byte aligned");
-        sets.count = n, sets.entries = (int)d->batch;
-        const int rc = launch_fp_chain(&all, plan, a[at], b[at], c[at], f[at], &sets, reinterpret_cast<hipStream_t>(stream));
-        if (rc != DITTO_OK) return rc;
-        at += n;
-        continue;
-      }
-    }
-    const int rc = ditto_bmm_chain_run(d, a[at], b[at], c[at], nullptr, f[at], nullptr, 0, stream);
-    if (rc != DITTO_OK) return rc;
-    ++at;
-  }
-  return DITTO_OK;
+  return for_sets_launches(d, count, a, b, c, f, [&](int at, const SetsPlan* together, const ditto::BmmSets& sets) {
+    if (!together) return ditto_bmm_chain_run(d, a[at], b[at], c[at], nullptr, f[at], nullptr, 0, stream);
+    if (!a[at] || !b[at] || !c[at] || !f[at]) return fail(DITTO_EINVAL, "null data pointer");
+    if (!aligned(a[at], 16) || !aligned(b[at], 16) || !aligned(c[at], 16) || !aligned(f[at], 16))
+      return fail(DITTO_EINVAL, "data pointers must be 16-byte aligned");
+    return launch_fp_chain(&together->desc, together->plan, a[at], b[at], c[at], f[at], &sets, reinterpret_cast<hipStream_t>(stream));
+  });
+}
+
+int ditto_bmm_chain_sets_launches(const ditto_bmm_chain_desc* d, int count, const void* const* a, const void* const* b,
+                                  const void* const* c, void* const* f) {
+  if (!d || count < 0 || (count > 0 && (!a || !b || !c || !f))) return fail(DITTO_EINVAL, "null argument or negative count");
+  int launches = 0;
+  for_sets_launches(d, count, a, b, c, f, [&](int, const SetsPlan*, const ditto::BmmSets&) { return ++launches, (int)DITTO_OK; });
+  return launches;
 }
 
 int ditto_conv_chain_select_tile(const ditto_conv_chain_desc* desc, ditto_tile_param* out) {

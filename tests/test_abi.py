@@ -66,6 +66,35 @@ def _desc(**kw):
     return d
 
 
+def _sets_launches(desc, count, step=1 << 24, out_step=1 << 22):
+    """Launches for ``count`` chains whose inputs lie ``step`` bytes behind one another (a list: where each one lies)."""
+    at = [i * step for i in range(count)] if isinstance(step, int) else step
+    ins = [[(1 << 40) + (j << 30) + i for i in at] for j in range(3)]
+    outs = [(1 << 41) + i * out_step for i in range(count)]
+    arrays = [(ctypes.c_void_p * count)(*v) for v in (*ins, outs)]
+    return _lib.load().ditto_bmm_chain_sets_launches(ctypes.byref(desc), count, *arrays)
+
+
+def _heads(batch, rows, d, **kw):
+    size = dict(batch=batch, M=rows, L=rows, K=d, N=d)
+    size.update({x + "_row_stride": d for x in "abcf"}, **{x + "_batch_stride": rows * d for x in "abcf"})
+    return _desc(**dict(size, **kw))
+
+
+def test_chains_that_share_launches_without_gpu():
+    # one launch holds sixteen chains; others than 16-bit softmax chains with keys as [L][K], and chains whose inputs lie apart
+    # by themselves, go out one by one
+    assert [_sets_launches(_heads(12, 99, 64), n) for n in (0, 1, 2, 16, 17, 33)] == [0, 1, 1, 1, 2, 3]
+    assert _sets_launches(_heads(12, 99, 64, inter_op=_lib.INTER_CAST), 5) == 5
+    assert _sets_launches(_heads(12, 99, 64, in_dtype=_lib.F32, out_dtype=_lib.F32), 5) == 5
+    assert _sets_launches(_heads(12, 99, 64, tile_variant=641), 5) == 5  # a kernel that takes one chain
+    assert _sets_launches(_heads(12, 99, 64), 4, [0, 1 << 24, (1 << 25) + 8, 3 << 24]) == 3
+    # together these are so large that a kernel is chosen which takes one chain; fewer of them share a launch all the same
+    assert _sets_launches(_heads(8, 64, 128), 12) <= 3
+    assert _sets_launches(_heads(8, 64, 128), 2) == 1
+    assert _sets_launches(_heads(96, 4096, 128), 6) == 6
+
+
 def test_select_tile_and_validation_without_gpu():
     lib = _lib.load()
     tile = _lib.TileParam()

@@ -344,7 +344,7 @@ def _attention_layers(heads, d, batch, M, dtype, count, scale=None):
 # 32 rows per wave, the large ones that take no sets), ragged rows among them
 @pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
 @pytest.mark.parametrize("heads,d,batch,M,count", [(2, 64, 1, 49, 2), (12, 64, 1, 99, 12), (8, 64, 2, 257, 17), (3, 80, 1, 130, 5),
-                                                   (2, 128, 1, 65, 3), (12, 64, 8, 512, 3), (4, 64, 1, 2100, 33)])
+                                                   (2, 128, 1, 65, 3), (8, 128, 1, 64, 12), (12, 64, 8, 512, 3), (4, 64, 1, 2100, 33)])
 def test_layers_that_share_a_launch_match_layers_run_one_by_one(heads, d, batch, M, count, dtype):
     graph, mods = _attention_layers(heads, d, batch, M, dtype, count)
     (func,) = mods.values()
