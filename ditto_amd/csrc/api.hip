@@ -1498,6 +1498,8 @@ bool plan_sets(const ditto_bmm_chain_desc* d, int n, SetsPlan* out) {
     all.a_batch_stride_outer = all.b_batch_stride_outer = all.c_batch_stride_outer = all.f_batch_stride_outer = 0;
   }
   if (plan_bmm(&all, &out->plan, true) != DITTO_OK || !plan_takes_sets(out->plan)) return false;
+  // (the plan of the 64-row kernel does not ask: one chain that a launch does not hold has nowhere to go, several have)
+  if (!launchable((long long)out->plan.nb * all.batch, out->plan.tile.block_threads)) return false;
   out->plan.split_ct = 0;  // (the key-splitting kernel for several chains has workgroups of all columns only)
   return true;
 }

@@ -95,6 +95,19 @@ def test_chains_that_share_launches_without_gpu():
     assert _sets_launches(_heads(96, 4096, 128), 6) == 6
 
 
+def test_chains_that_share_a_launch_fit_it_without_gpu():
+    # a launch holds fewer than 2^32 work items: 16 chains of 1.1 million one-row entries, 256 threads each, make 4.5e9
+    entries, rows = 1100000, 1
+    for count in (15, 16):
+        grid = _heads(entries * count, rows, 64)
+        assert (entries * count * 256 < 1 << 32) == (count == 15)
+        assert _sets_launches(_heads(entries, rows, 64), count) == (1 if count == 15 else 2)
+        tile = _lib.TileParam()
+        assert _lib.load().ditto_bmm_chain_select_tile(ctypes.byref(grid), ctypes.byref(tile)) == _lib.OK and tile.block_m == 64
+    # exactly 2^32 of them
+    assert _sets_launches(_heads(1 << 20, 16, 8), 16) == 2 and _sets_launches(_heads(1 << 20, 16, 8), 15) == 1
+
+
 def test_select_tile_and_validation_without_gpu():
     lib = _lib.load()
     tile = _lib.TileParam()
