@@ -320,11 +320,13 @@ PyObject* py_run_attention(PyObject*, PyObject* const* v, Py_ssize_t n) {
 // run_attention_sets(projections, outs, heads, hidden, scale, tile_variant, batch, rows): run_attention on several projections
 // [batch, rows, 3 * hidden], in as few launches as hold them -> return code, or None where that does not do: tensors that are
 // not the plain case, not of that shape or not alike, or an output that shares memory with another set's tensors (then the caller runs them in order)
-PyObject* py_run_attention_sets(PyObject*, PyObject* const* v, Py_ssize_t n) {
+// attention_sets_launches(the same): how many launches that call makes (or its return code where it fails), or None likewise
+template <typename Call>
+PyObject* attention_sets(PyObject* const* v, Py_ssize_t n, Call&& call) {
   return guarded([&]() -> PyObject* {
     if (n != 8 || !PyList_Check(v[0]) || !PyList_Check(v[1]) || PyList_GET_SIZE(v[0]) != PyList_GET_SIZE(v[1]) ||
         PyList_GET_SIZE(v[0]) == 0)
-      fail(PyExc_TypeError, "run_attention_sets takes two lists of tensors, equally long, and 6 numbers");
+      fail(PyExc_TypeError, "attention sets take two lists of tensors, equally long, and 6 numbers");
     const int64_t heads = integer(v[2]), hidden = integer(v[3]);
     const Py_ssize_t sets = PyList_GET_SIZE(v[0]);
     struct Span {
@@ -355,9 +357,14 @@ PyObject* py_run_attention_sets(PyObject*, PyObject* const* v, Py_ssize_t n) {
     ditto_bmm_chain_desc desc;
     fill_attention(&desc, x0, o0.scalar_type(), heads, hidden, (float)number(v[4]), (int)integer(v[5]));
     return PyLong_FromLong(on_current_stream(x0.device(), [&](void* stream) {
-      return ditto_bmm_chain_run_sets(&desc, (int)sets, q.data(), k.data(), c.data(), f.data(), stream);
+      return call(&desc, (int)sets, q.data(), k.data(), c.data(), f.data(), stream);
     }));
   });
+}
+PyObject* py_run_attention_sets(PyObject*, PyObject* const* v, Py_ssize_t n) { return attention_sets(v, n, ditto_bmm_chain_run_sets); }
+PyObject* py_attention_sets_launches(PyObject*, PyObject* const* v, Py_ssize_t n) {
+  return attention_sets(v, n, [](const ditto_bmm_chain_desc* d, int sets, const void* const* q, const void* const* k, const void* const* c,
+                                 void* const* f, void*) { return ditto_bmm_chain_sets_launches(d, sets, q, k, c, f); });
 }
 
 // ---- a built function's call -----------------------------------------------------------------
@@ -563,6 +570,7 @@ PyTypeObject conv_call_type = {PyVarObject_HEAD_INIT(nullptr, 0)};
 PyMethodDef methods[] = {FAST("fill_bmm_desc", py_fill_bmm_desc), FAST("run_bmm", py_run_bmm),
                          FAST("run_bmm_desc", py_run_bmm_desc), FAST("run_attention", py_run_attention),
                          FAST("run_attention_sets", py_run_attention_sets),
+                         FAST("attention_sets_launches", py_attention_sets_launches),
                          {nullptr, nullptr, 0, nullptr}};
 #undef FAST
 

@@ -388,19 +388,21 @@ class AttentionFunction:
     def sets(self, calls):
         """A callable that does what calling the function with each ``(query_key_value, out)`` of ``calls`` in order does.
         Calls that do not read or write what another of them writes share launches (``ditto_bmm_chain_run_sets``); else they
-        run one by one."""
+        run one by one.  Its ``launches`` says how many launches it makes."""
         m, host = self.sch.module, _lib.host()
-        xs, outs = [x for x, _ in calls], [o for _, o in calls]
-        batch, rows = self.tensors[0].shape[:2]
+        every = ([x for x, _ in calls], [o for _, o in calls], m.num_heads, m.hidden_size, m.scale, self.sch.tile_variant,
+                 *self.tensors[0].shape[:2])
 
         def run():
-            rc = host.run_attention_sets(xs, outs, m.num_heads, m.hidden_size, m.scale, self.sch.tile_variant, batch, rows)
+            rc = host.run_attention_sets(*every)
             if rc is None:
                 for args in calls:
                     self(*args)
             elif rc:
                 _lib.check(rc)
 
+        launches = host.attention_sets_launches(*every)
+        run.launches = len(calls) if launches is None else launches
         return run
 
 

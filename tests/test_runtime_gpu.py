@@ -374,6 +374,33 @@ def test_layers_that_share_a_launch_match_layers_run_one_by_one(heads, d, batch,
                 assert (got.float() - want.float()).norm() <= bound * want.float().norm()
             func(ins[0], alone[0])
 
+@pytest.mark.parametrize("dtype,alike", [("float32", True), ("float16", False), ("float16", True)])
+def test_layers_that_share_no_launch_are_recorded(dtype, alike):
+    """Five layers are as many launches where the kernel takes one chain (fp32) or their tensors are laid out differently."""
+    heads, d, M, count = 4, 64, 72, 5
+    graph, mods = _attention_layers(heads, d, 1, M, dtype, count)
+    (func,) = mods.values()
+    gen = torch.Generator(device="cuda").manual_seed(15)
+    width = 3 * heads * d
+    ins = [torch.empty(1, M, width + (0 if alike else 8 * i), dtype=getattr(torch, dtype), device="cuda").normal_(generator=gen)[..., :width]
+           for i in range(count)]
+    alone = [torch.empty(1, M, heads * d, dtype=x.dtype, device="cuda") for x in ins]
+    for x, o in zip(ins, alone):
+        func(x, o)
+    eng = runtime.create_hip_graph_engine(graph, mods, "cuda:0")
+    eng.set_inputs(ins)
+    eng.compile()
+    assert (eng._graph is None) == (dtype == "float16" and alike)
+    for _ in range(3):  # replays with eager work and synchronisations in between
+        for o in eng.get_outputs():
+            o.zero_()
+        torch.cuda.synchronize()
+        eng.run()
+        torch.cuda.synchronize()
+        for got, want in zip(eng.get_outputs(), alone):
+            assert (got - want).norm() <= (1e-3 if dtype == "float16" else 1e-5) * want.norm()
+        func(ins[0], alone[0])
+
 def test_calls_that_share_memory_run_in_order():
     """An output that is part of the next call's input: the calls are not independent and must not share a launch."""
     heads, d, M = 2, 64, 64
