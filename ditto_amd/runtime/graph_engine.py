@@ -105,7 +105,8 @@ class GraphEngine:
     def compile(self):
         if not self._init:
             self.init()
-        self._to_exe = []
+        self._to_exe = []  # until all of it is there: a compile that raises leaves nothing to run, and run compiles again
+        to_exe = []
         for li, layer in enumerate(self.graph.layers):
             key = layer.fingerprint
             if key not in self.built_mods:
@@ -116,10 +117,11 @@ class GraphEngine:
                 # fixed weights: repack them once, here, into a workspace this layer owns
                 func = func.specialize(*self.weight_buffer[li])
             args = [*self.input_buffer[li], *self.weight_buffer[li], *self.output_buffer[li]]
-            self._to_exe.append((func, args))
-        self._steps = self._make_steps()
+            to_exe.append((func, args))
+        self._steps = self._make_steps(to_exe)
         self._weights = [w for li in sorted(self.weight_buffer) for w in self.weight_buffer[li]]
         self._weight_versions = self._versions()
+        self._to_exe = to_exe
 
     def _versions(self):
         return [w._version for w in self._weights]
@@ -130,19 +132,19 @@ class GraphEngine:
         for step in self._steps:
             step()
 
-    def _make_steps(self):
+    def _make_steps(self, to_exe):
         """The calls of one run.  Consecutive layers of one function that takes several calls at once (attention blocks) make
         one step, up to a layer that reads what one of them makes: twelve such layers in a launch of their own each are twelve
         starts and twelve tails (12 x [96 heads, 512 rows of 64] 171 -> 131 us, 12 x [12 heads, 99 rows of 64] 50 -> 18)."""
         steps, li = [], 0
-        while li < len(self._to_exe):
-            func, args = self._to_exe[li]
+        while li < len(to_exe):
+            func, args = to_exe[li]
             end = li + 1
             if hasattr(func, "sets"):
-                while end < len(self._to_exe) and self._to_exe[end][0] is func and not self._reads(end, li):
+                while end < len(to_exe) and to_exe[end][0] is func and not self._reads(end, li):
                     end += 1
             if end - li > 1:
-                steps.append(func.sets([tuple(a) for _, a in self._to_exe[li:end]]))
+                steps.append(func.sets([tuple(a) for _, a in to_exe[li:end]]))
             else:
                 steps.append(functools.partial(func, *args))
             li = end
@@ -175,16 +177,20 @@ class HipGraphEngine(GraphEngine):
     MOST_CALLED = 4
 
     def compile(self):
-        super().compile()
         self._graph = None
-        GraphEngine.run(self)  # warm-up outside the capture (first-call set-up, cached workspaces)
-        torch.cuda.synchronize(self.dev)
-        if sum(getattr(step, "launches", 1) for step in self._steps) <= self.MOST_CALLED:
-            return
-        g = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(g):
-            GraphEngine.run(self)
-        self._graph = g
+        super().compile()
+        try:
+            GraphEngine.run(self)  # warm-up outside the capture (first-call set-up, cached workspaces)
+            torch.cuda.synchronize(self.dev)
+            if sum(getattr(step, "launches", 1) for step in self._steps) <= self.MOST_CALLED:
+                return
+            g = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(g):
+                GraphEngine.run(self)
+            self._graph = g
+        except BaseException:
+            self._to_exe = []  # (a graph that should have been recorded is not called instead)
+            raise
 
     def run(self):
         # (a recorded graph holds the repacked weights of compile time: weights updated in place since then

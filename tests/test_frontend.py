@@ -550,3 +550,87 @@ def test_the_reference_import_name_resolves():
     assert ac_ref is ditto_amd.auto_compute and at_ref is ditto_amd.auto_tensorize
     assert hardware_param is ditto_amd.hardware.hardware_param and ditto.build is ditto_amd.build
     assert ditto.chimera is ditto_amd.chimera and ditto.runtime.Graph is ditto_amd.runtime.Graph
+
+
+def _engine_of_adding_layers(make, fail):
+    """A graph of two layers on the CPU, x -> x + 1 and the same again, whose functions raise while ``fail`` is not empty."""
+    import types
+
+    import torch
+    from ditto_amd import runtime
+
+    def add_one(x, y):
+        if fail:
+            raise RuntimeError(fail[0])
+        torch.add(x, 1, out=y)
+
+    t = types.SimpleNamespace(name="t", shape=(3,), dtype="float32")
+    layers = [types.SimpleNamespace(name="l", fingerprint="f", inputs=[t], weights=[], ops=[types.SimpleNamespace(output=lambda i: t)])
+              for _ in range(2)]
+    return make(runtime.Graph(layers, {(1, 0): (0, 0)}), {"f": add_one}, "cpu")
+
+
+def test_a_compile_that_fails_leaves_nothing_to_run():
+    import torch
+    from ditto_amd import runtime
+
+    eng = _engine_of_adding_layers(runtime.create_graph_engine, [])
+    eng.set_inputs([torch.zeros(3)])
+    eng.run()
+    assert eng.get_outputs()[0].tolist() == [2.0] * 3
+    mods, eng.built_mods = eng.built_mods, {}
+    eng.set_inputs([torch.ones(3)])
+    for _ in range(2):  # not the first compile's calls on the tensors before
+        with pytest.raises(KeyError):
+            eng.run()
+    eng.built_mods = mods
+    second = eng.graph.layers[1]
+    second.fingerprint = "g"  # found missing behind a layer that is there
+    for _ in range(2):
+        with pytest.raises(KeyError):
+            eng.run()
+    second.fingerprint = "f"
+    eng.run()
+    assert eng.get_outputs()[0].tolist() == [3.0] * 3
+
+
+def test_a_recording_that_fails_is_tried_again(monkeypatch):
+    import torch
+    from ditto_amd import runtime
+
+    recordings = []
+
+    class Recording:
+        def replay(self):
+            recordings.append(self)
+
+    class Recorder:
+        def __init__(self, graph):
+            if refused:
+                raise RuntimeError(refused[0])
+
+        def __enter__(self):
+            return self
+
+        def __exit__(self, *error):
+            return False
+
+    monkeypatch.setattr(torch.cuda, "synchronize", lambda dev=None: None)
+    monkeypatch.setattr(torch.cuda, "CUDAGraph", Recording)
+    monkeypatch.setattr(torch.cuda, "graph", Recorder)
+    refused, fail = ["no recording"], []
+    eng = _engine_of_adding_layers(runtime.create_hip_graph_engine, fail)
+    eng.MOST_CALLED = 1
+    eng.set_inputs([torch.zeros(3)])
+    for _ in range(2):
+        with pytest.raises(RuntimeError, match="no recording"):
+            eng.run()
+    refused.clear()
+    fail.append("no warm-up")
+    for _ in range(2):
+        with pytest.raises(RuntimeError, match="no warm-up"):
+            eng.run()
+    fail.clear()
+    eng.run()
+    eng.run()
+    assert len(recordings) == 2 and eng._graph is recordings[0]
