@@ -366,16 +366,24 @@ int plan_bmm_rules(const ditto_bmm_chain_desc* d, BmmPlan* plan, int cus) {
       if (rt > 0) {
         plan->split_dt = dt, plan->split_rt = rt;
         plan->nb = (int)((d->M + 16 * rt - 1) / (16 * rt));
-        // Half of the columns to a workgroup (32 of 80), or a quarter of 128, where every workgroup still has a compute unit: 0.80 -
-        // 0.97 of the time in 105 of 112 random shapes, two workgroups to one 1.1 - 2.2 times as long.  With B as [K][L], whose
-        // rows of 32 keys are read in pieces of 64 bytes, more than 150 workgroups on long keys wait for L2: 1 x 1399 x 2056 x 64
-        // 7.8 against 9.2 us, 9 x 143 x 1848 x 128 13.0 / 14.0, while 32 x 22 x 1616 x 128 gains (11.2 -> 10.5); and a quarter of
-        // 128 columns is level with half (2 x 224 x 1808 x 128 11.0 / 10.2; B [L][K] 21 x 25 x 944 x 128 7.0 / 7.6).
-        const long long wgs = plan->nb * d->batch;
+        // Half of the columns to a workgroup (32 of 80), or a quarter of 128, where every workgroup still has a compute unit: 0.79 -
+        // 0.96 of the time in nine of ten of 24000 random shapes, two workgroups to one 1.1 - 2.2 times as long.  What they pull of B
+        // grows with the workgroups, and beyond these lines L2 gives it too slowly: with B as [K][L], whose rows of 32 keys are read
+        // in pieces of 64 bytes, three fifths of the compute units past 300 keys (3 x 418 x 976 x 80 7.2 us against 5.9, 2 x 959 x
+        // 944 x 64 6.2 / 5.6; at 300 all of them gain, 0.95) and two fifths past 800 (2 x 538 x 2320 x 64 8.7 against 7.7, 19 x 55 x
+        // 2528 x 128 18.9 / 17.3); [L][K] at 64 columns four fifths past 1000 (20 x 81 x 3910 x 64 10.8 against 10.1).  Nor where more
+        // batch entries than XCDs have so many keys that those an XCD's workgroups belong to pass its L2, 10 MB in all with [K][L]
+        // (10 x 72 x 3392 x 128 23.3 / 17.3, 11 x 56 x 3216 x 128 25.5 / 18.4) and 18 MB with [L][K] up to 80 columns (18 x 46 x 3903 x
+        // 80 15.3 / 14.0).  Within the lines one of the 24000 takes more than 1.03 (7 x 62 x 3728 x 128 [K][L], 1.04).  With [K][L] a quarter of 128 columns is level with
+        // half from 500 keys on (2 x 224 x 1808 x 128 11.0 / 10.2; B [L][K] 21 x 25 x 944 x 128 7.0 / 7.6).
+        const long long wgs = plan->nb * d->batch, bytes = 2 * d->batch * d->L * (d->K + d->N);
         auto blocks = [&](int ct) { return (d->N + 16 * ct - 1) / (16 * ct); };
         const int half = dt == 8 ? 4 : 2;
-        if (rt == 1 && blocks(half) > 1 && wgs * blocks(half) <= cus && !(kl_b && d->L > 1000 && 5 * wgs * blocks(half) > 3LL * cus))
-          plan->split_ct = dt == 8 && blocks(2) > blocks(4) && wgs * blocks(2) <= cus && (!kl_b || d->L <= 500) ? 2 : half;
+        const int fifths = kl_b ? (d->L <= 300 ? 5 : d->L <= 800 ? 3 : 2) : dt == 4 && d->L > 1000 ? 4 : 5;
+        const bool spills = d->batch > 8 && bytes > (kl_b ? 10 << 20 : 18 << 20) && (kl_b || dt != 8);
+        auto room = [&](int ct) { return 5 * wgs * blocks(ct) <= (long long)fifths * cus; };
+        if (rt == 1 && blocks(half) > 1 && room(half) && !spills)
+          plan->split_ct = dt == 8 && blocks(2) > blocks(4) && room(2) && (!kl_b || d->L <= 500) ? 2 : half;
         const int ct = plan->split_ct ? plan->split_ct : dt;
         ditto_tile_param& t = plan->tile;
         t.block_threads = 64 * ditto::kSplitWaves;

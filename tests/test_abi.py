@@ -326,3 +326,24 @@ def test_missing_library_fails_loudly(monkeypatch, tmp_path):
     monkeypatch.setattr(_lib, "LIB_PATH", str(tmp_path / "nope.so"))
     with pytest.raises(_lib.ChainLibraryError, match="no CPU or PyTorch fallback"):
         _lib.load()
+
+
+def test_columns_are_shared_out_where_that_pays():
+    """Workgroups of a few rows that share out the columns pull B once each: on many compute units and long keys that takes
+    longer than idle compute units (batch, rows, keys, columns, layout of B, softmax, columns of a workgroup)."""
+    tile = _lib.TileParam()
+    for batch, m, l, d, kl, sm, block in (
+            (3, 418, 976, 80, True, False, 80), (2, 959, 944, 64, True, False, 64), (2, 538, 2320, 64, True, False, 64),
+            (2, 972, 960, 64, True, True, 64), (19, 55, 2528, 128, True, True, 128), (2, 953, 944, 128, True, False, 128),
+            (12, 34, 4032, 80, True, True, 80), (20, 81, 3910, 64, False, False, 64),
+            (10, 72, 3392, 128, True, False, 128), (18, 46, 3903, 80, False, False, 80),
+            # and on the other side of the lines
+            (3, 418, 296, 80, True, False, 32), (2, 538, 800, 64, True, False, 32), (6, 55, 2528, 128, True, True, 64),
+            (15, 81, 3910, 64, False, False, 32), (21, 25, 944, 128, False, True, 32), (1, 710, 1408, 80, False, True, 32)):
+        desc = _heads(batch, m, d, L=l, inter_op=_lib.INTER_SOFTMAX if sm else _lib.INTER_CAST, b_batch_stride=l * d, c_batch_stride=l * d)
+        if kl:
+            desc.b_layout, desc.b_row_stride = _lib.B_KL, l
+        assert _lib.load().ditto_bmm_chain_select_tile(ctypes.byref(desc), ctypes.byref(tile)) == _lib.OK
+        assert tile.variant // 100 == 20 and tile.block_n == block, (batch, m, l, d, kl, sm, tile.variant, tile.block_n)
+        rows = -(-m // 16) * batch
+        assert tile.grid_x == rows * -(-d // block) <= 256 or block == d
