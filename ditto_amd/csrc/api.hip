@@ -107,8 +107,8 @@ struct BmmPrice {
   int variant, rows, threads, resident;
   float start, first[3], per_key[3];
 };
-// Least squares over 3300 random shapes (batch 1 - 160, 32 - 4096 rows and keys, fp16 and bf16), root mean square error
-// 4 - 12 %; the columns: head sizes up to 64 | 128, without | with softmax, B [L][K] | [K][L].
+// Least squares over 3300 random shapes (batch 1 - 160, 32 - 4096 rows and keys, fp16 and bf16), those of 2144 and of the 64-row
+// kernels with softmax over 3600 others, root mean square error 4 - 12 %; the columns: head sizes up to 64 | 128, without | with softmax, B [L][K] | [K][L].
 constexpr BmmPrice kPrices64[2][2][8] = {
     {{{641, 128, 256, 1, 0.71f, {3.38f}, {.0074f}}, {644, 64, 256, 3, 2.64f, {1.30f, 1.81f, 2.36f}, {.0049f, .0079f, .0121f}},
       {645, 64, 256, 2, 2.98f, {1.34f, 2.09f}, {.0042f, .0070f}}, {649, 256, 512, 1, 0, {5.03f}, {.0118f}},
@@ -140,33 +140,60 @@ constexpr BmmPrice kPrices128[2][2][7] = {
 // The kernel that is priced at least 7 % below `own`, the one the rules of plan_bmm name, or 0.  The rules draw their lines
 // along one size at a time and miss where the rounds of two kernels fall differently: one round of 256-row workgroups against
 // two of 128 rows (40 x 809 x 1608 x 128 softmax 59.2 -> 44.2 us), 1.2 rounds of 256 against 2.2 of 128 (30 x 2080 x 2032 x 128
-// 122 -> 79), without softmax 50 x 1520 x 576 x 64 24.7 -> 19.1, 5 x 432 x 144 x 128 7.6 -> 6.0.  Over 400 - 700 random shapes
-// a class the mean is 0.8 to 3.6 % lower, the best 0.50 of the time, the worst 1.06 - 1.11 of it.  Softmax chains of up to 64
-// columns have one other kernel to go to, 32 rows a wave, from 5 % on: of 1800 + 900 random shapes with B [L][K] | [K][L] it
-// takes 150 + 100 there, at 0.90 | 0.88 of the time, the worst 1.01 (1152 x 512 x 512 122 -> 107 us, 3268 x 197 x 197 110 -> 84,
-// 830 x 1024 x 1024 295 -> 258; long keys on few rows stay: 830 x 192 x 2048 114 against 136).
+// 122 -> 79), without softmax 50 x 1520 x 576 x 64 24.7 -> 19.1, 5 x 432 x 144 x 128 7.6 -> 6.0.  Softmax chains of up to 64
+// columns have one other kernel to go to, 32 rows a wave, from 5 % on (1152 x 512 x 512 122 -> 107 us, 3268 x 197 x 197 110 -> 84;
+// long keys on few rows stay: 830 x 192 x 2048 114 against 136).  A price misses a single shape by more than these margins, so
+// the pairs of kernels whose shapes went wrong are left out below: of 5000 random shapes whose kernel changes 1 in 1000 takes more
+// than 1.03 of its time, the worst 1.04, the mean 0.85 without softmax and at 128 columns and 0.90 with it at 64.
 int cheaper_variant(const ditto_bmm_chain_desc* d, int own, int cus) {
   const long long dmax = d->K > d->N ? d->K : d->N;
   const bool sm = d->inter_op == DITTO_INTER_SOFTMAX, kl = d->b_layout == DITTO_B_KL;
   // with softmax the kernels that find a row's first unmasked key wherever it lies (20xx, 21xx, 644, 645) keep what they have
   if (dmax > 64 && (dmax <= 80 || (sm && own >= 2000))) return 0;
   const BmmPrice* const prices = dmax <= 64 ? kPrices64[sm][kl] : kPrices128[sm][kl];
-  const int count = dmax <= 64 ? 8 : 7;
+  const BmmPrice* const end = prices + (dmax <= 64 ? 8 : 7);
+  auto workgroups = [&](const BmmPrice& p) { return ((d->M + p.rows - 1) / p.rows) * d->batch; };
+  auto rounds = [&](const BmmPrice& p) { return workgroups(p) / (p.resident * cus); };  // full ones
+  auto price = [&](const BmmPrice& p) {
+    const long long full = rounds(p);
+    const int left = (int)((workgroups(p) - full * p.resident * cus + cus - 1) / cus), r = p.resident - 1;
+    const float L = (float)d->L;
+    return p.start + full * (p.first[r] + p.per_key[r] * L) + (left > 0 ? p.first[left - 1] + p.per_key[left - 1] * L : 0.f);
+  };
+  const BmmPrice* const mine = std::find_if(prices, end, [&](const BmmPrice& p) { return p.variant == own; });
+  if (mine == end) return 0;
+  // what a kernel's price may be of the rules' kernel's: 2148 is level with the 64-row kernels where it is priced 5 - 10 % below
+  // (up to 64 keys 1.05 of the time, 43 x 741 x 34 4.68 -> 5.05 us)
+  auto margin = [&](const BmmPrice& p) { return p.variant == 2148 ? 0.90f : sm && dmax <= 64 ? 0.95f : 0.93f; };
+  auto taken = [&](const BmmPrice& p) {
+    if (!launchable(workgroups(p), p.threads)) return false;
+    switch (p.variant) {
+      case 2188:  // (beyond these keys its price fits by 4 - 9 %; against 256-row workgroups it takes 0.99 - 1.04 of the time)
+        return d->L >= 64 && d->L <= 700 && own != 1282 && own != 1289;
+      case 2144:
+        // fp16 64-row workgroups scale A beforehand, a fifth of the vector ALU's work in the softmax, which the one price for
+        // both types does not show: 1.00 of the time in the mean from 700 keys on, up to 1.05 (252 x 697 x 1083 65.5 -> 68.7 us;
+        // [K][L], whose transposing reads weigh more, from 1024 on)
+        if (sm && dmax <= 64 && d->in_dtype == DITTO_F16 && (own == 645 || (own == 644 && !kl && d->L > 700))) return false;
+        return d->L > (kl && own == 2148 ? 128 : 64) || (sm && rounds(p) > 0);
+      case 2081:
+      case 2082:
+        // (38 x 197 x 2717 without softmax 33.0 -> 34.6 us, 46 x 352 x 4037 48.5 -> 52.8; up to 300 keys 0.92.  With it where B and C
+        // pass the L2s several times over: 133 x 61 x 1924 33.9 -> 37.7 [L][K], 69 x 99 x 2768 47.5 -> 50.3 [K][L].)
+        return sm ? 2 * d->batch * d->L * (d->K + d->N) <= (kl ? 48 << 20 : 96 << 20) : kl || d->L <= 1024;
+      case 644:  // (117 x 1064 x 32 [K][L] 10.8 -> 11.7 us)
+        if (kl && own == 2148) return false;
+        [[fallthrough]];
+      default: return !sm || dmax > 64;
+    }
+  };
   int best = 0;
-  float own_price = 0, best_price = 0;
-  for (int i = 0; i < count && prices[i].variant != 0; ++i) {
-    const BmmPrice& p = prices[i];
-    const long long wgs = ((d->M + p.rows - 1) / p.rows) * d->batch, full = wgs / (p.resident * cus);
-    const int left = (int)((wgs - full * p.resident * cus + cus - 1) / cus), r = p.resident - 1;
-    const float L = (float)d->L, price = p.start + full * (p.first[r] + p.per_key[r] * L) +
-                                         (left > 0 ? p.first[left - 1] + p.per_key[left - 1] * L : 0.f);
-    if (p.variant == own) own_price = price;
-    // (beyond the lines their prices fit, by 4 - 9 %)
-    if ((p.variant == 2188 && (d->L < 64 || d->L > 700)) || (p.variant == 2144 && d->L <= 64 && !(sm && full > 0))) continue;
-    if (sm && dmax <= 64 && p.variant != 2144) continue;
-    if ((best == 0 || price < best_price) && launchable(wgs, p.threads)) best = p.variant, best_price = price;
-  }
-  return best != own && own_price > 0 && best_price < (sm && dmax <= 64 ? 0.95f : 0.93f) * own_price ? best : 0;
+  float best_price = 0;
+  const float own_price = price(*mine);
+  for (const BmmPrice* p = prices; p != end && p->variant != 0; ++p)
+    if (p != mine && taken(*p) && price(*p) < margin(*p) * own_price && (best == 0 || price(*p) < best_price))
+      best = p->variant, best_price = price(*p);
+  return best;
 }
 
 int plan_bmm_rules(const ditto_bmm_chain_desc* d, BmmPlan* plan, int cus);

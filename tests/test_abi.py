@@ -255,8 +255,9 @@ def test_kernels_are_priced_against_each_other():
     lib = _lib.load()
     tile = _lib.TileParam()
 
-    def plan(batch, M, L, D, inter, layout, variant=0):
-        d = _desc(batch=batch, M=M, N=D, K=D, L=L, inter_op=inter, b_layout=layout, a_batch_stride=M * D, a_row_stride=D,
+    def plan(batch, M, L, D, inter, layout, variant=0, bf16=False):
+        dt = _lib.BF16 if bf16 else _lib.F16
+        d = _desc(in_dtype=dt, out_dtype=dt, batch=batch, M=M, N=D, K=D, L=L, inter_op=inter, b_layout=layout, a_batch_stride=M * D, a_row_stride=D,
                   b_batch_stride=L * D, b_row_stride=L if layout == _lib.B_KL else D, c_batch_stride=L * D, c_row_stride=D,
                   f_batch_stride=M * D, f_row_stride=D, tile_variant=variant)
         for _ in range(2):  # planned, and kept
@@ -274,6 +275,15 @@ def test_kernels_are_priced_against_each_other():
     # one round of 128-row workgroups, several; not: 64 rows, long keys on few rows, a last block of 32 rows in 5 / 4 of a round
     assert plan(329, 197, 128, 64, SM, LK) == 2144 and plan(1152, 512, 512, 64, SM, KL) == 2144 and plan(2100, 96, 96, 64, SM, LK) == 2144
     assert plan(2202, 64, 64, 64, SM, LK) == 644 and plan(830, 192, 2048, 64, SM, LK) == 645 and plan(493, 160, 160, 64, SM, LK) == 644
+    # pairs of kernels whose prices tell the faster one wrongly: the rules' kernel stays
+    assert plan(43, 741, 34, 64, CAST, LK) == 644 and plan(22, 2258, 45, 64, CAST, LK) == 2148  # one and two rounds of 64 rows
+    assert plan(38, 197, 2717, 128, CAST, LK) == 1281 and plan(46, 352, 4037, 128, CAST, LK) == 1281
+    assert plan(160, 515, 512, 128, CAST, KL) == 1289 and plan(22, 2282, 624, 128, CAST, KL) == 1289
+    assert plan(252, 697, 1083, 64, SM, LK) == 645 and plan(42, 3995, 1065, 64, SM, LK) == 645  # fp16; bf16 scales the scores
+    assert plan(252, 697, 1083, 64, SM, LK, bf16=True) == 2144
+    assert plan(133, 61, 1924, 128, SM, LK) == 1281 and plan(69, 99, 2768, 128, SM, KL) == 1281
+    assert plan(147, 1628, 96, 64, CAST, KL) == 2148 and plan(117, 1064, 32, 64, CAST, KL) == 2148
+    assert plan(120, 1160, 1152, 64, SM, KL) == 645
     for M in (100, 300, 1000):
         for L in (64, 500, 1500):
             for batch in (1, 20, 200):
