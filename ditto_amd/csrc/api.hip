@@ -587,14 +587,16 @@ int plan_bmm_rules(const ditto_bmm_chain_desc* d, BmmPlan* plan, int cus) {
     const long long blocks_per_slice = (blocks256 + most_slices - 1) / most_slices;
     // Few rows: the kernel whose waves take units of 64 x 64 weights, with as many workgroups to a row block (slices of its
     // columns) as pay.  Prices in us per launch, least squares over 300 random shapes (64 - 8192 rows, K and N 16 - 1024, L 16 -
-    // 512) with 1 - 6 slices, root mean square error 5 %, the other kernel's over 800, 4 %, up to one round of its workgroups; by
-    // these prices the faster of the two is missed by 0.2 % in the mean, the worst of 640 1.11 (224 x 48 x 208 x 928 7.8 -> 4.8 us,
-    // 256 x 912 x 96 x 800 10.4 -> 6.2, 1120 x 32 x 48 x 16 4.8 -> 3.8).
+    // 512) with 1 - 6 slices, root mean square error 5 %, the other kernel's over 800, 4 %, up to one round of its workgroups.  `pulls`: every
+    // workgroup pulls all of B, and past two units of it a wave on all compute units L2 is the bound, 0.4 us a unit (6 x 208 x 992 x
+    // 368 x 144 14.9 us where the other kernel takes 11.6, 1 x 3456 x 656 x 432 x 16 12.1 / 10.7).  It has to win by 5 %: of 4300 random
+    // shapes that change kernels by that five take more than 1.03 of the other's time, the worst 1.07, the mean 0.78 (224 x 48 x 208 x 928
+    // 7.8 -> 4.8 us, 256 x 912 x 96 x 800 10.4 -> 6.2, 1120 x 32 x 48 x 16 4.8 -> 3.8).
     {
       const double nl = (double)((d->L + 63) / 64), units1 = nl * (double)((d->K + 63) / 64) / 8;
       const long long nbt = (d->N + 63) / 64;
       const double chunks1 = (double)(Lp / 256 * ((d->K + 127) / 128)), chunks2 = (double)((d->L + 127) / 128 * blocks_per_slice);
-      double best = 0.98 * (3.90 + 0.355 * chunks1 + 0.474 * chunks2 + 0.357e-6 * (double)(d->batch * d->M) * (double)d->N +
+      double best = 0.95 * (3.90 + 0.355 * chunks1 + 0.474 * chunks2 + 0.357e-6 * (double)(d->batch * d->M) * (double)d->N +
                             0.289 * (double)(rows32 * ((blocks256 + blocks_per_slice - 1) / blocks_per_slice)) / cus);
       if (d->tile_variant == 8101 || d->tile_variant == 8102) best = 1e30;
       for (int rt = 1; rt <= 2; ++rt) {
@@ -605,9 +607,10 @@ int plan_bmm_rules(const ditto_bmm_chain_desc* d, BmmPlan* plan, int cus) {
           if ((nbt + blocks - 1) / blocks != s || ditto::i8_units_lds_bytes_host(d->L, rt, (int)std::min(blocks, 1LL << 20)) > 160 * 1024) continue;
           if (!launchable(wgs * s, 512)) break;
           const double rounds = (double)((wgs * s + cus - 1) / cus), units2 = nl * (double)blocks / 8, grid = (double)(wgs * s) / cus;
-          const double price = rt == 1 ? 3.17 + rounds * (0.07 + 0.155 * nl + 0.158 * blocks + 0.417 * units1 + 0.206 * units2 +
+          const double pulls = 0.4 * std::max(0.0, grid * units1 - 2);
+          const double price = pulls + (rt == 1 ? 3.17 + rounds * (0.07 + 0.155 * nl + 0.158 * blocks + 0.417 * units1 + 0.206 * units2 +
                                                            0.056 * ceil(units1) + 0.183 * ceil(units2)) + 0.472 * grid
-                                       : 3.5 + rounds * (0.375 * nl + 0.306 * blocks + 0.582 * units1 + 0.474 * units2) + 0.568 * grid;
+                                       : 3.5 + rounds * (0.375 * nl + 0.306 * blocks + 0.582 * units1 + 0.474 * units2) + 0.568 * grid);
           if (price < best) best = price, plan->units_rt = rt, plan->slices = (int)s, plan->slice_blocks = (int)blocks;
         }
       }

@@ -357,3 +357,16 @@ def test_columns_are_shared_out_where_that_pays():
         assert tile.variant // 100 == 20 and tile.block_n == block, (batch, m, l, d, kl, sm, tile.variant, tile.block_n)
         rows = -(-m // 16) * batch
         assert tile.grid_x == rows * -(-d // block) <= 256 or block == d
+
+
+def test_int8_units_only_where_they_win():
+    """Workgroups of a few rows each pull all of B: not where the chunk kernel's ring of 32 rows is as fast."""
+    tile = _lib.TileParam()
+    for batch, m, k, l, n, units in ((6, 208, 992, 368, 144, False), (1, 3456, 656, 432, 16, False), (1, 3264, 640, 144, 32, False),
+                                     (1, 1168, 992, 160, 336, False), (1, 1312, 464, 352, 192, False),
+                                     (1, 224, 48, 208, 928, True), (1, 256, 912, 96, 800, True), (1, 1120, 32, 48, 16, True)):
+        desc = _desc(in_dtype=_lib.I8, acc_dtype=_lib.I32, out_dtype=_lib.I32, inter_op=_lib.INTER_REQUANT, b_layout=_lib.B_KL,
+                     batch=batch, M=m, K=k, L=l, N=n, requant_scale=0.01, a_batch_stride=m * k, a_row_stride=k, b_batch_stride=k * l,
+                     b_row_stride=l, c_batch_stride=l * n, c_row_stride=n, f_batch_stride=m * n, f_row_stride=n)
+        assert _lib.load().ditto_bmm_chain_select_tile(ctypes.byref(desc), ctypes.byref(tile)) == _lib.OK
+        assert (tile.variant // 100 == 81) == units, (m, k, l, n, tile.variant)
