@@ -776,14 +776,15 @@ bool plan_dw_tiles(const ditto_conv_chain_desc* d, long long P, long long Q, Con
   if (lds_of(1) > 160 * 1024) return false;
   // Rows per workgroup.  A workgroup of one pixel tile per wave takes two units alone on a compute unit and three (multiplier
   // 1: 2.6) beside another, one of two tiles 3 and 4.6 (5.2), with two waves to a tile 1.5 and 2.4 (1.9 and 2.3), with four 1.25
-  // and 2 (1.65 and 2); a compute unit holds two.  The height with the fewest units on the busiest compute unit wins, the smaller
+  // and 2 (1.65 and 2.1); a compute unit holds two.  The height with the fewest units on the busiest compute unit wins, the smaller
   // one on ties (32 x 64 x 56 x 56 times 16: one row 63 us, two 38, four 29.5; times 1: 22, 16.2, 18.3; 11 x 64 x 28 x 28 times
-  // 16: one row 13.1, two 10.6, four 13.7; times 1: 7.2, 6.3, 6.7).
+  // 16: one row 13.1, two 10.6, four 13.7; times 1: 7.2, 6.3, 6.7; 22 x 32 x 23 x 23 times 1: one
+  // row 5.8, three 5.2).
   int th = 1;
   double best = 0;
   for (int t = 1; t <= P && t * Q <= slots && lds_of(t) <= 160 * 1024; ++t) {
     const int k = t * Q > 16 * ditto::kDtWaves ? 0 : groups_of(t) == 1 ? 1 : groups_of(t) == 2 ? 2 : 3;
-    static constexpr double kAlone[2][4] = {{3, 2, 1.9, 1.65}, {3, 2, 1.5, 1.25}}, kPair[2][4] = {{5.2, 2.6, 2.3, 2}, {4.6, 3, 2.4, 2}};
+    static constexpr double kAlone[2][4] = {{3, 2, 1.9, 1.65}, {3, 2, 1.5, 1.25}}, kPair[2][4] = {{5.2, 2.6, 2.3, 2.1}, {4.6, 3, 2.4, 2}};
     const double alone = kAlone[mult == 16][k], pair = kPair[mult == 16][k];
     const long long wgs = d->N * ((P + t - 1) / t), per_round = 2LL * lds_of(t) <= 160 * 1024 ? 2 * cus : cus;
     const long long full = wgs / per_round, rest = wgs % per_round;

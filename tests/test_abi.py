@@ -370,3 +370,16 @@ def test_int8_units_only_where_they_win():
                      b_row_stride=l, c_batch_stride=l * n, c_row_stride=n, f_batch_stride=m * n, f_row_stride=n)
         assert _lib.load().ditto_bmm_chain_select_tile(ctypes.byref(desc), ctypes.byref(tile)) == _lib.OK
         assert (tile.variant // 100 == 81) == units, (m, k, l, n, tile.variant)
+
+
+def test_rows_of_a_depthwise_tile():
+    """Rows per workgroup by the units of its busiest compute unit (images, channels, extent, multiplier, stride, rows)."""
+    tile = _lib.TileParam()
+    for n, c, h, mult, stride, rows in ((22, 32, 23, 1, 1, 3), (20, 64, 25, 1, 1, 3), (11, 64, 28, 1, 1, 2), (11, 64, 28, 16, 1, 2),
+                                        (32, 64, 56, 16, 1, 4), (4, 64, 28, 16, 1, 1)):
+        d = _lib.ConvChainDesc()
+        d.abi_version, d.in_dtype, d.out_dtype, d.acc_dtype = _lib.ABI_VERSION, _lib.F16, _lib.F16, _lib.F32
+        d.N, d.C0, d.H, d.W, d.C1, d.R1, d.S1, d.pad1, d.stride1 = n, c, h, h, c * mult, 3, 3, 1, stride
+        d.C2, d.R2, d.S2, d.stride2, d.groups1 = 64, 1, 1, 1, c
+        assert _lib.load().ditto_conv_chain_select_tile(ctypes.byref(d), ctypes.byref(tile)) == _lib.OK
+        assert tile.variant == 4100 + rows, (n, c, h, mult, tile.variant)
