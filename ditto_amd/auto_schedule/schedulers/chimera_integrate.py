@@ -40,8 +40,10 @@ FP_ROWS_KEYS = 1024
 
 
 # int8 chain: 8000 + 10 * (row tiles of 32 per workgroup) + depth of the ring of staged weight chunks; 8100 + row tiles of 16 per
-# workgroup of the kernel for few rows (the library refuses it where the rows are many)
-I8_VARIANTS = (8012, 8014, 8022, 8023, 8101, 8102)
+# workgroup of the kernel for few rows.  Its workgroups each pull all of B, and the library's own choice looks at it up to one
+# block of 32 rows for a compute unit: beyond, it is left out here too (forced, it runs whatever fits LDS and a launch).
+I8_VARIANTS = (8012, 8014, 8022, 8023)
+I8_FEW_ROWS_VARIANTS = (8101, 8102)
 
 
 class TuneEntry:
@@ -76,10 +78,13 @@ def make_tile_variant_space(desc):
     auto.tile_variant = 0
     _lib.check(lib.ditto_bmm_chain_select_tile(ctypes.byref(auto), ctypes.byref(tile)))
     space = [tile.to_json()]
+    groups = int(query_hw_param("gpu.hip.MI355X").num_groups)
     if desc.in_dtype in (_lib.F16, _lib.BF16):
-        ids = _fp_variants(desc, int(query_hw_param("gpu.hip.MI355X").num_groups))
+        ids = _fp_variants(desc, groups)
+    elif desc.in_dtype == _lib.I8:
+        ids = I8_VARIANTS + (I8_FEW_ROWS_VARIANTS if -(-desc.M // 32) * desc.batch <= groups else ())
     else:
-        ids = I8_VARIANTS if desc.in_dtype == _lib.I8 else ()
+        ids = ()
     for variant in ids:
         d = copy.copy(desc)
         d.tile_variant = variant

@@ -242,6 +242,8 @@ def test_tile_variant_space_of_the_kernels_for_many_rows_of_64_columns_and_few_i
 
     few = ci.make_tile_variant_space(i8(688))
     assert {8101, 8102} <= {t["variant"] for t in few}
+    for M, tried in ((8192, True), (8208, False), (20000, False)):  # 256 blocks of 32 rows, 257
+        assert ({8101, 8102} <= {t["variant"] for t in ci.make_tile_variant_space(i8(M))}) == tried, M
     assert all(0 < ci.evaluate_param_hip(i8(688), t) < 1e10 for t in few)
 
 
