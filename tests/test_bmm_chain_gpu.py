@@ -295,6 +295,48 @@ def test_kernel_of_32_rows_per_wave_on_masked_keys(oracle, variant, D, dtype, ke
         assert mx <= 4e-2 and rel <= (REL_L2 if dtype == "float16" else 2.0e-3), (b_layout, mx, rel)
 
 
+# every kernel that takes several chains a launch, alone and with two levels of batch
+@pytest.mark.parametrize("variant,D", [(644, 64), (645, 64), (2041, 64), (2042, 56), (2051, 80), (2052, 72), (2081, 128), (2082, 96),
+                                       (2144, 64), (2148, 64), (2154, 80), (2158, 80), (2188, 128)])
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+@pytest.mark.parametrize("out", ["own", "float32"])
+def test_chains_in_one_launch_on_masked_keys_and_wide_outputs(oracle, variant, D, dtype, out):
+    import ctypes
+
+    from ditto_amd import _lib
+
+    batch, M, L, sets, scale = 4, 75, 280, 3, 0.2
+    out_dtype = "float32" if out == "float32" else dtype
+    dt, lib = TORCH_DTYPES[dtype], _lib.load()
+    for keys in sorted(MASKED_KEYS):
+        data = [masked_scores(oracle, batch, M, D, D, L, dtype, MASKED_KEYS[keys](L), seed=5 * i + D) for i in range(sets)]
+        # A, B as [L][K] and C of a set in one buffer, so that all of them lie equally far from the first set's
+        buf = torch.zeros(sets, batch, M + 2 * L, D, device="cuda", dtype=dt)
+        for i, (A, B, C) in enumerate(data):
+            buf[i] = torch.cat([to_dev(A, dtype), to_dev(np.ascontiguousarray(B.transpose(0, 2, 1)), dtype), to_dev(C, dtype)], 1)
+        f = torch.full((sets, batch, M, D), float("nan"), device="cuda", dtype=TORCH_DTYPES[out_dtype])
+        for inner in (0, 2):
+            x = buf[0].view(2, 2, M + 2 * L, D) if inner else buf[0]
+            y = f[0].view(2, 2, M, D) if inner else f[0]
+            a, b, c = x[..., :M, :], x[..., M:M + L, :].transpose(-1, -2), x[..., M + L:, :]
+            desc = chain.bmm_chain_desc(a, b, c, y, "softmax", scale, 1.0, variant)
+            step = buf[0].numel() * buf.element_size()
+            at = [[t.data_ptr() + i * step for i in range(sets)] for t in (a, b, c)] + [[f[i].data_ptr() for i in range(sets)]]
+            arrays = [(ctypes.c_void_p * sets)(*v) for v in at]
+            assert lib.ditto_bmm_chain_sets_launches(ctypes.byref(desc), sets, *arrays) == 1
+            f.fill_(float("nan"))
+            stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+            assert lib.ditto_bmm_chain_run_sets(ctypes.byref(desc), sets, *arrays, stream) == 0
+            torch.cuda.synchronize()
+            for i, (A, B, C) in enumerate(data):
+                got = f[i].float().cpu().numpy()
+                assert np.isfinite(got).all(), (keys, inner, i)
+                mx, rel = errors(got, oracle.bmm_chain_f64(A, B, C, inter="softmax", scale=scale))
+                # the probabilities' rounding over as little as one key, and the result's own
+                assert mx <= 4e-2 and rel <= (REL_L2 if dtype == "float16" else 2.0e-3 if out == "float32" else REL_L2_BF16_QUANT), \
+                    (keys, inner, i, mx, rel)
+
+
 @pytest.mark.parametrize("shape", [(1, 512, 64, 64, 64), (3, 100, 24, 40, 72), (2, 64, 128, 128, 200)])
 @pytest.mark.parametrize("inter", ["cast", "relu", "softmax"])
 def test_fp32_chain_vs_oracle(oracle, shape, inter):
