@@ -13,7 +13,8 @@
 //
 // Measured, us per launch (2.4 of them the launch), other kernel -> this one: 16 x 176 x 176 x 80 8.4 -> 4.9,
 // 8 x 461 x 461 x 80 12.7 -> 5.9, 2 x 2392 x 2392 x 80 38.5 -> 13.1, 2 x 4096 x 4096 x 128 60.9 -> 28.4,
-// 8 x 512 x 2048 x 64 17.5 -> 8.8, the chain 1 x 512 x 256 x 64 without softmax 4.7 -> 4.05 (3.83 with its columns shared out).
+// 8 x 512 x 2048 x 64 17.5 -> 8.8, the chain 1 x 512 x 256 x 64 without softmax 4.7 -> 4.05 (with its columns shared out the
+// kernel takes 3.72 of 4.45 in a trace; the call, which the launch bounds, the same 4.1 - 4.3).
 //
 // Where two or more workgroups to a row block still leave each a compute unit, they share out the columns of F (CT of the DT
 // tiles each) and repeat the first product: a workgroup then pulls all of B and its columns of C.  21 x 25 x 944 x 128 with softmax

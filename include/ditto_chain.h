@@ -168,7 +168,8 @@ typedef struct ditto_tile_param {
                              short tiles: 2144, 2148, 2154, 2158, 2188 = 2100 + 10 * (head size / 16
                              rounded up likewise) + (waves); conv chains: the ids listed at
                              ditto_conv_chain_desc.tile_variant; fp32 / fp64 1000 / 1001; int8
-                             8000 + 10 * (row tiles of 32) + ring depth */
+                             8000 + 10 * (row tiles of 32) + ring depth, on few rows 8100 + (row tiles
+                             of 16, 1 or 2) */
 } ditto_tile_param;
 
 /* ---- entry points ------------------------------------------------------- */

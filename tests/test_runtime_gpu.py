@@ -364,6 +364,8 @@ def test_layers_that_share_a_launch_match_layers_run_one_by_one(heads, d, batch,
         eng.set_inputs(ins)
         eng.compile()
         assert recorded is None or (eng._graph is not None) == recorded
+        # launches are shared: sixteen layers to one, or as many as a kernel takes
+        assert len(eng._steps) == 1 and eng._steps[0].launches == (2 if (heads, d) == (8, 128) else -(-count // 16))
         for _ in range(3):  # replays with eager work and synchronisations in between
             for o in eng.get_outputs():
                 o.zero_()
