@@ -1536,7 +1536,17 @@ bool plan_sets(const ditto_bmm_chain_desc* d, int n, SetsPlan* out) {
     all.batch_inner = d->batch;
     all.a_batch_stride_outer = all.b_batch_stride_outer = all.c_batch_stride_outer = all.f_batch_stride_outer = 0;
   }
-  if (plan_bmm(&all, &out->plan, true) != DITTO_OK || !plan_takes_sets(out->plan)) return false;
+  if (plan_bmm(&all, &out->plan, true) != DITTO_OK) return false;
+  // A chain that splits its keys by itself does so with others too, 16 | 32 rows a workgroup: every part of the keys has its own
+  // reference, whose probability is exact, and the kernels with one a row are 0.5 - 12 % further from 64 bits (12 x [8 heads, 172
+  // rows of 64] fp16 2.5e-4 against 2.8e-4).  That costs time, up to 3.5 times theirs (12 x [8 heads, 256 rows of 64] 11.7 us against
+  // 6.6, 12 x [16 heads, 197 rows of 80] 33 / 10.6; a launch each 48 and 61), and saves some where they take no sets (12 x [2 heads,
+  // 1024 rows of 128] 34 against 51).
+  if (alone.split_rt > 0 && out->plan.split_rt == 0) {
+    all.tile_variant = alone.tile.variant / 10 * 10 + (d->M <= 16 ? 1 : 2);
+    if (plan_bmm(&all, &out->plan, true) != DITTO_OK) return false;
+  }
+  if (!plan_takes_sets(out->plan)) return false;
   // (the plan of the 64-row kernel does not ask: one chain that a launch does not hold has nowhere to go, several have)
   if (!launchable((long long)out->plan.nb * all.batch, out->plan.tile.block_threads)) return false;
   out->plan.split_ct = 0;  // (the key-splitting kernel for several chains has workgroups of all columns only)

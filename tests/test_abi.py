@@ -90,8 +90,15 @@ def test_chains_that_share_launches_without_gpu():
     assert _sets_launches(_heads(12, 99, 64, tile_variant=641), 5) == 5  # a kernel that takes one chain
     assert _sets_launches(_heads(12, 99, 64), 4, [0, 1 << 24, (1 << 25) + 8, 3 << 24]) == 3
     # together these are so large that a kernel is chosen which takes one chain; fewer of them share a launch all the same
-    assert _sets_launches(_heads(8, 64, 128), 12) <= 3
-    assert _sets_launches(_heads(8, 64, 128), 2) == 1
+    assert _sets_launches(_heads(48, 300, 128), 12) == 3
+    assert _sets_launches(_heads(48, 300, 128), 3) == 1
+    # chains that split their keys by themselves do so together, whatever kernel is chosen for as many rows
+    for entries, rows, d in ((8, 64, 128), (24, 172, 128), (2, 1024, 128), (2, 4096, 64), (48, 16, 80)):
+        alone, together = _lib.TileParam(), _lib.TileParam()
+        for desc, tile in ((_heads(entries, rows, d), alone), (_heads(12 * entries, rows, d), together)):
+            assert _lib.load().ditto_bmm_chain_select_tile(ctypes.byref(desc), ctypes.byref(tile)) == _lib.OK
+        assert alone.variant // 100 == 20 and together.variant // 100 != 20, (entries, rows, d)
+        assert _sets_launches(_heads(entries, rows, d), 12) == 1
     assert _sets_launches(_heads(96, 4096, 128), 6) == 6
 
 

@@ -344,7 +344,7 @@ def _attention_layers(heads, d, batch, M, dtype, count, scale=None):
 # 32 rows per wave, the large ones that take no sets), ragged rows among them
 @pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
 @pytest.mark.parametrize("heads,d,batch,M,count", [(2, 64, 1, 49, 2), (12, 64, 1, 99, 12), (8, 64, 2, 257, 17), (3, 80, 1, 130, 5),
-                                                   (2, 128, 1, 65, 3), (8, 128, 1, 64, 12), (12, 64, 8, 512, 3), (4, 64, 1, 2100, 33)])
+                                                   (2, 128, 1, 65, 3), (8, 128, 1, 64, 12), (48, 128, 1, 300, 12), (12, 64, 8, 512, 3), (4, 64, 1, 2100, 33)])
 def test_layers_that_share_a_launch_match_layers_run_one_by_one(heads, d, batch, M, count, dtype):
     graph, mods = _attention_layers(heads, d, batch, M, dtype, count)
     (func,) = mods.values()
@@ -365,7 +365,7 @@ def test_layers_that_share_a_launch_match_layers_run_one_by_one(heads, d, batch,
         eng.compile()
         assert recorded is None or (eng._graph is not None) == recorded
         # launches are shared: sixteen layers to one, or as many as a kernel takes
-        assert len(eng._steps) == 1 and eng._steps[0].launches == (2 if (heads, d) == (8, 128) else -(-count // 16))
+        assert len(eng._steps) == 1 and eng._steps[0].launches == (3 if heads == 48 else -(-count // 16))
         for _ in range(3):  # replays with eager work and synchronisations in between
             for o in eng.get_outputs():
                 o.zero_()
@@ -449,14 +449,16 @@ def _attention_f64(x, heads, scale):
     q, k, v = x.double().cpu().view(b, m, 3, heads, w // 3 // heads).permute(2, 0, 3, 1, 4).unbind(0)
     return (torch.softmax(scale * (q @ k.transpose(-1, -2)), -1) @ v).permute(0, 2, 1, 3).reshape(b, m, w // 3)
 
-# (8 heads of 172 rows alone are a key-splitting chain, twelve layers together 64-row workgroups; 2100 rows: their form of two
-# key halves)
-@pytest.mark.parametrize("heads,M,count", [(8, 172, 12), (2, 2100, 12)])
+# (112 heads of 400 rows are a chain of 32 rows a wave alone and of 64-row workgroups together; the others by themselves are
+# key-splitting chains, whatever takes all of them together)
+@pytest.mark.parametrize("heads,d,M,count", [(112, 64, 400, 3), (8, 64, 172, 12), (2, 64, 2100, 12), (48, 80, 9, 12), (16, 128, 16, 12), (8, 80, 99, 12),
+                                             (4, 80, 450, 5), (8, 128, 64, 12), (2, 128, 1024, 12), (24, 128, 172, 3)])
 @pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
-def test_layers_that_share_a_launch_are_as_exact_as_alone(heads, M, count, dtype):
+def test_layers_that_share_a_launch_are_as_exact_as_alone(heads, d, M, count, dtype):
     """No operand is rounded that a layer by itself does not round: queries that leave the 16-bit range once they are scaled
-    come out, and the error against 64 bits is no larger than one layer's."""
-    d, scale = 64, 1.0
+    come out, and the error against 64 bits is no larger than one layer's.  Key-splitting chains have an exact probability, the
+    reference, in each part of the keys: together they stay such chains."""
+    scale = 1.0
     graph, mods = _attention_layers(heads, d, 1, M, dtype, count, scale)
     (func,) = mods.values()
     gen = torch.Generator(device="cuda").manual_seed(9)
@@ -476,7 +478,9 @@ def test_layers_that_share_a_launch_are_as_exact_as_alone(heads, M, count, dtype
             rel = [float((t.double().cpu() - want).norm() / want.norm()) for t in (o, alone)]
             # both round every probability and every result once, at most u = 2^-11 | 2^-9 of it each
             assert max(rel) <= (2 * 2 ** -11 if dtype == "float16" else 2 * 2 ** -9), rel
-            # and the same number of times.  The two roundings are of one size, so that the error is sqrt(2) times the result's own
-            # rounding; where a row's largest probabilities are exact, because they are the references of the keys' parts that a
-            # kernel walks apart, it is less, and no less than that one.
-            assert large or rel[0] <= 2 ** 0.5 * rel[1], rel
+            # eight waves with one tile of 32 keys each, on 16 rows or 32: the same sums.  (With more a wave raises the references of
+            # all its rows where one of them calls for it.)
+            assert M > 256 or torch.equal(o, alone), rel
+            # (the two kernels of the 112 heads have one exact probability a row each, and not the same one: at most the largest
+            # one's share of the probabilities' half of the squared error, e^6 / (400 e^2) for normal scores, 0.034 of the error)
+            assert large or rel[0] <= 1.034 * rel[1], rel
