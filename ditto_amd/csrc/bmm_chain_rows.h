@@ -62,7 +62,8 @@ __host__ __device__ constexpr int bmm_chain_rows_lds() {
 inline int bmm_chain_rows_lds(int dt, int nw, bool kl) {
   if (dt == 4 && nw == 4) return kl ? bmm_chain_rows_lds<4, true, 4>() : bmm_chain_rows_lds<4, false, 4>();
   if (dt == 4) return kl ? bmm_chain_rows_lds<4, true, 8>() : bmm_chain_rows_lds<4, false, 8>();
-  if (dt == 5) return kl ? bmm_chain_rows_lds<5, true, 8>() : bmm_chain_rows_lds<5, false, 8>();  // (the same for four waves)
+  if (dt == 5 && nw == 4) return kl ? bmm_chain_rows_lds<5, true, 4>() : bmm_chain_rows_lds<5, false, 4>();
+  if (dt == 5) return kl ? bmm_chain_rows_lds<5, true, 8>() : bmm_chain_rows_lds<5, false, 8>();
   return kl ? bmm_chain_rows_lds<8, true, 8>() : bmm_chain_rows_lds<8, false, 8>();
 }
 
