@@ -1586,10 +1586,11 @@ bool plan_sets(const ditto_bmm_chain_desc* d, int n, SetsPlan* out) {
   if (plan_bmm(&all, &out->plan, true, false) != DITTO_OK) return false;
   // A chain that the rules of plan_bmm have split its keys by itself does so with others too, 16 | 32 rows a workgroup: every part of
   // the keys has its own reference, whose probability is exact, and the kernels with one a row are 0.5 - 12 % further from 64 bits
-  // (12 x [8 heads, 172 rows of 64] fp16 2.5e-4 against 2.8e-4).  (Where few_rows_variant has it do so, the stack stays on the
-  // kernels with one: they were the chain's own until that kernel's start became a matter of less than they cost.)  That costs time, up to 3.5 times theirs (12 x [8 heads, 256 rows of 64] 11.7 us against
-  // 6.6, 12 x [16 heads, 197 rows of 80] 33 / 10.6; a launch each 48 and 61), and saves some where they take no sets (12 x [2 heads,
-  // 1024 rows of 128] 34 against 51).
+  // (12 x [8 heads, 172 rows of 64] fp16 2.5e-4 against 2.8e-4).  That costs time, up to 3.5 times theirs (12 x [8 heads, 256 rows of
+  // 64] 11.7 us against 6.6, 12 x [16 heads, 197 rows of 80] 33 / 10.6; a launch each 48 and 61), and saves some where they take no
+  // sets (12 x [2 heads, 1024 rows of 128] 34 against 51).  Where few_rows_variant has a chain split its keys, the stack stays on the
+  // kernels with one reference a row, which were the chain's own before: as exact as then, and 7 - 10 % (fp16 results) to 25 %
+  // (fp32 ones) further from 64 bits than the chain by itself now.
   if (alone.split_rt > 0 && out->plan.split_rt == 0) {
     all.tile_variant = alone.tile.variant / 10 * 10 + (d->M <= 16 ? 1 : 2);
     if (plan_bmm(&all, &out->plan, true, false) != DITTO_OK) return false;
