@@ -62,8 +62,13 @@ struct F32Lds {
   static __device__ int swz(int row) { return row & 15; }
 };
 
+// Waves of a SIMD that the compiler is held to where its own choice misses them by a few registers: two workgroups of eight waves to
+// a compute unit need 128, and two exact row tiles of 64 columns without softmax, B [L][K], take 130 since their rows come through
+// LDS.  us per launch at 130 / 128: 73 x 1022 x 75 40.3 / 30.9, 44 x 1346 x 169 43.9 / 36.7, 52 x 1057 x 599 96.3 / 86.7; on 50 random shapes
+// 0.88 in the mean, the worst 1.027 (0.92 and 1.006 of what the kernel took without the trip through LDS).
+constexpr int f32_min_waves(int DT, int RT, bool EXACT, bool KL, bool SM) { return DT == 4 && RT == 2 && EXACT && !KL && !SM ? 4 : 1; }
 template <int DT, int RT, bool EXACT, bool KL, bool SM, int W>
-__global__ __launch_bounds__(64 * kWaves) void gemm_chain_f32_kernel(F32ChainArgs p) {
+__global__ __launch_bounds__(64 * kWaves, f32_min_waves(DT, RT, EXACT, KL, SM)) void gemm_chain_f32_kernel(F32ChainArgs p) {
   constexpr int PW = W == 0 || W == 64 ? 4 : W / 16;                   // columns of a lane's piece of a row
   constexpr int G = W == 0 ? DT / 4 : 1, REM = W == 0 ? DT % 4 : 0;  // column groups of 16 PW, column tiles beyond them
   constexpr int NT = PW * G + REM;                                     // column tiles of the workgroup

@@ -11,6 +11,7 @@ invisible in its results:
 * no flat memory instructions: a pointer that has passed through an ``asm`` constraint is no longer known
   to point to global memory or LDS, and flat accesses count on both wait counters.
 """
+import ctypes
 import os
 import re
 import shutil
@@ -18,7 +19,7 @@ import subprocess
 
 import pytest
 
-from ditto_amd import build_ext
+from ditto_amd import _lib, build_ext
 
 CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "ditto_amd", "csrc")
 
@@ -461,3 +462,28 @@ def test_depthwise_tiles_of_one_group_walk_two_pairs_of_channels_a_step(tmp_path
             assert sum("v_mfma" in line for line in lines) == 2 * rt * (2 + nt), name
             seen += 1
     assert seen == 4
+
+
+def test_fp32_chain_of_two_row_tiles_fits_a_compute_unit_twice(tmp_path):
+    """The fp32 kernel for many rows of 64 columns without softmax, B stored [L][K], has few phases that overlap within a workgroup:
+    two workgroups of eight waves to a compute unit, so at most 128 registers, no scratch and half of the LDS."""
+    hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+    if not os.path.exists(hipcc):
+        pytest.skip("hipcc not available")
+    unit = [u for u in build_ext.UNITS if u[0] == "gemm_chain_f32"][0]
+    out = tmp_path / "f32.s"
+    flags = [f for f in build_ext.HIPCC_FLAGS if f != "-fPIC"]
+    cmd = [hipcc, *flags, "--cuda-device-only", "-S", *unit[2], os.path.join(CSRC, unit[1]), "-o", str(out)]
+    subprocess.run(cmd, check=True, capture_output=True)
+    text = out.read_text()
+    name = [k for k in kernel_metadata(text) if "gemm_chain_f32_kernelILi4ELi2ELb1ELb0ELb0ELi0EE" in k]
+    assert len(name) == 1 and kernel_metadata(text)[name[0]] == {"private_segment_fixed_size": 0, "vgpr_spill_count": 0}
+    registers = re.search(r"\.name:\s+%s\n.*?\.vgpr_count:\s+(\d+)" % re.escape(name[0]), text, re.S)
+    assert int(registers.group(1)) <= 128
+    d, tile = _lib.BmmChainDesc(), _lib.TileParam()
+    d.abi_version, d.in_dtype, d.out_dtype, d.acc_dtype, d.b_layout = _lib.ABI_VERSION, _lib.F32, _lib.F32, _lib.F32, _lib.B_LK
+    d.inter_op, d.batch, d.M, d.N, d.K, d.L = _lib.INTER_CAST, 64, 512, 64, 64, 512
+    d.a_row_stride = d.b_row_stride = d.c_row_stride = d.f_row_stride = 64
+    d.a_batch_stride = d.b_batch_stride = d.c_batch_stride = d.f_batch_stride = 512 * 64
+    _lib.check(_lib.load().ditto_bmm_chain_select_tile(ctypes.byref(d), ctypes.byref(tile)))
+    assert tile.block_m == 32 and 2 * tile.lds_bytes <= 160 * 1024
