@@ -584,12 +584,21 @@ int plan_bmm_rules(const ditto_bmm_chain_desc* d, BmmPlan* plan, int cus) {
     // (every B and C fragment fetched from L2 feeds two row tiles), and the fewer rounds over the compute units win.
     // Measured, us per launch, 16 / 32 rows: 12 x 512 x 512 x 64 14.4 / 12.9, 1 x 512 x 512 x 64 7.3 / 13.2,
     // 16 x 700 x 700 x 64 28.3 / 32.2, 64 x 512 x 512 x 64 49.9 / 49.5.  B stored [K][L] does not come through LDS and gains more from
-    // feeding two row tiles: from 5 rounds against 3 on (44 x 428 x 112 x 64 19.6 / 16.7, 42 x 431 x 521 x 64 44.5 / 41.5; twelve shapes of
-    // 64 columns 0.93 in the mean, the worst 0.99; 8 against 5 0.87 - 1.03), and from 7 against 4 with columns that are no
-    // whole tiles (52 x 469 x 51 x 64 21.5 / 16.3, 45 x 620 x 142 x 56 56.9 / 51.3; [L][K] there 1.12 - 1.16).  Beyond 80 columns two row tiles
-    // do not fit the registers.
+    // feeding two row tiles: from 5 rounds against 3 on (44 x 428 x 112 x 64 19.6 / 16.7, 42 x 431 x 521 x 64 44.5 / 41.5; forty shapes of
+    // 64 and 80 columns 0.93 in the mean, the worst 1.02; 8 against 5 0.87 - 1.03).  Rows that are loaded element by element do so with
+    // softmax up to 64 columns (27 x 630 x 264, 48 -> 64 51.3 / 45.8; 16 shapes 0.85 - 0.91) and without it beyond (38 x 457 x 246,
+    // 80 -> 64 60.4 / 55.0; 15 shapes 0.82 - 0.96); with columns that are no whole tiles from 7 against 4 on (41 x 664 x 462 x 43 85.4 /
+    // 73.3, 44 x 575 x 131 x 72 65.0 / 58.6; [L][K] there 1.12 - 1.16).  Without softmax up to 64 columns the loads of one row tile
+    // overlap better (42 x 642 x 149 x 32 31.7 / 37.3, 20 x 1292 x 87 x 56 37.2 / 42.4; 16 shapes 1.07 in the mean), and with softmax
+    // beyond, where two spill registers, it takes some 200 keys to make up for that (18 x 978 x 125, 80 -> 64 47.3 / 50.8, 41 x 603 x
+    // 92, 68 -> 75 47.0 / 50.4; 21 x 1236 x 466 x 72 124 / 113): 9 rounds against 5 there, as with [L][K].  Beyond 80 columns two row
+    // tiles do not fit the registers.
     auto rounds = [&](int rows) { return (((d->M + rows - 1) / rows) * d->batch + cus - 1) / cus; };
-    const double worth = d->b_layout != DITTO_B_KL ? 1.8 : d->K % 16 || d->N % 16 ? 1.7 : 1.65;
+    const bool wide = d->K > 64 || d->N > 64;
+    const bool exact = ditto::f32_chain_exact((int)d->K, (int)d->N, d->a_batch_stride | d->c_batch_stride | d->f_batch_stride |
+                                                                        d->a_row_stride | d->c_row_stride | d->f_row_stride);
+    const bool gains = exact || (d->inter_op == DITTO_INTER_SOFTMAX ? !wide || d->L > 200 : wide);
+    const double worth = d->b_layout != DITTO_B_KL || !gains ? 1.8 : d->K % 16 || d->N % 16 ? 1.7 : 1.65;
     plan->qt = !f64 && (d->K > 80 || d->N > 80 || (double)rounds(16) < worth * (double)rounds(32)) ? 1 : 2;
     plan->f32_width = f64 || plan->qt != 1 ? 0 : ditto::f32_chain_width((int)d->K, (int)d->N, ((d->M + 15) / 16) * d->batch, cus);
     plan->f32_cols = plan->f32_width ? (int)((d->N + plan->f32_width - 1) / plan->f32_width) : 1;

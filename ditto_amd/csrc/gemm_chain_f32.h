@@ -27,6 +27,7 @@ struct F32ChainArgs {
 
 int f32_chain_lds_bytes_host(int K, int N, int f64, int row_tiles, int width);
 int f32_chain_width(int K, int N, long long row_blocks, int cus);
+bool f32_chain_exact(int K, int N, long long strides);  // whole tiles of columns and rows in 16-byte pieces; the strides ORed together
 int f32_chain_max_dim();  // largest K and N the kernels take
 hipError_t launch_gemm_chain_f32(const F32ChainArgs& args, hipStream_t stream);
 

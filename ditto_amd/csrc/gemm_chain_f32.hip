@@ -490,6 +490,10 @@ int f32_chain_lds_bytes_host(int K, int N, int f64, int rt, int width) {
   if (rt == 2) return dt == 4 ? f32_lds_bytes<4, 2>(width) : f32_lds_bytes<5, 2>(width);
   return dt == 4 ? f32_lds_bytes<4, 1>(width) : dt == 5 ? f32_lds_bytes<5, 1>(width) : f32_lds_bytes<8, 1>(width);
 }
+bool f32_chain_exact(int K, int N, long long strides) {
+  const int columns = 16 * f32_tiles(K, N);
+  return K == columns && N == columns && strides % 4 == 0;
+}
 // The columns a workgroup owns, 0 for all: the fewest that leave every workgroup a compute unit of its own.
 int f32_chain_width(int K, int N, long long row_blocks, int cus) {
   const int dt = f32_tiles(K, N);
@@ -561,7 +565,7 @@ hipError_t launch_gemm_chain_f32(const F32ChainArgs& a, hipStream_t stream) {
   // 16-byte pieces of the rows of A, B (stored [L][K]), C and F; a [K][L] B is read one element per lane either way
   long long strides = a.a_bs | a.c_bs | a.f_bs | a.a_rs | a.c_rs | a.f_rs;
   if (a.b_lk) strides |= a.b_bs | a.b_rs;
-  const bool exact = a.K == 16 * dt && a.N == 16 * dt && strides % 4 == 0;
+  const bool exact = f32_chain_exact(a.K, a.N, strides);
   return dt == 4 ? launch_f32_rows<4>(a, exact, stream)
          : dt == 5 ? launch_f32_rows<5>(a, exact, stream)
                    : launch_f32_rows<8>(a, exact, stream);

@@ -471,16 +471,35 @@ def test_fp32_chain_staged_through_lds(shape, inter):
 @pytest.mark.parametrize("shape", [(44, 429, 64, 111), (52, 469, 64, 51), (45, 621, 56, 65), (31, 813, 80, 130)])  # (batch, M, columns, L)
 @pytest.mark.parametrize("inter", ["relu", "softmax"])
 def test_fp32_chain_of_two_row_tiles_a_workgroup(shape, inter):
-    """B stored [K][L] on 5 rounds of 16-row workgroups against 3 of 32-row ones, and 7 against 4: the 32-row ones run, and give what
-    64 bits give within the fp32 chain's bound."""
+    """B stored [K][L] on 5 rounds of 16-row workgroups against 3 of 32-row ones, and 7 against 4: the 32-row ones run (but for columns
+    that are no whole tiles without softmax, up to 64 of them), and give what 64 bits give within the fp32 chain's bound."""
     batch, M, D, L = shape
     gen = torch.Generator(device="cuda").manual_seed(M)
     a, b, c = (torch.randn(batch, *s, device="cuda", generator=gen) for s in ((M, D), (D, L), (L, D)))
     f = torch.full((batch, M, D + 4), float("nan"), device="cuda")[:, :, :D]
     chain.run_bmm_chain(a, b, c, f, inter, 0.2)
-    assert chain.select_tile(chain.bmm_chain_desc(a, b, c, f, inter, 0.2)).block_m == 32
+    assert chain.select_tile(chain.bmm_chain_desc(a, b, c, f, inter, 0.2)).block_m == (16 if D == 56 and inter == "relu" else 32)
     s = torch.bmm(a.double(), b.double())
     want = torch.bmm(torch.softmax(s * 0.2, -1) if inter == "softmax" else s.relu(), c.double())
+    assert torch.isfinite(f).all() and ((f.double() - want).norm() / want.norm()).item() <= 1e-5
+
+
+@pytest.mark.parametrize("K,N,L,inter,pad,rows", [
+    # 7 rounds of 16-row workgroups against 4 of 32: element by element up to 64 columns and beyond, with softmax on either side of 200 keys
+    (72, 72, 142, "softmax", 0, 16), (68, 75, 200, "softmax", 0, 16), (72, 72, 201, "softmax", 0, 32), (80, 64, 65, "softmax", 0, 16),
+    (64, 80, 33, "cast", 0, 32), (65, 65, 17, "relu", 0, 32), (80, 80, 40, "softmax", 1, 16), (80, 80, 40, "softmax", 4, 32),
+    (32, 32, 149, "relu", 0, 16), (63, 64, 31, "softmax", 0, 32), (64, 64, 50, "cast", 1, 16), (64, 64, 50, "cast", 4, 32),
+])
+def test_fp32_rows_loaded_element_by_element(K, N, L, inter, pad, rows):
+    """Two row tiles a workgroup only where they are ahead (`pad`: elements behind the rows of C), within the fp32 chain's bound."""
+    gen = torch.Generator(device="cuda").manual_seed(K + L)
+    a, b, c = (torch.randn(45, *s, device="cuda", generator=gen) for s in ((619, K), (K, L), (L, N + pad)))
+    c[:, :, N:] = float("nan")
+    c, f = c[:, :, :N], torch.full((45, 619, N), float("nan"), device="cuda")
+    chain.run_bmm_chain(a, b, c, f, inter, 0.2)
+    assert chain.select_tile(chain.bmm_chain_desc(a, b, c, f, inter, 0.2)).block_m == rows
+    s = torch.bmm(a.double(), b.double())
+    want = torch.bmm(torch.softmax(s * 0.2, -1) if inter == "softmax" else s.relu() if inter == "relu" else s, c.double().contiguous())
     assert torch.isfinite(f).all() and ((f.double() - want).norm() / want.norm()).item() <= 1e-5
 
 
