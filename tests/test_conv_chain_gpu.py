@@ -975,6 +975,17 @@ def test_halo_rows_staged_by_neighbouring_lanes(oracle, case):
 
 
 @pytest.mark.parametrize("case", [
+    # N, C0, H, W, C1, R, pad, stride, C2: one, two and three groups of eight pixels behind the last four, alone and behind others, rows of
+    # whole vectors and not, tasks below, at and above the threads of a workgroup
+    (1, 64, 1, 16, 16, 1, 0, 1, 16), (1, 64, 1, 24, 16, 1, 0, 1, 16), (1, 192, 1, 17, 16, 1, 0, 1, 16), (1, 96, 3, 40, 32, 1, 0, 1, 17),
+    (1, 192, 1, 66, 64, 1, 0, 1, 16), (3, 96, 6, 54, 64, 3, 1, 2, 8), (1, 192, 7, 20, 32, 3, 1, 1, 32), (2, 256, 11, 11, 32, 1, 0, 1, 32),
+    (1, 192, 22, 22, 192, 3, 1, 2, 64), (1, 192, 43, 24, 8, 3, 1, 2, 32),
+])
+def test_last_groups_of_the_halo_rows(oracle, case):
+    test_conv_chain_on_row_tiles(oracle, case, "float16")
+
+
+@pytest.mark.parametrize("case", [
     # N, C0, H, W, C1, R, pad, stride, C2: two, four and eight pixels to a lane of the second convolution, full and ragged, by each split of the
     # waves; one tile of output channels (no gap between the lanes' pixels in LDS) and more
     (1, 32, 1, 32, 64, 1, 0, 1, 17), (1, 32, 1, 33, 64, 1, 0, 1, 16), (2, 32, 3, 64, 64, 3, 1, 1, 80), (1, 64, 2, 65, 64, 3, 1, 1, 24),
