@@ -203,10 +203,13 @@ int cheaper_variant(const ditto_bmm_chain_desc* d, int own, int cus) {
 // plan_bmm weigh it at what it took before its rows of A came through LDS, and know no shares of the columns.  2.3 us and, for
 // every round of workgroups, a start and a share of the keys; fitted to 2200 random shapes (root mean square error 4 % at 64
 // columns, 7 at 128).  us per launch: 5 x 256 x 224 x 64 [K][L] 5.05 -> 3.96, 3 x 166 x 166 x 64 4.35 -> 3.76, 1 x 512 x 96 x 64 without
-// softmax 3.68 -> 3.22; 3 x 1552 x 272 x 128 [K][L] 10.9 -> 7.9, 13 x 608 x 256 x 128 without softmax 8.2 -> 6.7.  Of 1640 other
-// shapes at 128 columns 4 % change, to 0.87 of the time, the worst 0.98; of 780 at 64 columns 12 %, to 0.89, the worst 1.04.  Up to
+// softmax 3.68 -> 3.22; 3 x 1552 x 272 x 128 [K][L] 10.9 -> 7.9, 13 x 608 x 256 x 128 without softmax 8.2 -> 6.7.  Of 9300 other
+// shapes at 128 columns 3 % change, to 0.83 of the time, the worst 0.98; of 8200 at 64 columns 11 %, to 0.88, the worst 1.00.  Up to
 // 64 keys, and from 1600 keys on at 128 columns, the price misses by more than there is to gain (1 x 2848 x 64 x 64 1.075, 81 x 64 x 64 x
-// 128 0.99, 6 x 1808 x 3888 x 128 1.025).
+// 128 0.99, 6 x 1808 x 3888 x 128 1.025).  So it does, for 32 rows a workgroup, up to 128 keys of [K][L] without softmax at 64 columns
+// (nine shapes 1.01 - 1.05: 7 x 926 x 112 x 24 3.82 -> 4.00, 2 x 3309 x 120 x 64 4.00 -> 4.12; 5 x 1358 x 136 0.95), and for a second
+// round of workgroups at 128 columns where B and C of the batch do not fit the L2s, 32 MB in all (99 x 78 x 1312 [K][L] 22.0 -> 24.6,
+// 132 x 63 x 1228 25.5 -> 27.3, eight shapes of 55 MB and more 0.93 - 1.11; below 33 MB 0.89 - 0.98).
 int few_rows_variant(const ditto_bmm_chain_desc* d, int own, int cus) {
   const long long dmax = d->K > d->N ? d->K : d->N;
   if (dmax > 64 && dmax <= 80) return 0;
@@ -229,6 +232,7 @@ int few_rows_variant(const ditto_bmm_chain_desc* d, int own, int cus) {
   for (int rt = 1; rt <= 2; ++rt) {
     const long long wgs = ((d->M + 16 * rt - 1) / (16 * rt)) * d->batch, rounds = (wgs + cus - 1) / cus;
     if (!launchable(wgs, 64 * ditto::kSplitWaves)) continue;
+    if (dmax <= 64 ? rt == 2 && kl && !sm && d->L <= 128 : rounds > 1 && 2 * d->batch * d->L * (d->K + d->N) > 32 << 20) continue;
     const float cost = 2.3f + rounds * (split[rt - 1].first + split[rt - 1].per_key * per_kl * (float)d->L);
     if (cost < best) best = cost, variant = (dmax <= 64 ? 2040 : 2080) + rt;
   }
