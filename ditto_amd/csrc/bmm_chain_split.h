@@ -97,12 +97,29 @@ __global__ __launch_bounds__(64 * kSplitWaves) void bmm_chain_split_kernel(Args 
   // 16 bytes lie in another line, for each of which the address unit spends a cycle, in front of the first keys (20 x 304 x 752 x 128
   // with softmax 12.8 -> 10.1 us, 5 x 1248 x 624 x 128 12.6 -> 9.3, 2 x 77 x 77 x 128 4.7 -> 4.0, at 64 columns 0.95 of the time).  Rows past M
   // repeat the last one; columns past K are loaded from column 0 and replaced by zeros below.
+  // Not 16 rows of 65 to 80 columns with B [L][K] and no softmax, whose short start the detour through LDS and the barrier make longer
+  // by more than ten 16-byte pieces a row save: 53 x 133 x 372 x 80 8.49 us through LDS, 7.87 direct, 1 x 105 x 956 x 80 5.27 / 4.92; 175
+  // random shapes 1.017 - 1.06 by keys (rows a packed tensor apart 0.95 - 1.00; with softmax 0.98 - 1.01, packed 0.94 - 0.97).
+  constexpr bool kStagedA = !(DT == 5 && RT == 1 && !B_KL && !kSoftmax);
   typedef SplitRows<DT, RT> R;
   char* const rows_of_a = smem_sp + kSplitWaves * S::BYTES;
-  if (w < R::LOADS) {
+  if (kStagedA && w < R::LOADS) {
     const int ch = 64 * w + lane, row = min(ch / R::CPR, 16 * RT - 1), pc = ch - row * R::CPR, lc = S::POW2 ? pc ^ swz_rows(row) : pc;
     lds_dma_16_from(Ag + (long long)min(m0 + row, M - 1) * p.a_rs + (8 * lc < K ? 8 * lc : 0),
                     (unsigned)(size_t)(DITTO_LDS char*)rows_of_a + 1024 * w);
+  }
+  // A fragments (operand column = row of A); with B stored [K][L] in the contraction order its transposing reads give
+  V8 af[RT][KS];
+  if constexpr (!kStagedA) {
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+      for (int s = 0; s < KS; ++s) {
+        const int k = 32 * s + 8 * q;
+        const V8 none = {0, 0, 0, 0, 0, 0, 0, 0};
+        const V8 v = *reinterpret_cast<const V8*>(Ag + (long long)min(m0 + 16 * rt + c, M - 1) * p.a_rs + (k < K ? k : 0));
+        af[rt][s] = k < K ? v : none;
+      }
   }
 
   // source offsets of the lane's chunks relative to the step's first key; what is not there reads as zero (out of range)
@@ -179,28 +196,36 @@ __global__ __launch_bounds__(64 * kSplitWaves) void bmm_chain_split_kernel(Args 
   const float c2 = p.scale_log2;
 
   load_b(w);
-  load_c(w);
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(S::B_LOADS + S::C_LOADS) : "memory");
-  lds_barrier();
-  // A fragments (operand column = row of A); with B stored [K][L] in the contraction order its transposing reads give
-  V8 af[RT][KS];
+  if constexpr (kStagedA) {
+    load_c(w);
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(S::B_LOADS + S::C_LOADS) : "memory");
+    lds_barrier();
 #pragma unroll
-  for (int rt = 0; rt < RT; ++rt) {
-    const char* const row = rows_of_a + (16 * rt + c) * (16 * R::CPR);
-    const int swz = S::POW2 ? swz_rows(c) : 0;
+    for (int rt = 0; rt < RT; ++rt) {
+      const char* const row = rows_of_a + (16 * rt + c) * (16 * R::CPR);
+      const int swz = S::POW2 ? swz_rows(c) : 0;
 #pragma unroll
-    for (int s = 0; s < KS; ++s) {
-      if constexpr (B_KL) {
-        const int k = 32 * s + 4 * q, ch = 4 * s + (q >> 1), half = 8 * (q & 1);
-        const V4 lo = *reinterpret_cast<const V4*>(row + (ch ^ swz) * 16 + half), hi = *reinterpret_cast<const V4*>(row + ((ch + 2) ^ swz) * 16 + half);
-        const V4 none = {0, 0, 0, 0};
-        af[rt][s] = concat4<V4, V8>(k < K ? lo : none, k + 16 < K ? hi : none);
-      } else {
-        const int k = 32 * s + 8 * q;
-        const V8 v = *reinterpret_cast<const V8*>(row + ((4 * s + q) ^ swz) * 16), none = {0, 0, 0, 0, 0, 0, 0, 0};
-        af[rt][s] = k < K ? v : none;
+      for (int s = 0; s < KS; ++s) {
+        if constexpr (B_KL) {
+          const int k = 32 * s + 4 * q, ch = 4 * s + (q >> 1), half = 8 * (q & 1);
+          const V4 lo = *reinterpret_cast<const V4*>(row + (ch ^ swz) * 16 + half), hi = *reinterpret_cast<const V4*>(row + ((ch + 2) ^ swz) * 16 + half);
+          const V4 none = {0, 0, 0, 0};
+          af[rt][s] = concat4<V4, V8>(k < K ? lo : none, k + 16 < K ? hi : none);
+        } else {
+          const int k = 32 * s + 8 * q;
+          const V8 v = *reinterpret_cast<const V8*>(row + ((4 * s + q) ^ swz) * 16), none = {0, 0, 0, 0, 0, 0, 0, 0};
+          af[rt][s] = k < K ? v : none;
+        }
       }
     }
+  } else {
+    // the fragments are named between the first direct loads: the compiler's wait for them then falls here, once, and not at their
+    // first use inside the loop, where it would wait for the prefetches as well
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+      for (int s = 0; s < KS; ++s) asm volatile("" : "+v"(af[rt][s]));
+    load_c(w);
   }
   for (int step = w; step < nsteps; step += kSplitWaves) {
     // this step's B tile has landed (its C tile, requested after it, may still be on its way)

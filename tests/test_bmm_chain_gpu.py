@@ -174,6 +174,25 @@ def test_key_splitting_kernel_takes_nothing_from_beside_its_rows(K, b_layout):
             assert torch.isfinite(f).all() and torch.equal(f, g), (M, rows)
 
 
+@pytest.mark.parametrize("K", [72, 80])
+@pytest.mark.parametrize("inter", ["cast", "relu"])
+def test_key_splitting_kernel_loads_its_rows_directly(K, inter):
+    """16 rows of 65 to 80 columns, B stored [L][K], no softmax: the rows of A take no detour through LDS.  NaN between and behind
+    them stays out, the result is the bits of contiguous rows, and the columns' sums are those of 64 bits."""
+    gen = torch.Generator(device="cuda").manual_seed(K)
+    for M, L in ((1, 31), (16, 32), (17, 257), (70, 300), (300, 600)):
+        a, k, v = (torch.randn(2, n, K, device="cuda", generator=gen).half() * 0.25 for n in (M, L, L))
+        view = torch.full((2, M + 16, K + 8), float("nan"), device="cuda", dtype=torch.float16)[:, :M, :K]
+        view.copy_(a)
+        f, g = (torch.full((2, M, K), float("nan"), device="cuda") for _ in range(2))
+        chain.run_bmm_chain(a, k.transpose(1, 2), v, f, inter, tile_variant=2051)
+        chain.run_bmm_chain(view, k.transpose(1, 2), v, g, inter, tile_variant=2051)
+        s = torch.bmm(a.float(), k.float().transpose(1, 2).contiguous()).half().double()
+        want = torch.bmm(s.relu() if inter == "relu" else s, v.double())
+        # the middle result's rounding alone: 2^-11 of it, and its ties
+        assert torch.equal(f, g) and ((f.double() - want).norm() / want.norm()).item() <= 2.0 ** -11, (M, L)
+
+
 @pytest.mark.parametrize("K,variant", [(8, 2144), (64, 2144), (56, 2148), (72, 2154), (80, 2158), (88, 2188), (128, 2188)])
 @pytest.mark.parametrize("b_layout", ["KL", "LK"])
 def test_kernel_of_32_rows_a_wave_takes_nothing_from_beside_its_rows(K, variant, b_layout):
