@@ -43,7 +43,7 @@ constexpr unsigned kLaunchBlocks = 1u << 22;  // most fp32 workgroups of one lau
 // DT: column tiles of 16 that K and N are padded to.  EXACT: K = N = 16 DT and every row starts on a 16-byte boundary;
 // otherwise elements are loaded one by one and columns past K or N are zeros.
 //
-// EXACT, 64 or 128 columns: A and, with B stored [L][K], the steps' keys come through LDS.  Fetched the way the MFMA wants them, every
+// EXACT, 64 or 128 columns, but for f32_direct: A and, with B stored [L][K], the steps' keys come through LDS.  Fetched the way the MFMA wants them, every
 // lane's 16 bytes lie in another row, and the address unit, which takes four lanes at a time and spends a cycle on every line they
 // touch, was busy for 14 thousand of the 27 thousand cycles of 12 x 512 x 512 x 64; rows end to end take a quarter of that.  us per
 // launch before / here: 12 x 512 x 512 x 64 14.9 / 14.3, 8 x 627 x 61 x 64 5.7 / 5.0, 1 x 729 x 995 x 128 21.2 / 18.2, 5 x 1009 x 341
@@ -67,14 +67,15 @@ struct F32Lds {
 // LDS.  us per launch at 130 / 128: 73 x 1022 x 75 40.3 / 30.9, 44 x 1346 x 169 43.9 / 36.7, 52 x 1057 x 599 96.3 / 86.7; on 50 random shapes
 // 0.88 in the mean, the worst 1.027 (0.92 and 1.006 of what the kernel took without the trip through LDS).
 constexpr int f32_min_waves(int DT, int RT, bool EXACT, bool KL, bool SM) { return DT == 4 && RT == 2 && EXACT && !KL && !SM ? 4 : 1; }
-template <int DT, int RT, bool EXACT, bool KL, bool SM, int W>
+// DIRECT: for chains that f32_direct names, nothing but the merge through LDS.
+template <int DT, int RT, bool EXACT, bool KL, bool SM, int W, bool DIRECT>
 __global__ __launch_bounds__(64 * kWaves, f32_min_waves(DT, RT, EXACT, KL, SM)) void gemm_chain_f32_kernel(F32ChainArgs p) {
   constexpr int PW = W == 0 || W == 64 ? 4 : W / 16;                   // columns of a lane's piece of a row
   constexpr int G = W == 0 ? DT / 4 : 1, REM = W == 0 ? DT % 4 : 0;  // column groups of 16 PW, column tiles beyond them
   constexpr int NT = PW * G + REM;                                     // column tiles of the workgroup
   typedef F32Lds<DT, RT, W> S;
   constexpr int ORS = S::ORS;
-  constexpr bool kStagedA = EXACT && DT != 5, kStaged = kStagedA && !KL;
+  constexpr bool kStagedA = EXACT && DT != 5 && !DIRECT, kStaged = kStagedA && !KL;
   static_assert(ORS == 16 * NT + 4, "the columns of a workgroup");
   typedef __attribute__((ext_vector_type(PW == 1 ? 2 : PW))) float Piece;
   static_assert(REM <= 1, "columns beyond the groups of 64: at most one tile of 16");
@@ -527,17 +528,25 @@ static hipError_t launch_with_lds(Kernel kernel, unsigned threads, int lds, cons
   return e;
 }
 
-template <int DT, int RT, bool EXACT, bool KL, bool SM, int W>
+template <int DT, int RT, bool EXACT, bool KL, bool SM, int W, bool DIRECT>
 struct F32Tag {};
+
+// Chains without softmax on up to 24 keys (16 with two row tiles), B [L][K]: one wave or two have a step, too short for the trip through
+// LDS to pay.  us per launch through LDS / direct: 24 x 1348 x 8 x 64 10.3 / 8.9, 3 x 74 x 9 x 128 3.38 / 2.98, 31 x 879 x 9 x 128 22.1 /
+// 19.9; by columns and keys 1.02 - 1.16 up to 24, 0.96 - 1.01 from 25 to 32.
+static bool f32_direct(const F32ChainArgs& a) { return !a.softmax && a.b_lk && a.L <= (a.row_tiles == 1 ? 24 : 16); }
 
 template <int DT, int RT, bool EXACT, int W>
 static hipError_t launch_f32(const F32ChainArgs& a, hipStream_t stream) {
   const int lds = f32_chain_lds_bytes_host(a.K, a.N, 0, RT, W), threads = 64 * kWaves;
   if (a.softmax)
-    return a.b_lk ? launch_with_lds<F32Tag<DT, RT, EXACT, false, true, W>>(gemm_chain_f32_kernel<DT, RT, EXACT, false, true, W>, threads, lds, a, stream)
-                  : launch_with_lds<F32Tag<DT, RT, EXACT, true, true, W>>(gemm_chain_f32_kernel<DT, RT, EXACT, true, true, W>, threads, lds, a, stream);
-  return a.b_lk ? launch_with_lds<F32Tag<DT, RT, EXACT, false, false, W>>(gemm_chain_f32_kernel<DT, RT, EXACT, false, false, W>, threads, lds, a, stream)
-                : launch_with_lds<F32Tag<DT, RT, EXACT, true, false, W>>(gemm_chain_f32_kernel<DT, RT, EXACT, true, false, W>, threads, lds, a, stream);
+    return a.b_lk ? launch_with_lds<F32Tag<DT, RT, EXACT, false, true, W, false>>(gemm_chain_f32_kernel<DT, RT, EXACT, false, true, W, false>, threads, lds, a, stream)
+                  : launch_with_lds<F32Tag<DT, RT, EXACT, true, true, W, false>>(gemm_chain_f32_kernel<DT, RT, EXACT, true, true, W, false>, threads, lds, a, stream);
+  if constexpr (EXACT && DT != 5)
+    if (f32_direct(a))
+      return launch_with_lds<F32Tag<DT, RT, true, false, false, W, true>>(gemm_chain_f32_kernel<DT, RT, true, false, false, W, true>, threads, lds, a, stream);
+  return a.b_lk ? launch_with_lds<F32Tag<DT, RT, EXACT, false, false, W, false>>(gemm_chain_f32_kernel<DT, RT, EXACT, false, false, W, false>, threads, lds, a, stream)
+                : launch_with_lds<F32Tag<DT, RT, EXACT, true, false, W, false>>(gemm_chain_f32_kernel<DT, RT, EXACT, true, false, W, false>, threads, lds, a, stream);
 }
 
 template <int DT, bool EXACT>

@@ -487,6 +487,13 @@ def test_fp32_chain_staged_through_lds(shape, inter):
     assert torch.isfinite(got[0]).all() and torch.equal(got[0], got[1]) and torch.equal(got[0], got[2])
 
 
+@pytest.mark.parametrize("shape", [  # (batch, M, columns, L): on either side of the keys up to which rows are loaded directly
+    (3, 33, 64, 16), (40, 90, 64, 24), (40, 90, 64, 25), (2, 50, 128, 24), (2, 50, 128, 25), (50, 90, 128, 23), (13, 500, 64, 16), (13, 500, 64, 17)])
+@pytest.mark.parametrize("inter", ["cast", "relu"])
+def test_fp32_chain_of_few_keys(shape, inter):
+    test_fp32_chain_staged_through_lds(shape, inter)
+
+
 @pytest.mark.parametrize("shape", [(44, 429, 64, 111), (52, 469, 64, 51), (45, 621, 56, 65), (31, 813, 80, 130)])  # (batch, M, columns, L)
 @pytest.mark.parametrize("inter", ["relu", "softmax"])
 def test_fp32_chain_of_two_row_tiles_a_workgroup(shape, inter):

@@ -476,7 +476,7 @@ def test_fp32_chain_of_two_row_tiles_fits_a_compute_unit_twice(tmp_path):
     cmd = [hipcc, *flags, "--cuda-device-only", "-S", *unit[2], os.path.join(CSRC, unit[1]), "-o", str(out)]
     subprocess.run(cmd, check=True, capture_output=True)
     text = out.read_text()
-    name = [k for k in kernel_metadata(text) if "gemm_chain_f32_kernelILi4ELi2ELb1ELb0ELb0ELi0EE" in k]
+    name = [k for k in kernel_metadata(text) if "gemm_chain_f32_kernelILi4ELi2ELb1ELb0ELb0ELi0ELb0EE" in k]
     assert len(name) == 1 and kernel_metadata(text)[name[0]] == {"private_segment_fixed_size": 0, "vgpr_spill_count": 0}
     registers = re.search(r"\.name:\s+%s\n.*?\.vgpr_count:\s+(\d+)" % re.escape(name[0]), text, re.S)
     assert int(registers.group(1)) <= 128
