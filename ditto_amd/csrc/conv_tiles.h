@@ -100,15 +100,17 @@ __global__ void pack_conv_fragments_kernel(ConvFragments w1, ConvFragments w2, u
 // 1x1 -> 64 -> 3x3 64 10.6 / 9.8 / 9.2; 12 x 64 x 112 x 112 -> 128 -> 64 33.7 / 32.6 / 34.5, 20 x 64 x 56 x 56 -> 128 -> 64 17.1 / 16.8 / 18.7.
 // The last one to three groups of pixels, which fill no four, are neighbours among themselves: with lanes left idle for the missing
 // ones one pass over the threads became two (1 x 192 x 66 x 66 1x1 -> 64 -> 16 5.46 us, 4.76 here, 4.97 with channels on neighbouring
-// lanes; 3 x 192 x 22 x 22 stride 2 -> 64 -> 64 8.26 / 7.54 / 7.65).
+// lanes; 3 x 192 x 22 x 22 stride 2 -> 64 -> 64 8.26 / 7.54 / 7.65).  Not with eight waves, whose threads hardly ever miss the tasks by so
+// few: idle lanes cost them less than the index (100 random calls of 256 channels 1.007 with it, the worst 1.05).
 // cg: groups of 8 channels staged, a multiple of 4; zg: groups zeroed in the columns left and right.
 template <int NT, typename T>
 __device__ __forceinline__ void stage_halo_rows(T* Xs, const T* Xg, int h0, int pad, int rows_in, int cols_in, int CHS, int cg, int zg,
                                                 int C0, int H, int W, float inv_cg, float inv_ng, int tid) {
   typedef typename Elem<T>::v8 V8;
   typedef __attribute__((ext_vector_type(8), aligned(2))) T V8u;  // 16 bytes at any element's address
-  const int row_step = cols_in * CHS, ng = (W + 7) / 8, groups = rows_in * ng, tasks = groups * cg;
-  const int tail = groups & 3, body = tasks - tail * cg;
+  const int row_step = cols_in * CHS, ng = (W + 7) / 8, groups = rows_in * ng;
+  constexpr bool kTail = NT == 256;
+  const int tail = groups & 3, body = (groups - tail) * cg, tasks = body + (tail == 0 ? 0 : kTail ? tail : 4) * cg;
   const float inv_tail = tail == 1 ? 1.f : tail == 2 ? 1.f / 2 : 1.f / 3;
   const bool whole = W % 8 == 0;
   const int low = whole ? 4 : 2, per = whole ? cg >> 2 : cg;  // lane bits below `rest`, values of it
@@ -118,17 +120,19 @@ __device__ __forceinline__ void stage_halo_rows(T* Xs, const T* Xg, int h0, int 
     constexpr int U = decltype(both)::value;
     i32x4 xr[U][8];
     int col[U];
+    bool in[U];
     T* dst[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int t = t0 + u * NT, hi = t >> low, quad = div_by(hi, inv_per), rest = hi - quad * per;
       int chg = whole ? 4 * rest + ((t >> 1) & 3) : rest, grp = 4 * quad + (whole ? (t & 1) + ((t >> 2) & 2) : t & 3);
-      if (t >= body) chg = div_by(t - body, inv_tail), grp = groups - tail + (t - body) - chg * tail;
+      if (kTail && t >= body) chg = div_by(t - body, inv_tail), grp = groups - tail + (t - body) - chg * tail;
       const int ri = div_by(grp, inv_ng);
       const int w = min(8 * (grp - ri * ng), W - 8), h = h0 + ri;
       col[u] = w + pad;
       dst[u] = Xs + ri * row_step + (w + pad) * CHS + 8 * chg;
-      const bool live = t < tasks && h >= 0 && h < H;
+      in[u] = t < tasks && (kTail || grp < groups);
+      const bool live = in[u] && h >= 0 && h < H;
       const T* const src = Xg + (long long)(8 * chg) * hw + (long long)h * W + w;
 #pragma unroll
       for (int k = 0; k < 8; ++k) {
@@ -139,7 +143,7 @@ __device__ __forceinline__ void stage_halo_rows(T* Xs, const T* Xg, int h0, int 
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      if (t0 + u * NT >= tasks) break;
+      if (!in[u]) break;
 #pragma unroll
       for (int px = 0; px < 8; ++px) {
         i32x4 o;
