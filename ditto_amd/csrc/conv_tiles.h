@@ -111,7 +111,7 @@ __device__ __forceinline__ void stage_halo_rows(T* Xs, const T* Xg, int h0, int 
   const int row_step = cols_in * CHS, ng = (W + 7) / 8, groups = rows_in * ng;
   constexpr bool kTail = NT == 256;
   const int tail = groups & 3, body = (groups - tail) * cg, tasks = body + (tail == 0 ? 0 : kTail ? tail : 4) * cg;
-  const int by_tail = tail == 1 ? 1 << 16 : tail == 2 ? 1 << 15 : 21846;  // 2^16 / tail, rounded up
+  const float inv_tail = tail == 1 ? 1.f : tail == 2 ? 1.f / 2 : 1.f / 3;
   const bool whole = W % 8 == 0;
   const int low = whole ? 4 : 2, per = whole ? cg >> 2 : cg;  // lane bits below `rest`, values of it
   const float inv_per = whole ? 4.f * inv_cg : inv_cg;
@@ -126,7 +126,7 @@ __device__ __forceinline__ void stage_halo_rows(T* Xs, const T* Xg, int h0, int 
     for (int u = 0; u < U; ++u) {
       const int t = t0 + u * NT, hi = t >> low, quad = div_by(hi, inv_per), rest = hi - quad * per;
       int chg = whole ? 4 * rest + ((t >> 1) & 3) : rest, grp = 4 * quad + (whole ? (t & 1) + ((t >> 2) & 2) : t & 3);
-      if (kTail && t >= body) chg = __umul24(t - body, by_tail) >> 16, grp = groups - tail + (t - body) - chg * tail;
+      if (kTail && t >= body) chg = div_by(t - body, inv_tail), grp = groups - tail + (t - body) - chg * tail;
       const int ri = div_by(grp, inv_ng);
       const int w = min(8 * (grp - ri * ng), W - 8), h = h0 + ri;
       col[u] = w + pad;
