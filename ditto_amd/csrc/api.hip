@@ -109,6 +109,8 @@ struct BmmPrice {
 };
 // Least squares over 3300 random shapes (batch 1 - 160, 32 - 4096 rows and keys, fp16 and bf16), those of 2144 and of the 64-row
 // kernels with softmax over 3600 others, root mean square error 4 - 12 %; the columns: head sizes up to 64 | 128, without | with softmax, B [L][K] | [K][L].
+// (The 20xx, 2148 and 2188 as they were before their rows of A came through LDS, up to 0.2 of a short launch more; few_rows_variant has
+// prices of its own for the 20xx.)
 constexpr BmmPrice kPrices64[2][2][8] = {
     {{{641, 128, 256, 1, 0.71f, {3.38f}, {.0074f}}, {644, 64, 256, 3, 2.64f, {1.30f, 1.81f, 2.36f}, {.0049f, .0079f, .0121f}},
       {645, 64, 256, 2, 2.98f, {1.34f, 2.09f}, {.0042f, .0070f}}, {649, 256, 512, 1, 0, {5.03f}, {.0118f}},
@@ -392,7 +394,8 @@ int plan_bmm_rules(const ditto_bmm_chain_desc* d, BmmPlan* plan, int cus) {
       else if (sm && lk && n8 >= 2LL * cus) plan->qt = 6;
     }
     {
-      // Few rows: the kernel whose eight waves split the keys (bmm_chain_split.h), in workgroups of 16 or 32 rows.  Its cost
+      // Few rows: the kernel whose eight waves split the keys (bmm_chain_split.h), in workgroups of 16 or 32 rows.  (As it was before
+      // its rows of A came through LDS: few_rows_variant takes the chains that it has been ahead for since.)  Its cost
       // beyond the launch is a start and a merge plus a share of the keys, `a + b L` us, for every round of workgroups over
       // the compute units; the kernels above walk all keys in one go and their 64 or 128 rows per workgroup need fewer
       // rounds.  Fitted to measurements at head sizes 64, 80 and 128 (us per launch, other kernel -> this one, LK):
